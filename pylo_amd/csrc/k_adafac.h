@@ -541,6 +541,54 @@ __device__ __forceinline__ av16f hf2_mfma(const au32x4 (&w)[2], const au32x4 (&x
   return acc;
 }
 
+// Hidden and output layer of the two groups of 32 elements a wave holds, from the first layer's sums `h` (D layout):
+// the two outputs of the lane's own element.
+__device__ __forceinline__ void adafac_hidden_out(const av16f (&h)[2], const au32x4 (&w2)[2][2], const av16f& bh,
+                                                  const float (&wo)[16][2], float bo0, float bo1, float& o0, float& o1) {
+  av16f g2[2];
+#pragma unroll
+  for (int gq = 0; gq < 2; ++gq) {
+    // hidden values of the units this lane holds -> planes, four units (two dwords) per block j
+    unsigned hp[2][4][2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        hf2_split2(__builtin_amdgcn_fmed3f(h[gq][4 * j + 2 * i], 0.0f, 65000.0f),
+                   __builtin_amdgcn_fmed3f(h[gq][4 * j + 2 * i + 1], 0.0f, 65000.0f), hp[0][j][i], hp[1][j][i]);
+    // blocks 2 s and 2 s + 1 are the lane's eight slots of reduction step s as they stand
+    g2[gq] = bh;
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      au32x4 hb[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        hb[q] = au32x4{hp[q][2 * s2][0], hp[q][2 * s2][1], hp[q][2 * s2 + 1][0], hp[q][2 * s2 + 1][1]};
+      g2[gq] = hf2_mfma(w2[s2], hb, g2[gq]);
+    }
+  }
+  float part[2][2];
+#pragma unroll
+  for (int gq = 0; gq < 2; ++gq) {
+    float p0 = 0.0f, p1 = 0.0f;
+#pragma unroll
+    for (int r2 = 0; r2 < 16; ++r2) {
+      const float gv = relu(g2[gq][r2]);
+      p0 = fmaf(gv, wo[r2][0], p0);
+      p1 = fmaf(gv, wo[r2][1], p1);
+    }
+    part[gq][0] = p0;
+    part[gq][1] = p1;
+  }
+  // a lane's element belongs to group `half`; its other 16 units sit 32 lanes away
+  unsigned a0 = __float_as_uint(part[0][0]), b0 = __float_as_uint(part[1][0]);
+  unsigned a1 = __float_as_uint(part[0][1]), b1 = __float_as_uint(part[1][1]);
+  half_swap(a0, b0);
+  half_swap(a1, b1);
+  o0 = (__uint_as_float(a0) + __uint_as_float(b0)) + bo0;
+  o1 = (__uint_as_float(a1) + __uint_as_float(b1)) + bo1;
+}
+
 // PER: the tensor is an (O, I, k, ..) one walked as the matrix (O, I * P) (TDesc::aper): the vector that is not
 // indexed by the column has an entry per (row, column mod P), so a lane fetches the row's factor and first-layer
 // terms for its own columns (one per element group) instead of sharing one entry with the wave.
@@ -670,7 +718,7 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
     hf2_pack8(fhi, xb[1]);
     // The two groups of 32 elements go through the layers a phase apart, so that the matrix instructions of one
     // have the vector work of the other to run under: first layer of both, then per group split -> hidden layer,
-    // then the output layer (on the vector pipe) of both.
+    // then the output layer (on the vector pipe) of both (adafac_hidden_out).
     av16f h[2];
 #pragma unroll
     for (int gq = 0; gq < 2; ++gq) {
@@ -683,48 +731,8 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
       }
       h[gq] = hf2_mfma(w1, xb[gq], h[gq]);
     }
-    av16f g2[2];
-#pragma unroll
-    for (int gq = 0; gq < 2; ++gq) {
-      // hidden values of the units this lane holds -> planes, four units (two dwords) per block j
-      unsigned hp[2][4][2];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          hf2_split2(__builtin_amdgcn_fmed3f(h[gq][4 * j + 2 * i], 0.0f, 65000.0f),
-                     __builtin_amdgcn_fmed3f(h[gq][4 * j + 2 * i + 1], 0.0f, 65000.0f), hp[0][j][i], hp[1][j][i]);
-      // blocks 2 s and 2 s + 1 are the lane's eight slots of reduction step s as they stand
-      g2[gq] = bh;
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        au32x4 hb[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-          hb[q] = au32x4{hp[q][2 * s2][0], hp[q][2 * s2][1], hp[q][2 * s2 + 1][0], hp[q][2 * s2 + 1][1]};
-        g2[gq] = hf2_mfma(w2[s2], hb, g2[gq]);
-      }
-    }
-    float part[2][2];
-#pragma unroll
-    for (int gq = 0; gq < 2; ++gq) {
-      float p0 = 0.0f, p1 = 0.0f;
-#pragma unroll
-      for (int r2 = 0; r2 < 16; ++r2) {
-        const float gv = relu(g2[gq][r2]);
-        p0 = fmaf(gv, wo[r2][0], p0);
-        p1 = fmaf(gv, wo[r2][1], p1);
-      }
-      part[gq][0] = p0;
-      part[gq][1] = p1;
-    }
-    // a lane's element belongs to group `half`; its other 16 units sit 32 lanes away
-    unsigned a0 = __float_as_uint(part[0][0]), b0 = __float_as_uint(part[1][0]);
-    unsigned a1 = __float_as_uint(part[0][1]), b1 = __float_as_uint(part[1][1]);
-    half_swap(a0, b0);
-    half_swap(a1, b1);
-    const float o0 = (__uint_as_float(a0) + __uint_as_float(b0)) + bo0;
-    const float o1 = (__uint_as_float(a1) + __uint_as_float(b1)) + bo1;
+    float o0, o1;
+    adafac_hidden_out(h, w2, bh, wo, bo0, bo1, o0, o1);
     float pn[1];
     pn[0] = adafac_update(d, a, o0 * __builtin_amdgcn_exp2f(o1 * exp_scale), xp[0]);
     store_vec_o<1>(p, lo, pn);
@@ -732,6 +740,202 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
     fr += 4 * per; tr += kAH * per;
     cur = nxt;
   }
+}
+
+// ---- the same for every other tensor: 64 consecutive elements a wave and trip ------------------------------
+// Tensors that no column-resident walk takes -- rows that are not a multiple of 64 long, more than two dims with
+// other factored dims, fewer than two dims -- are taken in storage order, element `base + 256 trip + thread`, with
+// the element MLP on the matrix pipe exactly as above.  What differs is where the factors and first-layer terms
+// come from: every lane works out the two table entries of its two elements (e of either group of 32; its own is
+// one of them) and fetches them, 16 bytes a load, out of tables that stay in the L2.  A lane past the end works on
+// the tensor's last element and stores nothing.
+// K: kModeFac2D, kModeFacND, or kModeVec.  A tensor with fewer than two dims has 28 features of its own and no
+// terms: two reduction steps of 16 slots for the first layer (four slots empty) and the effective bias instead.
+// Bound by latency on the small tensors that come here and by vector instructions on large ones.  The all-VALU
+// kernel that it replaces on the matrix-pipe plans read the 1 600 weights of an element row by row through the
+// scalar cache, 32 dependent trips of it over 8 192 elements a block.  Whole steps: the 118 000-parameter classifier
+// (784 -> 128 -> 128 -> 10, ELO) 285 -> 88 us, its apply launch 207 us before; ResNet-50's set (AdafacLO: 161 tensors,
+// the vectors, the stem and the 1 x 1 kernels of 64 x 64 come here) 792 -> 729 us.
+template <int K>
+__device__ __forceinline__ void adafac_apply_lin_hf(const TDesc& d, const PyloTensorArgs& a, long long base, int trips,
+                                                    const EmaConsts& e, const PyloDecays& dec,
+                                                    const float* __restrict__ fac_tab,
+                                                    const float* __restrict__ term_tab, const float* wfold_t,
+                                                    const float* net, const float* bias_eff) {
+  constexpr bool VEC = K == kModeVec;
+  constexpr int S = VEC ? 2 : 1;       // reduction steps of the first layer
+  const int lane = threadIdx.x & 63, half = lane >> 5, el = lane & 31;
+  au32x4 w1[S][2], w2[2][2];
+  {
+    float x[8];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int c = 16 * s + 8 * half + i;
+        // a vector's feature c is channel c of the 30 without 1 and 14
+        const int row = VEC ? (c < 1 ? 0 : c < 13 ? c + 1 : c + 2) : adafac_elem_row(c);
+        x[i] = (VEC && c >= 28) ? 0.0f : *(const gfloat*)(net + kAW1 + row * kAH + el);
+      }
+      hf2_pack8(x, w1[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        x[i] = *(const gfloat*)(net + kAWH + (8 * (2 * s + (i >> 2)) + 4 * half + (i & 3)) * kAH + el);
+      hf2_pack8(x, w2[s]);
+    }
+  }
+  float fsc[VEC ? 30 : 16];   // the normalisers of the features, by channel (vectors) or by feature
+  {
+    const cfloat* sc = launder(wfold_t + 30 * kAH);
+#pragma unroll
+    for (int c = 0; c < (VEC ? 30 : 16); ++c) fsc[c] = sc[VEC ? c : adafac_elem_row(c)];
+  }
+  av16f bh, b1;
+  float wo[16][2];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int unit = 8 * (r >> 2) + 4 * half + (r & 3);
+    bh[r] = *(const gfloat*)(net + kABH + unit);
+    wo[r][0] = *(const gfloat*)(net + kAWO + unit * 2 + 0);
+    wo[r][1] = *(const gfloat*)(net + kAWO + unit * 2 + 1);
+    if constexpr (VEC) b1[r] = *(const gfloat*)(bias_eff + unit);
+  }
+  const cfloat* nw = launder(net);
+  const float bo0 = nw[kABO + 0], bo1 = nw[kABO + 1];
+  const float exp_scale = a.exp_mult * 1.44269504088896341f;
+  const long long n = d.n;
+  const unsigned last = (unsigned)(n - 1);     // n < 2^31
+  const unsigned wave0 = (unsigned)base + (threadIdx.x & ~63u);
+  // table entries of element u
+  auto entries = [&](unsigned u, unsigned& i0, unsigned& i1) {
+    if constexpr (K == kModeFac2D) {
+      i0 = fd_div(u, d.nd_div_blk[0]);
+      i1 = u - i0 * (unsigned)d.C0;
+    } else {
+      const unsigned s0 = (unsigned)d.nd_stride[0], s1 = (unsigned)d.nd_stride[1];
+      i0 = fd_div(u, d.nd_div_blk[0]) * s0 + (u - fd_div(u, d.nd_div_st[0]) * s0);
+      i1 = fd_div(u, d.nd_div_blk[1]) * s1 + (u - fd_div(u, d.nd_div_st[1]) * s1);
+    }
+  };
+  struct In { float g, p, m[3], rms, v[VEC ? 3 : 1]; };
+  auto fetch = [&](unsigned w0, In& x) {
+    const unsigned u = min(w0 + lane, last);
+    x.g = *(const gfloat*)(a.grad + u);
+    x.p = *(const gfloat*)(a.param + u);
+    x.rms = *(const gfloat*)(a.rms + u);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      x.m[k] = *(const gfloat*)(a.mom + k * n + u);
+      if constexpr (VEC) x.v[k] = *(const gfloat*)(a.fac_v + k * n + u);
+    }
+  };
+  In cur;
+  fetch(wave0, cur);
+  for (int it = 0; it < trips; ++it) {
+    const unsigned w0 = wave0 + (unsigned)it * kThreads;
+    if (w0 > last) break;                       // wave-uniform: every lane of a wave reaches the matrix instructions
+    In nxt;
+    fetch(w0 + (it + 1 < trips ? kThreads : 0), nxt);
+    const float g = cond_grad(cur.g, d.gscale, a.clip_val, d.nan0), p = cur.p;
+    float m[3] = {cur.m[0], cur.m[1], cur.m[2]}, rms = cur.rms, v[3] = {0.0f, 0.0f, 0.0f};
+    av16f h[2];
+    float f[16 * S];
+    if constexpr (VEC) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) v[k] = cur.v[k];
+      vec_update(e, dec, g, m, rms, v);
+      float f30[30];
+      vec_features(g, p, m, rms, v, 1e-6f, f30);
+      int q = 0;
+#pragma unroll
+      for (int c = 0; c < 30; ++c)
+        if (adafac_channel(c)) f[q++] = f30[c] * fsc[c];
+#pragma unroll
+      for (; q < 16 * S; ++q) f[q] = 0.0f;
+      h[0] = b1;
+      h[1] = b1;
+    } else {
+      unsigned i0[2], i1[2];
+#pragma unroll
+      for (int gq = 0; gq < 2; ++gq) entries(min(w0 + 32 * gq + el, last), i0[gq], i1[gq]);
+      float fa[4], fb[4];
+      load_vec_o<4>(fac_tab + d.fac_off[0], (half ? i0[1] : i0[0]) * 16u, fa);
+      load_vec_o<4>(fac_tab + d.fac_off[1], (half ? i1[1] : i1[0]) * 16u, fb);
+#pragma unroll
+      for (int gq = 0; gq < 2; ++gq) {
+        const float* t0 = term_tab + d.term_off[0] + (size_t)i0[gq] * kAH + 4 * half;
+        const float* t1 = term_tab + d.term_off[1] + (size_t)i1[gq] * kAH + 4 * half;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float4 ta = load_f4(t0 + 8 * j), tb = load_f4(t1 + 8 * j);
+          h[gq][4 * j + 0] = ta.x + tb.x;
+          h[gq][4 * j + 1] = ta.y + tb.y;
+          h[gq][4 * j + 2] = ta.z + tb.z;
+          h[gq][4 * j + 3] = ta.w + tb.w;
+        }
+      }
+      ema_update(e, g, m, rms);
+      const float rfcf[3] = {fa[0] * fb[0], fa[1] * fb[1], fa[2] * fb[2]};
+      float f18[kNStat];
+      lo_features(g, p, m, rms, rfcf, 1e-6f, f18);
+      const float fx[16] = {f18[0], f18[2], f18[3], f18[4], f18[5], f18[6], f18[7], f18[8], f18[9], f18[10],
+                            f18[11], f18[12], f18[13], f18[15], f18[16], f18[17]};
+#pragma unroll
+      for (int c = 0; c < 16; ++c) f[c] = fx[c] * fsc[c];
+    }
+    if (w0 + lane <= last) {
+      const unsigned u = w0 + lane;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        *(gfloat*)(a.mom + k * n + u) = m[k];
+        if constexpr (VEC) *(gfloat*)(a.fac_v + k * n + u) = v[k];
+      }
+      *(gfloat*)(a.rms + u) = rms;
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      float flo[8], fhi[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        unsigned x = __float_as_uint(f[16 * s + i]), y = __float_as_uint(f[16 * s + 8 + i]);
+        half_swap(x, y);
+        flo[i] = __uint_as_float(x);
+        fhi[i] = __uint_as_float(y);
+      }
+      au32x4 xb[2];
+      hf2_pack8(flo, xb);
+      h[0] = hf2_mfma(w1[s], xb, h[0]);
+      hf2_pack8(fhi, xb);
+      h[1] = hf2_mfma(w1[s], xb, h[1]);
+    }
+    float o0, o1;
+    adafac_hidden_out(h, w2, bh, wo, bo0, bo1, o0, o1);
+    if (w0 + lane <= last)
+      *(gfloat*)(a.param + w0 + lane) = adafac_update(d, a, o0 * __builtin_amdgcn_exp2f(o1 * exp_scale), p);
+    cur = nxt;
+  }
+}
+
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_adafac_apply_lin(
+    const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const Item* __restrict__ items,
+    const float* __restrict__ fac_tab, const float* __restrict__ term_tab, PyloDecays dec,
+    const float* __restrict__ wfold, const float* __restrict__ net, const float* __restrict__ bias_eff,
+    const Globals* __restrict__ gl) {
+  const Item it = items[blockIdx.x];
+  TDesc d = descs[it.tensor];
+  const PyloTensorArgs a = dyn[it.tensor];
+  if (a.grad == nullptr) return;
+  set_grad_scale(d, a, gl, it.tensor);
+  const EmaConsts e = make_ema(dec);
+  const float* w = wfold + (size_t)it.tensor * kAFold;
+  const float* be = bias_eff + (size_t)it.tensor * kAH;
+  const long long base = (long long)it.a * kThreads * it.b;
+  if (d.mode == kModeFac2D) adafac_apply_lin_hf<kModeFac2D>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
+  else if (d.mode == kModeFacND) adafac_apply_lin_hf<kModeFacND>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
+  else adafac_apply_lin_hf<kModeVec>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
 }
 
 __global__ __launch_bounds__(kThreads) void k_adafac_apply(const TDesc* __restrict__ descs,

@@ -141,6 +141,7 @@ struct Layout {
   std::vector<int> dc, dr;
   int H = 8;  // width of the first MLP layer (terms per row / column)
   int Tpad = 0;
+  bool lin_hf = false;       // AdafacLO: ga_items are k_adafac_apply_lin's (else k_adafac_apply's)
   bool global_norm = false;  // AdafacLO kind: every tensor has P0 items, the call may clip by global norm
   bool tensor_norm = false;  // ... or every tensor by its own norm (PYLO_F_TENSOR_NORM)
   size_t off_descs, off_dyn, off_p0_items, off_nd_items, off_sl_items, off_seg_items, off_segtot, off_el_items, off_ap_items, off_pp_items, off_ga_items, off_fin_items, off_finpart, off_finscale, off_tscale, off_v0a_items, off_v0b_items, off_fac_list,
@@ -780,6 +781,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
   L.dc.assign(T, -1);
   L.dr.assign(T, -1);
   long long part = 0, fac = 0, term = 0;
+  std::vector<int> lin_tensors;   // AdafacLO: tensors of the linear apply pass
   const int H = L.H;
   L.tensor_norm = (shapes[0].flags & PYLO_F_TENSOR_NORM) != 0;
   L.global_norm = (shapes[0].flags & PYLO_F_GLOBAL_NORM) != 0 || L.tensor_norm;
@@ -865,6 +867,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
         d.n_strips = (d.R0 + kP0Rows - 1) / kP0Rows;
         d.n_colblk = (d.C0 + 64 * d.vec - 1) / (64 * d.vec);
         d.npart[0] = d.n_colblk; d.npart[1] = d.n_strips;
+        d.nd_div_blk[0] = make_fastdiv((unsigned)std::max(d.C0, 1));   // element -> row (k_adafac_apply_lin)
       } else {
         d.vec = 1;
         d.vec0_is_r = 1;
@@ -973,9 +976,20 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
         d.atile_ntask = d.atile_nct * ((d.R0 + d.tile_rows - 1) / d.tile_rows);
         for (int b = 0; b * 4 < d.atile_ntask; ++b) (periodic ? L.pp_items : L.ap_items).push_back(Item{t, b, 0, 0});
       } else {
-        for (long long c = 0; c * chunk < n; ++c) L.ga_items.push_back(Item{t, (int)c, 0, 0});
+        lin_tensors.push_back(t);
       }
     }
+  }
+  // Blocks of AdafacLO's linear apply pass: on the matrix pipe Item::b trips of 256 elements each, as many as leave
+  // every SIMD the two waves it holds and no more than 16 (the set-up of a wave, its weights split into planes,
+  // costs about as much as a trip); else 8192- / 2048-element chunks.
+  L.lin_hf = env_matrix_pipe() && env_adafac_hf();
+  long long lin_elems = 0;
+  for (int t : lin_tensors) lin_elems += L.descs[t].n;
+  const int trips = (int)std::max<long long>(1, std::min<long long>(16, lin_elems / (2 * 256 * kThreads)));
+  for (int t : lin_tensors) {
+    const long long chunk = L.lin_hf ? (long long)kThreads * trips : (long long)kThreads * L.descs[t].vec * kElemIters;
+    for (long long c = 0; c * chunk < L.descs[t].n; ++c) L.ga_items.push_back(Item{t, (int)c, L.lin_hf ? trips : 0, 0});
   }
   if (kind == PYLO_KIND_CELO2 || kind == PYLO_KIND_VELO) build_elem_items(L, T, kind);
   long long ns_floats = 0;
@@ -2231,7 +2245,10 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   const Item* ga_items = P->at<Item>(L.off_ga_items);
   const Item* pp_items = P->at<Item>(L.off_pp_items);
   const int n_ap = (int)L.ap_items.size(), n_ga = (int)L.ga_items.size(), n_pp = (int)L.pp_items.size();
-  if (n_ga > 0)
+  if (n_ga > 0 && L.lin_hf)
+    hipLaunchKernelGGL(k_adafac_apply_lin, dim3(n_ga), dim3(kThreads), 0, s, descs, dyn, ga_items, fac_tab, term_tab, dec,
+                       wfold, net, (const float*)bias_eff, gl);
+  else if (n_ga > 0)
     hipLaunchKernelGGL(k_adafac_apply, dim3(n_ga), dim3(kThreads), 0, s, descs, dyn, ga_items, fac_tab, term_tab, dec,
                        wfold, net, (const float*)bias_eff, gl);
   if (n_pp > 0)
