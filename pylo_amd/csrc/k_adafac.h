@@ -42,9 +42,9 @@ __global__ __launch_bounds__(64) void k_adafac_bias(const float* __restrict__ ne
 template <int V, bool ND>
 __device__ __forceinline__ void adafac_stats_fac(const TDesc& d, const PyloTensorArgs& a, int chunk,
                                                  const EmaConsts& e, const float* __restrict__ fac_tab, VeloAcc& acc) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
 #pragma unroll 2
-  for (int it = 0; it < kElemIters; ++it) {
+  for (int it = 0; it < d.iters; ++it) {
     const long long idx = base + (long long)(it * kThreads + threadIdx.x) * V;
     if (idx >= d.n) break;
     ElemIn<V> x;
@@ -106,8 +106,8 @@ __device__ __forceinline__ void adafac_stats_tile(const TDesc& d, const PyloTens
 template <int V>
 __device__ __forceinline__ void adafac_stats_vec(const TDesc& d, const PyloTensorArgs& a, int chunk,
                                                  const EmaConsts& e, const PyloDecays& dec, VeloAcc& acc) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
-  for (int it = 0; it < kElemIters; ++it) {
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
+  for (int it = 0; it < d.iters; ++it) {
     const long long idx = base + (long long)(it * kThreads + threadIdx.x) * V;
     if (idx >= d.n) break;
     VecIn<V> x;

@@ -55,10 +55,10 @@ __device__ __forceinline__ void lo_features(float g, float p, const float (&m)[3
 template <int V>
 __device__ __forceinline__ void celo2_adam_chunk(const TDesc& d, const PyloTensorArgs& a, int chunk,
                                                  float scale, const EmaConsts& e) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
   const long long n = d.n;
 #pragma unroll 2
-  for (int it = 0; it < kElemIters; ++it) {
+  for (int it = 0; it < d.iters; ++it) {
     const long long idx = base + (long long)(it * kThreads + threadIdx.x) * V;
     if (idx >= n) break;
     float g[V], p[V], m0[V], m1[V], m2[V], r[V];
@@ -91,11 +91,11 @@ __device__ __forceinline__ void celo2_adam_chunk(const TDesc& d, const PyloTenso
 template <int V>
 __device__ __forceinline__ void celo2_adam_indep_chunk(const TDesc& d, const PyloTensorArgs& a, int chunk,
                                                        float scale, const PyloDecays& dec) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
   const long long n = d.n;
   const float b1 = dec.adam_beta1, ob1 = 1.0f - dec.adam_beta1, b2 = dec.adam_beta2, ob2 = 1.0f - dec.adam_beta2;
 #pragma unroll 2
-  for (int it = 0; it < kElemIters; ++it) {
+  for (int it = 0; it < d.iters; ++it) {
     const long long idx = base + (long long)(it * kThreads + threadIdx.x) * V;
     if (idx >= n) break;
     float g[V], p[V], m[V], v[V];
@@ -159,8 +159,7 @@ __device__ __forceinline__ void load_elems(const TDesc& d, const PyloTensorArgs&
 // V = elements per lane and access, VC = the tensor's vector width (which fixes the chunk size).
 template <int V, int VC = V>
 struct Cursor {
-  static constexpr int kChunkElems = kThreads * VC * kElemIters;
-  static constexpr int kIters = kElemIters * VC / V;
+  static constexpr int kTripsPerIter = VC / V;   // a chunk is TDesc::iters * kTripsPerIter trips
   unsigned off, i0, i1;  // lane's vector: element offset in the chunk, row, column
   unsigned lim;          // elements of the chunk that exist
   unsigned C0, sq, sr;   // row length; block stride = sq rows + sr columns
@@ -169,7 +168,8 @@ struct Cursor {
   __device__ __forceinline__ Cursor(const TDesc& d, long long base) {
     off = threadIdx.x * V;
     const long long left = d.n - base;
-    lim = left < (long long)kChunkElems ? (unsigned)left : (unsigned)kChunkElems;
+    const int chunk_elems = kThreads * VC * d.iters;
+    lim = left < (long long)chunk_elems ? (unsigned)left : (unsigned)chunk_elems;
     C0 = (unsigned)d.C0;
     const unsigned ub = (unsigned)base;  // n < 2^31
     c_i0 = ub / C0;
@@ -244,11 +244,11 @@ template <int V>
 __device__ __forceinline__ void celo2_stats_chunk(const TDesc& d, const PyloTensorArgs& a, int chunk,
                                                   float scale, const EmaConsts& e, const float* f0,
                                                   const float* f1, float (&acc)[kNStat]) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
   Cursor<V> cur(d, base);
   const ChunkPtrs cp(d, a, base);
 #pragma unroll 2
-  for (int it = 0; it < kElemIters; ++it, cur.advance()) {
+  for (int it = 0; it < d.iters; ++it, cur.advance()) {
     if (!cur.live()) break;
     ElemIn<V> x;
     load_elems_at<V>(d, a, cp, cur.off, cur.i0, cur.i1, scale, f0, f1, x);
@@ -475,11 +475,11 @@ __device__ __forceinline__ void celo2_apply_chunk(const TDesc& d, const PyloTens
                                                   float scale, const EmaConsts& e, const float* f0,
                                                   const float* f1, const float* t0, const float* t1,
                                                   const float* wbase) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
   const bool use_exp = a.exp_mult != 0.0f;
   Cursor<V> cur(d, base);
   const ChunkPtrs cp(d, a, base);
-  for (int it = 0; it < kElemIters; ++it, cur.advance()) {
+  for (int it = 0; it < d.iters; ++it, cur.advance()) {
     if (!cur.live()) break;
     ElemIn<V> x;
     load_elems_at<V>(d, a, cp, cur.off, cur.i0, cur.i1, scale, f0, f1, x);
@@ -574,7 +574,7 @@ __device__ __forceinline__ void celo2_apply_chunk_mfma(const TDesc& d, const Pyl
                                                        float scale, const EmaConsts& e, const float* f0,
                                                        const float* f1, const float* t0, const float* t1,
                                                        const float* wbase) {
-  const long long base = (long long)chunk * (kThreads * 4 * kElemIters);   // chunks are sized for vec == 4
+  const long long base = (long long)chunk * (kThreads * 4 * d.iters);   // chunks are sized for vec == 4
   const bool use_exp = a.exp_mult != 0.0f;
   const float exp_scale = a.exp_mult * 1.44269504088896341f;
   const int lane = threadIdx.x & 63;
@@ -585,7 +585,8 @@ __device__ __forceinline__ void celo2_apply_chunk_mfma(const TDesc& d, const Pyl
   const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
   Cursor<V, 4> cur(d, base);
   const ChunkPtrs cp(d, a, base);
-  for (int it = 0; it < Cursor<V, 4>::kIters; ++it, cur.advance()) {
+  const int trips = d.iters * Cursor<V, 4>::kTripsPerIter;
+  for (int it = 0; it < trips; ++it, cur.advance()) {
     // no early exit: every lane of the wave must reach the matrix instructions; lanes past the end
     // work on the chunk's first element and store nothing
     const bool live = cur.live();
@@ -866,7 +867,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PYLO_A
             for (int v = 0; v < kTileV; ++v) a.step_out[(size_t)r * d.C0 + tk.col + v] = nan;
         }
       } else {
-        const long long chunk = (long long)kThreads * d.vec * kElemIters, base = (long long)it.a * chunk;
+        const long long chunk = (long long)kThreads * d.vec * d.iters, base = (long long)it.a * chunk;
         for (long long i = base + threadIdx.x; i < base + chunk && i < d.n; i += kThreads) a.step_out[i] = nan;
       }
     }

@@ -97,9 +97,10 @@ __device__ __forceinline__ void p0_factored(const TDesc& d, const float* g, int 
 template <int V>
 __device__ __forceinline__ void p0_flat(const TDesc& d, const float* g, int chunk, float& gsq, float& amax) {
   const int nan0 = d.nan0;
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
 #pragma unroll
   for (int it = 0; it < kElemIters; ++it) {
+    if (it >= d.iters) break;
     const long long e = base + (long long)(it * kThreads + threadIdx.x) * V;
     if (e < d.n) {
       float x[V];

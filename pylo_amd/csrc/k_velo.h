@@ -176,9 +176,9 @@ __device__ __forceinline__ void lstm_sums(const float (&m)[3], float rms, VeloAc
 template <int V, bool ND>
 __device__ __forceinline__ void velo_stats_fac(const TDesc& d, const PyloTensorArgs& a, int chunk,
                                                const EmaConsts& e, const float* __restrict__ fac_tab, VeloAcc& acc) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
 #pragma unroll 2
-  for (int it = 0; it < kElemIters; ++it) {
+  for (int it = 0; it < d.iters; ++it) {
     const long long idx = base + (long long)(it * kThreads + threadIdx.x) * V;
     if (idx >= d.n) break;
     ElemIn<V> x;
@@ -312,8 +312,8 @@ __device__ __forceinline__ void vec_update(const EmaConsts& e, const PyloDecays&
 template <int V>
 __device__ __forceinline__ void velo_stats_vec(const TDesc& d, const PyloTensorArgs& a, int chunk,
                                                const EmaConsts& e, const PyloDecays& dec, VeloAcc& acc) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
-  for (int it = 0; it < kElemIters; ++it) {
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
+  for (int it = 0; it < d.iters; ++it) {
     const long long idx = base + (long long)(it * kThreads + threadIdx.x) * V;
     if (idx >= d.n) break;
     VecIn<V> x;
@@ -944,9 +944,9 @@ template <int V, bool ND>
 __device__ __forceinline__ void velo_apply_fac(const TDesc& d, const PyloTensorArgs& a, int chunk,
                                                const EmaConsts& e, const float* __restrict__ fac_tab,
                                                const float* __restrict__ term_tab, const float* wbase, NewSums& ns) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
   const long long n = d.n;
-  for (int it = 0; it < kElemIters; ++it) {
+  for (int it = 0; it < d.iters; ++it) {
     const long long idx = base + (long long)(it * kThreads + threadIdx.x) * V;
     if (idx >= n) break;
     ElemIn<V> x;
@@ -1092,9 +1092,9 @@ template <int V>
 __device__ __forceinline__ void velo_apply_vec(const TDesc& d, const PyloTensorArgs& a, int chunk,
                                                const EmaConsts& e, const PyloDecays& dec, const float* wbase,
                                                NewSums& ns) {
-  const long long base = (long long)chunk * (kThreads * V * kElemIters);
+  const long long base = (long long)chunk * (kThreads * V * d.iters);
   const long long n = d.n;
-  for (int it = 0; it < kElemIters; ++it) {
+  for (int it = 0; it < d.iters; ++it) {
     const long long idx = base + (long long)(it * kThreads + threadIdx.x) * V;
     if (idx >= n) break;
     VecIn<V> x;
@@ -1236,7 +1236,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             for (int v = 0; v < kTileV; ++v) a.param[(size_t)r * d.C0 + tk.col + v] = nan;
         }
       } else {
-        const long long chunk = (long long)kThreads * d.vec * kElemIters, base = (long long)it.a * chunk;
+        const long long chunk = (long long)kThreads * d.vec * d.iters, base = (long long)it.a * chunk;
         for (long long i = base + threadIdx.x; i < base + chunk && i < d.n; i += kThreads) a.param[i] = nan;
       }
     }

@@ -14,10 +14,10 @@ namespace pylo {
 constexpr int kThreads = 256;   // 4 waves of 64 lanes
 constexpr int kWaves = 4;
 constexpr int kP0Rows = 128;    // rows of one row/column-sum tile; tile columns = 64 * vec
-constexpr int kElemIters = 8;   // an element chunk is kThreads * vec * kElemIters elements
+constexpr int kElemIters = 8;   // an element chunk is kThreads * vec * TDesc::iters elements, iters <= kElemIters
 constexpr int kTileV = 2;       // column-resident walk: a wave owns 64 * kTileV columns ...
 constexpr int kTileCols = 64 * kTileV;
-constexpr int kTileRows = 16;   // ... and walks this many rows of them (TDesc::tile_rows; ELO-CELO2 plans may choose fewer)
+constexpr int kTileRows = 16;   // ... and walks TDesc::tile_rows of them, at most this many
 constexpr int kNStat = 18;      // feature channels that vary per element (the other 12 are
                                 // functions of the row or of the column only)
 constexpr int kV0aEnt = 64;     // vector entries per k_v0a block
@@ -73,6 +73,7 @@ struct TDesc {
   long long n;
   int mode;
   int vec;          // 4: 128-bit accesses (2-D with C0 % 4 == 0, flat/vec with n % 4 == 0); 1: dword
+  int iters;        // trips of an element chunk: kThreads * vec * iters elements (split_for)
   int R0, C0;       // 2-D: sizes of dim 0 / dim 1
   int vec0_is_r;    // vector 0 carries fac_r / row_factor (else fac_c / col_factor)
   int len[2];       // entries of vector 0 / 1

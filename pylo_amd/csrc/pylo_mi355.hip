@@ -188,10 +188,22 @@ long long env_keep_elems() {   // largest tensor whose inputs are still expected
   return (v && v[0]) ? std::atoll(v) : 8000000;
 }
 
-int tile_rows_for(int kind) {
+// How finely the element passes of a plan are cut: a block's 8192 elements (four wave tasks of 16 rows, or a chunk of
+// eight trips) are divided by this.  A block of a small plan is a serial chain of memory round trips while most
+// CUs have no block at all, so blocks are halved until there is one for each of the 256 CUs or a wave task is down to one
+// row.  Measured on a 118 000-parameter classifier, 1 against 16: k_celo2_elem 49 -> 21 us, k_velo_elem 48 -> 26 us,
+// AdafacLO's statistics and apply launches 49 -> 24 us together.  From 2.1 M elements on nothing is divided: with
+// 512 or 1024 blocks asked for, VeLO on 2.8 M elements went from 137 to 140 and 149 us, AdafacLO from 172 to 173
+// and 178 us (every block derives pivots and weights for itself and leaves a row of partial sums to add up).
+int split_for(long long elems) {
+  int f = 1;
+  while (f < kTileRows && elems * f < 256ll * 8192) f *= 2;
+  return f;
+}
+int tile_rows_for(int kind, int split) {
   const char* v = std::getenv("PYLO_MI355_TILE_ROWS");
   if (kind == PYLO_KIND_CELO2 && v && v[0] && std::atoi(v) > 0) return std::atoi(v);
-  return kTileRows;
+  return kTileRows / split;
 }
 
 // Items of k_celo2_elem.  Slabs are runs of whole tensors, last tensors first (their gradients are what
@@ -783,6 +795,13 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
   long long part = 0, fac = 0, term = 0;
   std::vector<int> lin_tensors;   // AdafacLO: tensors of the linear apply pass
   const int H = L.H;
+  long long total_elems = 0;
+  for (int t = 0; t < T; ++t) {
+    long long n = 1;
+    for (int i = 0; i < std::max(0, std::min(shapes[t].ndim, PYLO_MAX_DIMS)); ++i) n *= std::min<long long>(std::max<long long>(shapes[t].shape[i], 0), 1ll << 31) , n = std::min(n, 1ll << 31);
+    total_elems += n;
+  }
+  const int split = split_for(total_elems);
   L.tensor_norm = (shapes[0].flags & PYLO_F_TENSOR_NORM) != 0;
   L.global_norm = (shapes[0].flags & PYLO_F_GLOBAL_NORM) != 0 || L.tensor_norm;
   for (int t = 0; t < T; ++t) {
@@ -798,6 +817,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
     if (n >= (1ll << 31)) return fail("plan: tensors of 2^31 or more elements are not supported");
     TDesc& d = L.descs[t];
     d.n = n;
+    d.iters = std::max(1, kElemIters / split);
     d.gscale = 1.0f;
     if ((s.flags & (PYLO_F_NAN_TO_NUM | PYLO_F_WD_PRESTEP | PYLO_F_GLOBAL_NORM | PYLO_F_TENSOR_NORM)) &&
         kind != PYLO_KIND_ADAFAC)
@@ -910,7 +930,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
         }
       }
     }
-    const long long chunk = (long long)kThreads * d.vec * kElemIters;
+    const long long chunk = (long long)kThreads * d.vec * d.iters;
     // P0 items: tiles of 2-D factored tensors; flat chunks only where a global norm is needed
     // (CELO2's AdamW tensors, every other tensor of a PYLO_F_GLOBAL_NORM plan)
     d.p0_first = (int)L.p0_items.size();
@@ -940,7 +960,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       for (long long s0 = 0; s0 < n_slices && n > 0; s0 += per) L.sl_items.push_back(Item{t, (int)s0, 0, 0});
     } else if (wide && d.C0 % kTileCols == 0) {
       d.tile_nct = d.C0 / kTileCols;
-      d.tile_rows = tile_rows_for(kind);
+      d.tile_rows = tile_rows_for(kind, split);
       d.tile_ntask = d.tile_nct * ((d.R0 + d.tile_rows - 1) / d.tile_rows);
       for (int b = 0; b * 4 < d.tile_ntask; ++b) L.el_items.push_back(Item{t, b, 0, 0});
     } else {
@@ -972,7 +992,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       }
       if ((wide && d.C0 % 64 == 0) || periodic) {
         d.atile_nct = d.C0 / 64;
-        if (d.tile_rows == 0) d.tile_rows = tile_rows_for(kind);
+        if (d.tile_rows == 0) d.tile_rows = tile_rows_for(kind, split);
         d.atile_ntask = d.atile_nct * ((d.R0 + d.tile_rows - 1) / d.tile_rows);
         for (int b = 0; b * 4 < d.atile_ntask; ++b) (periodic ? L.pp_items : L.ap_items).push_back(Item{t, b, 0, 0});
       } else {
