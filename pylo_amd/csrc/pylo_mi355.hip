@@ -31,6 +31,7 @@
 #include "k_celo2_slices.h"
 #include "k_ns.h"
 #include "k_ns_hf.h"
+#include "k_ns_small.h"
 #include "k_slice_finish.h"
 #include "k_cast.h"
 #include "pylo_common.h"
@@ -86,6 +87,7 @@ struct NsGroup {
 // One batch of matrices: those whose operand planes share the plane workspace at one time.
 struct NsBatch { int mat0, n_mats, group0, n_groups; long long plane_elems; };
 
+constexpr int kNsSmallClasses = 3;
 struct Layout {
   std::vector<Item> mx_items;   // ELO-CELO2: statistics and apply items in slab order (k_celo2_elem)
   size_t off_mx_items = 0, off_sync = 0;
@@ -114,6 +116,15 @@ struct Layout {
   int slice_lds_l[kSliceLaneSets] = {}, slice_lds_w = 0, slice_lds_b = 0;
   size_t off_slice_mats = 0, off_slice_items_l[kSliceLaneSets] = {}, off_slice_items_w = 0, off_slice_items_b = 0;
   int ns_max_m = 0;
+  // Newton-Schulz: matrices that one launch takes from the raw step to the parameter (k_ns_small.h), by class (m up to
+  // 32, 64, 128)
+  std::vector<NsSmall> sm_mats;
+  std::vector<NsSmallItem> sm_items[kNsSmallClasses];
+  std::vector<char> small_of_tensor;  // per tensor: its matrices are in sm_mats
+  long long sm_part_floats = 0;
+  int sm_sums = 0, sm_sync = 0, sm_ticket0 = 0;
+  bool sm_meets[kNsSmallClasses] = {};   // the class has matrices of several blocks
+  size_t off_sm_mats = 0, off_sm_items[kNsSmallClasses] = {}, off_sm_part = 0, off_sm_sums = 0, off_sm_sync = 0;
   std::vector<Item> ns_flag_items;    // split-fp16 kernels: {matrix, chunk of its A} of k_ns_hf_chain_sumsq, group after group
   int ns_fpart_total = 0;
   size_t off_ns_flags = 0, off_ns_fpart = 0, off_ns_flag_items = 0;
@@ -421,6 +432,84 @@ void xcd_interleave(std::vector<NsItem>& items, const std::vector<std::pair<int,
   items.swap(out);
 }
 
+// PYLO_MI355_NS_SMALL=0: small matrices go through the tiled products like all others; read at plan creation.
+bool env_ns_small() {
+  const char* e = getenv("PYLO_MI355_NS_SMALL");
+  return !(e && e[0] == '0');
+}
+
+using SmSmall = SmDims<1, 1, 2>;
+using SmMid = SmDims<2, 1, 2>;
+using SmLarge = SmDims<4, 2, 1>;
+int ns_small_class(int m) { return m <= SmSmall::MP ? 0 : m <= SmMid::MP ? 1 : 2; }
+int ns_small_chunk(int cls) { return cls == 0 ? SmSmall::NB : cls == 1 ? SmMid::NB : SmLarge::NB; }
+int ns_small_edge(int cls) { return cls == 0 ? SmSmall::MP : cls == 1 ? SmMid::MP : SmLarge::MP; }
+
+// Which matrices the one-launch kernel takes: a smaller dim of at most 128 (its m x m matrices fit a CU's LDS) and a
+// longer one up to where its few blocks, each walking chunks of the long dim one after another, fall behind tiles on all CUs.
+// Whole steps of a classifier with one n x m matrix in front, small kernel against tiled products:
+//   m = 128: n = 4096 290 / 348 us, 8192 436 / 477, 16384 732 / 487        m = 64: 16384 226 / 419, 32768 341 / 466
+//   m = 32: 16384 206 / 340, 32768 297 / 365, 65536 475 / 410              m = 1: 32768 158 / 306
+// (three thousand odd matrices, the limit of m <= 16 at 1024, 16384, 65536: 3954, 3081, 2792 us)
+bool ns_small_takes(int R, int C) {
+  const int m = std::min(R, C), n = std::max(R, C);
+  if (m > SmLarge::MP) return false;
+  return n <= (m <= 16 ? 65536 : m <= SmMid::MP ? 32768 : 8192);
+}
+
+// Slabs (blocks) of each small matrix and the items of the launches.
+void build_small_items(Layout& L) {
+  // what a launch of the class holds at a time on 256 CUs (LDS), and an eighth of it: see k_ns_small.h
+  constexpr int kHolds[kNsSmallClasses] = {2048, 512, 256}, kSlabsMax[kNsSmallClasses] = {64, 32, 8};
+  auto cls_of = [](const NsSmall& b) { return ns_small_class(b.m); };
+  int lift[kNsSmallClasses] = {0, 1, 2};
+  // A plan with few small matrices takes them all in the class of the largest, one launch: the small ones end under it.
+  if ((int)L.sm_mats.size() <= 64) {
+    int top = 0;
+    for (const NsSmall& b : L.sm_mats) top = std::max(top, cls_of(b));
+    for (int& c : lift) c = top;
+  }
+  for (int cls = 0; cls < kNsSmallClasses; ++cls) {
+    std::vector<int> of;
+    const int nb = ns_small_chunk(cls);
+    auto chunks = [&](int q) { return (L.sm_mats[q].n + nb - 1) / nb; };
+    long long total = 0;
+    for (int q = 0; q < (int)L.sm_mats.size(); ++q)
+      if (lift[cls_of(L.sm_mats[q])] == cls) {
+        of.push_back(q);
+        total += chunks(q);
+      }
+    // one slab a chunk while the launch's blocks all run at once, longer ones when there are more
+    const int per = (int)std::max<long long>(1, total / kHolds[cls]);
+    for (int q : of) {
+      NsSmall& b = L.sm_mats[q];
+      const int c = chunks(q);
+      b.chunks = std::max(per, (c + kSlabsMax[cls] - 1) / kSlabsMax[cls]);
+      b.slabs = (c + b.chunks - 1) / b.chunks;
+      if (b.slabs == 1) { b.chunks = c; continue; }
+      b.chunks = (c + b.slabs - 1) / b.slabs;      // even slabs
+      b.slabs = (c + b.chunks - 1) / b.chunks;
+      b.part = L.sm_part_floats;
+      L.sm_part_floats += 2ll * b.slabs * ns_small_edge(cls) * ns_small_edge(cls);
+      b.sums = L.sm_sums;
+      L.sm_sums += 2 * b.slabs;
+      b.sync = L.sm_sync;
+      L.sm_sync += 2;
+      L.sm_meets[cls] = true;
+    }
+    // the blocks that meet first (they start together), then the longest
+    std::stable_sort(of.begin(), of.end(), [&](int x, int y) {
+      const NsSmall &a = L.sm_mats[x], &b = L.sm_mats[y];
+      if ((a.slabs > 1) != (b.slabs > 1)) return a.slabs > 1;
+      return a.chunks > b.chunks;
+    });
+    for (int q : of)
+      for (int sl = 0; sl < L.sm_mats[q].slabs; ++sl) L.sm_items[cls].push_back(NsSmallItem{q, sl});
+  }
+  L.sm_ticket0 = L.sm_sync;
+  L.sm_sync += kNsSmallClasses;
+}
+
 // Newton-Schulz tables: every 2-D MLP tensor (the fp32 kernels: those whose rows (C) and whose smaller dim are
 // multiples of 4).  `ws_floats` returns the floats of workspace behind off_ns_ws.
 void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long& ws_floats) {
@@ -428,6 +517,8 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
   L.ns_xalt.assign(T, -1);
   L.ns_of_tensor.assign(T, -1);
   L.ns_group_of_tensor.assign(T, -1);
+  L.small_of_tensor.assign(T, 0);
+  const bool small = L.ns_hf && env_ns_small();
   auto take = [&](long long n) { const long long o = ws_floats; ws_floats += (n + 63) / 64 * 64; return o; };
   for (int t = 0; t < T; ++t) {
     const TDesc& d = L.descs[t];
@@ -441,6 +532,19 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
     // the fp32 kernels load 16 bytes at a time along the contiguous dim of X, A and B'
     if (!L.ns_hf && (C % 4 != 0 || std::min(R, C) % 4 != 0)) continue;
     const int n_sl = slices ? (int)(d.n / ((long long)R * C)) : 1;
+    if (small && ns_small_takes(R, C)) {
+      L.small_of_tensor[t] = 1;
+      for (int sl = 0; sl < n_sl; ++sl) {
+        NsSmall b{};
+        b.tensor = t;
+        b.m = std::min(R, C);
+        b.n = std::max(R, C);
+        b.tall = R > C;
+        b.elem_off = (long long)sl * R * C;
+        L.sm_mats.push_back(b);
+      }
+      continue;
+    }
     for (int sl = 0; sl < n_sl; ++sl) {
     NsMat mt{};
     mt.tensor = t;
@@ -480,6 +584,7 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
     L.ns_mats.push_back(mt);
     }
   }
+  build_small_items(L);
   if (L.ns_hf) {
     // A plan with few matrices (a convolutional net's one classifier, a small MLP) has fewer Gram tile jobs than the
     // part has CUs, each a long reduction: split them along it, up to eight ways, until there are two jobs a CU.
@@ -581,7 +686,8 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
     L.ns_flag_items.clear();
     L.ns_fpart_total = 0;
     for (NsBatch& bt : L.ns_batches) {
-    const int n_groups = std::min<int>(env_ns_groups(), std::max(bt.n_mats / 8, 1));
+    // (one of the four hardware queues is left to the small matrices where there are any)
+    const int n_groups = std::min<int>(L.sm_mats.empty() ? env_ns_groups() : std::min(env_ns_groups(), 3), std::max(bt.n_mats / 8, 1));
     std::vector<std::vector<int>> members(n_groups);
     {
       // (tensor by tensor: the slices of a tensor with more than two dims share a group, which also finishes it)
@@ -742,7 +848,7 @@ int build_fin_tables(Layout& L, const PyloTensorShape* shapes, int T) {
     TDesc& d = L.descs[t];
     d.fin_unit0 = (int)L.fin_units.size();
     d.fin_units = 0;
-    if (d.mode == kModeFlat || d.n == 0) return;
+    if (d.mode == kModeFlat || d.n == 0 || L.small_of_tensor[t]) return;
     long long slices = 1, len = d.n;
     if (d.mode == kModeFacND) {
       if (L.slice_of_tensor[t] >= 0) return;
@@ -1099,6 +1205,11 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
     L.off_nsb_split_items = take(sizeof(NsTileItem) * L.nsb_split_items.size());
     L.off_ns_list = take(sizeof(int) * L.ns_list.size());
     L.off_ns_pw = take(sizeof(hbits) * (size_t)L.nsb_plane_elems);
+    L.off_sm_mats = take(sizeof(NsSmall) * L.sm_mats.size());
+    for (int k = 0; k < kNsSmallClasses; ++k) L.off_sm_items[k] = take(sizeof(NsSmallItem) * L.sm_items[k].size());
+    L.off_sm_part = take(sizeof(float) * (size_t)L.sm_part_floats);
+    L.off_sm_sums = take(sizeof(double) * (size_t)L.sm_sums);
+    L.off_sm_sync = take(sizeof(int) * (size_t)L.sm_sync);
     L.off_slice_mats = take(sizeof(SliceMat) * L.slice_mats.size());
     for (int k = 0; k < kSliceLaneSets; ++k) L.off_slice_items_l[k] = take(sizeof(Item) * L.slice_items_l[k].size());
     L.off_slice_items_w = take(sizeof(Item) * L.slice_items_w.size());
@@ -1221,6 +1332,11 @@ int pylo_mi355_plan_create(int kind, const PyloTensorShape* shapes, int n_tensor
     if (e == hipSuccess) e = up(L.off_slice_items_l[k], L.slice_items_l[k].data(), sizeof(Item) * L.slice_items_l[k].size());
   if (e == hipSuccess) e = up(L.off_slice_items_w, L.slice_items_w.data(), sizeof(Item) * L.slice_items_w.size());
   if (e == hipSuccess) e = up(L.off_slice_items_b, L.slice_items_b.data(), sizeof(Item) * L.slice_items_b.size());
+  if (e == hipSuccess) e = up(L.off_sm_mats, L.sm_mats.data(), sizeof(NsSmall) * L.sm_mats.size());
+  for (int k = 0; k < kNsSmallClasses; ++k)
+    if (e == hipSuccess) e = up(L.off_sm_items[k], L.sm_items[k].data(), sizeof(NsSmallItem) * L.sm_items[k].size());
+  // the meeting counters start at zero; every launch leaves them there
+  if (e == hipSuccess && L.sm_sync > 0) e = hipMemsetAsync(P->ws + L.off_sm_sync, 0, sizeof(int) * (size_t)L.sm_sync, s);
   // the padding of the operand planes is read by the products and written by nobody: zero, once
   if (e == hipSuccess && L.nsb_plane_elems > 0)
     e = hipMemsetAsync(P->ws + L.off_ns_pw, 0, sizeof(hbits) * (size_t)L.nsb_plane_elems, s);
@@ -1255,6 +1371,7 @@ int pylo_mi355_plan_create(int kind, const PyloTensorShape* shapes, int n_tensor
   }
   bool plan_has_slices = !L.slice_items_w.empty() || !L.slice_items_b.empty();
   for (const auto& v : L.slice_items_l) plan_has_slices = plan_has_slices || !v.empty();
+  plan_has_slices = plan_has_slices || !L.sm_mats.empty();   // the small matrices' launches ride on the same stream
   if (e == hipSuccess && plan_has_slices && ns_streams >= 1 && ns_streams <= 3) {   // main + groups + this one <= 4 queues
     e = hipStreamCreateWithFlags(&P->slice_side, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&P->slice_fork, hipEventDisableTiming);
@@ -1696,6 +1813,56 @@ __global__ __launch_bounds__(256) void k_ns_zero(u32x4* __restrict__ p, size_t n
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) p[i] = u32x4{0u, 0u, 0u, 0u};
 }
 
+int small_lds_once() {
+  static std::mutex mu;
+  static std::vector<int> done;
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(mu);
+  for (int d : done)
+    if (d == dev) return 0;
+  HIP_TRY(hipFuncSetAttribute((const void*)(k_ns_small<4, 2, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, SmLarge::kLds));
+  HIP_TRY(hipFuncSetAttribute((const void*)(k_ns_small<2, 1, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, SmMid::kLds));
+  HIP_TRY(hipFuncSetAttribute((const void*)(k_ns_small<1, 1, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, SmSmall::kLds));
+  done.push_back(dev);
+  return 0;
+}
+
+// The launches of the small matrices (k_ns_small.h): one per class, largest first.
+int enqueue_small(PyloPlan* P, hipStream_t s, const TDesc* descs, const PyloTensorArgs* dyn, const float* coeffs, int ns_iters,
+                  float ns_eps) {
+  const Layout& L = P->L;
+  if (int rc = small_lds_once()) return rc;
+  const int orth = coeffs != nullptr && ns_iters > 0;
+  NsSmallStep st{};
+  if (orth) {
+    const NsExps ex = ns_plane_exps(coeffs[0], coeffs[1], coeffs[2], ns_iters);
+    const int q2 = ex.q[std::min<size_t>(2, ex.q.size() - 1)];
+    st.x_s = pow2(ex.x); st.a_s = pow2(ex.a); st.b_s = pow2(ex.b); st.t_s = pow2(ex.t); st.q_s = pow2(q2);
+    st.gram = pow2(-2 * ex.x); st.poly = pow2(-2 * ex.a);
+    st.prod_t = pow2(-(ex.a + ex.b)); st.prod_a = pow2(-(ex.b + ex.t)); st.prod_q = pow2(-2 * ex.b);
+    st.upd_b = pow2(-(ex.x + ex.b)); st.upd_q = pow2(-(ex.x + q2));
+    st.c0 = coeffs[0]; st.c1 = coeffs[1]; st.c2 = coeffs[2]; st.eps = ns_eps;
+    // pairs, also where the environment asks for longer chains or a choice per matrix (which trade accuracy for
+    // the products over the long dim that small matrices do not have); single iterations where it asks for those
+    st.n_pairs = ns_iters / 2;
+    const std::vector<int> chains = ns_chains(ns_iters);
+    if (*std::max_element(chains.begin(), chains.end()) == 1) st.n_pairs = 0;
+    st.n_chains = ns_iters - st.n_pairs;
+  }
+  auto launch = [&](auto kern, int cls, int threads, int lds) {
+    if (!L.sm_items[cls].empty())
+      hipLaunchKernelGGL(kern, dim3((unsigned)L.sm_items[cls].size()), dim3(threads), lds, s, P->at<NsSmall>(L.off_sm_mats),
+                         P->at<NsSmallItem>(L.off_sm_items[cls]), descs, dyn, P->at<float>(L.off_sm_part),
+                         P->at<double>(L.off_sm_sums), P->at<int>(L.off_sm_sync), st, orth,
+                         L.sm_meets[cls] ? P->at<int>(L.off_sm_sync) + L.sm_ticket0 + cls : (int*)nullptr);
+  };
+  launch(k_ns_small<4, 2, 1>, 2, SmLarge::kThr, SmLarge::kLds);
+  launch(k_ns_small<2, 1, 2>, 1, SmMid::kThr, SmMid::kLds);
+  launch(k_ns_small<1, 1, 2>, 0, SmSmall::kThr, SmSmall::kLds);
+  return 0;
+}
+
 // Newton-Schulz (ns_iters > 0, on the tensors flagged PYLO_ARG_ORTHOGONALIZE) and the finishing pass.
 int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, int ns_iters, float ns_eps, void* stream,
                 const char* who) {
@@ -1703,7 +1870,7 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
   if (!P || P->kind != PYLO_KIND_CELO2) return fail(w + ": not an ELO-CELO2 plan");
   if (!args) return fail(w + ": null argument");
   const Layout& L = P->L;
-  bool any_ns = false, any_slices = false;
+  bool any_ns = false, any_slices = false, any_small = false;
   for (int t = 0; t < P->T; ++t) {
     const TDesc& d = L.descs[t];
     const PyloTensorArgs& a = args[t];
@@ -1719,12 +1886,17 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
       any_slices = true;
       continue;
     }
+    const bool small = L.small_of_tensor[t] != 0;
     const bool vec = d.fin_units > 0 && L.fin_units[d.fin_unit0].vec;
-    if (m % (vec ? 16 : 4) != 0) return fail(w + ": misaligned pointer" + at);
+    if (!small && m % (vec ? 16 : 4) != 0) return fail(w + ": misaligned pointer" + at);
+    if (small && (reinterpret_cast<uintptr_t>(a.step_out) % 4 != 0 || reinterpret_cast<uintptr_t>(a.param) % (d.store != 0 ? 2 : 4) != 0))
+      return fail(w + ": misaligned pointer" + at);
+    any_small = any_small || small;
     if (coeffs && ns_iters == 0 && (a.flags & PYLO_ARG_ORTHOGONALIZE))
       return fail(w + ": PYLO_ARG_ORTHOGONALIZE with ns_iters = 0 on a tensor that the tiled products orthogonalise "
                   "(the division by the norm alone is the caller's)" + at);
     if (ns_iters > 0 && (a.flags & PYLO_ARG_ORTHOGONALIZE)) {
+      if (small) continue;
       if (L.ns_of_tensor[t] < 0) return fail(w + ": PYLO_ARG_ORTHOGONALIZE on a tensor the library cannot orthogonalise" + at);
       any_ns = true;
     }
@@ -1741,15 +1913,17 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
   const int n_fin = (int)L.fin_items.size();
   // The per-slice launches touch only their own tensors: next to the matrices' chains of products they run on a stream
   // of their own (forked from and joined into the caller's like the groups').
-  const bool slices_aside = any_slices && any_ns && L.ns_hf && P->slice_side != nullptr;
+  const bool slices_aside = (any_slices || any_small) && any_ns && L.ns_hf && P->slice_side != nullptr;
+  if (slices_aside) {
+    HIP_TRY(hipEventRecord(P->slice_fork, s));
+    HIP_TRY(hipStreamWaitEvent(P->slice_side, P->slice_fork, 0));
+  }
+  if (any_small)
+    if (int rc = enqueue_small(P, slices_aside ? P->slice_side : s, descs, dyn, coeffs, ns_iters, ns_eps)) return rc;
   if (any_slices) {
     // tensors with more than two dims: everything per slice, in LDS (k_slice_finish.h)
     if (int rc = slice_lds_once()) return rc;
     hipStream_t caller = s;
-    if (slices_aside) {
-      HIP_TRY(hipEventRecord(P->slice_fork, caller));
-      HIP_TRY(hipStreamWaitEvent(P->slice_side, P->slice_fork, 0));
-    }
     hipStream_t s = slices_aside ? P->slice_side : caller;
     const SliceMat* smats = P->at<SliceMat>(L.off_slice_mats);
     const float c0 = coeffs ? coeffs[0] : 0.0f, c1 = coeffs ? coeffs[1] : 0.0f, c2 = coeffs ? coeffs[2] : 0.0f;
@@ -1770,8 +1944,8 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
     if (!L.slice_items_b.empty())
       hipLaunchKernelGGL(k_celo2_slice_finish<true>, dim3((unsigned)L.slice_items_b.size()), dim3(256), L.slice_lds_b, s,
                          smats, P->at<Item>(L.off_slice_items_b), descs, dyn, orth_call, ns_iters, ns_eps, c0, c1, c2);
-    if (slices_aside) HIP_TRY(hipEventRecord(P->slice_join, P->slice_side));
   }
+  if (slices_aside) HIP_TRY(hipEventRecord(P->slice_join, P->slice_side));
   if (n_fin == 0) {
     HIP_TRY(hipGetLastError());
     return 0;
@@ -2013,7 +2187,7 @@ extern "C" int pylo_mi355_plan_finish_supported(const PyloPlan* P, int tensor) {
 extern "C" int pylo_mi355_plan_orthogonalize_supported(const PyloPlan* P, int tensor) {
   if (!P || tensor < 0 || tensor >= P->T || P->kind != PYLO_KIND_CELO2) return 0;
   if (P->L.slice_of_tensor[tensor] >= 0) return P->L.slice_mats[P->L.slice_of_tensor[tensor]].no_orth ? 0 : 2;
-  return P->L.ns_of_tensor[tensor] >= 0 ? 1 : 0;
+  return P->L.ns_of_tensor[tensor] >= 0 || P->L.small_of_tensor[tensor] ? 1 : 0;
 }
 
 extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, const PyloDecays* decays,

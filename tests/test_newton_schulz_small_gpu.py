@@ -1,0 +1,77 @@
+"""Small matrices (smaller dim at most 128) that one launch takes from the raw step to the parameter: every class of
+sizes at its edges, matrices of one block and of several that meet, against the literal formula in fp64.
+
+The bound is that of the tiled products' tests: no further from fp64 than 1.5 times what the formula in fp32 torch
+products is, plus 5e-5 of the result's unit RMS (the operands' two fp16 planes and the pairing of iterations)."""
+
+import numpy as np
+import pytest
+import torch
+
+from test_newton_schulz_gpu import _orthogonalise_direct, _reference_direct
+
+pytestmark = pytest.mark.gpu
+
+SETS = {
+    "up to 32": [(1, 1), (1, 7), (7, 1), (31, 33), (32, 32), (5, 128), (129, 5), (32, 1025), (3000, 17), (1, 30000), (16, 65536), (17, 32769)],
+    "up to 64": [(33, 33), (33, 128), (129, 40), (64, 64), (64, 2048), (4099, 37), (37, 8191), (32768, 33)],
+    "up to 128": [(65, 65), (65, 128), (129, 100), (128, 128), (784, 128), (128, 4096), (1027, 127), (96, 257), (8193, 80)],
+}
+
+
+@pytest.mark.parametrize("iters", [1, 2, 5])
+@pytest.mark.parametrize("which", list(SETS))
+def test_small_matrices_against_fp64(which, iters):
+    gen = torch.Generator(device="cuda").manual_seed(iters)
+    mats = [torch.randn(s, generator=gen, device="cuda") * 10.0 ** (-(i % 5)) for i, s in enumerate(SETS[which])]
+    got = _orthogonalise_direct(mats, iters)
+    again = _orthogonalise_direct(mats, iters)
+    prev = torch.backends.cuda.matmul.allow_tf32
+    torch.backends.cuda.matmul.allow_tf32 = False
+    try:
+        for x, y, z in zip(mats, got, again):
+            want = _reference_direct(x, iters)
+            e = float((y.double() - want).abs().max())
+            e32 = float((_reference_direct(x, iters, dtype=torch.float32).double() - want).abs().max())
+            print(tuple(x.shape), iters, e, e32)
+            assert torch.equal(y, z), tuple(x.shape)
+            assert e <= 1.5 * e32 + 5e-5, (tuple(x.shape), e, e32)
+    finally:
+        torch.backends.cuda.matmul.allow_tf32 = prev
+
+
+def test_many_that_meet_and_repeated_calls():
+    """More matrices of several blocks than may wait at a time (longer slabs are taken), a plan used again and again,
+    a NaN that stays in its matrix, and a call that only normalises and applies."""
+    from pylo_amd import _lib
+
+    shapes = [(128, 784)] * 24 + [(60, 1500)] * 30 + [(3, 5000)] * 20 + [(128, 784), (200, 300)]
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    mats = [torch.randn(s, generator=gen, device="cuda") for s in shapes]
+    mats[5][3, 700] = float("nan")
+    plan = _lib.Plan(_lib.KIND_CELO2, shapes, [0] * len(shapes), torch.device("cuda:0"))
+    fin = np.zeros(len(mats), dtype=_lib.ARGS_DTYPE)
+    want = None
+    for call in range(4):
+        steps = [x.clone() for x in mats]
+        params = [torch.zeros_like(x) for x in mats]
+        for i in range(len(mats)):
+            fin["grad"][i], fin["param"][i], fin["step_out"][i] = 1, params[i].data_ptr(), steps[i].data_ptr()
+            fin["lr"][i], fin["weight_decay"][i], fin["step_mult"][i] = -1.0, 0.0, 1.0
+            fin["flags"][i] = _lib.ARG_ORTHOGONALIZE if call < 3 else 0
+        plan.celo2_orthogonalize_finish(fin, (3.4445, -4.775, 2.0315), 5, 1e-8, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.isnan(params[5]).all()
+        if call == 0:
+            want = params
+            for i in (0, 23, 24, 53, 54, 73, 75):
+                assert float((params[i].double() - _reference_direct(mats[i])).abs().max()) <= 2e-4, i
+            assert float((params[74].double() - _reference_direct(mats[74])).abs().max()) <= 2e-4
+        elif call < 3:
+            assert all(torch.equal(a, b) for i, (a, b) in enumerate(zip(params, want)) if i != 5)
+        else:
+            for i, x in enumerate(mats):
+                if i != 5:
+                    r = x.double() * torch.rsqrt(1e-9 + x.double().pow(2).mean())
+                    assert float((params[i].double() - r).abs().max()) <= 1e-5, i
+    plan.close()
