@@ -1194,6 +1194,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 // block folds this step's channel normalisers, param_scale and lr_mult into the block the apply
 // items read.
 // ---------------------------------------------------------------------------------------------
+template <bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_velo_elem(const TDesc* __restrict__ descs,
                                                         const PyloTensorArgs* __restrict__ dyn,
                                                         const Item* __restrict__ items,
@@ -1208,7 +1209,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   __shared__ float sc[30];
   __shared__ int s_flag;
   const Item it = items[blockIdx.x];
-  const TDesc d = descs[it.tensor];
+  const TDesc d = elem_desc<SPLIT>(descs + it.tensor);
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
   if (it.c & kElemApply) {

@@ -90,6 +90,7 @@ struct NsBatch { int mat0, n_mats, group0, n_groups; long long plane_elems; };
 constexpr int kNsSmallClasses = 3;
 struct Layout {
   std::vector<Item> mx_items;   // ELO-CELO2: statistics and apply items in slab order (k_celo2_elem)
+  bool split = false;           // element blocks smaller than 8192 elements (split_for)
   size_t off_mx_items = 0, off_sync = 0;
   size_t off_newsum = 0, off_piv = 0, off_wmix = 0;   // VeLO: sums carried to the next step, pivots, un-folded MLPs
   // ELO-CELO2: Newton-Schulz on the 2-D tensors (k_ns.h)
@@ -908,6 +909,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
     total_elems += n;
   }
   const int split = split_for(total_elems);
+  L.split = split > 1;
   L.tensor_norm = (shapes[0].flags & PYLO_F_TENSOR_NORM) != 0;
   L.global_norm = (shapes[0].flags & PYLO_F_GLOBAL_NORM) != 0 || L.tensor_norm;
   for (int t = 0; t < T; ++t) {
@@ -1734,12 +1736,10 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
   if (n_mx > 0) {
     const Item* mx_items = P->at<Item>(L.off_mx_items);
     int* sync = P->at<int>(L.off_sync);
-    if (P->mlp_on_matrix_pipe)
-      hipLaunchKernelGGL(k_celo2_elem<true>, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, mx_items, fac_tab, term_tab,
-                         gl, dec, mlp, wfold, chan_ms, stats, sync, P->T);
-    else
-      hipLaunchKernelGGL(k_celo2_elem<false>, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, mx_items, fac_tab, term_tab,
-                         gl, dec, mlp, wfold, chan_ms, stats, sync, P->T);
+    const auto elem = P->mlp_on_matrix_pipe ? (L.split ? k_celo2_elem<true, true> : k_celo2_elem<true, false>)
+                                            : (L.split ? k_celo2_elem<false, true> : k_celo2_elem<false, false>);
+    hipLaunchKernelGGL(elem, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, mx_items, fac_tab, term_tab, gl, dec, mlp,
+                       wfold, chan_ms, stats, sync, P->T);
     HIP_TRY(mark());
   } else {
     if (n_el > 0) hipLaunchKernelGGL(k_celo2_stats, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, gl, dec, stats);
@@ -2298,7 +2298,8 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
     if (n_v0b > 0)
       hipLaunchKernelGGL(k_terms<4>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, bscale, canon, kVCanon, term_tab);
     HIP_TRY(mark());
-    hipLaunchKernelGGL(k_velo_elem, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, P->at<Item>(L.off_mx_items), fac_tab, term_tab,
+    const auto elem = L.split ? k_velo_elem<true> : k_velo_elem<false>;
+    hipLaunchKernelGGL(elem, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, P->at<Item>(L.off_mx_items), fac_tab, term_tab,
                        dec, (const float*)wmix, wfold, stats, (const float*)piv, newsum, P->at<int>(L.off_sync), T);
     HIP_TRY(mark());
     mark.done();
