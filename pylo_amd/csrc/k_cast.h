@@ -7,6 +7,12 @@
 // through a substituted argument record (k_stage_args), and what the step wrote to the parameter is rounded
 // to nearest-even back into the caller's buffer (k_cast_out).  Against 72 bytes per element of a factored
 // tensor this adds 18 (16-bit types) or 36 (fp64) bytes; tensors without a tag are not touched by any of it.
+//
+// VeLO's 2-D tensors on the column-resident walk skip the staging where they are stored in 16 bits (TDesc::direct):
+// its three passes over them take the storage type as a template argument, widen in the load and round in the store.
+// Two casts with 18 bytes an element less, and passes that move 12 bytes an element less.  On 86 M bf16 elements (ViT-B/16)
+// casts 327 us -> 15 us (what is still staged), k_p0 105 -> 59, k_velo_stats 307 -> 299, k_velo_apply 694 -> 617, whole
+// step 1.51 -> 1.04 ms, every result bit for bit the same.
 #pragma once
 
 #include "pylo_common.h"
@@ -39,6 +45,42 @@ __device__ __forceinline__ void store_stored(void* base, long long i, int store,
   if (store == kStoreF64) ((double*)base)[i] = (double)x;
   else if (store == kStoreF32) ((float*)base)[i] = x;
   else ((unsigned short*)base)[i] = narrow16(x, store);
+}
+
+// Rows of a tensor as the column-resident walks see them: fp32 (ST = kStoreF32) or the 16-bit type ST.
+template <int ST> struct StoredAs { typedef unsigned short E; };
+template <> struct StoredAs<kStoreF32> { typedef float E; };
+
+// V consecutive elements at a wave-uniform base plus `off` elements per lane.  16-bit elements: V * 2 bytes a lane, aligned
+// to as much where `off` and the row pitch are multiples of V (buffers of tagged tensors are 16-byte aligned).
+template <int V, int ST, bool NT>
+__device__ __forceinline__ void load_row(const typename StoredAs<ST>::E* base, unsigned off, float (&x)[V]) {
+  if constexpr (ST == kStoreF32) {
+    if constexpr (NT) load_vec_nt<V>(base, off * 4u, x);
+    else load_vec_o<V>(base, off * 4u, x);
+  } else {
+    typedef unsigned short E __attribute__((ext_vector_type(V)));
+    typedef __attribute__((address_space(1))) E gE;
+    const gE* p = (const gE*)((const gchar*)base + off * 2u);
+    E w;
+    if constexpr (NT) w = __builtin_nontemporal_load(p);
+    else w = *p;
+#pragma unroll
+    for (int v = 0; v < V; ++v) x[v] = widen16(w[v], ST);
+  }
+}
+template <int V, int ST>
+__device__ __forceinline__ void store_row(typename StoredAs<ST>::E* base, unsigned off, const float (&x)[V]) {
+  if constexpr (ST == kStoreF32) {
+    store_vec_o<V>(base, off * 4u, x);
+  } else {
+    typedef unsigned short E __attribute__((ext_vector_type(V)));
+    typedef __attribute__((address_space(1))) E gE;
+    E w;
+#pragma unroll
+    for (int v = 0; v < V; ++v) w[v] = narrow16(x[v], ST);
+    *(gE*)((gchar*)base + off * 2u) = w;
+  }
 }
 
 // src (storage type) -> dst (fp32), elements [0, lim) of a block's piece; both 16-byte aligned when vec.
@@ -82,10 +124,10 @@ __device__ __forceinline__ void narrow_piece(const float* src, void* dst, unsign
   }
 }
 
-// Per tagged tensor: floats into the staging area of its gradient and of its parameter (-1: not tagged).
+// Per staged tensor: floats into the staging area of its gradient and of its parameter (-1: not staged).
 struct StageOfs { long long g, p; };
 
-// dyn[t] = user[t], with grad / param of a tagged tensor that takes part pointing into the staging.
+// dyn[t] = user[t], with grad / param of a staged tensor that takes part pointing into the staging.
 __global__ __launch_bounds__(256) void k_stage_args(int T, const TDesc* __restrict__ descs,
                                                     const PyloTensorArgs* __restrict__ user,
                                                     PyloTensorArgs* __restrict__ dyn, const StageOfs* __restrict__ ofs,
@@ -93,7 +135,7 @@ __global__ __launch_bounds__(256) void k_stage_args(int T, const TDesc* __restri
   const int t = blockIdx.x * 256 + threadIdx.x;
   if (t >= T) return;
   PyloTensorArgs a = user[t];
-  if (descs[t].store != kStoreF32 && a.grad != nullptr) {
+  if (descs[t].store != kStoreF32 && !descs[t].direct && a.grad != nullptr) {
     a.grad = stage + ofs[t].g;
     a.param = stage + ofs[t].p;
   }

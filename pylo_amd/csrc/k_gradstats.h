@@ -2,6 +2,7 @@
 // gradient norm, and the Adafactor row / column vectors with everything derived from them (V0).
 #pragma once
 
+#include "k_cast.h"
 #include "pylo_common.h"
 
 namespace pylo {
@@ -16,8 +17,9 @@ __device__ __forceinline__ float abs_or_inf(float x, int nan0) {
   return (nan0 && ax != ax) ? __builtin_inff() : ax;
 }
 
-template <int V, bool exact>
-__device__ __forceinline__ void p0_factored(const TDesc& d, const float* g, int strip, int cb,
+// ST: storage type of the gradient (k_cast.h).
+template <int V, bool exact, int ST = kStoreF32>
+__device__ __forceinline__ void p0_factored(const TDesc& d, const typename StoredAs<ST>::E* g, int strip, int cb,
                                             float scale, float clipv, int nan0, float* __restrict__ rowpart,
                                             float* __restrict__ colpart, float* lds_col, float* lds_row,
                                             float& gsq, float& amax) {
@@ -37,12 +39,14 @@ __device__ __forceinline__ void p0_factored(const TDesc& d, const float* g, int 
   // flight).  Measured, it does not change the pass's time inside a step (0.125 ms where a bare streaming kernel
   // reads the same bytes in 0.07 - 0.08 ms): what holds it back there is the write-back of the lines that the
   // kernels before it left dirty, not the bytes it has in flight.
-  const float* gc = g + (in ? c : 0);
+  const typename StoredAs<ST>::E* gc = g + (in ? c : 0);
   auto load_trip = [&](int rb, float (&x)[4][V]) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int r = rb + u * kWaves;
-      load_vec<V>(gc + (size_t)(r < r1 ? r : rb) * C0, x[u]);
+      const typename StoredAs<ST>::E* row = gc + (size_t)(r < r1 ? r : rb) * C0;
+      if constexpr (ST == kStoreF32) load_vec<V>(row, x[u]);
+      else load_row<V, ST, false>(row, 0u, x[u]);
     }
   };
   int trip = 0;
@@ -149,6 +153,8 @@ __device__ __forceinline__ void p0_nd_block(const TDesc* __restrict__ descs, con
 // pass 0: tensors with clip_norm > 0 are summed raw (the scale factors out of g^2) and flag
 //         elements beyond the clamp; tensors without global-norm clipping are clamped directly.
 // pass 1: only if the flag was raised: redo clip_norm > 0 tensors with scale and clamp applied.
+// TYPED: plans with tensors whose 16-bit gradient is read here (TDesc::direct; their rows are multiples of 128).
+template <bool TYPED>
 __global__ __launch_bounds__(kThreads) void k_p0(const TDesc* __restrict__ descs,
                                                  const PyloTensorArgs* __restrict__ dyn,
                                                  const Item* __restrict__ items, float* __restrict__ part,
@@ -177,7 +183,13 @@ __global__ __launch_bounds__(kThreads) void k_p0(const TDesc* __restrict__ descs
       const float scale = (pass == 1) ? grad_scale(d, a, gl, it.tensor) : 1.0f;
       float* p0r = part + d.part_off[0];
       float* p0c = part + d.part_off[1];
-      if (d.vec == 4 && exact) p0_factored<4, true>(d, a.grad, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
+      if (TYPED && d.direct) {
+        const unsigned short* g16 = reinterpret_cast<const unsigned short*>(a.grad);
+        if (d.store == kStoreBF16 && exact) p0_factored<4, true, kStoreBF16>(d, g16, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
+        else if (d.store == kStoreBF16) p0_factored<4, false, kStoreBF16>(d, g16, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
+        else if (exact) p0_factored<4, true, kStoreF16>(d, g16, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
+        else p0_factored<4, false, kStoreF16>(d, g16, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
+      } else if (d.vec == 4 && exact) p0_factored<4, true>(d, a.grad, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
       else if (d.vec == 4) p0_factored<4, false>(d, a.grad, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
       else if (exact) p0_factored<1, true>(d, a.grad, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
       else p0_factored<1, false>(d, a.grad, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);

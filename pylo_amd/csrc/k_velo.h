@@ -3,6 +3,7 @@
 // emits each tensor's MLP weights.
 #pragma once
 
+#include "k_cast.h"
 #include "k_celo2.h"
 #include "k_gradstats.h"
 #include "pylo_common.h"
@@ -130,12 +131,12 @@ struct NewSums {
   float v[9];
   float piv[4];
   __device__ __forceinline__ void clear(const TDesc& d, const PyloTensorArgs& a, const EmaConsts& e,
-                                        const float* __restrict__ old_first) {
+                                        const float* __restrict__ old_first, float raw_first) {
 #pragma unroll
     for (int c = 0; c < 9; ++c) v[c] = 0.0f;
     float of[4];
     load_uniform<4>(old_first, of);
-    const float g0 = d.n > 0 ? cond_grad(*(const cfloat*)a.grad, d.gscale, a.clip_val, d.nan0) : 0.0f;
+    const float g0 = d.n > 0 ? cond_grad(raw_first, d.gscale, a.clip_val, d.nan0) : 0.0f;
     float m[3] = {of[0], of[1], of[2]};
     float r = of[3];
     ema_update(e, g0, m, r);
@@ -199,7 +200,8 @@ __device__ __forceinline__ void velo_stats_fac(const TDesc& d, const PyloTensorA
 // factors through the scalar cache, six streams per row.
 // KEEP: plain loads, which leave the lines in the memory-side cache for the apply items that follow
 // (k_velo_elem); otherwise non-temporal loads (see celo2_stats_tile).
-template <bool KEEP>
+// ST: storage type of gradient and parameter (k_cast.h).
+template <bool KEEP, int ST>
 __device__ __forceinline__ void velo_stats_tile(const TDesc& d, const PyloTensorArgs& a, int task,
                                                 const EmaConsts& e, const float* __restrict__ fac_tab,
                                                 VeloAcc& acc) {
@@ -210,23 +212,22 @@ __device__ __forceinline__ void velo_stats_tile(const TDesc& d, const PyloTensor
   float fb[V][4];
 #pragma unroll
   for (int v = 0; v < V; ++v) load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
-  const unsigned lo = (threadIdx.x & 63) * (V * 4u);
-  const float *g = a.grad + tk.first, *p = a.param + tk.first, *m0 = a.mom + tk.first,
-              *m1 = a.mom + d.n + tk.first, *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
+  const unsigned le = (threadIdx.x & 63) * V, lo = le * 4u;
+  typedef typename StoredAs<ST>::E E;
+  const E *g = reinterpret_cast<const E*>(a.grad) + tk.first, *p = reinterpret_cast<const E*>(a.param) + tk.first;
+  const float *m0 = a.mom + tk.first, *m1 = a.mom + d.n + tk.first, *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
   const float* fr = f0 + (size_t)tk.r0 * 4;
 #pragma unroll 2
   for (int r = tk.r0; r < tk.r1; ++r) {
     float xg[V], xp[V], x0[V], x1[V], x2[V], xr[V], fa[4];
+    load_row<V, ST, !KEEP>(g, le, xg);
+    load_row<V, ST, !KEEP>(p, le, xp);
     if constexpr (KEEP) {
-      load_vec_o<V>(g, lo, xg);
-      load_vec_o<V>(p, lo, xp);
       load_vec_o<V>(m0, lo, x0);
       load_vec_o<V>(m1, lo, x1);
       load_vec_o<V>(m2, lo, x2);
       load_vec_o<V>(rms, lo, xr);
     } else {
-      load_vec_nt<V>(g, lo, xg);
-      load_vec_nt<V>(p, lo, xp);
       load_vec_nt<V>(m0, lo, x0);
       load_vec_nt<V>(m1, lo, x1);
       load_vec_nt<V>(m2, lo, x2);
@@ -332,7 +333,7 @@ __device__ __forceinline__ void velo_stats_vec(const TDesc& d, const PyloTensorA
 
 // One block of the statistics pass (channel sums and, when nobody carried them over, the LSTM's sums).
 // Returns after a barrier with the four waves' sums in `red`.
-template <bool LSTM_SUMS, bool KEEP>
+template <bool LSTM_SUMS, bool KEEP, bool TYPED = false>
 __device__ __forceinline__ void velo_stats_block(const TDesc& d, const PyloTensorArgs& a, const Item& it,
                                                  const float* __restrict__ fac_tab, const PyloDecays& dec,
                                                  float (*red)[38]) {
@@ -345,7 +346,11 @@ __device__ __forceinline__ void velo_stats_block(const TDesc& d, const PyloTenso
   lstm_pivots(d, a, acc.piv);
   if (d.tile_nct > 0) {
     const int task = it.a * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (task < d.tile_ntask) velo_stats_tile<KEEP>(d, a, task, e, fac_tab, acc);
+    if (task < d.tile_ntask) {
+      if (TYPED && d.direct && d.store == kStoreBF16) velo_stats_tile<KEEP, kStoreBF16>(d, a, task, e, fac_tab, acc);
+      else if (TYPED && d.direct) velo_stats_tile<KEEP, kStoreF16>(d, a, task, e, fac_tab, acc);
+      else velo_stats_tile<KEEP, kStoreF32>(d, a, task, e, fac_tab, acc);
+    }
   } else if (d.mode == kModeFac2D) {
     if (d.vec == 4) velo_stats_fac<4, false>(d, a, it.a, e, fac_tab, acc);
     else velo_stats_fac<1, false>(d, a, it.a, e, fac_tab, acc);
@@ -371,6 +376,7 @@ __device__ __forceinline__ void velo_stats_block(const TDesc& d, const PyloTenso
   __syncthreads();
 }
 
+template <bool TYPED>
 __global__ __launch_bounds__(kThreads) void k_velo_stats(const TDesc* __restrict__ descs,
                                                          const PyloTensorArgs* __restrict__ dyn,
                                                          const Item* __restrict__ items,
@@ -381,7 +387,7 @@ __global__ __launch_bounds__(kThreads) void k_velo_stats(const TDesc* __restrict
   const TDesc d = descs[it.tensor];
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
-  velo_stats_block<true, false>(d, a, it, fac_tab, dec, red);
+  velo_stats_block<true, false, TYPED>(d, a, it, fac_tab, dec, red);
   if (threadIdx.x < 38) {
     const int c = threadIdx.x;
     stats_part[(size_t)blockIdx.x * kStatW + c] =
@@ -990,7 +996,8 @@ __device__ __forceinline__ void velo_apply_fac(const TDesc& d, const PyloTensorA
 // The apply pass over one wave task of the column-resident walk, with the 30->4->4->2 MLP as
 // lane-local 4x4x1 fp32 outer products on the matrix pipe: weight group v (four consecutive floats
 // of the folded block) sits in lanes 4*(v%16).. of register v/16; biases enter as a rank-1 update
-// with the constant 1.
+// with the constant 1.  ST: storage type of gradient and parameter (k_cast.h).
+template <int ST>
 __device__ __forceinline__ void velo_apply_tile(const TDesc& d, const PyloTensorArgs& a, int task,
                                                 const EmaConsts& e, const float* __restrict__ fac_tab,
                                                 const float* __restrict__ term_tab, const float* wbase, NewSums& ns,
@@ -1017,17 +1024,18 @@ __device__ __forceinline__ void velo_apply_tile(const TDesc& d, const PyloTensor
     load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
     load_vec_o<4>(t1 + v * 4, tk.col * 16u, tb[v]);
   }
-  const unsigned lo = lane * (V * 4u);
-  const float* g = a.grad + tk.first;
-  float *p = a.param + tk.first, *m0 = a.mom + tk.first, *m1 = a.mom + d.n + tk.first,
-        *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
+  const unsigned le = lane * V, lo = le * 4u;
+  typedef typename StoredAs<ST>::E E;
+  const E* g = reinterpret_cast<const E*>(a.grad) + tk.first;
+  E* p = reinterpret_cast<E*>(a.param) + tk.first;
+  float *m0 = a.mom + tk.first, *m1 = a.mom + d.n + tk.first, *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
   const float* fr = f0 + (size_t)tk.r0 * 4;
   const float* tr = t0 + (size_t)tk.r0 * 4;
   const float wd_lr = a.weight_decay * a.lr;
   for (int r = tk.r0; r < tk.r1; ++r) {
     float xg[V], xp[V], x0[V], x1[V], x2[V], xr[V], fa[4], ta[4];
-    load_vec_nt<V>(g, lo, xg);
-    load_vec_nt<V>(p, lo, xp);
+    load_row<V, ST, true>(g, le, xg);
+    load_row<V, ST, true>(p, le, xp);
     load_vec_nt<V>(m0, lo, x0);
     load_vec_nt<V>(m1, lo, x1);
     load_vec_nt<V>(m2, lo, x2);
@@ -1082,7 +1090,7 @@ __device__ __forceinline__ void velo_apply_tile(const TDesc& d, const PyloTensor
       const float mm[3] = {x0[v], x1[v], x2[v]};
       ns.add(q, mm, xr[v]);
     }
-    store_vec_o<V>(p, lo, pn);
+    store_row<V, ST>(p, le, pn);
     g += d.C0; p += d.C0; m0 += d.C0; m1 += d.C0; m2 += d.C0; rms += d.C0;
     fr += 4; tr += 4;
   }
@@ -1131,7 +1139,9 @@ __device__ __forceinline__ void velo_apply_vec(const TDesc& d, const PyloTensorA
   }
 }
 
-// One block of the apply pass; its sums over the written values go to row `row` of newsum_part.
+// One block of the apply pass; its sums over the written values go to row `row` of newsum_part (nobody reads those of
+// plans with 16-bit tensors: the next step starts from the rounded parameter).
+template <bool TYPED = false>
 __device__ __forceinline__ void velo_apply_block(const TDesc& d, const PyloTensorArgs& a, const Item& it,
                                                  const float* __restrict__ fac_tab,
                                                  const float* __restrict__ term_tab, const PyloDecays& dec,
@@ -1140,10 +1150,17 @@ __device__ __forceinline__ void velo_apply_block(const TDesc& d, const PyloTenso
   const EmaConsts e = make_ema(dec);
   const float* w = wfold + (size_t)it.tensor * kVFold;
   NewSums ns;
-  ns.clear(d, a, e, piv + (size_t)it.tensor * 4);
+  float raw_first = 0.0f;
+  if (TYPED && d.direct) raw_first = load_stored(a.grad, 0, d.store);
+  else if (d.n > 0) raw_first = *(const cfloat*)a.grad;
+  ns.clear(d, a, e, piv + (size_t)it.tensor * 4, raw_first);
   if (d.tile_nct > 0) {
     const int task = it.a * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (task < d.tile_ntask) velo_apply_tile(d, a, task, e, fac_tab, term_tab, w, ns, coh);
+    if (task < d.tile_ntask) {
+      if (TYPED && d.direct && d.store == kStoreBF16) velo_apply_tile<kStoreBF16>(d, a, task, e, fac_tab, term_tab, w, ns, coh);
+      else if (TYPED && d.direct) velo_apply_tile<kStoreF16>(d, a, task, e, fac_tab, term_tab, w, ns, coh);
+      else velo_apply_tile<kStoreF32>(d, a, task, e, fac_tab, term_tab, w, ns, coh);
+    }
   } else if (d.mode == kModeFac2D) {
     if (d.vec == 4) velo_apply_fac<4, false>(d, a, it.a, e, fac_tab, term_tab, w, ns);
     else velo_apply_fac<1, false>(d, a, it.a, e, fac_tab, term_tab, w, ns);
@@ -1168,6 +1185,7 @@ __device__ __forceinline__ void velo_apply_block(const TDesc& d, const PyloTenso
 }
 
 // Apply pass as a launch of its own.
+template <bool TYPED>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_velo_apply(const TDesc* __restrict__ descs,
                                                          const PyloTensorArgs* __restrict__ dyn,
                                                          const Item* __restrict__ items,
@@ -1181,7 +1199,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   const TDesc d = descs[it.tensor];
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
-  velo_apply_block(d, a, it, fac_tab, term_tab, dec, wfold, piv, newsum_part, (int)blockIdx.x, false, red);
+  velo_apply_block<TYPED>(d, a, it, fac_tab, term_tab, dec, wfold, piv, newsum_part, (int)blockIdx.x, false, red);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -112,6 +112,7 @@ struct TDesc {
   int nan0;                // gradients pass through torch.nan_to_num (PYLO_F_NAN_TO_NUM)
   int wd_prestep;          // p -= lr * (step + wd * p) against the pre-step parameter (PYLO_F_WD_PRESTEP)
   int store;               // storage type of the caller's grad / param buffers (kStore*, k_cast.h); 0 = fp32
+  int direct;              // ... which the passes read and write themselves: no fp32 staging (k_cast.h)
   int own_norm;            // clip_norm bounds the tensor's own gradient norm (PYLO_F_TENSOR_NORM), not the call's
   int p0_first, p0_n;      // the tensor's blocks of the first statistics launch (rows of its sum-of-squares partials)
   float gscale;            // 1 in the plan; AdafacLO-family kernels overwrite their copy with the clip scale

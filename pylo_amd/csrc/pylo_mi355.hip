@@ -940,14 +940,6 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
     d.own_norm = L.tensor_norm ? 1 : 0;
     d.nan0 = (s.flags & PYLO_F_NAN_TO_NUM) != 0;
     d.store = (s.flags & PYLO_F_STORE_MASK) >> 8;
-    L.stage_ofs.push_back(StageOfs{-1, -1});
-    if (d.store != kStoreF32 && n > 0) {
-      const long long pitch = (n + 63) / 64 * 64;
-      L.stage_ofs.back() = StageOfs{L.stage_floats, L.stage_floats + pitch};
-      L.stage_floats += 2 * pitch;
-      for (long long c = 0; c * kCastElems < n; ++c) L.cast_items.push_back(Item{t, (int)c, 0, 0});
-      L.typed = true;
-    }
     d.wd_prestep = (s.flags & PYLO_F_WD_PRESTEP) != 0;
     d.fac_slot = -1;
     d.rank = rank < 4 ? rank : 4;
@@ -1070,6 +1062,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       d.tile_nct = d.C0 / kTileCols;
       d.tile_rows = tile_rows_for(kind, split);
       d.tile_ntask = d.tile_nct * ((d.R0 + d.tile_rows - 1) / d.tile_rows);
+      d.direct = kind == PYLO_KIND_VELO && (d.store == kStoreF16 || d.store == kStoreBF16);
       for (int b = 0; b * 4 < d.tile_ntask; ++b) L.el_items.push_back(Item{t, b, 0, 0});
     } else {
       for (long long c = 0; c * chunk < n; ++c) L.el_items.push_back(Item{t, (int)c, 0, 0});
@@ -1126,6 +1119,18 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
     build_slice_tables(L, shapes, T);
     build_ns_tables(L, shapes, T, ns_floats);
     if (int rc = build_fin_tables(L, shapes, T)) return rc;
+  }
+  // fp32 staging of tensors in other storage types (k_cast.h)
+  for (int t = 0; t < T; ++t) {
+    const TDesc& d = L.descs[t];
+    L.stage_ofs.push_back(StageOfs{-1, -1});
+    if (d.store == kStoreF32 || d.n == 0) continue;
+    L.typed = true;
+    if (d.direct) continue;
+    const long long pitch = (d.n + 63) / 64 * 64;
+    L.stage_ofs.back() = StageOfs{L.stage_floats, L.stage_floats + pitch};
+    L.stage_floats += 2 * pitch;
+    for (long long c = 0; c * kCastElems < d.n; ++c) L.cast_items.push_back(Item{t, (int)c, 0, 0});
   }
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -1558,6 +1563,7 @@ void stage_in(PyloPlan* P, hipStream_t s, int what) {
   hipLaunchKernelGGL(k_stage_args, dim3((P->T + 255) / 256), dim3(256), 0, s, P->T, P->at<TDesc>(L.off_descs),
                      P->at<PyloTensorArgs>(L.off_dyn_user), P->at<PyloTensorArgs>(L.off_dyn),
                      P->at<StageOfs>(L.off_stage_ofs), P->at<float>(L.off_stage));
+  if (L.cast_items.empty()) return;   // every tensor is read in place
   hipLaunchKernelGGL(k_cast_in, dim3((unsigned)L.cast_items.size()), dim3(kThreads), 0, s, P->at<TDesc>(L.off_descs),
                      P->at<PyloTensorArgs>(L.off_dyn_user), P->at<Item>(L.off_cast_items),
                      P->at<StageOfs>(L.off_stage_ofs), P->at<float>(L.off_stage), what);
@@ -1565,7 +1571,7 @@ void stage_in(PyloPlan* P, hipStream_t s, int what) {
 
 void stage_out(PyloPlan* P, hipStream_t s, int flat_only) {
   const Layout& L = P->L;
-  if (!L.typed) return;
+  if (L.cast_items.empty()) return;
   hipLaunchKernelGGL(k_cast_out, dim3((unsigned)L.cast_items.size()), dim3(kThreads), 0, s, P->at<TDesc>(L.off_descs),
                      P->at<PyloTensorArgs>(L.off_dyn_user), P->at<Item>(L.off_cast_items),
                      P->at<StageOfs>(L.off_stage_ofs), P->at<float>(L.off_stage), flat_only);
@@ -1714,14 +1720,14 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
   const bool exact_pass = exact_pass_possible(P, args);
   HIP_TRY(mark());
   if (n_p0 > 0)
-    hipLaunchKernelGGL(k_p0, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
+    hipLaunchKernelGGL(k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
                        (const Item*)nullptr, n_p0);
   HIP_TRY(mark());
   hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, gsq, flag, n_p0, gl, exact_pass ? 1 : 0,
                      P->at<int>(L.off_sync), 2 * P->T);
   HIP_TRY(mark());
   if (n_p0 > 0 && exact_pass)
-    hipLaunchKernelGGL(k_p0, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
+    hipLaunchKernelGGL(k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
                        (const Item*)nullptr, n_p0);
   if (n_nd > 0) hipLaunchKernelGGL(k_p0_nd, dim3(n_nd), dim3(kThreads), 0, s, descs, dyn, nd_items, part, gl);
   HIP_TRY(mark());
@@ -2265,9 +2271,10 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   };
   // clip_norm is 0 for VeLO tensors: k_p0 clamps directly; its norm / flag outputs are not used
   // no global norm to wait for: the N-D tensors' sums ride in the tail blocks of the same launch
+  const bool typed = L.typed;
   auto gradient_sums = [&]() {
     if (n_p0 + n_nd > 0)
-      hipLaunchKernelGGL(k_p0, dim3(n_p0 + n_nd), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
+      hipLaunchKernelGGL(typed ? k_p0<true> : k_p0<false>, dim3(n_p0 + n_nd), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
                          nd_items, n_p0);
   };
   auto factor_tables = [&]() {
@@ -2313,7 +2320,7 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   HIP_TRY(mark());
   if (n_mx == 0) HIP_TRY(mark());
   if (int rc = factor_tables()) return rc;
-  if (n_el > 0) hipLaunchKernelGGL(k_velo_stats, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, dec, stats);
+  if (n_el > 0) hipLaunchKernelGGL(typed ? k_velo_stats<true> : k_velo_stats<false>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, dec, stats);
   if (n_mx == 0) HIP_TRY(mark());
   const Item* seg_items = P->at<Item>(L.off_seg_items);
   double* seg_tot = P->at<double>(L.off_segtot);
@@ -2327,7 +2334,7 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
     hipLaunchKernelGGL(k_terms<4>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, bscale, canon, kVCanon, term_tab);
   HIP_TRY(mark());
   if (n_el > 0)
-    hipLaunchKernelGGL(k_velo_apply, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, term_tab, dec, wfold,
+    hipLaunchKernelGGL(typed ? k_velo_apply<true> : k_velo_apply<false>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, term_tab, dec, wfold,
                        (const float*)piv, newsum);
   HIP_TRY(mark());
   mark.done();
@@ -2400,7 +2407,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   // without global-norm clipping the N-D tensors' sums ride in the tail blocks of the first launch
   const int n_tail = clips ? 0 : n_nd;
   if (n_p0 + n_tail > 0)
-    hipLaunchKernelGGL(k_p0, dim3(n_p0 + n_tail), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
+    hipLaunchKernelGGL(k_p0<false>, dim3(n_p0 + n_tail), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
                        nd_items, n_p0);
   if (clips && L.tensor_norm) {
     // every tensor against its own norm (AdafacLO_naive.py:199-200): no clamp on such tensors, no exact pass
@@ -2409,7 +2416,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
     const bool exact_pass = exact_pass_possible(P, args);
     hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, gsq, flag, n_p0, gl, exact_pass ? 1 : 0, (int*)nullptr, 0);
     if (n_p0 > 0 && exact_pass)
-      hipLaunchKernelGGL(k_p0, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
+      hipLaunchKernelGGL(k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
                          (const Item*)nullptr, n_p0);
   }
   HIP_TRY(mark());
