@@ -1,8 +1,8 @@
 // ELO-CELO2 / CELO2 element kernels: statistics pass, weight folding, apply pass.
 #pragma once
 
-#include "pylo_common.h"
 #include "k_cast.h"
+#include "pylo_common.h"
 
 #ifndef PYLO_STATS_UNROLL
 #define PYLO_STATS_UNROLL 2   // rows of the statistics walk whose loads are issued together
@@ -293,8 +293,8 @@ struct TileTask {
 // the scalar cache, and the only per-row vector memory traffic is the six streams.
 // KEEP: plain loads, which leave the lines in the memory-side cache for the apply items that follow a
 // few thousand blocks later (k_celo2_elem); otherwise non-temporal loads, the faster way to stream
-// data that will have been evicted before anyone reads it again.
-template <bool KEEP>
+// data that will have been evicted before anyone reads it again.  ST: storage type of gradient and parameter (k_cast.h).
+template <bool KEEP, int ST>
 __device__ __forceinline__ void celo2_stats_tile(const TDesc& d, const PyloTensorArgs& a, int task, float scale,
                                                  const EmaConsts& e, const float* f0, const float* f1,
                                                  float (&acc)[kNStat]) {
@@ -303,23 +303,22 @@ __device__ __forceinline__ void celo2_stats_tile(const TDesc& d, const PyloTenso
   float fb[V][4];
 #pragma unroll
   for (int v = 0; v < V; ++v) load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
-  const unsigned lo = (threadIdx.x & 63) * (V * 4u);
-  const float *g = a.grad + tk.first, *p = a.param + tk.first, *m0 = a.mom + tk.first,
-              *m1 = a.mom + d.n + tk.first, *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
+  const unsigned le = (threadIdx.x & 63) * V, lo = le * 4u;
+  typedef typename StoredAs<ST>::E E;
+  const E *g = reinterpret_cast<const E*>(a.grad) + tk.first, *p = reinterpret_cast<const E*>(a.param) + tk.first;
+  const float *m0 = a.mom + tk.first, *m1 = a.mom + d.n + tk.first, *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
   const float* fr = f0 + (size_t)tk.r0 * 4;
 #pragma unroll PYLO_STATS_UNROLL
   for (int r = tk.r0; r < tk.r1; ++r) {
     float xg[V], xp[V], x0[V], x1[V], x2[V], xr[V], fa[4];
+    load_row<V, ST, !KEEP>(g, le, xg);
+    load_row<V, ST, !KEEP>(p, le, xp);
     if constexpr (KEEP) {
-      load_vec_o<V>(g, lo, xg);
-      load_vec_o<V>(p, lo, xp);
       load_vec_o<V>(m0, lo, x0);
       load_vec_o<V>(m1, lo, x1);
       load_vec_o<V>(m2, lo, x2);
       load_vec_o<V>(rms, lo, xr);
     } else {
-      load_vec_nt<V>(g, lo, xg);
-      load_vec_nt<V>(p, lo, xp);
       load_vec_nt<V>(m0, lo, x0);
       load_vec_nt<V>(m1, lo, x1);
       load_vec_nt<V>(m2, lo, x2);
@@ -345,7 +344,7 @@ __device__ __forceinline__ void celo2_stats_tile(const TDesc& d, const PyloTenso
 // One block of the statistics pass: sum of squares of the 18 per-element channels over the block's
 // elements, with the accumulators advanced in registers only (nothing is written back); an AdamW tensor
 // is updated completely instead.  Returns true when `red` holds the four waves' sums (after a barrier).
-template <bool KEEP>
+template <bool KEEP, bool TYPED = false>
 __device__ __forceinline__ bool celo2_stats_block(const TDesc& d, const PyloTensorArgs& a, const Item& it,
                                                   const float* __restrict__ fac_tab, const Globals* __restrict__ gl,
                                                   const PyloDecays& dec, float (*red)[kNStat]) {
@@ -369,7 +368,11 @@ __device__ __forceinline__ bool celo2_stats_block(const TDesc& d, const PyloTens
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (d.tile_nct > 0) {
     const int task = it.a * 4 + __builtin_amdgcn_readfirstlane(wave);
-    if (task < d.tile_ntask) celo2_stats_tile<KEEP>(d, a, task, scale, e, f0, f1, acc);
+    if (task < d.tile_ntask) {
+      if (TYPED && d.direct && d.store == kStoreBF16) celo2_stats_tile<KEEP, kStoreBF16>(d, a, task, scale, e, f0, f1, acc);
+      else if (TYPED && d.direct) celo2_stats_tile<KEEP, kStoreF16>(d, a, task, scale, e, f0, f1, acc);
+      else celo2_stats_tile<KEEP, kStoreF32>(d, a, task, scale, e, f0, f1, acc);
+    }
   } else if (d.vec == 4) {
     celo2_stats_chunk<4>(d, a, it.a, scale, e, f0, f1, acc);
   } else {
@@ -390,6 +393,7 @@ __device__ __forceinline__ double stats_block_total(const float (*red)[kNStat], 
 
 // Statistics pass as a launch of its own (each pass over all tensors; the fused element pass,
 // k_celo2_elem, is the default).
+template <bool TYPED>
 __global__ __launch_bounds__(kThreads) void k_celo2_stats(const TDesc* __restrict__ descs,
                                                           const PyloTensorArgs* __restrict__ dyn,
                                                           const Item* __restrict__ items,
@@ -401,7 +405,7 @@ __global__ __launch_bounds__(kThreads) void k_celo2_stats(const TDesc* __restric
   const TDesc d = descs[it.tensor];
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
-  if (!celo2_stats_block<false>(d, a, it, fac_tab, gl, dec, red)) return;
+  if (!celo2_stats_block<false, TYPED>(d, a, it, fac_tab, gl, dec, red)) return;
   if (threadIdx.x < kNStat)
     stats_part[(size_t)blockIdx.x * kStatW + stat_channel(threadIdx.x)] = stats_block_total(red, threadIdx.x);
 }
@@ -675,8 +679,9 @@ __device__ __forceinline__ void celo2_apply_chunk_mfma(const TDesc& d, const Pyl
 }
 
 // The matrix-pipe apply pass over one wave task of the column-resident walk: column factors and
-// column terms stay in registers, row factors and row terms arrive through the scalar cache.
-template <bool COH>
+// column terms stay in registers, row factors and row terms arrive through the scalar cache.  ST: storage type of
+// gradient and parameter (k_cast.h).
+template <bool COH, int ST>
 __device__ __forceinline__ void celo2_apply_tile(const TDesc& d, const PyloTensorArgs& a, int task, float scale,
                                                  const EmaConsts& e, const float* f0, const float* f1,
                                                  const float* t0, const float* t1, const float* wbase) {
@@ -696,16 +701,17 @@ __device__ __forceinline__ void celo2_apply_tile(const TDesc& d, const PyloTenso
     load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
     load_row8(t1 + v * 8, tk.col, tb[v]);
   }
-  const unsigned lo = lane * (V * 4u);
-  const float *g = a.grad + tk.first, *p = a.param + tk.first;
+  const unsigned le = lane * V, lo = le * 4u;
+  typedef typename StoredAs<ST>::E E;
+  const E *g = reinterpret_cast<const E*>(a.grad) + tk.first, *p = reinterpret_cast<const E*>(a.param) + tk.first;
   float *m0 = a.mom + tk.first, *m1 = a.mom + d.n + tk.first, *m2 = a.mom + 2 * d.n + tk.first,
         *rms = a.rms + tk.first, *out = a.step_out + tk.first;
   const float* fr = f0 + (size_t)tk.r0 * 4;
   const float* tr = t0 + (size_t)tk.r0 * 8;
   for (int r = tk.r0; r < tk.r1; ++r) {
     float xg[V], xp[V], x0[V], x1[V], x2[V], xr[V], fa[4], ta[8];
-    load_vec_nt<V>(g, lo, xg);
-    load_vec_nt<V>(p, lo, xp);
+    load_row<V, ST, true>(g, le, xg);
+    load_row<V, ST, true>(p, le, xp);
     load_vec_nt<V>(m0, lo, x0);
     load_vec_nt<V>(m1, lo, x1);
     load_vec_nt<V>(m2, lo, x2);
@@ -775,7 +781,7 @@ __device__ __forceinline__ void celo2_apply_tile(const TDesc& d, const PyloTenso
 
 // One block of the apply pass: accumulators advanced and written, features, MLP, raw step.
 // COH: the tensor's folded weights were written by another block of the running kernel.
-template <bool MFMA, bool COH>
+template <bool MFMA, bool COH, bool TYPED = false>
 __device__ __forceinline__ void celo2_apply_block(const TDesc& d, const PyloTensorArgs& a, const Item& it,
                                                   const float* __restrict__ fac_tab,
                                                   const float* __restrict__ term_tab, const Globals* __restrict__ gl,
@@ -785,9 +791,14 @@ __device__ __forceinline__ void celo2_apply_block(const TDesc& d, const PyloTens
   const float* w = wfold + (size_t)d.fac_slot * kC2Fold;
   if (MFMA && d.tile_nct > 0) {
     const int task = it.a * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (task < d.tile_ntask)
-      celo2_apply_tile<COH>(d, a, task, scale, e, fac_tab + d.fac_off[0], fac_tab + d.fac_off[1],
-                            term_tab + d.term_off[0], term_tab + d.term_off[1], w);
+    if (task < d.tile_ntask) {
+      const float *f0 = fac_tab + d.fac_off[0], *f1 = fac_tab + d.fac_off[1], *t0 = term_tab + d.term_off[0],
+                  *t1 = term_tab + d.term_off[1];
+      if (TYPED && d.direct && d.store == kStoreBF16)
+        celo2_apply_tile<COH, kStoreBF16>(d, a, task, scale, e, f0, f1, t0, t1, w);
+      else if (TYPED && d.direct) celo2_apply_tile<COH, kStoreF16>(d, a, task, scale, e, f0, f1, t0, t1, w);
+      else celo2_apply_tile<COH, kStoreF32>(d, a, task, scale, e, f0, f1, t0, t1, w);
+    }
   } else if (MFMA && d.vec == 4)
     celo2_apply_chunk_mfma<kMfmaV, COH>(d, a, it.a, scale, e, fac_tab + d.fac_off[0], fac_tab + d.fac_off[1],
                                         term_tab + d.term_off[0], term_tab + d.term_off[1], w);
@@ -800,7 +811,7 @@ __device__ __forceinline__ void celo2_apply_block(const TDesc& d, const PyloTens
 }
 
 // Apply pass as a launch of its own (see k_celo2_stats).
-template <bool MFMA>
+template <bool MFMA, bool TYPED>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PYLO_APPLY_WAVES))) void k_celo2_apply(const TDesc* __restrict__ descs,
                                                           const PyloTensorArgs* __restrict__ dyn,
                                                           const Item* __restrict__ items,
@@ -813,7 +824,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PYLO_A
   if (d.mode == kModeFlat) return;
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
-  celo2_apply_block<MFMA, false>(d, a, it, fac_tab, term_tab, gl, dec, wfold);
+  celo2_apply_block<MFMA, false, TYPED>(d, a, it, fac_tab, term_tab, gl, dec, wfold);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -840,7 +851,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PYLO_A
 //     rather than hang the GPU.
 // k_gnorm zeroes `sync` before every launch.
 // ---------------------------------------------------------------------------------------------
-template <bool MFMA, bool SPLIT>
+// TYPED: plans with tensors of 16-bit storage that are read in place (TDesc::direct).
+template <bool MFMA, bool SPLIT, bool TYPED = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PYLO_APPLY_WAVES))) void k_celo2_elem(
     const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const Item* __restrict__ items,
     const float* __restrict__ fac_tab, const float* __restrict__ term_tab, const Globals* __restrict__ gl,
@@ -866,7 +878,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PYLO_A
     }
     __syncthreads();
     if (s_flag) {
-      celo2_apply_block<MFMA, true>(d, a, it, fac_tab, term_tab, gl, dec, wfold);
+      celo2_apply_block<MFMA, true, TYPED>(d, a, it, fac_tab, term_tab, gl, dec, wfold);
     } else {
       // gave up: NaN steps for this block's elements (tile items: the wave tasks' rows; else the chunk)
       const float nan = __builtin_nanf("");
@@ -884,8 +896,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PYLO_A
     }
     return;
   }
-  const bool counted = (it.c & kElemKeep) ? celo2_stats_block<true>(d, a, it, fac_tab, gl, dec, red)
-                                          : celo2_stats_block<false>(d, a, it, fac_tab, gl, dec, red);
+  const bool counted = (it.c & kElemKeep) ? celo2_stats_block<true, TYPED>(d, a, it, fac_tab, gl, dec, red)
+                                          : celo2_stats_block<false, TYPED>(d, a, it, fac_tab, gl, dec, red);
   if (!counted) return;
   if (threadIdx.x < kNStat)
     coh_store_wait(stats_part + (size_t)it.b * kStatW + stat_channel(threadIdx.x), stats_block_total(red, threadIdx.x));

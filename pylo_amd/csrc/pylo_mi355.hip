@@ -139,6 +139,7 @@ struct Layout {
          off_ns_scale = 0, off_ns_ws = 0;
   // tensors whose grad / param are not fp32 (PYLO_F_STORE_*): fp32 staging, pieces of the cast kernels
   bool typed = false;
+  bool in_place = false;   // some tensor of 16-bit storage is read in place (TDesc::direct)
   std::vector<StageOfs> stage_ofs;
   std::vector<Item> cast_items;
   long long stage_floats = 0;
@@ -1062,7 +1063,8 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       d.tile_nct = d.C0 / kTileCols;
       d.tile_rows = tile_rows_for(kind, split);
       d.tile_ntask = d.tile_nct * ((d.R0 + d.tile_rows - 1) / d.tile_rows);
-      d.direct = kind == PYLO_KIND_VELO && (d.store == kStoreF16 || d.store == kStoreBF16);
+      d.direct = kind != PYLO_KIND_ADAFAC && (d.store == kStoreF16 || d.store == kStoreBF16);
+      L.in_place = L.in_place || d.direct;
       for (int b = 0; b * 4 < d.tile_ntask; ++b) L.el_items.push_back(Item{t, b, 0, 0});
     } else {
       for (long long c = 0; c * chunk < n; ++c) L.el_items.push_back(Item{t, (int)c, 0, 0});
@@ -1715,19 +1717,20 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
   const int n_p0 = (int)L.p0_items.size(), n_el = (int)L.el_items.size(), n_fac = (int)L.fac_list.size();
   const int n_v0a = (int)L.v0a_items.size(), n_v0b = (int)L.v0b_items.size();
   const PyloDecays dec = *decays;
+  const bool in_place = L.in_place;   // tensors of 16-bit storage without staging (the matrix pipe's walks only)
   Marks mark(P, s);
 
   const bool exact_pass = exact_pass_possible(P, args);
   HIP_TRY(mark());
   if (n_p0 > 0)
-    hipLaunchKernelGGL(k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
+    hipLaunchKernelGGL(in_place ? k_p0<true> : k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
                        (const Item*)nullptr, n_p0);
   HIP_TRY(mark());
   hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, gsq, flag, n_p0, gl, exact_pass ? 1 : 0,
                      P->at<int>(L.off_sync), 2 * P->T);
   HIP_TRY(mark());
   if (n_p0 > 0 && exact_pass)
-    hipLaunchKernelGGL(k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
+    hipLaunchKernelGGL(in_place ? k_p0<true> : k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
                        (const Item*)nullptr, n_p0);
   if (n_nd > 0) hipLaunchKernelGGL(k_p0_nd, dim3(n_nd), dim3(kThreads), 0, s, descs, dyn, nd_items, part, gl);
   HIP_TRY(mark());
@@ -1742,13 +1745,14 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
   if (n_mx > 0) {
     const Item* mx_items = P->at<Item>(L.off_mx_items);
     int* sync = P->at<int>(L.off_sync);
-    const auto elem = P->mlp_on_matrix_pipe ? (L.split ? k_celo2_elem<true, true> : k_celo2_elem<true, false>)
-                                            : (L.split ? k_celo2_elem<false, true> : k_celo2_elem<false, false>);
+    const auto elem = in_place              ? (L.split ? k_celo2_elem<true, true, true> : k_celo2_elem<true, false, true>)
+                      : P->mlp_on_matrix_pipe ? (L.split ? k_celo2_elem<true, true> : k_celo2_elem<true, false>)
+                                              : (L.split ? k_celo2_elem<false, true> : k_celo2_elem<false, false>);
     hipLaunchKernelGGL(elem, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, mx_items, fac_tab, term_tab, gl, dec, mlp,
                        wfold, chan_ms, stats, sync, P->T);
     HIP_TRY(mark());
   } else {
-    if (n_el > 0) hipLaunchKernelGGL(k_celo2_stats, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, gl, dec, stats);
+    if (n_el > 0) hipLaunchKernelGGL(in_place ? k_celo2_stats<true> : k_celo2_stats<false>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, gl, dec, stats);
     HIP_TRY(mark());
     const Item* seg_items = P->at<Item>(L.off_seg_items);
     double* seg_tot = P->at<double>(L.off_segtot);
@@ -1759,12 +1763,10 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
                          chan_ms);
     HIP_TRY(mark());
     if (n_el > 0) {
-      if (P->mlp_on_matrix_pipe)
-        hipLaunchKernelGGL(k_celo2_apply<true>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab,
-                           term_tab, gl, dec, wfold);
-      else
-        hipLaunchKernelGGL(k_celo2_apply<false>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab,
-                           term_tab, gl, dec, wfold);
+      const auto apply = in_place                ? k_celo2_apply<true, true>
+                         : P->mlp_on_matrix_pipe ? k_celo2_apply<true, false>
+                                                 : k_celo2_apply<false, false>;
+      hipLaunchKernelGGL(apply, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, term_tab, gl, dec, wfold);
     }
   }
   if (n_sl > 0)
@@ -2271,7 +2273,7 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   };
   // clip_norm is 0 for VeLO tensors: k_p0 clamps directly; its norm / flag outputs are not used
   // no global norm to wait for: the N-D tensors' sums ride in the tail blocks of the same launch
-  const bool typed = L.typed;
+  const bool typed = L.in_place;
   auto gradient_sums = [&]() {
     if (n_p0 + n_nd > 0)
       hipLaunchKernelGGL(typed ? k_p0<true> : k_p0<false>, dim3(n_p0 + n_nd), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,

@@ -1,4 +1,4 @@
-"""VeLO on 2-D tensors of 16-bit storage that its passes read and write in place (no fp32 staging).
+"""2-D tensors of 16-bit storage that the passes of VeLO and ELO-CELO2 read and write in place (no fp32 staging).
 
 Checked against the float32 step of the same class on the widened values: accumulators to rel 1e-5 / abs 1e-6, the
 parameter as that step's value rounded into the type, to one spacing (a float32 difference of an ulp can fall on the other
@@ -20,22 +20,28 @@ SETS = [
 ]
 
 
-def _run(params, grads, loss):
-    from pylo_amd import VeLO_CUDA
-    from pylo_amd.models import VeLOMLP, VeLORNN
+def _run(cls, params, grads, loss):
+    from pylo_amd import ELO_CELO2_CUDA, VeLO_CUDA
+    from pylo_amd.models import CELO2MLP, VeLOMLP, VeLORNN
 
     torch.manual_seed(1)
-    opt = VeLO_CUDA(params, lr=1.0, num_steps=100, weight_decay=0.01, rnn=VeLORNN(), mlp=VeLOMLP())
     for p, g in zip(params, grads):
         p.grad = g
-    opt.step(loss)
+    if cls == "VeLO":
+        opt = VeLO_CUDA(params, lr=1.0, num_steps=100, weight_decay=0.01, rnn=VeLORNN(), mlp=VeLOMLP())
+        opt.step(loss)
+    else:
+        opt = ELO_CELO2_CUDA(params, lr=1e-2, weight_decay=0.01, clip_grad=cls == "ELO_CELO2 clipped", clip_norm=1.0,
+                             network=CELO2MLP(), hf_key=None)
+        opt.step()
     return opt
 
 
+@pytest.mark.parametrize("cls", ["VeLO", "ELO_CELO2", "ELO_CELO2 clipped"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shapes", SETS)
 @pytest.mark.parametrize("mixed", [False, True])
-def test_step_in_place_matches_float32(shapes, dtype, mixed):
+def test_step_in_place_matches_float32(shapes, dtype, mixed, cls):
     gen = torch.Generator().manual_seed(3)
     dts = [torch.float32 if mixed and i == len(shapes) - 1 and i > 0 else dtype for i in range(len(shapes))]
     init = [(torch.randn(s, generator=gen) * 0.3).to(dt) for s, dt in zip(shapes, dts)]
@@ -43,11 +49,11 @@ def test_step_in_place_matches_float32(shapes, dtype, mixed):
     p16 = [torch.nn.Parameter(v.clone().cuda()) for v in init]
     p32 = [torch.nn.Parameter(v.float().cuda()) for v in init]
     loss = torch.tensor(2.0, device="cuda")
-    o16 = _run(p16, [g.cuda() for g in grads], loss)
-    o32 = _run(p32, [g.float().cuda() for g in grads], loss)
+    o16 = _run(cls, p16, [g.cuda() for g in grads], loss)
+    o32 = _run(cls, p32, [g.float().cuda() for g in grads], loss)
     torch.cuda.synchronize()
     for a, b, s, dt in zip(p16, p32, shapes, dts):
-        for k in ("mom", "rms", "fac_vec_row", "fac_vec_col", "fac_vec_v"):
+        for k in (k for k, v in o32.state[b].items() if torch.is_tensor(v) and v.is_cuda and k != "rank_onehot"):
             assert max_err(o16.state[a][k], o32.state[b][k].cpu(), 1e-5, 1e-6) <= 1.0, (s, k)
         got, want = a.detach().cpu(), b.detach().cpu()
         if dt == torch.float32:
