@@ -6,6 +6,7 @@
 // same for every element of a step and are folded into the first-layer bias.
 #pragma once
 
+#include "k_cast.h"
 #include "k_velo.h"
 
 namespace pylo {
@@ -61,7 +62,9 @@ __device__ __forceinline__ void adafac_stats_fac(const TDesc& d, const PyloTenso
   }
 }
 
-// Column-resident walk of one wave task (wide 2-D tensors), as in VeLO's statistics pass.
+// Column-resident walk of one wave task (wide 2-D tensors), as in VeLO's statistics pass.  ST: storage type of gradient
+// and parameter (k_cast.h).
+template <int ST>
 __device__ __forceinline__ void adafac_stats_tile(const TDesc& d, const PyloTensorArgs& a, int task,
                                                   const EmaConsts& e, const float* __restrict__ fac_tab,
                                                   VeloAcc& acc) {
@@ -72,15 +75,16 @@ __device__ __forceinline__ void adafac_stats_tile(const TDesc& d, const PyloTens
   float fb[V][4];
 #pragma unroll
   for (int v = 0; v < V; ++v) load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
-  const unsigned lo = (threadIdx.x & 63) * (V * 4u);
-  const float *g = a.grad + tk.first, *p = a.param + tk.first, *m0 = a.mom + tk.first,
-              *m1 = a.mom + d.n + tk.first, *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
+  const unsigned le = (threadIdx.x & 63) * V, lo = le * 4u;
+  typedef typename StoredAs<ST>::E E;
+  const E *g = reinterpret_cast<const E*>(a.grad) + tk.first, *p = reinterpret_cast<const E*>(a.param) + tk.first;
+  const float *m0 = a.mom + tk.first, *m1 = a.mom + d.n + tk.first, *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
   const float* fr = f0 + (size_t)tk.r0 * 4;
 #pragma unroll 2
   for (int r = tk.r0; r < tk.r1; ++r) {
     float xg[V], xp[V], x0[V], x1[V], x2[V], xr[V], fa[4];
-    load_vec_nt<V>(g, lo, xg);
-    load_vec_nt<V>(p, lo, xp);
+    load_row<V, ST, true>(g, le, xg);
+    load_row<V, ST, true>(p, le, xp);
     load_vec_nt<V>(m0, lo, x0);
     load_vec_nt<V>(m1, lo, x1);
     load_vec_nt<V>(m2, lo, x2);
@@ -124,6 +128,7 @@ __device__ __forceinline__ void adafac_stats_vec(const TDesc& d, const PyloTenso
   }
 }
 
+template <bool TYPED>
 __global__ __launch_bounds__(kThreads) void k_adafac_stats(const TDesc* __restrict__ descs,
                                                            const PyloTensorArgs* __restrict__ dyn,
                                                            const Item* __restrict__ items,
@@ -142,7 +147,11 @@ __global__ __launch_bounds__(kThreads) void k_adafac_stats(const TDesc* __restri
   for (int c = 0; c < 30; ++c) acc.ch[c] = 0.0f;
   if (d.tile_nct > 0) {
     const int task = it.a * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (task < d.tile_ntask) adafac_stats_tile(d, a, task, e, fac_tab, acc);
+    if (task < d.tile_ntask) {
+      if (TYPED && d.direct && d.store == kStoreBF16) adafac_stats_tile<kStoreBF16>(d, a, task, e, fac_tab, acc);
+      else if (TYPED && d.direct) adafac_stats_tile<kStoreF16>(d, a, task, e, fac_tab, acc);
+      else adafac_stats_tile<kStoreF32>(d, a, task, e, fac_tab, acc);
+    }
   } else if (d.mode == kModeFac2D) {
     if (d.vec == 4) adafac_stats_fac<4, false>(d, a, it.a, e, fac_tab, acc);
     else adafac_stats_fac<1, false>(d, a, it.a, e, fac_tab, acc);
@@ -592,7 +601,8 @@ __device__ __forceinline__ void adafac_hidden_out(const av16f (&h)[2], const au3
 // PER: the tensor is an (O, I, k, ..) one walked as the matrix (O, I * P) (TDesc::aper): the vector that is not
 // indexed by the column has an entry per (row, column mod P), so a lane fetches the row's factor and first-layer
 // terms for its own columns (one per element group) instead of sharing one entry with the wave.
-template <bool PER>
+// ST: storage type of gradient and parameter (k_cast.h).
+template <bool PER, int ST>
 __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloTensorArgs& a, int task,
                                                      const EmaConsts& e, const float* __restrict__ fac_tab,
                                                      const float* __restrict__ term_tab, const float* wfold_t,
@@ -651,18 +661,20 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
     for (int gq = 0; gq < 2; ++gq) trow_off[gq] += ((tk.col - lane + 32 * gq + el) % (unsigned)per) * (kAH * 4u);
   }
   const unsigned lo = lane * 4u;
-  const float* g = a.grad + tk.first;
-  float *p = a.param + tk.first, *m0 = a.mom + tk.first, *m1 = a.mom + d.n + tk.first,
+  typedef typename StoredAs<ST>::E E;
+  const E* g = reinterpret_cast<const E*>(a.grad) + tk.first;
+  E* p = reinterpret_cast<E*>(a.param) + tk.first;
+  float *m0 = a.mom + tk.first, *m1 = a.mom + d.n + tk.first,
         *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
   const float* fr = fac_tab + pick(d.fac_off, pv) + (size_t)tk.r0 * 4 * per;
   const float* tr = term_tab + pick(d.term_off, pv) + (size_t)tk.r0 * kAH * per;
   // Everything a row reads from memory.  The loop keeps one row in flight: the loads of row r + 1 are issued
   // before row r is worked on (a wave shares its SIMD with one other wave only, too few to cover a memory round
   // trip per row otherwise).
-  struct RowIn { float g[1], p[1], m0[1], m1[1], m2[1], rms[1], fa[4], ta[PER ? 2 : 1][4][4]; };
+  struct RowIn { E g, p; float m0[1], m1[1], m2[1], rms[1], fa[4], ta[PER ? 2 : 1][4][4]; };
   auto fetch = [&](RowIn& x, long long eo, const float* fr_, const float* tr_) {
-    load_vec_nt<1>(g + eo, lo, x.g);
-    load_vec_nt<1>(p + eo, lo, x.p);
+    x.g = load_raw<ST>(g + eo, lane);
+    x.p = load_raw<ST>(p + eo, lane);
     load_vec_nt<1>(m0 + eo, lo, x.m0);
     load_vec_nt<1>(m1 + eo, lo, x.m1);
     load_vec_nt<1>(m2 + eo, lo, x.m2);
@@ -682,7 +694,7 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
       const bool more = r + 1 < tk.r1;
       fetch(nxt, more ? d.C0 : 0, fr + (more ? 4 * per : 0), tr + (more ? kAH * per : 0));
     }
-    float xg[1] = {cur.g[0]}, xp[1] = {cur.p[0]}, x0[1] = {cur.m0[0]}, x1[1] = {cur.m1[0]}, x2[1] = {cur.m2[0]},
+    float xg[1] = {widen_raw<ST>(cur.g)}, xp[1] = {widen_raw<ST>(cur.p)}, x0[1] = {cur.m0[0]}, x1[1] = {cur.m1[0]}, x2[1] = {cur.m2[0]},
           xr_[1] = {cur.rms[0]};
     const float (&fa)[4] = cur.fa;
     const float (&ta)[PER ? 2 : 1][4][4] = cur.ta;
@@ -735,7 +747,7 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
     adafac_hidden_out(h, w2, bh, wo, bo0, bo1, o0, o1);
     float pn[1];
     pn[0] = adafac_update(d, a, o0 * __builtin_amdgcn_exp2f(o1 * exp_scale), xp[0]);
-    store_vec_o<1>(p, lo, pn);
+    store_row<1, ST>(p, lane, pn);
     g += d.C0; p += d.C0; m0 += d.C0; m1 += d.C0; m2 += d.C0; rms += d.C0;
     fr += 4 * per; tr += kAH * per;
     cur = nxt;
@@ -963,7 +975,8 @@ __global__ __launch_bounds__(kThreads) void k_adafac_apply(const TDesc* __restri
 
 // The apply pass for tensors walked column-resident (items hold four wave tasks each).  BF: the element MLP on
 // the fp16 matrix instructions (two-plane operands), else on the fp32 ones.
-template <bool BF, bool PER = false>
+// TYPED: plans with tensors of 16-bit storage that are read in place (TDesc::direct).
+template <bool BF, bool PER = false, bool TYPED = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BF ? 2 : PYLO_ADAFAC_WAVES)))
 void k_adafac_apply_tile(const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn,
                          const Item* __restrict__ items, const float* __restrict__ fac_tab,
@@ -979,9 +992,15 @@ void k_adafac_apply_tile(const TDesc* __restrict__ descs, const PyloTensorArgs* 
   const int task = it.a * 4 + wave;
   if (task >= d.atile_ntask) return;
   static_assert(BF || !PER, "tensors with more than two dims are walked by the fp16 variant only");
-  if constexpr (BF)
-    adafac_apply_tile_hf<PER>(d, a, task, make_ema(dec), fac_tab, term_tab, wfold + (size_t)it.tensor * kAFold, net);
-  else
+  if constexpr (BF) {
+    const float* w = wfold + (size_t)it.tensor * kAFold;
+    if (TYPED && d.direct && d.store == kStoreBF16)
+      adafac_apply_tile_hf<PER, kStoreBF16>(d, a, task, make_ema(dec), fac_tab, term_tab, w, net);
+    else if (TYPED && d.direct)
+      adafac_apply_tile_hf<PER, kStoreF16>(d, a, task, make_ema(dec), fac_tab, term_tab, w, net);
+    else
+      adafac_apply_tile_hf<PER, kStoreF32>(d, a, task, make_ema(dec), fac_tab, term_tab, w, net);
+  } else
     adafac_apply_tile(d, a, task, make_ema(dec), fac_tab, term_tab, wfold + (size_t)it.tensor * kAFold, net, xch[wave]);
 }
 

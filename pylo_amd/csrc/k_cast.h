@@ -8,12 +8,12 @@
 // to nearest-even back into the caller's buffer (k_cast_out).  Against 72 bytes per element of a factored
 // tensor this adds 18 (16-bit types) or 36 (fp64) bytes; tensors without a tag are not touched by any of it.
 //
-// 2-D tensors on the column-resident walks of VeLO and ELO-CELO2 skip the staging where they are stored in 16 bits
-// (TDesc::direct): the three passes over them take the storage type as a template argument, widen in the load and
-// (VeLO) round in the store.  Both casts less, and passes that move half the gradient's and parameter's bytes.
+// 2-D tensors on the column-resident walks skip the staging where they are stored in 16 bits (TDesc::direct): the three
+// passes over them take the storage type as a template argument, widen in the load and round in the store.  Both casts less, and passes that move half the gradient's and parameter's bytes.
 //   VeLO, 86 M bf16 elements (ViT-B/16): casts 327 us -> 15 us (what is still staged), k_p0 105 -> 59, k_velo_stats
 //     307 -> 299, k_velo_apply 694 -> 617, whole step 1.51 -> 1.04 ms
 //   ELO-CELO2, 124 M bf16 elements (GPT-2-small): whole step 7.07 -> 6.71 ms
+//   AdafacLO, 1.1 G elements (Llama-1.1B): bf16 27.1 -> 21.5 ms, fp16 27.1 -> 22.0 ms (fp32 22.8 ms)
 // every result bit for bit the same.  Linear chunks, vectors, tensors with more than two dims and fp64 stay staged.
 #pragma once
 
@@ -70,6 +70,17 @@ __device__ __forceinline__ void load_row(const typename StoredAs<ST>::E* base, u
 #pragma unroll
     for (int v = 0; v < V; ++v) x[v] = widen16(w[v], ST);
   }
+}
+// One element as it is stored, for a load that is in flight over other work: widened where it is used.
+template <int ST>
+__device__ __forceinline__ typename StoredAs<ST>::E load_raw(const typename StoredAs<ST>::E* base, unsigned off) {
+  typedef __attribute__((address_space(1))) typename StoredAs<ST>::E gE;
+  return __builtin_nontemporal_load((const gE*)((const gchar*)base + off * (unsigned)sizeof(typename StoredAs<ST>::E)));
+}
+template <int ST>
+__device__ __forceinline__ float widen_raw(typename StoredAs<ST>::E w) {
+  if constexpr (ST == kStoreF32) return w;
+  else return widen16(w, ST);
 }
 template <int V, int ST>
 __device__ __forceinline__ void store_row(typename StoredAs<ST>::E* base, unsigned off, const float (&x)[V]) {

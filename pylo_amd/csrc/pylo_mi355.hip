@@ -1063,7 +1063,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       d.tile_nct = d.C0 / kTileCols;
       d.tile_rows = tile_rows_for(kind, split);
       d.tile_ntask = d.tile_nct * ((d.R0 + d.tile_rows - 1) / d.tile_rows);
-      d.direct = kind != PYLO_KIND_ADAFAC && (d.store == kStoreF16 || d.store == kStoreBF16);
+      d.direct = (kind != PYLO_KIND_ADAFAC || env_adafac_hf()) && (d.store == kStoreF16 || d.store == kStoreBF16);
       L.in_place = L.in_place || d.direct;
       for (int b = 0; b * 4 < d.tile_ntask; ++b) L.el_items.push_back(Item{t, b, 0, 0});
     } else {
@@ -2393,6 +2393,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   const PyloDecays dec = *decays;
   VeloStep vs;
   std::memset(&vs, 0, sizeof(vs));
+  const bool in_place = L.in_place;   // tensors of 16-bit storage without staging (the fp16 matrix instructions' walk only)
   Marks mark(P, s);
 
   // ELO's global-norm clipping (ELO_cuda.py:153-161): the norm, then the exact sums where an element
@@ -2409,7 +2410,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   // without global-norm clipping the N-D tensors' sums ride in the tail blocks of the first launch
   const int n_tail = clips ? 0 : n_nd;
   if (n_p0 + n_tail > 0)
-    hipLaunchKernelGGL(k_p0<false>, dim3(n_p0 + n_tail), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
+    hipLaunchKernelGGL(in_place ? k_p0<true> : k_p0<false>, dim3(n_p0 + n_tail), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
                        nd_items, n_p0);
   if (clips && L.tensor_norm) {
     // every tensor against its own norm (AdafacLO_naive.py:199-200): no clamp on such tensors, no exact pass
@@ -2418,7 +2419,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
     const bool exact_pass = exact_pass_possible(P, args);
     hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, gsq, flag, n_p0, gl, exact_pass ? 1 : 0, (int*)nullptr, 0);
     if (n_p0 > 0 && exact_pass)
-      hipLaunchKernelGGL(k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
+      hipLaunchKernelGGL(in_place ? k_p0<true> : k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
                          (const Item*)nullptr, n_p0);
   }
   HIP_TRY(mark());
@@ -2433,7 +2434,9 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
     hipLaunchKernelGGL(k_v0b<kAH>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, v0part, 1e-5f,
                        net + kAW1, (const float*)bias_eff, kAH, fac_tab, term_tab, bscale);
   HIP_TRY(mark());
-  if (n_el > 0) hipLaunchKernelGGL(k_adafac_stats, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, dec, stats, gl);
+  if (n_el > 0)
+    hipLaunchKernelGGL(in_place ? k_adafac_stats<true> : k_adafac_stats<false>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn,
+                       el_items, fac_tab, dec, stats, gl);
   HIP_TRY(mark());
   const Item* seg_items = P->at<Item>(L.off_seg_items);
   double* seg_tot = P->at<double>(L.off_segtot);
@@ -2459,12 +2462,10 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
     hipLaunchKernelGGL((k_adafac_apply_tile<true, true>), dim3(n_pp), dim3(kThreads), 0, s, descs, dyn, pp_items, fac_tab,
                        term_tab, dec, wfold, net, gl);
   if (n_ap > 0) {
-    if (P->adafac_hf)
-      hipLaunchKernelGGL(k_adafac_apply_tile<true>, dim3(n_ap), dim3(kThreads), 0, s, descs, dyn, ap_items, fac_tab,
-                         term_tab, dec, wfold, net, gl);
-    else
-      hipLaunchKernelGGL(k_adafac_apply_tile<false>, dim3(n_ap), dim3(kThreads), 0, s, descs, dyn, ap_items, fac_tab,
-                         term_tab, dec, wfold, net, gl);
+    const auto apply = in_place       ? k_adafac_apply_tile<true, false, true>
+                       : P->adafac_hf ? k_adafac_apply_tile<true, false, false>
+                                      : k_adafac_apply_tile<false, false, false>;
+    hipLaunchKernelGGL(apply, dim3(n_ap), dim3(kThreads), 0, s, descs, dyn, ap_items, fac_tab, term_tab, dec, wfold, net, gl);
   }
   HIP_TRY(mark());
   mark.done();

@@ -1,4 +1,4 @@
-"""2-D tensors of 16-bit storage that the passes of VeLO and ELO-CELO2 read and write in place (no fp32 staging).
+"""2-D tensors of 16-bit storage that the passes of VeLO, ELO-CELO2 and AdafacLO read and write in place (no fp32 staging).
 
 Checked against the float32 step of the same class on the widened values: accumulators to rel 1e-5 / abs 1e-6, the
 parameter as that step's value rounded into the type, to one spacing (a float32 difference of an ulp can fall on the other
@@ -21,8 +21,8 @@ SETS = [
 
 
 def _run(cls, params, grads, loss):
-    from pylo_amd import ELO_CELO2_CUDA, VeLO_CUDA
-    from pylo_amd.models import CELO2MLP, VeLOMLP, VeLORNN
+    from pylo_amd import ELO_CELO2_CUDA, AdafacLO_CUDA, VeLO_CUDA
+    from pylo_amd.models import CELO2MLP, MetaMLP, VeLOMLP, VeLORNN
 
     torch.manual_seed(1)
     for p, g in zip(params, grads):
@@ -30,6 +30,10 @@ def _run(cls, params, grads, loss):
     if cls == "VeLO":
         opt = VeLO_CUDA(params, lr=1.0, num_steps=100, weight_decay=0.01, rnn=VeLORNN(), mlp=VeLOMLP())
         opt.step(loss)
+    elif cls.startswith("AdafacLO"):
+        opt = AdafacLO_CUDA(params, lr=1.0, weight_decay=0.01, max_grad_norm=0.5 if "clipped" in cls else None,
+                            network=MetaMLP(39, 32, 1))
+        opt.step()
     else:
         opt = ELO_CELO2_CUDA(params, lr=1e-2, weight_decay=0.01, clip_grad=cls == "ELO_CELO2 clipped", clip_norm=1.0,
                              network=CELO2MLP(), hf_key=None)
@@ -37,7 +41,7 @@ def _run(cls, params, grads, loss):
     return opt
 
 
-@pytest.mark.parametrize("cls", ["VeLO", "ELO_CELO2", "ELO_CELO2 clipped"])
+@pytest.mark.parametrize("cls", ["VeLO", "ELO_CELO2", "ELO_CELO2 clipped", "AdafacLO", "AdafacLO clipped"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shapes", SETS)
 @pytest.mark.parametrize("mixed", [False, True])
