@@ -520,7 +520,9 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
   L.ns_of_tensor.assign(T, -1);
   L.ns_group_of_tensor.assign(T, -1);
   L.small_of_tensor.assign(T, 0);
-  const bool small = L.ns_hf && env_ns_small();
+  // Chains of other lengths than pairs and singles, where the environment asks for them, are the tiled products' only.
+  const char* chains = getenv("PYLO_MI355_NS_CHAINS");
+  const bool small = L.ns_hf && env_ns_small() && !(chains && chains[0]) && !ns_adaptive();
   auto take = [&](long long n) { const long long o = ws_floats; ws_floats += (n + 63) / 64 * 64; return o; };
   for (int t = 0; t < T; ++t) {
     const TDesc& d = L.descs[t];
@@ -1851,8 +1853,8 @@ int enqueue_small(PyloPlan* P, hipStream_t s, const TDesc* descs, const PyloTens
     st.prod_t = pow2(-(ex.a + ex.b)); st.prod_a = pow2(-(ex.b + ex.t)); st.prod_q = pow2(-2 * ex.b);
     st.upd_b = pow2(-(ex.x + ex.b)); st.upd_q = pow2(-(ex.x + q2));
     st.c0 = coeffs[0]; st.c1 = coeffs[1]; st.c2 = coeffs[2]; st.eps = ns_eps;
-    // pairs, also where the environment asks for longer chains or a choice per matrix (which trade accuracy for
-    // the products over the long dim that small matrices do not have); single iterations where it asks for those
+    // pairs, or single iterations where the environment asks for those (plans made while it asks for other chains have no
+    // small matrices)
     st.n_pairs = ns_iters / 2;
     const std::vector<int> chains = ns_chains(ns_iters);
     if (*std::max_element(chains.begin(), chains.end()) == 1) st.n_pairs = 0;

@@ -1,0 +1,33 @@
+"""Which launches take a plan's small matrices, seen in the workspace that a plan asks for (no GPU needed).
+
+A matrix that goes through the tiled products has operand planes and tile tables there, one that goes aside (k_ns_small.h)
+partial sums: 2 x blocks x (32, 64 or 128)^2 floats, the edge being that of the class it runs in."""
+
+import ctypes as C
+
+import pytest
+
+from pylo_amd import _lib
+
+
+def _bytes(shapes):
+    lib = _lib.load()
+    arr = (_lib.TensorShape * len(shapes))()
+    for i, s in enumerate(shapes):
+        arr[i].ndim = len(s)
+        for d, v in enumerate(s):
+            arr[i].shape[d] = v
+    n = C.c_size_t()
+    assert lib.pylo_mi355_plan_workspace_bytes(_lib.KIND_CELO2, arr, len(shapes), C.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("name,value", [("PYLO_MI355_NS_CHAINS", "3,2"), ("PYLO_MI355_NS_ADAPTIVE", "1")])
+def test_other_chain_lengths_reach_small_matrices(name, value, monkeypatch):
+    """Chains other than pairs and singles are the tiled products': a plan made while the environment asks for them has no
+    small launches."""
+    shapes = [(128, 784), (128, 128), (10, 128)]
+    monkeypatch.setenv(name, value)
+    asked = _bytes(shapes)
+    monkeypatch.setenv("PYLO_MI355_NS_SMALL", "0")
+    assert asked == _bytes(shapes)
