@@ -24,8 +24,8 @@
 // (norm, three Gram products, RMS), leaving their partial sums in the workspace and adding all of them in slab order.
 // Blocks wait for blocks of their own matrix only.  The wait ends: a block draws its place in the item table when it
 // starts, so that of all matrices with a block running at most one still has blocks to start -- as many as wait in
-// it, and no more than an eighth of what the chip holds (kSlabsMax), so that the launches that four hardware queues can
-// run at once never fill it with them; all others have their blocks running, end, and make room.  After
+// it, at most 64, 32 or 8 by class of the 2048, 512 or 256 that the chip holds (kSlabsMax), so that the launches that four
+// hardware queues can run at once never fill it with them; all others have their blocks running, end, and make room.  After
 // kSpinLimit polls a block gives up and leaves NaN in its part of the parameter.
 // Measured: the kernel is a chain on one CU -- on 128 x 784 (seven blocks, 92 us) five products of an m x m pair phase
 // take 13.7 us of which the matrix instructions are 1.3 us each, a meeting with its partial sums 8.5 us, a Gram or

@@ -461,15 +461,29 @@ bool ns_small_takes(int R, int C) {
 
 // Slabs (blocks) of each small matrix and the items of the launches.
 void build_small_items(Layout& L) {
-  // what a launch of the class holds at a time on 256 CUs (LDS), and an eighth of it: see k_ns_small.h
+  // what a launch of the class holds at a time on 256 CUs (LDS), and the most blocks one matrix may have waiting
+  // (k_ns_small.h)
   constexpr int kHolds[kNsSmallClasses] = {2048, 512, 256}, kSlabsMax[kNsSmallClasses] = {64, 32, 8};
   auto cls_of = [](const NsSmall& b) { return ns_small_class(b.m); };
   int lift[kNsSmallClasses] = {0, 1, 2};
-  // A plan with few small matrices takes them all in the class of the largest, one launch: the small ones end under it.
+  // A plan with few small matrices takes them in the class of the largest, one launch: the small ones end under it,
+  // unless the fewer and larger blocks of that class walk more than eight chunks each, what its own longest matrix walks
+  // (a chunk is 15 to 25 us of a block's chain).  Whole steps, a class of 65 x 65 or 100 x 100 next to others, lifted /
+  // in their own classes: 784 -> 128 -> 128 -> 10 148 / 177 us, 784 -> 64 (x 4) -> 10 112 / 121, twenty of 64 x 8192 (eight
+  // chunks) 548 / 613; 16 x 65536 (64 chunks) 1028 / 397, 64 x 32768 (32) 1092 / 405, 63 of 16 x 65536 (126) 4319 / 3000.
   if ((int)L.sm_mats.size() <= 64) {
     int top = 0;
     for (const NsSmall& b : L.sm_mats) top = std::max(top, cls_of(b));
-    for (int& c : lift) c = top;
+    const int nb = ns_small_chunk(top);
+    for (int c = top - 1; c >= 0; --c) {
+      long long total = 0, most = 0;
+      for (const NsSmall& b : L.sm_mats) {
+        if (lift[cls_of(b)] != top && cls_of(b) != c) continue;
+        total += (b.n + nb - 1) / nb;
+        if (cls_of(b) == c) most = std::max<long long>(most, (b.n + nb - 1) / nb);
+      }
+      if (std::max(total / kHolds[top], (most + kSlabsMax[top] - 1) / kSlabsMax[top]) <= 8) lift[c] = top;
+    }
   }
   for (int cls = 0; cls < kNsSmallClasses; ++cls) {
     std::vector<int> of;
@@ -481,7 +495,7 @@ void build_small_items(Layout& L) {
         of.push_back(q);
         total += chunks(q);
       }
-    // one slab a chunk while the launch's blocks all run at once, longer ones when there are more
+    // one slab a chunk while no more blocks are started than twice what runs at once, longer ones when there are more
     const int per = (int)std::max<long long>(1, total / kHolds[cls]);
     for (int q : of) {
       NsSmall& b = L.sm_mats[q];

@@ -31,3 +31,10 @@ def test_other_chain_lengths_reach_small_matrices(name, value, monkeypatch):
     asked = _bytes(shapes)
     monkeypatch.setenv("PYLO_MI355_NS_SMALL", "0")
     assert asked == _bytes(shapes)
+
+
+@pytest.mark.parametrize("longs", [[(16, 65536)], [(65536, 9)], [(16, 65536)] * 20])
+def test_long_thin_matrices_keep_their_class(longs):
+    """Next to one 100 x 100 their blocks and partial sums are those that they have without it (64 x 32^2 floats, twice; the
+    largest class would give them 8 x 128^2)."""
+    assert _bytes(longs + [(100, 100)]) - _bytes(longs) <= _bytes([(100, 100)])
