@@ -440,6 +440,21 @@ bool env_ns_small() {
   return !(e && e[0] == '0');
 }
 
+// The products of an m x n matrix in the unit of the rules below: five iterations in pairs are three Gram products on
+// the upper blocks, three updates and eleven m x m products.
+double ns_work(int m, int n) { return (double)m * m * (4.6 * n + 5.9 * m); }
+
+// Into how many groups (streams) the matrices of a plan are dealt: as many as have eight of its matrices each, those that
+// go aside to k_ns_small counted (which launch takes them says nothing about the others), and 55 G of work each.  Below that a
+// group's launches are bound by their number, and more streams only add to it.  Whole steps, 1 / 2 / 3 groups (one
+// decoder layer of width 256, 384, 512, 1024: 1.3, 4.3, 10, 82 G; two embeddings of 4000 rows: 2.6, 6, 11, 50 G):
+//   width 256, 12 layers (18 G) 856 / 903 / 957 us      384, 8 layers (43 G) 1294 / 1293 / 1331, 12 (60 G) 1667 / 1593 / 1648
+//   512, 4 layers (52 G) 1244 / 1291 / 1331, 6 (72 G) 1691 / 1621 / 1633, 8 (93 G) 2057 / 1896 / 1945, 12 (133 G) 2551 / 2446 / 2405
+//   1024, 2 layers (210 G) 2799 / 2547 / 2542, 3 layers 3367 / 3103 / 3091 us
+int ns_group_count(int mats, double work) {
+  return (int)std::min<double>(std::min(env_ns_groups(), std::max(mats / 8, 1)), 1.0 + std::floor(work / 55e9));
+}
+
 using SmSmall = SmDims<1, 1, 2>;
 using SmMid = SmDims<2, 1, 2>;
 using SmLarge = SmDims<4, 2, 1>;
@@ -457,6 +472,24 @@ bool ns_small_takes(int R, int C) {
   const int m = std::min(R, C), n = std::max(R, C);
   if (m > SmLarge::MP) return false;
   return n <= (m <= 16 ? 65536 : m <= SmMid::MP ? 32768 : 8192);
+}
+
+// Whether a plan's small matrices go aside to their own launches, or with the larger ones through the tiled launches that
+// run anyway.  Aside they cost a fork and a join (10 us and more of a chain on one stream) and, in the largest class, a CU
+// a block; in the tiled launches they are a few more tiles, free while the launches leave CUs idle.  So they stay with larger
+// matrices that are one group, if these are less than 22 G of work (or the small one is alone) and the small ones add
+// no more than 512 update tiles, two a CU.  Whole steps, tiled / aside:
+//   classifier 784 -> 1024 -> 1024 -> 10 (17 G) 978 / 1013 us, 784 -> 384 -> 384 -> 10 477 / 508, 784 -> 2048 (x 4) -> 10
+//     (280 G, one small) 3144 / 3171
+//   one 512 x 512 (1.4 G) and 8, 32, 64 of 16 x 1024 564 / 580, 582 / 643, 652 / 708
+//   decoder of width 256 with k, v of 32, 1, 4, 12 layers 530 / 543, 576 / 583, 858 / 867; width 384, 48, 1 layer 643 / 677
+//   four 1024 x 1024 (44 G) and 8, 16, 64 of 16 x 1024 1118 / 1092, 1144 / 1107, 1458 / 1202
+//   two 1024 x 1024 (22 G) and 4, 16 of 64 x 2000 979 / 956, 1026 / 1013
+//   decoder of width 512 with k, v of 64 (32 G) 994 / 987, 8 layers (93 G, two groups) 1896 / 1877
+//   three thousand odd tensors (1720 small matrices) 4.35 / 2.79 ms
+bool ns_small_aside(int n_large, double work_large, int n_small, long long small_tiles) {
+  if (n_large == 0 || small_tiles > 512 || ns_group_count(n_large + n_small, work_large) > 1) return true;
+  return n_small > 1 && work_large >= 22e9;
 }
 
 // Slabs (blocks) of each small matrix and the items of the launches.
@@ -534,22 +567,44 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
   L.ns_of_tensor.assign(T, -1);
   L.ns_group_of_tensor.assign(T, -1);
   L.small_of_tensor.assign(T, 0);
-  // Chains of other lengths than pairs and singles, where the environment asks for them, are the tiled products' only.
-  const char* chains = getenv("PYLO_MI355_NS_CHAINS");
-  const bool small = L.ns_hf && env_ns_small() && !(chains && chains[0]) && !ns_adaptive();
   auto take = [&](long long n) { const long long o = ws_floats; ws_floats += (n + 63) / 64 * 64; return o; };
-  for (int t = 0; t < T; ++t) {
+  // The matrices of a tensor: R x C, n_sl of them; none if the products do not take it.
+  auto matrices = [&](int t, int& R, int& C, int& n_sl) {
     const TDesc& d = L.descs[t];
-    if (d.n == 0 || (shapes[t].flags & PYLO_F_NO_ORTHOGONALIZE)) continue;
+    if (d.n == 0 || (shapes[t].flags & PYLO_F_NO_ORTHOGONALIZE)) return false;
     // two dims; or more, as one matrix per slice of the last two, where the per-slice launches do not take the
     // slices (k_slice_finish.h) -- the split-fp16 kernels only, whose tables carry a matrix's place in its tensor
     const bool slices = d.mode == kModeFacND && L.ns_hf && L.slice_of_tensor[t] < 0;
-    if (d.mode != kModeFac2D && !slices) continue;
-    const int R = slices ? (int)shapes[t].shape[shapes[t].ndim - 2] : d.R0;
-    const int C = slices ? (int)shapes[t].shape[shapes[t].ndim - 1] : d.C0;
+    if (d.mode != kModeFac2D && !slices) return false;
+    R = slices ? (int)shapes[t].shape[shapes[t].ndim - 2] : d.R0;
+    C = slices ? (int)shapes[t].shape[shapes[t].ndim - 1] : d.C0;
     // the fp32 kernels load 16 bytes at a time along the contiguous dim of X, A and B'
-    if (!L.ns_hf && (C % 4 != 0 || std::min(R, C) % 4 != 0)) continue;
-    const int n_sl = slices ? (int)(d.n / ((long long)R * C)) : 1;
+    if (!L.ns_hf && (C % 4 != 0 || std::min(R, C) % 4 != 0)) return false;
+    n_sl = slices ? (int)(d.n / ((long long)R * C)) : 1;
+    return true;
+  };
+  int R = 0, C = 0, n_sl = 0;
+  // Chains of other lengths than pairs and singles, where the environment asks for them, are the tiled products' only.
+  const char* chains = getenv("PYLO_MI355_NS_CHAINS");
+  bool small = L.ns_hf && env_ns_small() && !(chains && chains[0]) && !ns_adaptive();
+  if (small) {
+    int n_large = 0, n_small = 0;
+    double work = 0.0;
+    long long tiles = 0;
+    for (int t = 0; t < T; ++t) {
+      if (!matrices(t, R, C, n_sl)) continue;
+      if (ns_small_takes(R, C)) {
+        n_small += n_sl;
+        tiles += (long long)n_sl * ((std::max(R, C) + kNsTile - 1) / kNsTile);
+      } else {
+        n_large += n_sl;
+        work += n_sl * ns_work(std::min(R, C), std::max(R, C));
+      }
+    }
+    small = ns_small_aside(n_large, work, n_small, tiles);
+  }
+  for (int t = 0; t < T; ++t) {
+    if (!matrices(t, R, C, n_sl)) continue;
     if (small && ns_small_takes(R, C)) {
       L.small_of_tensor[t] = 1;
       for (int sl = 0; sl < n_sl; ++sl) {
@@ -704,8 +759,12 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
     L.ns_flag_items.clear();
     L.ns_fpart_total = 0;
     for (NsBatch& bt : L.ns_batches) {
-    // (one of the four hardware queues is left to the small matrices where there are any)
-    const int n_groups = std::min<int>(L.sm_mats.empty() ? env_ns_groups() : std::min(env_ns_groups(), 3), std::max(bt.n_mats / 8, 1));
+    double batch_work = 0.0;
+    for (int q = bt.mat0; q < bt.mat0 + bt.n_mats; ++q) batch_work += ns_work(L.nsb_mats[q].m, L.nsb_mats[q].n);
+    // (one of the four hardware queues is left to the small matrices where there are any: 3 / 4 groups next to them, 1024
+    // wide 8117 / 8162 us, 512 wide 3203 / 3281)
+    const int n_groups = std::min({L.sm_mats.empty() ? 4 : 3, bt.n_mats,
+                                   ns_group_count(bt.n_mats + (int)L.sm_mats.size(), batch_work)});
     std::vector<std::vector<int>> members(n_groups);
     {
       // (tensor by tensor: the slices of a tensor with more than two dims share a group, which also finishes it)
@@ -713,8 +772,7 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
       std::vector<Run> runs;
       for (int q = bt.mat0; q < bt.mat0 + bt.n_mats; ++q) {
         const NsHfMat& b = L.nsb_mats[q];
-        // (five iterations in pairs: three Gram products on the upper blocks and three updates, eleven m x m products)
-        const double w = (double)b.m * b.m * (4.6 * b.n + 5.9 * b.m);
+        const double w = ns_work(b.m, b.n);
         if (!runs.empty() && L.nsb_mats[runs.back().q0].tensor == b.tensor) { runs.back().q1 = q + 1; runs.back().work += w; }
         else runs.push_back(Run{q, q + 1, w});
       }

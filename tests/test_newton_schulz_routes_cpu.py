@@ -22,6 +22,38 @@ def _bytes(shapes):
     return n.value
 
 
+def _decoder(width, kv, layers):
+    return [(width, width), (width, kv), (width, kv), (width, width), (width, 3 * width)] * layers
+
+
+# few small matrices next to one group of larger ones ride with them: the plan is the one that has no small launches
+@pytest.mark.parametrize("shapes", [
+    [(1024, 784), (1024, 1024), (10, 1024)],
+    [(384, 784), (384, 384), (10, 384)],
+    [(512, 512)] + [(16, 1024), (1024, 16)] * 8,
+    _decoder(256, 32, 3),
+], ids=["classifier 1024", "classifier 384", "adapters beside one matrix", "decoder 256"])
+def test_small_matrices_ride_with_larger_ones(shapes, monkeypatch):
+    monkeypatch.delenv("PYLO_MI355_NS_SMALL", raising=False)
+    default = _bytes(shapes)
+    monkeypatch.setenv("PYLO_MI355_NS_SMALL", "0")
+    assert default == _bytes(shapes)
+
+
+# no larger ones, many small ones, or larger ones with launches that fill the chip: aside
+@pytest.mark.parametrize("shapes", [
+    [(128, 784), (128, 128), (10, 128)],
+    [(512, 512)] + [(60, 100)] * 600,
+    [(1024, 1024)] * 4 + [(16, 1024), (1024, 16)] * 8,
+    _decoder(512, 64, 8),
+], ids=["classifier 128", "many", "adapters beside four matrices", "decoder 512"])
+def test_small_matrices_aside(shapes, monkeypatch):
+    monkeypatch.delenv("PYLO_MI355_NS_SMALL", raising=False)
+    default = _bytes(shapes)
+    monkeypatch.setenv("PYLO_MI355_NS_SMALL", "0")
+    assert default != _bytes(shapes)
+
+
 @pytest.mark.parametrize("name,value", [("PYLO_MI355_NS_CHAINS", "3,2"), ("PYLO_MI355_NS_ADAPTIVE", "1")])
 def test_other_chain_lengths_reach_small_matrices(name, value, monkeypatch):
     """Chains other than pairs and singles are the tiled products': a plan made while the environment asks for them has no
