@@ -550,6 +550,32 @@ __device__ __forceinline__ av16f hf2_mfma(const au32x4 (&w)[2], const au32x4 (&x
   return acc;
 }
 
+// Output layer of the two groups of 32 elements a wave holds, from the hidden layer's sums `g2` (D layout): the two outputs
+// of the lane's own element.
+__device__ __forceinline__ void adafac_output(const av16f (&g2)[2], const float (&wo)[16][2], float bo0, float bo1, float& o0,
+                                              float& o1) {
+  float part[2][2];
+#pragma unroll
+  for (int gq = 0; gq < 2; ++gq) {
+    float p0 = 0.0f, p1 = 0.0f;
+#pragma unroll
+    for (int r2 = 0; r2 < 16; ++r2) {
+      const float gv = relu(g2[gq][r2]);
+      p0 = fmaf(gv, wo[r2][0], p0);
+      p1 = fmaf(gv, wo[r2][1], p1);
+    }
+    part[gq][0] = p0;
+    part[gq][1] = p1;
+  }
+  // a lane's element belongs to group `half`; its other 16 units sit 32 lanes away
+  unsigned a0 = __float_as_uint(part[0][0]), b0 = __float_as_uint(part[1][0]);
+  unsigned a1 = __float_as_uint(part[0][1]), b1 = __float_as_uint(part[1][1]);
+  half_swap(a0, b0);
+  half_swap(a1, b1);
+  o0 = (__uint_as_float(a0) + __uint_as_float(b0)) + bo0;
+  o1 = (__uint_as_float(a1) + __uint_as_float(b1)) + bo1;
+}
+
 // Hidden and output layer of the two groups of 32 elements a wave holds, from the first layer's sums `h` (D layout):
 // the two outputs of the lane's own element.
 __device__ __forceinline__ void adafac_hidden_out(const av16f (&h)[2], const au32x4 (&w2)[2][2], const av16f& bh,
@@ -576,26 +602,7 @@ __device__ __forceinline__ void adafac_hidden_out(const av16f (&h)[2], const au3
       g2[gq] = hf2_mfma(w2[s2], hb, g2[gq]);
     }
   }
-  float part[2][2];
-#pragma unroll
-  for (int gq = 0; gq < 2; ++gq) {
-    float p0 = 0.0f, p1 = 0.0f;
-#pragma unroll
-    for (int r2 = 0; r2 < 16; ++r2) {
-      const float gv = relu(g2[gq][r2]);
-      p0 = fmaf(gv, wo[r2][0], p0);
-      p1 = fmaf(gv, wo[r2][1], p1);
-    }
-    part[gq][0] = p0;
-    part[gq][1] = p1;
-  }
-  // a lane's element belongs to group `half`; its other 16 units sit 32 lanes away
-  unsigned a0 = __float_as_uint(part[0][0]), b0 = __float_as_uint(part[1][0]);
-  unsigned a1 = __float_as_uint(part[0][1]), b1 = __float_as_uint(part[1][1]);
-  half_swap(a0, b0);
-  half_swap(a1, b1);
-  o0 = (__uint_as_float(a0) + __uint_as_float(b0)) + bo0;
-  o1 = (__uint_as_float(a1) + __uint_as_float(b1)) + bo1;
+  adafac_output(g2, wo, bo0, bo1, o0, o1);
 }
 
 // PER: the tensor is an (O, I, k, ..) one walked as the matrix (O, I * P) (TDesc::aper): the vector that is not
@@ -754,30 +761,60 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
   }
 }
 
-// ---- the same for every other tensor: 64 consecutive elements a wave and trip ------------------------------
+// ---- every other tensor: 64 consecutive elements a wave and trip -----------------------------------------
 // Tensors that no column-resident walk takes -- rows that are not a multiple of 64 long, more than two dims with
-// other factored dims, fewer than two dims -- are taken in storage order, element `base + 256 trip + thread`, with
-// the element MLP on the matrix pipe exactly as above.  What differs is where the factors and first-layer terms
-// come from: every lane works out the two table entries of its two elements (e of either group of 32; its own is
-// one of them) and fetches them, 16 bytes a load, out of tables that stay in the L2.  A lane past the end works on
-// the tensor's last element and stores nothing.
+// other factored dims, fewer than two dims -- are taken in storage order, element `base + 256 trip + thread`.  The element
+// MLP has the layouts of the walk above, on the folded fp32 weights and the features as they are, and every operand
+// is three bfloat16 planes: rounded, what is left rounded, and the rest, which is exact -- all 24 bits of an fp32 number over
+// its whole range, nothing scaled or clamped.  Six of the nine products of planes are taken (v_mfma_f32_32x32x16_bf16);
+// the others are below 2^-25 of a product together, half of what one fp32 rounding of it may be.  In fp32 throughout for all
+// that can be seen of it: against fp64 no further off than the all-VALU kernel (AdafacLO's linear-apply test).
+// The factors and first-layer terms: every lane works out the two table entries of its two elements (e of either group
+// of 32; its own is one of them) and fetches them, 16 bytes a load, out of tables that stay in the L2.  A lane past the end
+// works on the tensor's last element and stores nothing.
 // K: kModeFac2D, kModeFacND, or kModeVec.  A tensor with fewer than two dims has 28 features of its own and no
 // terms: two reduction steps of 16 slots for the first layer (four slots empty) and the effective bias instead.
-// Bound by latency on the small tensors that come here and by vector instructions on large ones.  The all-VALU
-// kernel that it replaces on the matrix-pipe plans read the 1 600 weights of an element row by row through the
-// scalar cache, 32 dependent trips of it over 8 192 elements a block.  Whole steps: the 118 000-parameter classifier
-// (784 -> 128 -> 128 -> 10, ELO) 285 -> 88 us, its apply launch 207 us before; ResNet-50's set (AdafacLO: 161 tensors,
-// the vectors, the stem and the 1 x 1 kernels of 64 x 64 come here) 792 -> 729 us.
+// Bound by latency on the small tensors that come here and by vector instructions (features, planes) on large ones.
+// Whole AdafacLO steps, all-VALU kernel / fp32 matrix instructions (32x32x2) / three planes: transformer of width 700
+// 2.85 / 2.32 / 1.89 ms, of width 701 2.35 / 1.86 / 1.54, vectors of 30 M elements 2.14 / 1.38 / 1.09; classifier 784 -> 128 ->
+// 128 -> 10 290 / 85 / 85 us.  (Two fp16 planes, 23 bits, are faster by a tenth and less accurate than fp32: 1.70, 1.40, 0.86.)
+typedef __bf16 ab16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 ab16x8 __attribute__((ext_vector_type(8)));
+
+// eight values (consecutive inputs of a matrix operand) as three planes of eight bfloat16
+__device__ __forceinline__ void bf3_pack8(const float (&x)[8], au32x4 (&pl)[3]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a = x[2 * i], b = x[2 * i + 1];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(af32x2{a, b}, ab16x2));
+      pl[q][i] = h;
+      a -= __uint_as_float(h << 16);
+      b -= __uint_as_float(h & 0xffff0000u);
+    }
+  }
+}
+
+// acc += W (three planes) x act (three planes), smallest terms first
+__device__ __forceinline__ av16f bf3_mfma(const au32x4 (&w)[3], const au32x4 (&x)[3], av16f acc) {
+  constexpr int pw[6] = {2, 0, 1, 1, 0, 0}, px[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+  for (int t = 0; t < 6; ++t)
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(ab16x8, w[pw[t]]), __builtin_bit_cast(ab16x8, x[px[t]]),
+                                                  acc, 0, 0, 0);
+  return acc;
+}
+
 template <int K>
-__device__ __forceinline__ void adafac_apply_lin_hf(const TDesc& d, const PyloTensorArgs& a, long long base, int trips,
-                                                    const EmaConsts& e, const PyloDecays& dec,
-                                                    const float* __restrict__ fac_tab,
-                                                    const float* __restrict__ term_tab, const float* wfold_t,
-                                                    const float* net, const float* bias_eff) {
+__device__ __forceinline__ void adafac_apply_lin(const TDesc& d, const PyloTensorArgs& a, long long base, int trips,
+                                                 const EmaConsts& e, const PyloDecays& dec,
+                                                 const float* __restrict__ fac_tab, const float* __restrict__ term_tab,
+                                                 const float* wfold_t, const float* net, const float* bias_eff) {
   constexpr bool VEC = K == kModeVec;
   constexpr int S = VEC ? 2 : 1;       // reduction steps of the first layer
   const int lane = threadIdx.x & 63, half = lane >> 5, el = lane & 31;
-  au32x4 w1[S][2], w2[2][2];
+  au32x4 w1[S][3], w2[2][3];
   {
     float x[8];
 #pragma unroll
@@ -787,23 +824,17 @@ __device__ __forceinline__ void adafac_apply_lin_hf(const TDesc& d, const PyloTe
         const int c = 16 * s + 8 * half + i;
         // a vector's feature c is channel c of the 30 without 1 and 14
         const int row = VEC ? (c < 1 ? 0 : c < 13 ? c + 1 : c + 2) : adafac_elem_row(c);
-        x[i] = (VEC && c >= 28) ? 0.0f : *(const gfloat*)(net + kAW1 + row * kAH + el);
+        x[i] = (VEC && c >= 28) ? 0.0f : *(const gfloat*)(wfold_t + row * kAH + el);
       }
-      hf2_pack8(x, w1[s]);
+      bf3_pack8(x, w1[s]);
     }
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
 #pragma unroll
       for (int i = 0; i < 8; ++i)
         x[i] = *(const gfloat*)(net + kAWH + (8 * (2 * s + (i >> 2)) + 4 * half + (i & 3)) * kAH + el);
-      hf2_pack8(x, w2[s]);
+      bf3_pack8(x, w2[s]);
     }
-  }
-  float fsc[VEC ? 30 : 16];   // the normalisers of the features, by channel (vectors) or by feature
-  {
-    const cfloat* sc = launder(wfold_t + 30 * kAH);
-#pragma unroll
-    for (int c = 0; c < (VEC ? 30 : 16); ++c) fsc[c] = sc[VEC ? c : adafac_elem_row(c)];
   }
   av16f bh, b1;
   float wo[16][2];
@@ -817,7 +848,6 @@ __device__ __forceinline__ void adafac_apply_lin_hf(const TDesc& d, const PyloTe
   }
   const cfloat* nw = launder(net);
   const float bo0 = nw[kABO + 0], bo1 = nw[kABO + 1];
-  const float exp_scale = a.exp_mult * 1.44269504088896341f;
   const long long n = d.n;
   const unsigned last = (unsigned)(n - 1);     // n < 2^31
   const unsigned wave0 = (unsigned)base + (threadIdx.x & ~63u);
@@ -864,7 +894,7 @@ __device__ __forceinline__ void adafac_apply_lin_hf(const TDesc& d, const PyloTe
       int q = 0;
 #pragma unroll
       for (int c = 0; c < 30; ++c)
-        if (adafac_channel(c)) f[q++] = f30[c] * fsc[c];
+        if (adafac_channel(c)) f[q++] = f30[c];
 #pragma unroll
       for (; q < 16 * S; ++q) f[q] = 0.0f;
       h[0] = b1;
@@ -896,7 +926,7 @@ __device__ __forceinline__ void adafac_apply_lin_hf(const TDesc& d, const PyloTe
       const float fx[16] = {f18[0], f18[2], f18[3], f18[4], f18[5], f18[6], f18[7], f18[8], f18[9], f18[10],
                             f18[11], f18[12], f18[13], f18[15], f18[16], f18[17]};
 #pragma unroll
-      for (int c = 0; c < 16; ++c) f[c] = fx[c] * fsc[c];
+      for (int c = 0; c < 16; ++c) f[c] = fx[c];
     }
     if (w0 + lane <= last) {
       const unsigned u = w0 + lane;
@@ -917,16 +947,29 @@ __device__ __forceinline__ void adafac_apply_lin_hf(const TDesc& d, const PyloTe
         flo[i] = __uint_as_float(x);
         fhi[i] = __uint_as_float(y);
       }
-      au32x4 xb[2];
-      hf2_pack8(flo, xb);
-      h[0] = hf2_mfma(w1[s], xb, h[0]);
-      hf2_pack8(fhi, xb);
-      h[1] = hf2_mfma(w1[s], xb, h[1]);
+      au32x4 xb[3];
+      bf3_pack8(flo, xb);
+      h[0] = bf3_mfma(w1[s], xb, h[0]);
+      bf3_pack8(fhi, xb);
+      h[1] = bf3_mfma(w1[s], xb, h[1]);
     }
+    av16f g2[2] = {bh, bh};
+#pragma unroll
+    for (int gq = 0; gq < 2; ++gq)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        // registers 8 s .. 8 s + 7 are the lane's eight slots of reduction step s as they stand
+        float x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = __builtin_amdgcn_fmed3f(h[gq][8 * s + i], 0.0f, __builtin_inff());
+        au32x4 xb[3];
+        bf3_pack8(x, xb);
+        g2[gq] = bf3_mfma(w2[s], xb, g2[gq]);
+      }
     float o0, o1;
-    adafac_hidden_out(h, w2, bh, wo, bo0, bo1, o0, o1);
+    adafac_output(g2, wo, bo0, bo1, o0, o1);
     if (w0 + lane <= last)
-      *(gfloat*)(a.param + w0 + lane) = adafac_update(d, a, o0 * __builtin_amdgcn_exp2f(o1 * exp_scale), p);
+      *(gfloat*)(a.param + w0 + lane) = adafac_update(d, a, o0 * expf(o1 * a.exp_mult), p);
     cur = nxt;
   }
 }
@@ -945,9 +988,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   const float* w = wfold + (size_t)it.tensor * kAFold;
   const float* be = bias_eff + (size_t)it.tensor * kAH;
   const long long base = (long long)it.a * kThreads * it.b;
-  if (d.mode == kModeFac2D) adafac_apply_lin_hf<kModeFac2D>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
-  else if (d.mode == kModeFacND) adafac_apply_lin_hf<kModeFacND>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
-  else adafac_apply_lin_hf<kModeVec>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
+  if (d.mode == kModeFac2D) adafac_apply_lin<kModeFac2D>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
+  else if (d.mode == kModeFacND) adafac_apply_lin<kModeFacND>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
+  else adafac_apply_lin<kModeVec>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
 }
 
 __global__ __launch_bounds__(kThreads) void k_adafac_apply(const TDesc* __restrict__ descs,

@@ -154,7 +154,7 @@ struct Layout {
   std::vector<int> dc, dr;
   int H = 8;  // width of the first MLP layer (terms per row / column)
   int Tpad = 0;
-  bool lin_hf = false;       // AdafacLO: ga_items are k_adafac_apply_lin's (else k_adafac_apply's)
+  bool lin_matrix = false;   // AdafacLO: ga_items are k_adafac_apply_lin's (else k_adafac_apply's)
   bool global_norm = false;  // AdafacLO kind: every tensor has P0 items, the call may clip by global norm
   bool tensor_norm = false;  // ... or every tensor by its own norm (PYLO_F_TENSOR_NORM)
   size_t off_descs, off_dyn, off_p0_items, off_nd_items, off_sl_items, off_seg_items, off_segtot, off_el_items, off_ap_items, off_pp_items, off_ga_items, off_fin_items, off_finpart, off_finscale, off_tscale, off_v0a_items, off_v0b_items, off_fac_list,
@@ -1178,15 +1178,15 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
     }
   }
   // Blocks of AdafacLO's linear apply pass: on the matrix pipe Item::b trips of 256 elements each, as many as leave
-  // every SIMD the two waves it holds and no more than 16 (the set-up of a wave, its weights split into planes,
+  // every SIMD the two waves it holds and no more than 16 (the set-up of a wave, its weights,
   // costs about as much as a trip); else 8192- / 2048-element chunks.
-  L.lin_hf = env_matrix_pipe() && env_adafac_hf();
+  L.lin_matrix = env_matrix_pipe();
   long long lin_elems = 0;
   for (int t : lin_tensors) lin_elems += L.descs[t].n;
   const int trips = (int)std::max<long long>(1, std::min<long long>(16, lin_elems / (2 * 256 * kThreads)));
   for (int t : lin_tensors) {
-    const long long chunk = L.lin_hf ? (long long)kThreads * trips : (long long)kThreads * L.descs[t].vec * kElemIters;
-    for (long long c = 0; c * chunk < L.descs[t].n; ++c) L.ga_items.push_back(Item{t, (int)c, L.lin_hf ? trips : 0, 0});
+    const long long chunk = L.lin_matrix ? (long long)kThreads * trips : (long long)kThreads * L.descs[t].vec * kElemIters;
+    for (long long c = 0; c * chunk < L.descs[t].n; ++c) L.ga_items.push_back(Item{t, (int)c, L.lin_matrix ? trips : 0, 0});
   }
   if (kind == PYLO_KIND_CELO2 || kind == PYLO_KIND_VELO) build_elem_items(L, T, kind);
   long long ns_floats = 0;
@@ -2526,7 +2526,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   const Item* ga_items = P->at<Item>(L.off_ga_items);
   const Item* pp_items = P->at<Item>(L.off_pp_items);
   const int n_ap = (int)L.ap_items.size(), n_ga = (int)L.ga_items.size(), n_pp = (int)L.pp_items.size();
-  if (n_ga > 0 && L.lin_hf)
+  if (n_ga > 0 && L.lin_matrix)
     hipLaunchKernelGGL(k_adafac_apply_lin, dim3(n_ga), dim3(kThreads), 0, s, descs, dyn, ga_items, fac_tab, term_tab, dec,
                        wfold, net, (const float*)bias_eff, gl);
   else if (n_ga > 0)

@@ -1,12 +1,9 @@
 """AdafacLO's apply pass in storage order (tensors that no column-resident walk takes) with the element MLP on the
 matrix pipe: one step at the edges of its groups of 64 elements, blocks of 256 and trips, against the oracle in fp64.
 
-The bound: an operand of two fp16 planes carries 23 significant bits and a product is off by about 2^-23 of itself (root
-mean square over its three kept terms and the dropped one), unbiased, so the errors of a layer's products add in
-quadrature.  With this network's uniform weights and features of unit second moment the products of the three layers
-have root sums of squares of 0.6, 0.3 and 0.15, the later layers' gains are below one, and a step is off by about
-0.3 * 2^-23 = 3.6e-8; the largest of some hundreds is four times that.  The fp32 accumulation, which both pipes share, comes on top
-(1.5 times what the fp32 oracle and the all-VALU kernel show)."""
+The bound: its operands' three bfloat16 planes are the fp32 numbers, so an error is that of an fp32 sum in another order,
+no larger than one and a half times the largest that the fp32 oracle and the all-VALU kernel show on the same tensor
+(each the largest of up to some hundred thousand), or than half a spacing of the result where these have almost none."""
 
 import copy
 
@@ -56,4 +53,4 @@ def test_adafac_linear_apply_against_fp64(which, monkeypatch):
         err = float((outs["0"][i] - ref64[i]).abs().max())
         size = float((ref64[i] - init[i].double().cuda()).abs().max())
         print(s, "largest step", size, "fp32 oracle", own, "vector pipe", valu, "matrix pipe", err)
-        assert err <= 1.5 * max(own, valu) + 1.2 * 2.0 ** -23, (s, err, own, valu)
+        assert err <= max(1.5 * max(own, valu), 2.0 ** -25 * size), (s, err, own, valu)
