@@ -299,9 +299,9 @@ __global__ __launch_bounds__(64 * (MT / RT) * MT) void k_ns_small(
   int meets = 0;
   bool good = true;
   // sum over the matrix of the block's sums `s` (per lane), the same for every block
-  auto total = [&](float s) {
+  auto total = [&](double s) {
     s = wave_sum(s);
-    if (lane == 0) red[wave] = (double)s;
+    if (lane == 0) red[wave] = s;
     __syncthreads();
     double t = 0.0;
 #pragma unroll
@@ -327,14 +327,19 @@ __global__ __launch_bounds__(64 * (MT / RT) * MT) void k_ns_small(
       if (c + 1 < n_ch) x = nx;
     }
   };
-  float sq = 0.0f;
+  // sums of squares: a lane's 32 values of a chunk in fp32, chunks, lanes and waves in fp64 (as k_celo2_sumsq, whose lanes
+  // have 32 values too)
+  static_assert(16 * RT * J == 32, "values of a lane and chunk");
+  double sq = 0.0;
   auto square = [&]() {
+    float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
       for (int j = 0; j < J; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sq = fmaf(x.t[i][j][r], x.t[i][j][r], sq);
+        for (int r = 0; r < 16; ++r) s = fmaf(x.t[i][j][r], x.t[i][j][r], s);
+    sq += (double)s;
   };
   each_chunk(false, [&](int) { square(); });
   if (orth_call && (a.flags & kArgOrthogonalize)) {
@@ -465,7 +470,7 @@ __global__ __launch_bounds__(64 * (MT / RT) * MT) void k_ns_small(
       }
       // X <- Q X
       const float inv = pair ? st.upd_q : st.upd_b;
-      if (last) sq = 0.0f;
+      if (last) sq = 0.0;
       each_chunk(resident, [&](int c) {
 #pragma unroll
         for (int i = 0; i < RT; ++i)

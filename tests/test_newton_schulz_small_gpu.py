@@ -75,3 +75,28 @@ def test_many_that_meet_and_repeated_calls():
                     r = x.double() * torch.rsqrt(1e-9 + x.double().pow(2).mean())
                     assert float((params[i].double() - r).abs().max()) <= 1e-5, i
     plan.close()
+
+
+@pytest.mark.parametrize("square", [1.0 + 1.4e-5, 1.0 + 2.9e-6, 1.21])
+def test_sums_of_squares_of_long_matrices(square):
+    """Equal entries, whose roundings all fall to the same side: the normaliser of a call that only applies the step.
+    Sums of at most 32 squares run in fp32, so the mean square is off by at most 31 * 2^-24 of itself and the
+    normaliser by half of that; the normaliser, the squares and the result are rounded by 2^-23 each at the most."""
+    from pylo_amd import _lib
+
+    shapes = [(16, 65536), (65536, 3), (64, 32768), (128, 4096), (8192, 128), (32, 1025)]
+    mats = [torch.full(s, square ** 0.5, device="cuda") for s in shapes]
+    plan = _lib.Plan(_lib.KIND_CELO2, shapes, [0] * len(shapes), torch.device("cuda:0"))
+    fin = np.zeros(len(mats), dtype=_lib.ARGS_DTYPE)
+    params = [torch.zeros_like(x) for x in mats]
+    for i in range(len(mats)):
+        fin["grad"][i], fin["param"][i], fin["step_out"][i] = 1, params[i].data_ptr(), mats[i].data_ptr()
+        fin["lr"][i], fin["weight_decay"][i], fin["step_mult"][i] = -1.0, 0.0, 1.0
+    want = [float(x.double().mul(torch.rsqrt(1e-9 + x.double().pow(2).mean()))[0, 0]) for x in mats]
+    plan.celo2_orthogonalize_finish(fin, (3.4445, -4.775, 2.0315), 5, 1e-8, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for s, p, w in zip(shapes, params, want):
+        off = float((p.double() / w - 1.0).abs().max())
+        print(s, off)
+        assert off <= 31 * 2.0 ** -25 + 3 * 2.0 ** -23, (s, off)
+    plan.close()
