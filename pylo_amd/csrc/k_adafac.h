@@ -128,7 +128,7 @@ __device__ __forceinline__ void adafac_stats_vec(const TDesc& d, const PyloTenso
   }
 }
 
-template <bool TYPED>
+template <bool TYPED, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void k_adafac_stats(const TDesc* __restrict__ descs,
                                                            const PyloTensorArgs* __restrict__ dyn,
                                                            const Item* __restrict__ items,
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kThreads) void k_adafac_stats(const TDesc* __restri
                                                            const Globals* __restrict__ gl) {
   __shared__ float red[kWaves][30];
   const Item it = items[blockIdx.x];
-  TDesc d = descs[it.tensor];
+  TDesc d = elem_desc<SPLIT>(descs + it.tensor);
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
   set_grad_scale(d, a, gl, it.tensor);

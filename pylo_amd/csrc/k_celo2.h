@@ -10,17 +10,6 @@
 
 namespace pylo {
 
-// The descriptor of a fused element pass.  Chunks of fewer than kElemIters trips (TDesc::iters) are an instantiation of
-// their own: the trip count as one more run-time value made the compiler cut the registers of every loop of the kernel
-// differently, the column-resident walk's among them (k_velo_elem on 86 M elements 0.86 -> 0.92 ms, whole step 1.00 ->
-// 1.06 ms).
-template <bool SPLIT>
-__device__ __forceinline__ TDesc elem_desc(const TDesc* __restrict__ p) {
-  TDesc d = *p;
-  if constexpr (!SPLIT) d.iters = kElemIters;
-  return d;
-}
-
 struct EmaConsts {
   float bm[3], obm[3];  // momentum decays and 1-decay
   float br, obr;        // rms
@@ -393,7 +382,7 @@ __device__ __forceinline__ double stats_block_total(const float (*red)[kNStat], 
 
 // Statistics pass as a launch of its own (each pass over all tensors; the fused element pass,
 // k_celo2_elem, is the default).
-template <bool TYPED>
+template <bool TYPED, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void k_celo2_stats(const TDesc* __restrict__ descs,
                                                           const PyloTensorArgs* __restrict__ dyn,
                                                           const Item* __restrict__ items,
@@ -402,7 +391,7 @@ __global__ __launch_bounds__(kThreads) void k_celo2_stats(const TDesc* __restric
                                                           double* __restrict__ stats_part) {
   __shared__ float red[kWaves][kNStat];
   const Item it = items[blockIdx.x];
-  const TDesc d = descs[it.tensor];
+  const TDesc d = elem_desc<SPLIT>(descs + it.tensor);
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
   if (!celo2_stats_block<false, TYPED>(d, a, it, fac_tab, gl, dec, red)) return;
@@ -811,7 +800,7 @@ __device__ __forceinline__ void celo2_apply_block(const TDesc& d, const PyloTens
 }
 
 // Apply pass as a launch of its own (see k_celo2_stats).
-template <bool MFMA, bool TYPED>
+template <bool MFMA, bool TYPED, bool SPLIT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PYLO_APPLY_WAVES))) void k_celo2_apply(const TDesc* __restrict__ descs,
                                                           const PyloTensorArgs* __restrict__ dyn,
                                                           const Item* __restrict__ items,
@@ -820,7 +809,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(PYLO_A
                                                           const Globals* __restrict__ gl, PyloDecays dec,
                                                           const float* __restrict__ wfold) {
   const Item it = items[blockIdx.x];
-  const TDesc d = descs[it.tensor];
+  const TDesc d = elem_desc<SPLIT>(descs + it.tensor);
   if (d.mode == kModeFlat) return;
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;

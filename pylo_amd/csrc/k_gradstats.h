@@ -154,7 +154,7 @@ __device__ __forceinline__ void p0_nd_block(const TDesc* __restrict__ descs, con
 //         elements beyond the clamp; tensors without global-norm clipping are clamped directly.
 // pass 1: only if the flag was raised: redo clip_norm > 0 tensors with scale and clamp applied.
 // TYPED: plans with tensors whose 16-bit gradient is read here (TDesc::direct; their rows are multiples of 128).
-template <bool TYPED>
+template <bool TYPED, bool SPLIT>
 __global__ __launch_bounds__(kThreads) void k_p0(const TDesc* __restrict__ descs,
                                                  const PyloTensorArgs* __restrict__ dyn,
                                                  const Item* __restrict__ items, float* __restrict__ part,
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(kThreads) void k_p0(const TDesc* __restrict__ descs
     return;
   }
   const Item it = items[blockIdx.x];
-  const TDesc d = descs[it.tensor];
+  const TDesc d = elem_desc<SPLIT>(descs + it.tensor);
   const PyloTensorArgs a = dyn[it.tensor];
   const bool clip_on = a.clip_norm > 0.0f;
   if (pass == 1 && (!clip_on || d.mode != kModeFac2D || gl->flag == 0)) return;

@@ -236,6 +236,18 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// The descriptor of an element pass.  Chunks of fewer than kElemIters trips (TDesc::iters; SPLIT) are an instantiation of
+// their own: the trip count as one more run-time value made the compiler cut the registers of every loop of a kernel
+// differently, the column-resident walk's among them (k_velo_elem on 86 M elements 0.86 -> 0.92 ms, whole step 1.00 ->
+// 1.06 ms; with k_velo_stats' own registers bounded, k_velo_stats on 30 M elements of vectors 265 -> 250 us, on 8 M of
+// 512 x 512 x 5 kernels 72 -> 64 us).
+template <bool SPLIT>
+__device__ __forceinline__ TDesc elem_desc(const TDesc* __restrict__ p) {
+  TDesc d = *p;
+  if constexpr (!SPLIT) d.iters = kElemIters;
+  return d;
+}
+
 // torch.clamp semantics (NaN propagates); c <= 0 disables the clamp.  Branch-free: the bound is a
 // wave-uniform select that the compiler hoists out of element loops.
 __device__ __forceinline__ float clampf(float x, float c) {

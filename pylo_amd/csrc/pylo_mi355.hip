@@ -1757,6 +1757,15 @@ struct Marks {  // per-launch HIP events when timing is on
 
 }  // namespace
 
+// The instantiation <TYPED, SPLIT> of a kernel, from all four of them.
+template <class F>
+F variant(bool typed, bool split, F plain, F split_only, F typed_only, F both) {
+  return typed ? (split ? both : typed_only) : (split ? split_only : plain);
+}
+inline auto p0_kernel(bool typed, bool split) {
+  return variant(typed, split, k_p0<false, false>, k_p0<false, true>, k_p0<true, false>, k_p0<true, true>);
+}
+
 extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, const PyloDecays* decays,
                                      const float* mlp, void* stream) {
   if (!P || !args || !decays || !mlp) return fail("celo2_step: null argument");
@@ -1797,14 +1806,14 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
   const bool exact_pass = exact_pass_possible(P, args);
   HIP_TRY(mark());
   if (n_p0 > 0)
-    hipLaunchKernelGGL(in_place ? k_p0<true> : k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
+    hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
                        (const Item*)nullptr, n_p0);
   HIP_TRY(mark());
   hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, gsq, flag, n_p0, gl, exact_pass ? 1 : 0,
                      P->at<int>(L.off_sync), 2 * P->T);
   HIP_TRY(mark());
   if (n_p0 > 0 && exact_pass)
-    hipLaunchKernelGGL(in_place ? k_p0<true> : k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
+    hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
                        (const Item*)nullptr, n_p0);
   if (n_nd > 0) hipLaunchKernelGGL(k_p0_nd, dim3(n_nd), dim3(kThreads), 0, s, descs, dyn, nd_items, part, gl);
   HIP_TRY(mark());
@@ -1826,7 +1835,9 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
                        wfold, chan_ms, stats, sync, P->T);
     HIP_TRY(mark());
   } else {
-    if (n_el > 0) hipLaunchKernelGGL(in_place ? k_celo2_stats<true> : k_celo2_stats<false>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, gl, dec, stats);
+    const auto stats_pass = variant(in_place, L.split, k_celo2_stats<false, false>, k_celo2_stats<false, true>,
+                                    k_celo2_stats<true, false>, k_celo2_stats<true, true>);
+    if (n_el > 0) hipLaunchKernelGGL(stats_pass, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, gl, dec, stats);
     HIP_TRY(mark());
     const Item* seg_items = P->at<Item>(L.off_seg_items);
     double* seg_tot = P->at<double>(L.off_segtot);
@@ -1837,9 +1848,9 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
                          chan_ms);
     HIP_TRY(mark());
     if (n_el > 0) {
-      const auto apply = in_place                ? k_celo2_apply<true, true>
-                         : P->mlp_on_matrix_pipe ? k_celo2_apply<true, false>
-                                                 : k_celo2_apply<false, false>;
+      const auto apply = in_place                ? (L.split ? k_celo2_apply<true, true, true> : k_celo2_apply<true, true, false>)
+                         : P->mlp_on_matrix_pipe ? (L.split ? k_celo2_apply<true, false, true> : k_celo2_apply<true, false, false>)
+                                                 : (L.split ? k_celo2_apply<false, false, true> : k_celo2_apply<false, false, false>);
       hipLaunchKernelGGL(apply, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, term_tab, gl, dec, wfold);
     }
   }
@@ -2350,7 +2361,7 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   const bool typed = L.in_place;
   auto gradient_sums = [&]() {
     if (n_p0 + n_nd > 0)
-      hipLaunchKernelGGL(typed ? k_p0<true> : k_p0<false>, dim3(n_p0 + n_nd), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
+      hipLaunchKernelGGL(p0_kernel(typed, L.split), dim3(n_p0 + n_nd), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
                          nd_items, n_p0);
   };
   auto factor_tables = [&]() {
@@ -2396,7 +2407,11 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   HIP_TRY(mark());
   if (n_mx == 0) HIP_TRY(mark());
   if (int rc = factor_tables()) return rc;
-  if (n_el > 0) hipLaunchKernelGGL(typed ? k_velo_stats<true> : k_velo_stats<false>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, dec, stats);
+  const auto stats_pass = variant(typed, L.split, k_velo_stats<false, false>, k_velo_stats<false, true>, k_velo_stats<true, false>,
+                                  k_velo_stats<true, true>);
+  const auto apply_pass = variant(typed, L.split, k_velo_apply<false, false>, k_velo_apply<false, true>, k_velo_apply<true, false>,
+                                  k_velo_apply<true, true>);
+  if (n_el > 0) hipLaunchKernelGGL(stats_pass, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, dec, stats);
   if (n_mx == 0) HIP_TRY(mark());
   const Item* seg_items = P->at<Item>(L.off_seg_items);
   double* seg_tot = P->at<double>(L.off_segtot);
@@ -2410,7 +2425,7 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
     hipLaunchKernelGGL(k_terms<4>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, bscale, canon, kVCanon, term_tab);
   HIP_TRY(mark());
   if (n_el > 0)
-    hipLaunchKernelGGL(typed ? k_velo_apply<true> : k_velo_apply<false>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, term_tab, dec, wfold,
+    hipLaunchKernelGGL(apply_pass, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, term_tab, dec, wfold,
                        (const float*)piv, newsum);
   HIP_TRY(mark());
   mark.done();
@@ -2484,7 +2499,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   // without global-norm clipping the N-D tensors' sums ride in the tail blocks of the first launch
   const int n_tail = clips ? 0 : n_nd;
   if (n_p0 + n_tail > 0)
-    hipLaunchKernelGGL(in_place ? k_p0<true> : k_p0<false>, dim3(n_p0 + n_tail), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
+    hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0 + n_tail), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
                        nd_items, n_p0);
   if (clips && L.tensor_norm) {
     // every tensor against its own norm (AdafacLO_naive.py:199-200): no clamp on such tensors, no exact pass
@@ -2493,7 +2508,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
     const bool exact_pass = exact_pass_possible(P, args);
     hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, gsq, flag, n_p0, gl, exact_pass ? 1 : 0, (int*)nullptr, 0);
     if (n_p0 > 0 && exact_pass)
-      hipLaunchKernelGGL(in_place ? k_p0<true> : k_p0<false>, dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
+      hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
                          (const Item*)nullptr, n_p0);
   }
   HIP_TRY(mark());
@@ -2508,8 +2523,10 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
     hipLaunchKernelGGL(k_v0b<kAH>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, v0part, 1e-5f,
                        net + kAW1, (const float*)bias_eff, kAH, fac_tab, term_tab, bscale);
   HIP_TRY(mark());
+  const auto stats_pass = variant(in_place, L.split, k_adafac_stats<false, false>, k_adafac_stats<false, true>,
+                                  k_adafac_stats<true, false>, k_adafac_stats<true, true>);
   if (n_el > 0)
-    hipLaunchKernelGGL(in_place ? k_adafac_stats<true> : k_adafac_stats<false>, dim3(n_el), dim3(kThreads), 0, s, descs, dyn,
+    hipLaunchKernelGGL(stats_pass, dim3(n_el), dim3(kThreads), 0, s, descs, dyn,
                        el_items, fac_tab, dec, stats, gl);
   HIP_TRY(mark());
   const Item* seg_items = P->at<Item>(L.off_seg_items);
