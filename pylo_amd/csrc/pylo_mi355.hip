@@ -121,7 +121,7 @@ struct Layout {
   // 32, 64, 128)
   std::vector<NsSmall> sm_mats;
   std::vector<NsSmallItem> sm_items[kNsSmallClasses];
-  std::vector<char> small_of_tensor;  // per tensor: its matrices are in sm_mats
+  std::vector<char> small_of_tensor;  // per tensor: its matrices are in sm_mats (2: they are multiples of four elements long)
   long long sm_part_floats = 0;
   int sm_sums = 0, sm_sync = 0, sm_ticket0 = 0;
   bool sm_meets[kNsSmallClasses] = {};   // the class has matrices of several blocks
@@ -606,7 +606,7 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
   for (int t = 0; t < T; ++t) {
     if (!matrices(t, R, C, n_sl)) continue;
     if (small && ns_small_takes(R, C)) {
-      L.small_of_tensor[t] = 1;
+      L.small_of_tensor[t] = (long long)R * C % 4 == 0 ? 2 : 1;
       for (int sl = 0; sl < n_sl; ++sl) {
         NsSmall b{};
         b.tensor = t;
@@ -1980,10 +1980,8 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
       continue;
     }
     const bool small = L.small_of_tensor[t] != 0;
-    const bool vec = d.fin_units > 0 && L.fin_units[d.fin_unit0].vec;
-    if (!small && m % (vec ? 16 : 4) != 0) return fail(w + ": misaligned pointer" + at);
-    if (small && (reinterpret_cast<uintptr_t>(a.step_out) % 4 != 0 || reinterpret_cast<uintptr_t>(a.param) % (d.store != 0 ? 2 : 4) != 0))
-      return fail(w + ": misaligned pointer" + at);
+    const bool vec = small ? L.small_of_tensor[t] == 2 : d.fin_units > 0 && L.fin_units[d.fin_unit0].vec;
+    if (m % (vec ? 16 : 4) != 0) return fail(w + ": misaligned pointer" + at);   // the same whatever launch takes the tensor
     any_small = any_small || small;
     if (coeffs && ns_iters == 0 && (a.flags & PYLO_ARG_ORTHOGONALIZE))
       return fail(w + ": PYLO_ARG_ORTHOGONALIZE with ns_iters = 0 on a tensor that the tiled products orthogonalise "

@@ -100,3 +100,30 @@ def test_sums_of_squares_of_long_matrices(square):
         print(s, off)
         assert off <= 31 * 2.0 ** -25 + 3 * 2.0 ** -23, (s, off)
     plan.close()
+
+
+@pytest.mark.parametrize("shape,offset,refused", [((128, 128), 4, True), ((2, 128, 128), 8, True), ((3, 4), 8, True), ((7, 9), 4, False)])
+def test_alignment_of_the_finishing_call(shape, offset, refused):
+    """Steps and parameters of whole groups of four elements are 16-byte aligned, others 4-byte: what the finishing pass
+    of every other matrix asks for.  A refused call launches nothing."""
+    from pylo_amd import _lib
+
+    n = int(np.prod(shape))
+    raw = torch.randn(n + 8, device="cuda")
+    step = raw[offset // 4:offset // 4 + n]
+    param = torch.zeros(n, device="cuda")
+    plan = _lib.Plan(_lib.KIND_CELO2, [shape], [0], torch.device("cuda:0"))
+    fin = np.zeros(1, dtype=_lib.ARGS_DTYPE)
+    fin["grad"][0], fin["param"][0], fin["step_out"][0] = 1, param.data_ptr(), step.data_ptr()
+    fin["lr"][0], fin["step_mult"][0] = -1.0, 1.0
+    args = (fin, (3.4445, -4.775, 2.0315), 5, 1e-8, torch.cuda.current_stream().cuda_stream)
+    if refused:
+        with pytest.raises(RuntimeError, match="misaligned"):
+            plan.celo2_orthogonalize_finish(*args)
+        torch.cuda.synchronize()
+        assert not param.any()
+    else:
+        plan.celo2_orthogonalize_finish(*args)
+        x = step.double()
+        assert float((param.double() - x * torch.rsqrt(1e-9 + x.pow(2).mean())).abs().max()) <= 1e-5
+    plan.close()
