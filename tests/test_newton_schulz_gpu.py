@@ -80,14 +80,18 @@ def test_library_kernels_take_these_shapes(pipe, monkeypatch):
     [(37, 4099), (4099, 37), (255, 257), (129, 129), (1, 300), (300, 1), (2, 3)],   # odd dims, single rows and columns
     [(300, 260), (300, 260), (300, 260), (64,)],                         # a bucket of equal shapes
 ])
-@pytest.mark.parametrize("pipe", ["fp16x2", "fp16x2-literal", "fp16x2-chains-3,2", "fp32"])
+@pytest.mark.parametrize("pipe", ["fp16x2", "fp16x2-tiled", "fp16x2-literal", "fp16x2-chains-3,2", "fp32"])
 def test_library_newton_schulz_matches_oracle(shapes, pipe, monkeypatch):
     """The sets of product kernels: the default (operands split into two scaled fp16 planes, three fp16 matrix
     products per fp32 product, two iterations sharing one Gram product and one update), the same with one Gram product and
     one update per iteration (PYLO_MI355_NS_PAIRS=0), with a chain of three iterations and one of two
-    (PYLO_MI355_NS_CHAINS="3,2"), and the fp32 matrix instructions (PYLO_MI355_NS_F32=1, read at plan creation)."""
+    (PYLO_MI355_NS_CHAINS="3,2"), and the fp32 matrix instructions (PYLO_MI355_NS_F32=1, read at plan creation).  Matrices
+    with a smaller dim of at most 128 have launches of their own by default in some of these sets; "tiled"
+    (PYLO_MI355_NS_SMALL=0) and the chains take all through the tiled products."""
     if pipe == "fp32":
         monkeypatch.setenv("PYLO_MI355_NS_F32", "1")
+    if pipe == "fp16x2-tiled":
+        monkeypatch.setenv("PYLO_MI355_NS_SMALL", "0")
     if pipe == "fp16x2-literal":
         monkeypatch.setenv("PYLO_MI355_NS_PAIRS", "0")
     if pipe.startswith("fp16x2-chains-"):

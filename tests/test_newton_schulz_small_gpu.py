@@ -15,6 +15,9 @@ pytestmark = pytest.mark.gpu
 SETS = {
     "up to 32": [(1, 1), (1, 7), (7, 1), (31, 33), (32, 32), (5, 128), (129, 5), (32, 1025), (3000, 17), (1, 30000), (16, 65536), (17, 32769)],
     "up to 64": [(33, 33), (33, 128), (129, 40), (64, 64), (64, 2048), (4099, 37), (37, 8191), (32768, 33)],
+    "past the limits": [(65537, 5), (32769, 33), (8193, 96), (70, 8200)],       # the tiled products', with no small ones
+    "beside a higher class": [(16, 65536), (64, 8192), (65, 65), (3, 9)],       # lifted, and too long to be
+    "beside larger ones": [(10, 512), (512, 300), (100, 300), (31, 33)],        # in the larger ones' launches
     "up to 128": [(65, 65), (65, 128), (129, 100), (128, 128), (784, 128), (128, 4096), (1027, 127), (96, 257), (8193, 80)],
 }
 
@@ -40,12 +43,16 @@ def test_small_matrices_against_fp64(which, iters):
         torch.backends.cuda.matmul.allow_tf32 = prev
 
 
-def test_many_that_meet_and_repeated_calls():
-    """More matrices of several blocks than may wait at a time (longer slabs are taken), a plan used again and again,
-    a NaN that stays in its matrix, and a call that only normalises and applies."""
+@pytest.mark.parametrize("counts", [(24, 30, 20), (80, 100, 60)])
+def test_many_that_meet_and_repeated_calls(counts):
+    """Matrices of several blocks: all of them running at once, and more of them than a launch holds at a time (longer
+    slabs, blocks that start when others end).  A plan used again and again, a NaN that stays in its matrix, and a call that
+    only normalises and applies."""
     from pylo_amd import _lib
 
-    shapes = [(128, 784)] * 24 + [(60, 1500)] * 30 + [(3, 5000)] * 20 + [(128, 784), (200, 300)]
+    a, b, c = counts
+    n = a + b + c
+    shapes = [(128, 784)] * a + [(60, 1500)] * b + [(3, 5000)] * c + [(128, 784), (200, 300)]
     gen = torch.Generator(device="cuda").manual_seed(1)
     mats = [torch.randn(s, generator=gen, device="cuda") for s in shapes]
     mats[5][3, 700] = float("nan")
@@ -64,11 +71,11 @@ def test_many_that_meet_and_repeated_calls():
         assert torch.isnan(params[5]).all()
         if call == 0:
             want = params
-            for i in (0, 23, 24, 53, 54, 73, 75):
+            for i in (0, a - 1, a, a + b - 1, a + b, n - 1, n + 1):
                 assert float((params[i].double() - _reference_direct(mats[i])).abs().max()) <= 2e-4, i
-            assert float((params[74].double() - _reference_direct(mats[74])).abs().max()) <= 2e-4
+            assert float((params[n].double() - _reference_direct(mats[n])).abs().max()) <= 2e-4
         elif call < 3:
-            assert all(torch.equal(a, b) for i, (a, b) in enumerate(zip(params, want)) if i != 5)
+            assert all(torch.equal(x, y) for i, (x, y) in enumerate(zip(params, want)) if i != 5)
         else:
             for i, x in enumerate(mats):
                 if i != 5:
@@ -127,3 +134,14 @@ def test_alignment_of_the_finishing_call(shape, offset, refused):
         x = step.double()
         assert float((param.double() - x * torch.rsqrt(1e-9 + x.pow(2).mean())).abs().max()) <= 1e-5
     plan.close()
+
+
+def test_slices_aside():
+    """Tensors of more than two dims whose slices are small matrices, with no larger one in the plan."""
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    mats = [torch.randn(s, generator=gen, device="cuda") for s in [(2, 128, 128), (3, 64, 300), (2, 2, 100, 201), (1, 8100, 40)]]
+    for x, y in zip(mats, _orthogonalise_direct(mats)):
+        for xs, ys in zip(x.reshape(-1, *x.shape[-2:]), y.reshape(-1, *x.shape[-2:])):
+            want = _reference_direct(xs)
+            e32 = float((_reference_direct(xs, dtype=torch.float32).double() - want).abs().max())
+            assert float((ys.double() - want).abs().max()) <= 1.5 * e32 + 5e-5, tuple(x.shape)

@@ -14,12 +14,22 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("rows", [100, 900, 2000, 3501, 6001])     # 16, 8, 4, 2 parts and whole blocks
 @pytest.mark.parametrize("family", ["elo_celo2", "velo", "adafac"])
 def test_every_cut_against_the_oracle(family, rows):
+    _three_steps(family, [(rows, 256), (rows, 130), (1000,), (33, 128)], rows)
+
+
+# The same with tensors of more than two dims: convolution kernels walked as matrices or by slices, channels last to first.
+@pytest.mark.parametrize("rows", [10, 100, 400, 900])     # 16, 8, 2 parts and whole blocks
+@pytest.mark.parametrize("family", ["elo_celo2", "velo", "adafac"])
+def test_every_cut_with_more_than_two_dims(family, rows):
+    _three_steps(family, [(rows, 64, 3, 3), (3, 5, rows, 7), (rows, 128, 9), (1, 1, 64), (rows,)], rows)
+
+
+def _three_steps(family, shapes, rows):
     from oracle import pylo_oracle as O
     from pylo_amd import ELO_CELO2_CUDA, AdafacLO_CUDA, VeLO_CUDA
     from pylo_amd.models import CELO2MLP, MetaMLP, VeLOMLP, VeLORNN
 
     torch.manual_seed(rows)
-    shapes = [(rows, 256), (rows, 130), (1000,), (33, 128)]
     gen = torch.Generator(device="cuda").manual_seed(rows)
     init = [torch.randn(s, generator=gen, device="cuda") * 0.05 for s in shapes]
     ref = [v.double() for v in init]

@@ -21,7 +21,7 @@ SETS = [
 
 
 def _run(cls, params, grads, loss):
-    from pylo_amd import ELO_CELO2_CUDA, AdafacLO_CUDA, VeLO_CUDA
+    from pylo_amd import ELO_CELO2_CUDA, ELO_CUDA, AdafacLO_CUDA, VeLO_CUDA
     from pylo_amd.models import CELO2MLP, MetaMLP, VeLOMLP, VeLORNN
 
     torch.manual_seed(1)
@@ -30,6 +30,10 @@ def _run(cls, params, grads, loss):
     if cls == "VeLO":
         opt = VeLO_CUDA(params, lr=1.0, num_steps=100, weight_decay=0.01, rnn=VeLORNN(), mlp=VeLOMLP())
         opt.step(loss)
+    elif cls.startswith("ELO ") or cls == "ELO":
+        opt = ELO_CUDA(params, lr=1e-2, weight_decay=0.01, clip_grad="clipped" in cls, clip_norm=0.5, network=MetaMLP(39, 32, 1),
+                       hf_key=None)
+        opt.step()
     elif cls.startswith("AdafacLO"):
         opt = AdafacLO_CUDA(params, lr=1.0, weight_decay=0.01, max_grad_norm=0.5 if "clipped" in cls else None,
                             network=MetaMLP(39, 32, 1))
@@ -56,7 +60,12 @@ def test_step_in_place_matches_float32(shapes, dtype, mixed, cls):
     o16 = _run(cls, p16, [g.cuda() for g in grads], loss)
     o32 = _run(cls, p32, [g.float().cuda() for g in grads], loss)
     torch.cuda.synchronize()
-    for a, b, s, dt in zip(p16, p32, shapes, dts):
+    _compare(o16, o32, p16, p32, init)
+
+
+def _compare(o16, o32, p16, p32, init):
+    for a, b, v in zip(p16, p32, init):
+        s, dt = tuple(v.shape), v.dtype
         for k in (k for k, v in o32.state[b].items() if torch.is_tensor(v) and v.is_cuda and k != "rank_onehot"):
             assert max_err(o16.state[a][k], o32.state[b][k].cpu(), 1e-5, 1e-6) <= 1.0, (s, k)
         got, want = a.detach().cpu(), b.detach().cpu()
@@ -64,4 +73,50 @@ def test_step_in_place_matches_float32(shapes, dtype, mixed, cls):
             assert max_err(got, want, 1e-5, 1e-6) <= 1.0, s
         else:
             assert float(((got.double() - want.to(dt).double()).abs() / _spacing(want, dt)).max()) <= 1.0, s
-            assert not torch.equal(got, init[[id(x) for x in p16].index(id(a))]), s
+            assert not torch.equal(got, v), s
+
+
+# Plans above 2.1 M elements, whose passes are not cut finer (instantiations of their own): tasks of sixteen rows, a last
+# one of fewer, a staged neighbour, and a tensor too large to be kept in the cache between its statistics and its apply.
+@pytest.mark.parametrize("cls", ["VeLO", "ELO_CELO2", "ELO_CELO2 clipped", "AdafacLO", "ELO clipped"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shapes", [[(4099, 768), (130, 36)], [(12801, 640), (256, 128)]])
+def test_plans_that_are_not_cut(shapes, dtype, cls):
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    init = [(torch.randn(s, generator=gen, device="cuda") * 0.3).to(dtype) for s in shapes]
+    grads = [(torch.randn(s, generator=gen, device="cuda") * 0.1).to(dtype) for s in shapes]
+    p16 = [torch.nn.Parameter(v.clone()) for v in init]
+    p32 = [torch.nn.Parameter(v.float()) for v in init]
+    loss = torch.tensor(2.0, device="cuda")
+    o16 = _run(cls, p16, grads, loss)
+    o32 = _run(cls, p32, [g.float() for g in grads], loss)
+    torch.cuda.synchronize()
+    _compare(o16, o32, p16, p32, [v.cpu() for v in init])
+
+
+# ELO replaces NaN and infinite gradients after clipping (torch.nan_to_num): elements that are only known after the norm
+# is, and that send the gradient sums through their second pass.
+@pytest.mark.parametrize("cls", ["ELO", "ELO clipped"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("odd", [float("nan"), float("inf"), 0.0])
+def test_elo_in_place_with_gradients_that_are_replaced(dtype, cls, odd):
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    shapes = [(33, 128), (257, 384), (130, 36)]
+    init = [(torch.randn(s, generator=gen, device="cuda") * 0.3).to(dtype) for s in shapes]
+    grads = [(torch.randn(s, generator=gen, device="cuda") * 0.1).to(dtype) for s in shapes]
+    if odd != 0.0:
+        grads[1][200, 17] = odd
+    p16 = [torch.nn.Parameter(v.clone()) for v in init]
+    p32 = [torch.nn.Parameter(v.float()) for v in init]
+    o16 = _run(cls, p16, grads, None)
+    o32 = _run(cls, p32, [g.float() for g in grads], None)
+    torch.cuda.synchronize()
+    for a, b in zip(p16, p32):
+        for k in (k for k, v in o32.state[b].items() if torch.is_tensor(v) and v.is_cuda):
+            x, y = o16.state[a][k], o32.state[b][k].cpu()
+            assert torch.equal(x.isfinite().cpu(), y.isfinite())
+            assert max_err(x.nan_to_num(0.0, 0.0, 0.0), y.nan_to_num(0.0, 0.0, 0.0), 1e-5, 1e-6) <= 1.0, k
+        got, want = a.detach().cpu(), b.detach().cpu().to(dtype)
+        assert torch.equal(got.isfinite(), want.isfinite())
+        fin = got.isfinite()
+        assert float(((got[fin].double() - want[fin].double()).abs() / _spacing(want[fin].float(), dtype)).max()) <= 1.0
