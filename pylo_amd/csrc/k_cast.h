@@ -9,11 +9,13 @@
 // tensor this adds 18 (16-bit types) or 36 (fp64) bytes; tensors without a tag are not touched by any of it.
 //
 // 2-D tensors on the column-resident walks skip the staging where they are stored in 16 bits (TDesc::direct): the three
-// passes over them take the storage type as a template argument, widen in the load and round in the store.  Both casts less, and passes that move half the gradient's and parameter's bytes.
+// passes over them take the storage type as a template argument, widen in the load and round in the store.  Both casts
+// less, and passes that move half the gradient's and parameter's bytes.
 //   VeLO, 86 M bf16 elements (ViT-B/16): casts 327 us -> 15 us (what is still staged), k_p0 105 -> 59, k_velo_stats
 //     307 -> 299, k_velo_apply 694 -> 617, whole step 1.51 -> 1.04 ms
 //   ELO-CELO2, 124 M bf16 elements (GPT-2-small): whole step 7.07 -> 6.71 ms
-//   AdafacLO, 1.1 G elements (Llama-1.1B): bf16 27.1 -> 21.5 ms, fp16 27.1 -> 22.0 ms (fp32 22.8 ms)
+//   59 M bf16 elements (transformer of width 768, six layers, 20 000 x 768 embedding), staged / in place / fp32: AdafacLO 1.48 /
+//     1.22 / 1.28 ms, VeLO 1.05 / 0.75 / 0.78, ELO-CELO2 without Newton-Schulz 1.05 / 0.85 / 0.91
 // every result bit for bit the same.  Linear chunks, vectors, tensors with more than two dims and fp64 stay staged.
 #pragma once
 
