@@ -443,6 +443,11 @@ bool env_ns_small() {
 // The products of an m x n matrix in the unit of the rules below: five iterations in pairs are three Gram products on
 // the upper blocks, three updates and eleven m x m products.
 double ns_work(int m, int n) { return (double)m * m * (4.6 * n + 5.9 * m); }
+// ... as the tiled launches do it, in whole tiles (a thousand 130 x 130, 176 G and not 23: 1917 us on four streams, 2145 on one)
+double ns_tiled_work(int m, int n) {
+  auto up = [](int x) { return (x + kNsTile - 1) / kNsTile * kNsTile; };
+  return ns_work(up(m), up(n));
+}
 
 // Into how many groups (streams) the matrices of a plan are dealt: as many as have eight of its matrices each, those that
 // go aside to k_ns_small counted (which launch takes them says nothing about the others), and 55 G of work each.  Below that a
@@ -451,6 +456,7 @@ double ns_work(int m, int n) { return (double)m * m * (4.6 * n + 5.9 * m); }
 //   width 256, 12 layers (18 G) 856 / 903 / 957 us      384, 8 layers (43 G) 1294 / 1293 / 1331, 12 (60 G) 1667 / 1593 / 1648
 //   512, 4 layers (52 G) 1244 / 1291 / 1331, 6 (72 G) 1691 / 1621 / 1633, 8 (93 G) 2057 / 1896 / 1945, 12 (133 G) 2551 / 2446 / 2405
 //   1024, 2 layers (210 G) 2799 / 2547 / 2542, 3 layers 3367 / 3103 / 3091 us
+//   64 of 256 x 256 (11 G) 533 / 588 us, four streams 664; 500 of 200 x 200 (88 G) 1817 / 1643 / four 1676
 int ns_group_count(int mats, double work) {
   return (int)std::min<double>(std::min(env_ns_groups(), std::max(mats / 8, 1)), 1.0 + std::floor(work / 55e9));
 }
@@ -598,7 +604,7 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
         tiles += (long long)n_sl * ((std::max(R, C) + kNsTile - 1) / kNsTile);
       } else {
         n_large += n_sl;
-        work += n_sl * ns_work(std::min(R, C), std::max(R, C));
+        work += n_sl * ns_tiled_work(std::min(R, C), std::max(R, C));
       }
     }
     small = ns_small_aside(n_large, work, n_small, tiles);
@@ -760,7 +766,7 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
     L.ns_fpart_total = 0;
     for (NsBatch& bt : L.ns_batches) {
     double batch_work = 0.0;
-    for (int q = bt.mat0; q < bt.mat0 + bt.n_mats; ++q) batch_work += ns_work(L.nsb_mats[q].m, L.nsb_mats[q].n);
+    for (int q = bt.mat0; q < bt.mat0 + bt.n_mats; ++q) batch_work += ns_tiled_work(L.nsb_mats[q].m, L.nsb_mats[q].n);
     // (one of the four hardware queues is left to the small matrices where there are any: 3 / 4 groups next to them, 1024
     // wide 8117 / 8162 us, 512 wide 3203 / 3281)
     const int n_groups = std::min({L.sm_mats.empty() ? 4 : 3, bt.n_mats,
