@@ -64,7 +64,6 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short hbits;   // one number of a plane in memory (an fp16)
 constexpr int kNsPl = 2;                      // planes per matrix
 constexpr int kNsRowB = 32 * kNsPl;           // bytes of one row in a block of 16 reduction steps
-constexpr int kNsRowPc = 2 * kNsPl;           // the same in 16-byte pieces
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) u32x4 luint4;
 
@@ -72,18 +71,20 @@ constexpr int kHfBK = 16;                     // reduction steps per stage
 // LDS of a tile job with 64 WN columns: two stages of (128 + 64 WN) rows x 2 planes x 32 bytes
 constexpr int hf_gemm_lds(int wn) { return 2 * (128 + 64 * wn) * kNsRowB; }
 
-// Planes of one matrix with `rows` rows and a (padded) reduction length: stored in blocks of 16 reduction
-// steps, [k / 16][row][plane][k % 16], so that the 128 rows x 3 planes x 16 steps a tile job stages at a
-// time are 12 KB of consecutive memory (whole cache lines; with row-major planes a stage was 32 bytes
-// out of every row and each 128-byte line was fetched from L2 four times).
+// Planes of one matrix with `rows` rows (a multiple of the tiles' rows; rows past the matrix hold zeros) and a (padded)
+// reduction length: blocks of 16 reduction steps x 16 rows, [k / 16][row / 16], of 1 KB each, inside a block [half: k / 8 % 2]
+// [plane][row % 16][k % 8].  The rows x 2 planes x 16 steps a tile job stages at a time are consecutive memory, a block is
+// what one wave-wide 16-byte load or store moves in lane order, and in LDS, where a stage lies as in memory, sixteen lanes
+// read the same piece of sixteen rows from 256 consecutive bytes.
 struct HfPlanes {
   const hbits* base;
-  int rows;   // rows allocated (a multiple of the tiles' rows; rows past the matrix hold zeros)
+  int rows;
 };
+constexpr int kNsBlock = 16 * 16 * kNsPl;   // numbers of a block
 
-// element offset of (row, k) in plane 0; plane 1 is 16 elements further
-__device__ __forceinline__ size_t hf_off(int rows, int row, int k) {
-  return ((size_t)(k >> 4) * rows + row) * (16 * kNsPl) + (k & 15);
+// the block with row and reduction step (row, k), elements from the planes' first
+__device__ __forceinline__ size_t hf_block(int rows, int row, int k) {
+  return (size_t)(k >> 4) * rows * (16 * kNsPl) + (size_t)(row >> 4) * kNsBlock;
 }
 
 struct NsHfMat {
@@ -91,12 +92,11 @@ struct NsHfMat {
   int R, C, m, n, tall;      // X is R x C row-major; m = min, n = max; tall: R > C
   int pad_m, pad_n;          // m and n rounded up to the 16 reduction steps of a stage (the padding holds zeros)
   int rows_m, rows_n;        // rows allocated for the planes whose rows are the m / n index (whole tiles)
-  int lda;                   // row pitch of the fp32 A and of the partial matrices: m rounded up to 4
   int n_slabs;
   long long off_xs;          // elements (hbits) into the plane workspace: planes of Xs (m rows, reduction n)
   long long off_xl[2];       // planes of Xl (n rows, reduction m), two buffers (a product reads one and writes the other)
   long long off_p, p_stride; // planes of the m x m matrices (m rows, reduction m): buffer b at off_p + b p_stride
-  long long off_a;           // floats into the fp32 workspace: A (m x m)
+  long long off_a, a_floats; // floats into the fp32 workspace: A (hf_a32); its size, and a partial matrix's
   long long off_part;        // floats: partial matrices of a split Gram product
   long long elem_off;        // elements from the tensor's raw step to this matrix (a slice of a tensor with more dims)
   int fpart0, n_fpart;       // its partial sums of squares of A (k_ns_hf_chain_sumsq): first, count
@@ -110,43 +110,53 @@ enum : int { kNsProd = 3, kNsProdA = 4 };
 // product's values (the reciprocal of the operands' plane scales) and the scale of the planes written
 struct NsBufs { int s1, s2, d; float acc_scale, out_scale; };
 
-// x (already times its plane scale) = h + l + what is left below 2^-22 |x|.  The clamp never acts on a matrix
-// within the bounds the scales were chosen for; it keeps a stray value from becoming an infinity.
-__device__ __forceinline__ void hf_split(float x, hbits& h, hbits& l) {
-  const float c = __builtin_amdgcn_fmed3f(x, -65000.0f, 65000.0f);
-  x = x == x ? c : x;   // (the median of three takes a NaN for the smallest: keep it a NaN)
-  const _Float16 hb = (_Float16)x;
-  const _Float16 lb = (_Float16)(x - (float)hb);
-  h = __builtin_bit_cast(hbits, hb);
-  l = __builtin_bit_cast(hbits, lb);
+// The fp32 copy of a symmetric m x m matrix (and of the partial matrices that add up to it): the 128 x 128 tiles on and
+// above the diagonal, row by row, each as the accumulators of the job that computes it, [wave][hi][hj][r / 4][lane][r % 4]
+// -- the job that reads it again (Poly) is the same tile's, so both move 16 bytes a lane in lane order.
+__host__ __device__ __forceinline__ int hf_tiles_upper(int m) {
+  const int nt = (m + kNsTile - 1) / kNsTile;
+  return nt * (nt + 1) / 2;
+}
+__device__ __forceinline__ int hf_tile_index(int m, int tm, int tn) {
+  const int nt = (m + kNsTile - 1) / kNsTile;
+  return tm * nt - tm * (tm - 1) / 2 + tn - tm;
+}
+constexpr int kNsTileFloats = kNsTile * kNsTile;
+// floats from A's first to the lane's registers 4 q .. 4 q + 3 of sub-tile (hi, hj)
+__device__ __forceinline__ size_t hf_a32(int tile, int wave, int hi, int hj, int q, int lane) {
+  return ((((size_t)tile * 4 + wave) * 4 + hi * 2 + hj) * 4 + q) * 256 + lane * 4;
 }
 
-// A stage of one operand in LDS: [row][plane][half], 64 bytes a row, as in memory, except that the four
-// 16-byte pieces of a row are permuted: piece s of row r sits in slot s ^ ((r / 4) % 4), so that sixteen
-// consecutive rows, read one piece each by sixteen lanes, touch sixteen different 16-byte bank groups (rows 4
-// apart would share them).
-// A wave-wide load instruction moves 64 consecutive 16-byte pieces of the stage from global memory into LDS
-// (the hardware puts lane l's piece at the instruction's LDS base + 16 l); the permutation is done on the global
-// side: lane l fetches the piece whose place in LDS it fills.  ROWS x 4 pieces = ROWS x 4 / 256 instructions
-// per thread; `off[]` holds the lane's byte offsets into the stage in memory (they do not change with k).
+// Two values (times their plane scale already) as two dwords, one of each plane: x = h + l + what is left below 2^-22 |x|.
+// No clamp: a matrix within the bounds the scales were chosen for stays below 24 000, and what is not -- a raw step with an
+// infinity or a NaN, whose norm is neither -- has to stay visible.
+__device__ __forceinline__ void hf_split2(float a, float b, unsigned& h, unsigned& l) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  const h2 hh = __builtin_convertvector(f2{a, b}, h2);
+  const h2 ll = __builtin_convertvector(f2{a - (float)hh[0], b - (float)hh[1]}, h2);
+  h = __builtin_bit_cast(unsigned, hh);
+  l = __builtin_bit_cast(unsigned, ll);
+}
+
 #define PYLO_LDS __attribute__((address_space(3)))
 #define PYLO_GLB __attribute__((address_space(1)))
 
-// (NW: waves of the block)
+// A stage of ROWS rows of one operand from memory into LDS, as it lies there: one wave-wide load a block (the hardware
+// puts lane l's 16 bytes at the instruction's LDS base + 16 l), blocks dealt to the waves in turn.  `g`: the stage's first
+// byte plus 16 lane.  (NW: waves of the block)
 template <int ROWS, int NW = 4>
-__device__ __forceinline__ void hf_stage_offsets(int wave, int lane, int (&off)[ROWS * kNsRowPc / (64 * NW)]) {
+__device__ __forceinline__ void hf_stage_issue(const char* g, PYLO_LDS char* lds, int wave) {
 #pragma unroll
-  for (int j = 0; j < ROWS * kNsRowPc / (64 * NW); ++j) {
-    const int p = (j * NW + wave) * 64 + lane;
-    off[j] = (p ^ ((p >> 4) & 3)) * 16;   // row p / 4: its four pieces permuted by (row / 4) % 4
-  }
+  for (int j = 0; j < ROWS * kNsRowB / (1024 * NW); ++j)
+    __builtin_amdgcn_global_load_lds((const PYLO_GLB void*)(g + (j * NW + wave) * 1024), (PYLO_LDS void*)(lds + (j * NW + wave) * 1024), 16, 0, 0);
 }
 
-template <int ROWS, int NW = 4>
-__device__ __forceinline__ void hf_stage_issue(const char* g, const int (&off)[ROWS * kNsRowPc / (64 * NW)], PYLO_LDS char* lds, int wave) {
-#pragma unroll
-  for (int j = 0; j < ROWS * kNsRowPc / (64 * NW); ++j)
-    __builtin_amdgcn_global_load_lds((const PYLO_GLB void*)(g + off[j]), (PYLO_LDS void*)(lds + (j * NW + wave) * 1024), 16, 0, 0);
+// The lane's fragment of row `row0 + lane % 32` (row0 a multiple of 16) in a stage in LDS: byte offset of plane 0, plane 1 is
+// 256 bytes further, the row 32 further down 2048.
+__device__ __forceinline__ int hf_frag(int row0, int lane) {
+  const int lo = lane & 31, kg = lane >> 5;
+  return (row0 + (lo & 16)) * kNsRowB + kg * 512 + (lo & 15) * 16;
 }
 
 // acc[hi][hj] += (rows i0.. of P1) x (rows j0.. of P2)^T over the reduction range [k0, k1) (multiples of 16);
@@ -159,29 +169,23 @@ __device__ __forceinline__ void hf_tile_product(const HfPlanes& P1, int i0, cons
   constexpr int RA = 32 * NW, RB = 64 * WN, SA = RA * kNsRowB, STAGE = SA + RB * kNsRowB;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wi = (wave >> 1) * 64, wj = (wave & 1) * 32 * WN;
-  const int kg = lane >> 5, lo = lane & 31;
-  int offa[RA * kNsRowPc / (64 * NW)], offb[RB * kNsRowPc / (64 * NW)];
-  hf_stage_offsets<RA, NW>(wave, lane, offa);
-  hf_stage_offsets<RB, NW>(wave, lane, offb);
-  const char* ga = (const char*)P1.base + ((size_t)(k0 >> 4) * P1.rows + i0) * kNsRowB;
-  const char* gb = (const char*)P2.base + ((size_t)(k0 >> 4) * P2.rows + j0) * kNsRowB;
+  const char* ga = (const char*)P1.base + ((size_t)(k0 >> 4) * P1.rows + i0) * kNsRowB + 16 * lane;
+  const char* gb = (const char*)P2.base + ((size_t)(k0 >> 4) * P2.rows + j0) * kNsRowB + 16 * lane;
   const size_t sa = (size_t)P1.rows * kNsRowB, sb = (size_t)P2.rows * kNsRowB;
   // a diagonal tile of X X^T or A A: both operands are the same 128 rows, staged once
   const bool same = WN == 2 && P1.base == P2.base && i0 == j0;
-  hf_stage_issue<RA, NW>(ga, offa, lds, wave);
-  if (!same) hf_stage_issue<RB, NW>(gb, offb, lds + SA, wave);
+  hf_stage_issue<RA, NW>(ga, lds, wave);
+  if (!same) hf_stage_issue<RB, NW>(gb, lds + SA, wave);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  // the lane's rows are lo, lo + 32, ..: all with the same (row / 4) % 4; plane q, half kg is piece 2 q + kg
-  const int sw = 16 * (kg ^ ((lo >> 2) & 3));
-  const int oa = (wi + lo) * kNsRowB + sw, ob = (same ? 0 : SA) + (wj + lo) * kNsRowB + sw;
+  const int oa = hf_frag(wi, lane), ob = (same ? 0 : SA) + hf_frag(wj, lane);
   int cur = 0;
   for (int k = k0; k < k1; k += kHfBK) {
     if (k + kHfBK < k1) {
       ga += sa;
       gb += sb;
-      hf_stage_issue<RA, NW>(ga, offa, lds + (STAGE - cur), wave);
-      if (!same) hf_stage_issue<RB, NW>(gb, offb, lds + (STAGE - cur) + SA, wave);
+      hf_stage_issue<RA, NW>(ga, lds + (STAGE - cur), wave);
+      if (!same) hf_stage_issue<RB, NW>(gb, lds + (STAGE - cur) + SA, wave);
     }
     if (compute) {
       f16x8 a[2][kNsPl], b[WN][kNsPl];
@@ -189,10 +193,10 @@ __device__ __forceinline__ void hf_tile_product(const HfPlanes& P1, int i0, cons
       for (int q = 0; q < kNsPl; ++q) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-          a[i][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + cur + ((oa + i * 32 * kNsRowB) ^ (q * 32))));
+          a[i][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + cur + oa + i * 32 * kNsRowB + q * 256));
 #pragma unroll
         for (int j = 0; j < WN; ++j)
-          b[j][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + cur + ((ob + j * 32 * kNsRowB) ^ (q * 32))));
+          b[j][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + cur + ob + j * 32 * kNsRowB + q * 256));
       }
       // smallest terms first: l h, h l, h h
 #pragma unroll
@@ -226,27 +230,24 @@ __device__ __forceinline__ void hf_tile_product_direct(const HfPlanes& P1, int i
   typedef PYLO_GLB u32x4 gu32x4;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wi = (wave >> 1) * 64, wj = (wave & 1) * 32 * WN;
-  const int kg = lane >> 5, lo = lane & 31;
-  int offb[RB * kNsRowPc / 256];
-  hf_stage_offsets<RB>(wave, lane, offb);
-  const char* ga = (const char*)P1.base + ((size_t)(k0 >> 4) * P1.rows + i0 + wi + lo) * kNsRowB + 16 * kg;
-  const char* gb = (const char*)P2.base + ((size_t)(k0 >> 4) * P2.rows + j0) * kNsRowB;
+  const char* ga = (const char*)P1.base + ((size_t)(k0 >> 4) * P1.rows + i0) * kNsRowB + hf_frag(wi, lane);
+  const char* gb = (const char*)P2.base + ((size_t)(k0 >> 4) * P2.rows + j0) * kNsRowB + 16 * lane;
   const size_t sa = (size_t)P1.rows * kNsRowB, sb = (size_t)P2.rows * kNsRowB;
   u32x4 an[2][2][kNsPl];   // the fragments of this step and the next (slot = step % 2), refilled for two steps on
   auto fetch_a = [&](auto slot, const char* g) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int q = 0; q < kNsPl; ++q) an[slot.value][i][q] = *(const gu32x4*)(g + i * 32 * kNsRowB + q * 32);
+      for (int q = 0; q < kNsPl; ++q) an[slot.value][i][q] = *(const gu32x4*)(g + i * 32 * kNsRowB + q * 256);
   };
   typedef std::integral_constant<int, 0> S0;
   typedef std::integral_constant<int, 1> S1;
-  hf_stage_issue<RB>(gb, offb, lds, wave);
+  hf_stage_issue<RB>(gb, lds, wave);
   fetch_a(S0(), ga);
   if (k0 + kHfBK < k1) fetch_a(S1(), ga + sa);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  const int ob = (wj + lo) * kNsRowB + 16 * (kg ^ ((lo >> 2) & 3));
+  const int ob = hf_frag(wj, lane);
   int cur = 0;
   ga += sa;
   auto step = [&](auto slot, int k) {
@@ -258,7 +259,7 @@ __device__ __forceinline__ void hf_tile_product_direct(const HfPlanes& P1, int i
     const bool more_b = k + kHfBK < k1, more_a = k + 2 * kHfBK < k1;
     if (more_b) {
       gb += sb;
-      hf_stage_issue<RB>(gb, offb, lds + (STAGE - cur), wave);
+      hf_stage_issue<RB>(gb, lds + (STAGE - cur), wave);
     }
     if (more_a) {
       ga += sa;
@@ -268,7 +269,7 @@ __device__ __forceinline__ void hf_tile_product_direct(const HfPlanes& P1, int i
     for (int q = 0; q < kNsPl; ++q)
 #pragma unroll
       for (int j = 0; j < WN; ++j)
-        b[j][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + cur + ((ob + j * 32 * kNsRowB) ^ (q * 32))));
+        b[j][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + cur + ob + j * 32 * kNsRowB + q * 256));
 #pragma unroll
     for (int term = 0; term < 3; ++term) {
       constexpr int pa[3] = {1, 0, 0}, pb[3] = {0, 1, 0};
@@ -294,75 +295,94 @@ __device__ __forceinline__ void hf_tile_product_direct(const HfPlanes& P1, int i
   }
 }
 
-// one value (times its plane scale already) into both planes
-__device__ __forceinline__ void hf_store1(hbits* base, int rows, int row, int k, float v) {
-  hbits h, l;
-  hf_split(v, h, l);
-  hbits* p = base + hf_off(rows, row, k);
-  p[0] = h;
-  p[16] = l;
-}
-
-// The block's 128 x 64 WN values (accumulator layout) times `scale` into planes, in one or both orientations, every
-// value split once.
-//   D   planes whose reduction index is the tile's column index: through the wave's own LDS patch
-//       ([row][plane][32 WN columns], 2 bytes each), 16 rows at a time; the wave reads the patch back as
-//       16-byte pieces in the order the planes have in memory ([16 columns][row][plane][half]: 64 pieces for the
-//       patch's 16 rows, one a lane).
-//   D4  (when not null) planes whose reduction index is the tile's row index: four consecutive rows of a
-//       lane are four consecutive reduction indices, one 8-byte store per plane straight from the registers.
-// Only the lanes of one wave meet in a patch and a wave's LDS instructions execute in order, so the passes
-// need no barrier, just the compiler kept from moving the reads over the writes.
-template <int WN>
-__device__ __forceinline__ void hf_store_planes(PYLO_LDS char* lds, const v16f (&acc)[2][WN], hbits* __restrict__ D,
-                                                int rows_total, int i0, int j0, int n_rows, int n_cols,
+// A wave's 32 HI x 32 WN values (accumulator layout) times `scale` into planes, in one or both orientations, every value
+// split once.  Rows and columns past the matrix hold zeros (hf_mask_edge).
+//   D   planes whose reduction index is the values' column: through the wave's own LDS patch, [column][16 rows] a plane,
+//       sixteen rows at a time, read back transposed (ds_read_b64_tr_b16: of the 4 columns x 16 rows that sixteen lanes
+//       address, lane i gets row i's four columns)
+//   D4  (when not null) planes whose reduction index is the row: straight from the registers
+// A lane's two quads of sixteen rows (8 g + 4 (lane / 32) ..) become eight consecutive ones by one swap between the
+// halves of the wave: 16 bytes of a plane, LDS takes them as they are, and one more swap between neighbouring sixteens of
+// lanes puts the pieces of sixteen columns into the order of a block: every store is 1 KB in lane order.  Before, the mirrored
+// planes went out 8 bytes a lane, 64 apart, and the others 2 bytes a value into the patch.  GPT-2-small set, one stream,
+// before / now: update 640 / 553 us, Gram 386 / 374, Poly (whose fp32 A was a dword a load) 161 / 113, A' 152 / 126, other
+// m x m products 124 / 116, the split of the raw steps 328 / 277; whole ELO-CELO2 step 6.65 / 6.23 ms, CELO2 on ResNet-50
+// 1.63 / 1.49 ms.
+// Only the lanes of one wave meet in a patch (2 KB a 32 columns) and a wave's LDS instructions execute in order, so the
+// passes need no barrier, just the compiler kept from moving the reads over the writes.
+template <int HI, int WN>
+__device__ __forceinline__ void hf_store_planes(PYLO_LDS char* patch, const v16f (&acc)[HI][WN], hbits* __restrict__ D,
+                                                int rows_d, int wi, int wj, int n_rows, int n_cols,
                                                 hbits* __restrict__ D4, int rows4, float scale) {
-  constexpr int kPlane = 64 * WN + 16;        // bytes: 32 WN columns x 2 + 16 (bank spread)
-  constexpr int kRow = kNsPl * kPlane, kWave = 16 * kRow;
-  typedef PYLO_LDS hbits lbf;
-  typedef unsigned long long u64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  PYLO_LDS char* patch = lds + wave * kWave;
-  const int wi = i0 + (wave >> 1) * 64, wj = j0 + (wave & 1) * 32 * WN;   // origin of the wave's values
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  typedef PYLO_LDS s16x4 ls4;
+  const int lane = threadIdx.x & 63;
+  PYLO_LDS char* const put = patch + (lane & 31) * 32 + (lane >> 5) * 16;
+  // the block's piece that the lane stores: sixteen lanes a (half, plane)
+  PYLO_LDS char* const get = patch + ((lane >> 4) & 1) * 1024 + (lane >> 5) * 256 + (lane & 15) * 8;
 #pragma unroll
-  for (int pass = 0; pass < 4; ++pass) {
-    const int hi = pass >> 1, half = pass & 1;   // rows 32 hi + 16 half .. + 15 of the wave's 64
+  for (int pass = 0; pass < 2 * HI; ++pass) {
+    const int hi = pass >> 1, b = pass & 1, row = wi + 32 * hi + 16 * b;
+    if (row >= n_rows) break;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the patch is free: the previous pass has read it
 #pragma unroll
-    for (int hj = 0; hj < WN; ++hj)
+    for (int hj = 0; hj < WN; ++hj) {
+      const v16f& v = acc[hi][hj];
+      u32x4 h, l;
 #pragma unroll
-      for (int g4 = 0; g4 < 2; ++g4) {
-        hbits h[4], l[4];
-        const int col_l = 32 * hj + (lane & 31);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          hf_split(acc[hi][hj][8 * half + 4 * g4 + r] * scale, h[r], l[r]);
-          lbf* q = (lbf*)(patch + (8 * g4 + 4 * (lane >> 5) + r) * kRow + col_l * 2);
-          q[0] = h[r];
-          q[kPlane / 2] = l[r];
-        }
-        if (D4 != nullptr) {
-          const int row = wi + 32 * hi + 16 * half + 8 * g4 + 4 * (lane >> 5), col = wj + col_l;
-          if (col < n_cols && row < n_rows) {   // values past n_rows are zeros, into the padding
-            hbits* p = D4 + hf_off(rows4, col, row);
-            *(u64*)p = (u64)h[0] | (u64)h[1] << 16 | (u64)h[2] << 32 | (u64)h[3] << 48;
-            *(u64*)(p + 16) = (u64)l[0] | (u64)l[1] << 16 | (u64)l[2] << 32 | (u64)l[3] << 48;
-          }
-        }
+      for (int u = 0; u < 4; ++u) {
+        unsigned h1, l1;
+        hf_split2(v[8 * b + 2 * u] * scale, v[8 * b + 2 * u + 1] * scale, h1, l1);
+        h[u] = h1;
+        l[u] = l1;
       }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    const int row_w0 = wi + 32 * hi + 16 * half;
 #pragma unroll
-    for (int c = 0; c < 2 * WN; ++c) {     // 16 columns = one block of the planes' layout
+      for (int u = 0; u < 2; ++u) {
+        const u32x2 a = __builtin_amdgcn_permlane32_swap(h[u], h[u + 2], false, false);
+        const u32x2 c = __builtin_amdgcn_permlane32_swap(l[u], l[u + 2], false, false);
+        h[u] = a[0]; h[u + 2] = a[1];
+        l[u] = c[0]; l[u + 2] = c[1];
+      }
+      *(luint4*)(put + hj * 2048) = h;
+      *(luint4*)(put + hj * 2048 + 1024) = l;
+      if (D4 != nullptr) {
+        const int col = wj + 32 * hj;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const u32x2 a = __builtin_amdgcn_permlane16_swap(h[u], l[u], false, false);
+          h[u] = a[0];
+          l[u] = a[1];
+        }
+        hbits* p = D4 + hf_block(rows4, col, row) + lane * 8;
+        if (col < n_cols) *(u32x4*)p = h;
+        if (col + 16 < n_cols) *(u32x4*)(p + kNsBlock) = l;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int c = 0; c < 2 * WN; ++c) {     // 16 columns = one block
       const int col = wj + 16 * c;
       if (col >= n_cols) continue;
-      hbits* dst = D + hf_off(rows_total, row_w0, col);
-      const int row_l = lane >> 2, plane = (lane >> 1) & 1, hf = lane & 1;   // piece `lane` of [row][plane][half]
-      if (row_w0 + row_l >= n_rows) continue;
-      const u32x4 w = *(const luint4*)(patch + row_l * kRow + plane * kPlane + (16 * c + 8 * hf) * 2);
-      *(u32x4*)(dst + (size_t)lane * 8) = w;
+      const s16x4 w0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls4*)(get + c * 512 + (c >> 1) * 1024));
+      const s16x4 w1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls4*)(get + c * 512 + (c >> 1) * 1024 + 128));
+      const u32x2 x = __builtin_bit_cast(u32x2, w0), y = __builtin_bit_cast(u32x2, w1);
+      *(u32x4*)(D + hf_block(rows_d, row, col) + lane * 8) = u32x4{x[0], x[1], y[0], y[1]};
     }
   }
+}
+
+// Values past the matrix's edge are products of padding: zeros, unless a NaN or an infinity met them.
+template <int HI, int WN>
+__device__ __forceinline__ void hf_mask_edge(v16f (&acc)[HI][WN], int wi, int wj, int n_rows, int n_cols) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < HI; ++i)
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (wi + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3) >= n_rows || wj + 32 * j + (lane & 31) >= n_cols) acc[i][j][r] = 0.0f;
 }
 
 // One launch = one product of one iteration, for every tensor (see the head of this file).
@@ -404,7 +424,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WN == 4 ? 2
   const NsHfMat mt = mats[it.mat];
   const PyloTensorArgs a = dyn[mt.tensor];
   if (a.grad == nullptr || !(a.flags & kArgOrthogonalize)) return;
-  const int m = mt.m, n = mt.n, lda = mt.lda;
+  const int m = mt.m, n = mt.n;
   v16f acc[2][WN];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -441,101 +461,130 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WN == 4 ? 2
     for (int j = 0; j < WN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] *= bufs.acc_scale;
-  float* A32 = ws + mt.off_a;
   const int n_i = OP == kNsUpdate ? n : m;   // rows of the output; its columns are always m
   const bool partial = OP == kNsGram && it.slab >= 0;
-  const bool mirror = OP != kNsUpdate && !partial && (it.tm != it.tn || wave_u == 1);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  float* xout = a.step_out + mt.elem_off;
-  const bool vec_out = (mt.C & 3) == 0;   // rows of the tensor are 16-byte aligned
-  // fp32 outputs (and Poly's transform of the accumulators) straight from the registers
-  if (OP == kNsGram || OP == kNsPoly || OP == kNsProdA || (OP == kNsUpdate && last)) {
+  const bool mirror = OP != kNsUpdate && (it.tm != it.tn || wave_u == 1);
+  const int lane = threadIdx.x & 63;
+  const int wi = i0 + (wave_u >> 1) * 64, wj = j0 + (wave_u & 1) * 32 * WN;   // origin of the wave's values
+  if (wi + 64 > n_i || wj + 32 * WN > m) hf_mask_edge<2, WN>(acc, wi, wj, n_i, m);
+  if (OP == kNsGram || OP == kNsPoly || OP == kNsProdA) {
+    // the fp32 A: written, or Poly's transform of the accumulators
+    float* A = ws + (partial ? mt.off_part + (size_t)it.slab * mt.a_floats : mt.off_a) + hf_a32(hf_tile_index(m, it.tm, it.tn), wave_u, 0, 0, 0, lane);
 #pragma unroll
     for (int hi = 0; hi < 2; ++hi)
 #pragma unroll
-      for (int hj = 0; hj < WN; ++hj) {
-        const int col = j0 + (wave & 1) * 32 * WN + hj * 32 + (lane & 31);
+      for (int hj = 0; hj < WN; ++hj)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int row = i0 + ns_acc_row(hi, 4 * q);   // rows row .. row + 3
-          if (col >= m || row >= n_i) continue;
-          float v[4];
+          gv4f* p = (gv4f*)(A + ((hi * 2 + hj) * 4 + q) * 256);
+          if (OP == kNsPoly) {
+            const v4f aij = *p;
+            const int d = wj + hj * 32 + (lane & 31) - (wi + hi * 32 + 8 * q + 4 * (lane >> 5));   // the register on the diagonal, if 0 .. 3
+            const bool in = wj + hj * 32 + (lane & 31) < m;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            float x = acc[hi][hj][4 * q + r];
-            if (OP == kNsPoly) {
-              const bool in = row + r < m;
-              const float aij = in ? A32[(size_t)(row + r) * lda + col] : 0.0f;
-              x = in ? c2 * x + c1 * aij + ((row + r) == col ? c0 : 0.0f) : 0.0f;
+            for (int r = 0; r < 4; ++r) {
+              float x = acc[hi][hj][4 * q + r];
+              x = c2 * x + c1 * aij[r] + (d == r && in ? c0 : 0.0f);
               acc[hi][hj][4 * q + r] = x;
             }
-            v[r] = x;
-          }
-          if (OP == kNsGram || OP == kNsProdA) {
-            float* out = partial ? ws + mt.off_part + (size_t)it.slab * m * lda : A32;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (row + r < m) out[(size_t)(row + r) * lda + col] = v[r];
-            if (mirror) *(gv4f*)(out + (size_t)col * lda + row) = v4f{v[0], v[1], v[2], v[3]};   // past m: zeros into the pitch's padding
-          } else if (OP == kNsUpdate) {
-            if (mt.tall) {   // X = Xl, n x m
-#pragma unroll
-              for (int r = 0; r < 4; ++r)
-                if (row + r < n) xout[(size_t)(row + r) * m + col] = v[r];
-            } else if (vec_out) {   // X = Xs, m x n: four consecutive columns of row `col` (n is a multiple of 4)
-              *(gv4f*)(xout + (size_t)col * n + row) = v4f{v[0], v[1], v[2], v[3]};
-            } else {
-#pragma unroll
-              for (int r = 0; r < 4; ++r)
-                if (row + r < n) xout[(size_t)col * n + row + r] = v[r];
-            }
+          } else {
+            *p = v4f{acc[hi][hj][4 * q], acc[hi][hj][4 * q + 1], acc[hi][hj][4 * q + 2], acc[hi][hj][4 * q + 3]};
           }
         }
-      }
+    if (partial) return;
   }
-  // planes: A and B' in both halves (the tile itself through LDS, the mirrored tile from the registers), Xl'
-  // (through LDS) and Xs' (registers)
-  if (partial || (OP == kNsUpdate && last)) return;
+  if (OP == kNsUpdate && last) {
+    // fp32 X in place of the raw step
+    float* xout = a.step_out + mt.elem_off;
+    if (!mt.tall && (mt.C & 3) == 0) {
+      // X = Xs, m x n, 16-byte aligned rows: 32 x 32 values through the wave's LDS patch (rows of 36 floats), so that eight
+      // lanes store 128 consecutive bytes of a row
+      typedef PYLO_LDS v4f lv4f;
+      PYLO_LDS char* patch = lds + wave_u * (32 * 144);
+#pragma unroll
+      for (int hi = 0; hi < 2; ++hi)
+#pragma unroll
+        for (int hj = 0; hj < WN; ++hj) {
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            *(lv4f*)(patch + (lane & 31) * 144 + 32 * q + 16 * (lane >> 5)) =
+                v4f{acc[hi][hj][4 * q], acc[hi][hj][4 * q + 1], acc[hi][hj][4 * q + 2], acc[hi][hj][4 * q + 3]};
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int cl = 8 * q + (lane >> 3), col = wj + hj * 32 + cl, row = wi + hi * 32 + 4 * (lane & 7);
+            const v4f v = *(lv4f*)(patch + cl * 144 + 16 * (lane & 7));
+            if (col < m && row < n) *(gv4f*)(xout + (size_t)col * n + row) = v;
+          }
+        }
+    } else {
+#pragma unroll
+      for (int hi = 0; hi < 2; ++hi)
+#pragma unroll
+        for (int hj = 0; hj < WN; ++hj) {
+          const int col = wj + hj * 32 + (lane & 31);
+          if (col >= m) continue;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int row = wi + hi * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+            if (row < n) xout[mt.tall ? (size_t)row * m + col : (size_t)col * n + row] = acc[hi][hj][r];
+          }
+        }
+    }
+    return;
+  }
+  // planes: A and B' in both halves (the mirrored tile is the other orientation), Xl' and Xs'
+  PYLO_LDS char* patch = lds + wave_u * (2048 * WN);
   if (OP == kNsUpdate) {
-    hf_store_planes<WN>(lds, acc, pw + (par ? mt.off_xl[0] : mt.off_xl[1]), mt.rows_n, i0, j0, n, m, pw + mt.off_xs, mt.rows_m,
-                        bufs.out_scale);
+    hf_store_planes<2, WN>(patch, acc, pw + (par ? mt.off_xl[0] : mt.off_xl[1]), mt.rows_n, wi, wj, n, m, pw + mt.off_xs, mt.rows_m,
+                           bufs.out_scale);
   } else {
     hbits* D = pw + mt.off_p + (OP == kNsGram ? (int)kNsBufA : bufs.d) * mt.p_stride;
-    hf_store_planes<WN>(lds, acc, D, mt.rows_m, i0, j0, m, m, mirror ? D : nullptr, mt.rows_m, bufs.out_scale);
+    hf_store_planes<2, WN>(patch, acc, D, mt.rows_m, wi, wj, m, m, mirror ? D : nullptr, mt.rows_m, bufs.out_scale);
   }
 }
 
-// A = sum over the slabs' partial matrices, in slab order, as fp32 and as planes (both halves).
-__global__ __launch_bounds__(256) void k_ns_hf_gram_reduce(const NsHfMat* __restrict__ mats, const int* __restrict__ split_mats,
-                                                           const PyloTensorArgs* __restrict__ dyn, float* __restrict__ ws,
-                                                           hbits* __restrict__ pw, NsPick pick, float out_scale) {
+// A = sum over the slabs' partial matrices, in slab order, as fp32 and as planes (both halves): a wave for each 32 x 32 of
+// the tiles on and above the diagonal.
+__global__ __launch_bounds__(64) void k_ns_hf_gram_reduce(const NsHfMat* __restrict__ mats, const int* __restrict__ split_mats,
+                                                          const PyloTensorArgs* __restrict__ dyn, float* __restrict__ ws,
+                                                          hbits* __restrict__ pw, NsPick pick, float out_scale) {
+  __shared__ __attribute__((aligned(16))) char patch[2048];
   if (pick.sel == kNsShortOnly && pick.flags[split_mats[blockIdx.y]] != 0) return;
   const NsHfMat mt = mats[split_mats[blockIdx.y]];
   const PyloTensorArgs a = dyn[mt.tensor];
   if (a.grad == nullptr || !(a.flags & kArgOrthogonalize)) return;
-  const int m = mt.m, lda = mt.lda;
-  const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (e >= (long long)m * m) return;
-  const int i = (int)(e / m), j = (int)(e - (long long)i * m);
-  if (i / 64 > j / 64) return;   // the Gram jobs compute the 64 x 64 blocks on and above the diagonal
-  const size_t mm = (size_t)m * lda;
-  const float* p = ws + mt.off_part + (size_t)i * lda + j;
-  float s = 0.0f;
-  for (int q0 = 0; q0 < mt.n_slabs; q0 += 8) {
-    float v[8];
+  const int m = mt.m, nt = (m + kNsTile - 1) / kNsTile, lane = threadIdx.x;
+  const int tile = blockIdx.x >> 4, wave = (blockIdx.x >> 2) & 3, hi = (blockIdx.x >> 1) & 1, hj = blockIdx.x & 1;
+  if (tile >= hf_tiles_upper(m)) return;
+  int tm = 0, left = tile;
+  while (left >= nt - tm) left -= nt - tm++;
+  const int tn = tm + left;
+  if (tm == tn && wave == 2) return;   // the mirror image of wave 1's
+  const int wi = tm * kNsTile + (wave >> 1) * 64 + hi * 32, wj = tn * kNsTile + (wave & 1) * 64 + hj * 32;
+  const size_t e = hf_a32(tile, wave, hi, hj, 0, lane);
+  const float* p = ws + mt.off_part + e;
+  v16f acc[1][1];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = q0 + q < mt.n_slabs ? *(const gfloat*)(p + (size_t)(q0 + q) * mm) : 0.0f;
+  for (int r = 0; r < 16; ++r) acc[0][0][r] = 0.0f;
+  for (int s0 = 0; s0 < mt.n_slabs; s0 += 4) {
+    v4f v[4][4];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) s += v[q];
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        v[u][q] = s0 + u < mt.n_slabs ? *(const gv4f*)(p + (size_t)(s0 + u) * mt.a_floats + q * 256) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[0][0][r] += v[u][r >> 2][r & 3];
   }
-  float* A = ws + mt.off_a;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    *(gv4f*)(ws + mt.off_a + e + q * 256) = v4f{acc[0][0][4 * q], acc[0][0][4 * q + 1], acc[0][0][4 * q + 2], acc[0][0][4 * q + 3]};
   hbits* P = pw + mt.off_p;   // buffer A
-  A[(size_t)i * lda + j] = s;
-  hf_store1(P, mt.rows_m, i, j, s * out_scale);
-  if (i / 64 != j / 64) {
-    A[(size_t)j * lda + i] = s;
-    hf_store1(P, mt.rows_m, j, i, s * out_scale);
-  }
+  hf_store_planes<1, 1>((PYLO_LDS char*)patch, acc, P, mt.rows_m, wi, wj, m, m, tm != tn || wave == 1 ? P : nullptr, mt.rows_m, out_scale);
 }
 
 // X0 = raw * s (s = 1 / (||raw|| + eps), scale[mat]) as planes in both layouts.  One block = one 64 x 64
@@ -545,9 +594,8 @@ __global__ __launch_bounds__(256) void k_ns_hf_gram_reduce(const NsHfMat* __rest
 // the largest eigenvalue of A from above; what a chain of three iterations adds to the error of the result is
 // proportional to it, 196 eps_A lambda_max against 16 eps_A lambda_max for a pair (head of this file), so three
 // iterations are taken where ||A||_F^2 <= tau^2, with tau = 16 / 196: no worse there than a pair is on any matrix.
-// Two launches, sums in a fixed order: 4096 elements of A per block, then one block per matrix.
-constexpr int kNsFlagChunk = 4096;
-// items[b] = {matrix, chunk of 4096 elements of its A}
+// Two launches, sums in a fixed order: 64 x 64 elements of A per block, then one block per matrix.
+// items[b] = {matrix, 64 x 64 part (tile x 4 + wave) of its fp32 A}: parts off the diagonal count twice
 __global__ __launch_bounds__(256) void k_ns_hf_chain_sumsq(const NsHfMat* __restrict__ mats, const Item* __restrict__ items,
                                                            const PyloTensorArgs* __restrict__ dyn, const float* __restrict__ ws,
                                                            float* __restrict__ part) {
@@ -556,21 +604,24 @@ __global__ __launch_bounds__(256) void k_ns_hf_chain_sumsq(const NsHfMat* __rest
   const NsHfMat mt = mats[it.tensor];
   const PyloTensorArgs a = dyn[mt.tensor];
   if (a.grad == nullptr || !(a.flags & kArgOrthogonalize)) return;
-  const long long mm = (long long)mt.m * mt.m, e0 = (long long)it.a * kNsFlagChunk;
-  const float* A = ws + mt.off_a;
+  const int nt = (mt.m + kNsTile - 1) / kNsTile, wave = it.a & 3;
+  int tm = 0, left = it.a >> 2;
+  while (left >= nt - tm) left -= nt - tm++;
+  if (left == 0 && wave == 2) {   // the mirror image of wave 1's, which nobody writes
+    if (threadIdx.x == 0) part[mt.fpart0 + it.a] = 0.0f;
+    return;
+  }
+  const float* A = ws + mt.off_a + (size_t)it.a * 4096;
   float s = 0.0f;
-  for (int i = 0; i < kNsFlagChunk / 256; ++i) {
-    const long long e = e0 + threadIdx.x + 256 * i;
-    if (e < mm) {
-      const int r = (int)(e / mt.m), c = (int)(e - (long long)r * mt.m);
-      const float v = *(const gfloat*)(A + (size_t)r * mt.lda + c);
-      s = fmaf(v, v, s);
-    }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const v4f v = *(const gv4f*)(A + 1024 * i + 4 * threadIdx.x);
+    s = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, s))));
   }
   s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) part[mt.fpart0 + it.a] = (red[0] + red[1]) + (red[2] + red[3]);
+  if (threadIdx.x == 0) part[mt.fpart0 + it.a] = (left > 0 || wave == 1 ? 2.0f : 1.0f) * ((red[0] + red[1]) + (red[2] + red[3]));
 }
 
 __global__ __launch_bounds__(64) void k_ns_hf_chain_flag(const NsHfMat* __restrict__ mats, const int* __restrict__ list,
@@ -607,17 +658,14 @@ __global__ __launch_bounds__(256) void k_ns_hf_split(const NsHfMat* __restrict__
   const int rows_d = mt.tall ? mt.rows_n : mt.rows_m, rows_t = mt.tall ? mt.rows_m : mt.rows_n;
   const int r0 = it.tr * 64, c0 = it.tc * 64;
   const int t = threadIdx.x;
-  // Eight consecutive columns of one row a lane and pass: 32 bytes read, one 16-byte piece per plane written
-  // to the direct planes (the two lanes of a 16-column block fill its 64 bytes) and to the tile in LDS.
-  // Columns and rows past the matrix read as zero; where a piece straddles the edge the zeros land in the
-  // planes' padding, which holds zeros anyway.
+  // Eight consecutive columns of one row a lane and pass: 32 bytes read, 16 bytes per plane into the tile in LDS.  Columns and
+  // rows past the matrix are zeros, which land in the planes' padding.
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
     const int u = pass * 256 + t, lr = u >> 3, lc = 8 * (u & 7);
     const int r = r0 + lr, c = c0 + lc;
     float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    const bool in = r < R && c < C;
-    if (in) {
+    if (r < R && c < C) {
       const float* src = raw + (size_t)r * C + c;
       if (vec_in) {
         const v4f x = *(const gv4f*)src;
@@ -632,42 +680,33 @@ __global__ __launch_bounds__(256) void k_ns_hf_split(const NsHfMat* __restrict__
           if (c + e < C) v[e] = *(const gfloat*)(src + e) * s;
       }
     }
-    u32x4 pl[kNsPl];
+    u32x4 h, l;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      hbits h0, l0, h1, l1;
-      hf_split(v[2 * q], h0, l0);
-      hf_split(v[2 * q + 1], h1, l1);
-      pl[0][q] = (unsigned)h0 | (unsigned)h1 << 16;
-      pl[1][q] = (unsigned)l0 | (unsigned)l1 << 16;
+      unsigned h1, l1;
+      hf_split2(v[2 * q], v[2 * q + 1], h1, l1);
+      h[q] = h1;
+      l[q] = l1;
     }
-#pragma unroll
-    for (int q = 0; q < kNsPl; ++q) *(luint4*)&tile[q][lr][lc] = pl[q];
-    if (in) {
-      hbits* p = direct + hf_off(rows_d, r, c);
-#pragma unroll
-      for (int q = 0; q < kNsPl; ++q) *(u32x4*)(p + 16 * q) = pl[q];
-    }
+    *(luint4*)&tile[0][lr][lc] = h;
+    *(luint4*)&tile[1][lr][lc] = l;
   }
   __syncthreads();
-  // transposed: a lane takes one column and sixteen rows of the tile, i.e. one row and one 16-step block of
-  // the transposed planes: 64 consecutive bytes, and the lanes of a wave (consecutive columns) the next 64
-  {
-    const int lc = t & 63, rb = t >> 6;
-    const int c = c0 + lc, r = r0 + 16 * rb;
-    if (c < C && r < R) {
-      hbits* p = transp + hf_off(rows_t, c, r);
+  // Sixteen blocks of each orientation, four a wave (those of sixteen rows of the tile), every store a block in lane order:
+  // sixteen lanes a (half, plane).  Transposed pieces are read with ds_read_b64_tr_b16 (lane i of sixteen gets column i of four rows).
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  typedef PYLO_LDS s16x4 ls4;
+  const int lane = t & 63, rb = 16 * (t >> 6), plane = (lane >> 4) & 1, half = lane >> 5, i = lane & 15;
+  if (r0 + rb >= R) return;
 #pragma unroll
-      for (int q = 0; q < kNsPl; ++q)
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-          u32x4 w;
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            w[i] = (unsigned)tile[q][16 * rb + 8 * hf + 2 * i][lc] | (unsigned)tile[q][16 * rb + 8 * hf + 2 * i + 1][lc] << 16;
-          *(u32x4*)(p + 16 * q + 8 * hf) = w;
-        }
-    }
+  for (int cb = 0; cb < 64; cb += 16) {
+    if (c0 + cb >= C) break;
+    *(u32x4*)(direct + hf_block(rows_d, r0 + rb, c0 + cb) + lane * 8) = *(const luint4*)&tile[plane][rb + i][cb + 8 * half];
+    const s16x4 w0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls4*)&tile[plane][rb + 8 * half + (i >> 2)][cb + 4 * (i & 3)]);
+    const s16x4 w1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls4*)&tile[plane][rb + 8 * half + 4 + (i >> 2)][cb + 4 * (i & 3)]);
+    const u32x2 x = __builtin_bit_cast(u32x2, w0), y = __builtin_bit_cast(u32x2, w1);
+    *(u32x4*)(transp + hf_block(rows_t, c0 + cb, r0 + rb) + lane * 8) = u32x4{x[0], x[1], y[0], y[1]};
   }
 }
 

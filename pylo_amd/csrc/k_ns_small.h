@@ -170,17 +170,6 @@ __device__ __forceinline__ void sm_product(const PYLO_LDS char* a, int ra, int p
   if (k < ks) multiply(0);
 }
 
-// Two values as two dwords, one of each plane.  No clamp: nothing here leaves the bounds that the scales were chosen
-// for (a matrix enters with unit norm), and an infinite raw step has an infinite norm and becomes NaN before this.
-__device__ __forceinline__ void sm_split2(float a, float b, unsigned& h, unsigned& l) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  const h2 hh = __builtin_convertvector(f2{a, b}, h2);
-  const h2 ll = __builtin_convertvector(f2{a - (float)hh[0], b - (float)hh[1]}, h2);
-  h = __builtin_bit_cast(unsigned, hh);
-  l = __builtin_bit_cast(unsigned, ll);
-}
-
 // A tile into planes whose contiguous index is the tile's row: element (row, col) at [col][row].  Groups of rows from
 // `ng` on are zero and only the first `nz` are read as reduction steps.
 __device__ __forceinline__ void sm_put_t(PYLO_LDS char* buf, int pitch, int plane, int row0, int col0, int ng, int nz,
@@ -195,8 +184,8 @@ __device__ __forceinline__ void sm_put_t(PYLO_LDS char* buf, int pitch, int plan
     u32x2 h = {0u, 0u}, l = {0u, 0u};
     if (g < ng) {
       unsigned h0, l0, h1, l1;
-      sm_split2(v[4 * g] * s, v[4 * g + 1] * s, h0, l0);
-      sm_split2(v[4 * g + 2] * s, v[4 * g + 3] * s, h1, l1);
+      hf_split2(v[4 * g] * s, v[4 * g + 1] * s, h0, l0);
+      hf_split2(v[4 * g + 2] * s, v[4 * g + 3] * s, h1, l1);
       h = u32x2{h0, h1};
       l = u32x2{l0, l1};
     }
@@ -217,7 +206,7 @@ __device__ __forceinline__ void sm_put_n(PYLO_LDS char* buf, int pitch, int plan
 #pragma unroll
     for (int r = 0; r < 4; r += 2) {
       unsigned h, l;
-      sm_split2(v[4 * g + r] * s, v[4 * g + r + 1] * s, h, l);
+      hf_split2(v[4 * g + r] * s, v[4 * g + r + 1] * s, h, l);
       PYLO_LDS char* o = p + (8 * g + r) * pitch;
       *(lhb*)o = (hbits)h;
       *(lhb*)(o + plane) = (hbits)l;

@@ -718,7 +718,7 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
       const bool wide_tiles = up(b.m, 256) <= 1.06 * up(b.m, 128);
       b.rows_m = up(b.m, wide_tiles ? 256 : kNsTile);
       b.rows_n = up(b.n, kNsTile);
-      b.lda = up(b.m, 4);
+      b.a_floats = (long long)hf_tiles_upper(b.m) * kNsTileFloats;
       b.n_slabs = f.n_slabs;
       b.p_stride = ((long long)kNsPl * b.rows_m * b.pad_m + 63) / 64 * 64;
       // (the matrices of one tensor -- the slices of one with more than two dims -- stay in one batch)
@@ -737,8 +737,8 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
       b.off_xl[0] = take_p((long long)kNsPl * b.rows_n * b.pad_m);
       b.off_xl[1] = take_p((long long)kNsPl * b.rows_n * b.pad_m);
       b.off_p = take_p(kNsBufs * b.p_stride);
-      b.off_a = take((long long)b.m * b.lda);
-      b.off_part = b.n_slabs > 1 ? take((long long)b.n_slabs * b.m * b.lda) : 0;
+      b.off_a = take(b.a_floats);
+      b.off_part = b.n_slabs > 1 ? take((long long)b.n_slabs * b.a_floats) : 0;
       b.elem_off = f.elem_off;
       L.ns_mats[q].off_a = b.off_a;   // the fp32 tables stay consistent for k_ns_scale (tensor index only)
       L.nsb_mats.push_back(b);
@@ -806,7 +806,7 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
         {
           NsHfMat& bw = L.nsb_mats[q];
           bw.fpart0 = L.ns_fpart_total;
-          bw.n_fpart = (int)(((long long)bw.m * bw.m + kNsFlagChunk - 1) / kNsFlagChunk);
+          bw.n_fpart = 4 * hf_tiles_upper(bw.m);
           L.ns_fpart_total += bw.n_fpart;
           for (int c = 0; c < bw.n_fpart; ++c) L.ns_flag_items.push_back(Item{q, c, 0, 0});
         }
@@ -2194,8 +2194,7 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
                 hipLaunchKernelGGL((k_ns_hf_gemm<kNsGram, 2>), dim3(G.n_gram), dim3(256), hf_gemm_lds(2), sg, bmats,
                                    gram + G.gram0, dyn, ns_ws, pw, op.par, op.last, op.b, c0, c1, c2, op.pick);
               if (G.n_split > 0)
-                hipLaunchKernelGGL(k_ns_hf_gram_reduce, dim3(((size_t)G.split_max_m * G.split_max_m + 255) / 256, G.n_split),
-                                   dim3(256), 0, sg, bmats, split + G.split0, dyn, ns_ws, pw, op.pick, op.b.out_scale);
+                hipLaunchKernelGGL(k_ns_hf_gram_reduce, dim3(16 * hf_tiles_upper(G.split_max_m), G.n_split), dim3(64), 0, sg, bmats, split + G.split0, dyn, ns_ws, pw, op.pick, op.b.out_scale);
               break;
             case kOpFlag:
               if (G.n_list > 0) {
@@ -2912,25 +2911,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   } else {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wi = (wave >> 1) * 64, wj = (wave & 1) * 32 * WN;
-    const int kg = lane >> 5, lo = lane & 31;
-    int offa[128 * kNsRowPc / 256], offb[RB * kNsRowPc / 256];
-    hf_stage_offsets<128>(wave, lane, offa);
-    hf_stage_offsets<RB>(wave, lane, offb);
-    hf_stage_issue<128>((const char*)X + (size_t)i0 * kNsRowB, offa, lds, wave);
-    hf_stage_issue<RB>((const char*)B + (size_t)j0 * kNsRowB, offb, lds + SA, wave);
+    hf_stage_issue<128>((const char*)X + (size_t)i0 * kNsRowB + 16 * lane, lds, wave);
+    hf_stage_issue<RB>((const char*)B + (size_t)j0 * kNsRowB + 16 * lane, lds + SA, wave);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    const int sw = 16 * (kg ^ ((lo >> 2) & 3));
-    const int oa = (wi + lo) * kNsRowB + sw, ob = SA + (wj + lo) * kNsRowB + sw;
+    const int oa = hf_frag(wi, lane), ob = SA + hf_frag(wj, lane);
     f16x8 a[2][kNsPl], b[WN][kNsPl];
     for (int k = 0; k < K; k += kHfBK) {
       if (MODE == 1 || k == 0) {
 #pragma unroll
         for (int q = 0; q < kNsPl; ++q) {
 #pragma unroll
-          for (int i = 0; i < 2; ++i) a[i][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + ((oa + i * 32 * kNsRowB) ^ (q * 32))));
+          for (int i = 0; i < 2; ++i) a[i][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + oa + i * 32 * kNsRowB + q * 256));
 #pragma unroll
-          for (int j = 0; j < WN; ++j) b[j][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + ((ob + j * 32 * kNsRowB) ^ (q * 32))));
+          for (int j = 0; j < WN; ++j) b[j][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + ob + j * 32 * kNsRowB + q * 256));
         }
       }
 #pragma unroll
