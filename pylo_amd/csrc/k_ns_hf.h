@@ -48,7 +48,9 @@
 // Tile job: 128 x 128 (Gram, Poly, narrow updates) or 128 x 256 outputs (updates with m > 128) by 256 threads =
 // 2 x 2 waves of 64 x 64 / 64 x 128 = 2 x 2 / 2 x 4 accumulators of 32 x 32; 16 reduction steps per stage,
 // double buffered in LDS (32 / 48 KB), staged from global memory straight into LDS (global_load_lds_dwordx4: no
-// staging registers, no LDS store instructions), one 16-byte read per lane, plane and 32-row block per stage.
+// staging registers, no LDS store instructions), one 16-byte read per lane, plane and 32-row block per stage.  A launch with
+// less than a tile of 128 x 128 a CU takes 64 x 64 (a 32 x 32 a wave) and 64 steps a stage: such a job is a chain of loads
+// that waits for memory once a stage, and four times as many blocks wait together.
 // The planes are allocated with their rows rounded up to whole tiles and the padding holds zeros, so the main
 // loop has no bounds checks; any two dims are taken (the raw step is read and the result written per element
 // where the tensor's rows are not 16-byte aligned).
@@ -68,8 +70,8 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) u32x4 luint4;
 
 constexpr int kHfBK = 16;                     // reduction steps per stage
-// LDS of a tile job with 64 WN columns: two stages of (128 + 64 WN) rows x 2 planes x 32 bytes
-constexpr int hf_gemm_lds(int wn) { return 2 * (128 + 64 * wn) * kNsRowB; }
+// LDS of a tile job with 64 WI rows and 64 WN columns: two stages of (64 WI + 64 WN) rows x 2 planes x 32 KS bytes
+constexpr int hf_gemm_lds(int wi, int wn, int ks) { return 2 * ks * (64 * wi + 64 * wn) * kNsRowB; }
 
 // Planes of one matrix with `rows` rows (a multiple of the tiles' rows; rows past the matrix hold zeros) and a (padded)
 // reduction length: blocks of 16 reduction steps x 16 rows, [k / 16][row / 16], of 1 KB each, inside a block [half: k / 8 % 2]
@@ -160,54 +162,70 @@ __device__ __forceinline__ int hf_frag(int row0, int lane) {
 }
 
 // acc[hi][hj] += (rows i0.. of P1) x (rows j0.. of P2)^T over the reduction range [k0, k1) (multiples of 16);
-// 128 rows of P1, 64 WN rows of P2.  LDS: two stages of (128 + 64 WN) x 64 bytes.
+// 16 NW WI rows of P1, 64 WN rows of P2, KS times 16 reduction steps a stage.  LDS: two stages of (16 NW WI + 64 WN) x 64 KS
+// bytes.
 // `compute` (the same for all lanes of a wave): false for a wave whose values nobody needs -- it stages and meets the
 // barriers, and leaves the matrix pipe to the other waves of its SIMD.
-template <int WN, int NW = 4>
+template <int WI, int WN, int KS = 1, int NW = 4>
 __device__ __forceinline__ void hf_tile_product(const HfPlanes& P1, int i0, const HfPlanes& P2, int j0, int k0, int k1,
-                                                PYLO_LDS char* lds, v16f (&acc)[2][WN], bool compute = true) {
-  constexpr int RA = 32 * NW, RB = 64 * WN, SA = RA * kNsRowB, STAGE = SA + RB * kNsRowB;
+                                                PYLO_LDS char* lds, v16f (&acc)[WI][WN], bool compute = true) {
+  constexpr int RA = 16 * NW * WI, RB = 64 * WN, SA = RA * kNsRowB, STEP = SA + RB * kNsRowB, STAGE = KS * STEP;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wi = (wave >> 1) * 64, wj = (wave & 1) * 32 * WN;
+  const int wi = (wave >> 1) * 32 * WI, wj = (wave & 1) * 32 * WN;
   const char* ga = (const char*)P1.base + ((size_t)(k0 >> 4) * P1.rows + i0) * kNsRowB + 16 * lane;
   const char* gb = (const char*)P2.base + ((size_t)(k0 >> 4) * P2.rows + j0) * kNsRowB + 16 * lane;
   const size_t sa = (size_t)P1.rows * kNsRowB, sb = (size_t)P2.rows * kNsRowB;
-  // a diagonal tile of X X^T or A A: both operands are the same 128 rows, staged once
-  const bool same = WN == 2 && P1.base == P2.base && i0 == j0;
-  hf_stage_issue<RA, NW>(ga, lds, wave);
-  if (!same) hf_stage_issue<RB, NW>(gb, lds + SA, wave);
+  // a diagonal tile of X X^T or A A: both operands are the same rows, staged once
+  const bool same = RA == RB && P1.base == P2.base && i0 == j0;
+  auto issue = [&](int k, PYLO_LDS char* to) {   // the stage that starts at k
+#pragma unroll
+    for (int u = 0; u < KS; ++u) {
+      if (u > 0 && k + u * kHfBK >= k1) break;
+      hf_stage_issue<RA, NW>(ga, to + u * STEP, wave);
+      if (!same) hf_stage_issue<RB, NW>(gb, to + u * STEP + SA, wave);
+      ga += sa;
+      gb += sb;
+    }
+  };
+  issue(k0, lds);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   const int oa = hf_frag(wi, lane), ob = (same ? 0 : SA) + hf_frag(wj, lane);
-  int cur = 0;
-  for (int k = k0; k < k1; k += kHfBK) {
-    if (k + kHfBK < k1) {
-      ga += sa;
-      gb += sb;
-      hf_stage_issue<RA, NW>(ga, lds + (STAGE - cur), wave);
-      if (!same) hf_stage_issue<RB, NW>(gb, lds + (STAGE - cur) + SA, wave);
-    }
-    if (compute) {
-      f16x8 a[2][kNsPl], b[WN][kNsPl];
+  auto multiply = [&](auto steps, const PYLO_LDS char* from) {
+    constexpr int N = steps.value;
+    f16x8 a[N][WI][kNsPl], b[N][WN][kNsPl];
+#pragma unroll
+    for (int u = 0; u < N; ++u)
 #pragma unroll
       for (int q = 0; q < kNsPl; ++q) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-          a[i][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + cur + oa + i * 32 * kNsRowB + q * 256));
+        for (int i = 0; i < WI; ++i)
+          a[u][i][q] = __builtin_bit_cast(f16x8, *(const luint4*)(from + u * STEP + oa + i * 32 * kNsRowB + q * 256));
 #pragma unroll
         for (int j = 0; j < WN; ++j)
-          b[j][q] = __builtin_bit_cast(f16x8, *(const luint4*)(lds + cur + ob + j * 32 * kNsRowB + q * 256));
+          b[u][j][q] = __builtin_bit_cast(f16x8, *(const luint4*)(from + u * STEP + ob + j * 32 * kNsRowB + q * 256));
       }
-      // smallest terms first: l h, h l, h h
+    // smallest terms first: l h, h l, h h
+#pragma unroll
+    for (int u = 0; u < N; ++u)
 #pragma unroll
       for (int term = 0; term < 3; ++term) {
         constexpr int pa[3] = {1, 0, 0}, pb[3] = {0, 1, 0};
 #pragma unroll
-        for (int hi = 0; hi < 2; ++hi)
+        for (int hi = 0; hi < WI; ++hi)
 #pragma unroll
           for (int hj = 0; hj < WN; ++hj)
-            acc[hi][hj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[hi][pa[term]], b[hj][pb[term]], acc[hi][hj], 0, 0, 0);
+            acc[hi][hj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u][hi][pa[term]], b[u][hj][pb[term]], acc[hi][hj], 0, 0, 0);
       }
+  };
+  int cur = 0;
+  for (int k = k0; k < k1; k += KS * kHfBK) {
+    if (k + KS * kHfBK < k1) issue(k + KS * kHfBK, lds + (STAGE - cur));
+    if (compute) {
+      // (a whole stage's fragments are read before its first product: one wait for LDS, not one a step)
+      if (KS == 1 || k + KS * kHfBK <= k1) multiply(std::integral_constant<int, KS>(), lds + cur);
+      else
+        for (int u = 0; k + u * kHfBK < k1; ++u) multiply(std::integral_constant<int, 1>(), lds + cur + u * STEP);
     }
     // the loads into the other stage have landed (they are counted like any other vector-memory load) and
     // every wave has read this one
@@ -391,7 +409,8 @@ __device__ __forceinline__ void hf_mask_edge(v16f (&acc)[HI][WN], int wi, int wj
 //   kNsProd    (buffer s1) (buffer s2) as planes (buffer d), both halves
 //   kNsProdA   the same, into buffer d and into the fp32 copy of A
 //   kNsUpdate  Xl' = Xl (buffer s1): planes of Xl' (buffer 1 - par) and Xs', or fp32 X in place of the raw step (`last`)
-// WN: the tile has 64 WN columns (Gram and Poly: 2; updates: 2 or 4, a table of jobs each).
+// WI, WN: the tile has 64 WI rows and 64 WN columns: 2, 2; updates with enough of them 2, 4; 1, 1 where a launch has less
+// than a 128 x 128 tile a CU (ns_tile_edge).  KS: reduction steps of 16 a stage.
 // Registers: 64 / 128 accumulator registers plus what the epilogues need; tiles of 256 columns are held to two
 // waves per SIMD (256 registers: left alone the epilogue takes 296 and a CU runs one job at a time).
 // Which matrices a launch is for, when the chain length is chosen per matrix (k_ns_hf_chain_flag): all of them; those
@@ -403,7 +422,7 @@ struct NsPick {
   float acc_scale_short;   // with s1_short: that buffer's planes have a scale of their own
 };
 
-template <int OP, int WN>
+template <int OP, int WI, int WN, int KS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WN == 4 ? 2 : 3))) void k_ns_hf_gemm(const NsHfMat* __restrict__ mats, const NsItem* __restrict__ items,
                                                     const PyloTensorArgs* __restrict__ dyn, float* __restrict__ ws,
                                                     hbits* __restrict__ pw, int par, int last, NsBufs bufs, float c0,
@@ -425,58 +444,60 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WN == 4 ? 2
   const PyloTensorArgs a = dyn[mt.tensor];
   if (a.grad == nullptr || !(a.flags & kArgOrthogonalize)) return;
   const int m = mt.m, n = mt.n;
-  v16f acc[2][WN];
+  v16f acc[WI][WN];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < WI; ++i)
 #pragma unroll
     for (int j = 0; j < WN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-  const int i0 = it.tm * kNsTile, j0 = it.tn * 64 * WN;
-  // A tile on the diagonal of a symmetric product: the 64 x 64 quadrant below the diagonal is the mirror image of the
+  const int i0 = it.tm * 64 * WI, j0 = it.tn * 64 * WN;
+  // A 128 x 128 tile on the diagonal of a symmetric product: the 64 x 64 quadrant below the diagonal is the mirror image of the
   // one above it, which its own wave (wave 1) writes to both places; wave 2 computes and stores nothing.
   const int wave_u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool diag = OP != kNsUpdate && WN == 2 && it.tm == it.tn;
+  const bool diag = OP != kNsUpdate && WI == 2 && it.tm == it.tn;
   const bool idle = diag && wave_u == 2;
   if (OP == kNsGram) {
     const HfPlanes X{pw + mt.off_xs, mt.rows_m};
-    hf_tile_product<WN>(X, i0, X, j0, it.k0, it.k1, lds, acc, !idle);
+    hf_tile_product<WI, WN, KS>(X, i0, X, j0, it.k0, it.k1, lds, acc, !idle);
   } else if (OP == kNsPoly) {
     const HfPlanes A{pw + mt.off_p, mt.rows_m};
-    hf_tile_product<WN>(A, i0, A, j0, it.k0, it.k1, lds, acc, !idle);
+    hf_tile_product<WI, WN, KS>(A, i0, A, j0, it.k0, it.k1, lds, acc, !idle);
   } else if (OP == kNsUpdate) {
     const HfPlanes X{pw + (par ? mt.off_xl[1] : mt.off_xl[0]), mt.rows_n};   // no run-time index: the struct stays in registers
     const HfPlanes B{pw + mt.off_p + bufs.s1 * mt.p_stride, mt.rows_m};
-    hf_tile_product<WN>(X, i0, B, j0, it.k0, it.k1, lds, acc);
+    hf_tile_product<WI, WN, KS>(X, i0, B, j0, it.k0, it.k1, lds, acc);
   } else {
     const HfPlanes P1{pw + mt.off_p + bufs.s1 * mt.p_stride, mt.rows_m};
     const HfPlanes P2{pw + mt.off_p + bufs.s2 * mt.p_stride, mt.rows_m};
-    hf_tile_product<WN>(P1, i0, P2, j0, it.k0, it.k1, lds, acc, !idle);
+    hf_tile_product<WI, WN, KS>(P1, i0, P2, j0, it.k0, it.k1, lds, acc, !idle);
   }
   if (idle) return;
   // the operands' planes hold their matrices times a power of two each
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < WI; ++i)
 #pragma unroll
     for (int j = 0; j < WN; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] *= bufs.acc_scale;
   const int n_i = OP == kNsUpdate ? n : m;   // rows of the output; its columns are always m
   const bool partial = OP == kNsGram && it.slab >= 0;
-  const bool mirror = OP != kNsUpdate && (it.tm != it.tn || wave_u == 1);
+  const bool mirror = OP != kNsUpdate && (it.tm != it.tn || (WI == 2 && wave_u == 1));
   const int lane = threadIdx.x & 63;
-  const int wi = i0 + (wave_u >> 1) * 64, wj = j0 + (wave_u & 1) * 32 * WN;   // origin of the wave's values
-  if (wi + 64 > n_i || wj + 32 * WN > m) hf_mask_edge<2, WN>(acc, wi, wj, n_i, m);
+  const int wi = i0 + (wave_u >> 1) * 32 * WI, wj = j0 + (wave_u & 1) * 32 * WN;   // origin of the wave's values
+  if (wi + 32 * WI > n_i || wj + 32 * WN > m) hf_mask_edge<WI, WN>(acc, wi, wj, n_i, m);
   if (OP == kNsGram || OP == kNsPoly || OP == kNsProdA) {
     // the fp32 A: written, or Poly's transform of the accumulators
-    float* A = ws + (partial ? mt.off_part + (size_t)it.slab * mt.a_floats : mt.off_a) + hf_a32(hf_tile_index(m, it.tm, it.tn), wave_u, 0, 0, 0, lane);
+    const size_t e = WI == 2 ? hf_a32(hf_tile_index(m, it.tm, it.tn), wave_u, 0, 0, 0, lane)
+                             : hf_a32(hf_tile_index(m, it.tm >> 1, it.tn >> 1), (it.tm & 1) * 2 + (it.tn & 1), wave_u >> 1, wave_u & 1, 0, lane);
+    float* A = ws + (partial ? mt.off_part + (size_t)it.slab * mt.a_floats : mt.off_a) + e;
 #pragma unroll
-    for (int hi = 0; hi < 2; ++hi)
+    for (int hi = 0; hi < WI; ++hi)
 #pragma unroll
       for (int hj = 0; hj < WN; ++hj)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          gv4f* p = (gv4f*)(A + ((hi * 2 + hj) * 4 + q) * 256);
+          gv4f* p = (gv4f*)(A + ((hi * WN + hj) * 4 + q) * 256);
           if (OP == kNsPoly) {
             const v4f aij = *p;
             const int d = wj + hj * 32 + (lane & 31) - (wi + hi * 32 + 8 * q + 4 * (lane >> 5));   // the register on the diagonal, if 0 .. 3
@@ -502,7 +523,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WN == 4 ? 2
       typedef PYLO_LDS v4f lv4f;
       PYLO_LDS char* patch = lds + wave_u * (32 * 144);
 #pragma unroll
-      for (int hi = 0; hi < 2; ++hi)
+      for (int hi = 0; hi < WI; ++hi)
 #pragma unroll
         for (int hj = 0; hj < WN; ++hj) {
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -520,7 +541,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WN == 4 ? 2
         }
     } else {
 #pragma unroll
-      for (int hi = 0; hi < 2; ++hi)
+      for (int hi = 0; hi < WI; ++hi)
 #pragma unroll
         for (int hj = 0; hj < WN; ++hj) {
           const int col = wj + hj * 32 + (lane & 31);
@@ -537,11 +558,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WN == 4 ? 2
   // planes: A and B' in both halves (the mirrored tile is the other orientation), Xl' and Xs'
   PYLO_LDS char* patch = lds + wave_u * (2048 * WN);
   if (OP == kNsUpdate) {
-    hf_store_planes<2, WN>(patch, acc, pw + (par ? mt.off_xl[0] : mt.off_xl[1]), mt.rows_n, wi, wj, n, m, pw + mt.off_xs, mt.rows_m,
+    hf_store_planes<WI, WN>(patch, acc, pw + (par ? mt.off_xl[0] : mt.off_xl[1]), mt.rows_n, wi, wj, n, m, pw + mt.off_xs, mt.rows_m,
                            bufs.out_scale);
   } else {
     hbits* D = pw + mt.off_p + (OP == kNsGram ? (int)kNsBufA : bufs.d) * mt.p_stride;
-    hf_store_planes<2, WN>(patch, acc, D, mt.rows_m, wi, wj, m, m, mirror ? D : nullptr, mt.rows_m, bufs.out_scale);
+    hf_store_planes<WI, WN>(patch, acc, D, mt.rows_m, wi, wj, m, m, mirror ? D : nullptr, mt.rows_m, bufs.out_scale);
   }
 }
 

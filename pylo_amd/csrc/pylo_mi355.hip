@@ -78,6 +78,7 @@ bool factored_dims(int kind, const PyloTensorShape& s, int* dc, int* dr) {
 // One group of matrices of the split-fp16 Newton-Schulz kernels: its ranges in the job tables.
 struct NsGroup {
   int gram0, n_gram, poly0, n_poly, upd0, n_upd, upd40, n_upd4, split0, n_split, split_max_m;
+  int gram_edge, poly_edge, upd_edge;   // output tiles of the three tables: 64 or 128 (upd4: 128 x 256)
   int list0, n_list;       // its matrices (ns_list)
   int sitem0, n_sitems;    // its tiles of the pass that splits the raw steps into planes
   int fitem0, n_fitems;    // its blocks of the pass that sums the squares of A (chain length per matrix)
@@ -565,6 +566,15 @@ void build_small_items(Layout& L) {
   L.sm_sync += kNsSmallClasses;
 }
 
+// The output tiles of a launch with `jobs` tiles of 128 x 128: those, or 64 x 64 where they are fewer than the CUs.  A tile job
+// is a chain of stages that wait for memory; few long ones leave most of the part idle and each of them half of its CU.
+// The m x m products' bare loop, 128 x 128 / 64 x 64 tiles (four steps a stage): one 1024 x 1024 with 63 steps (36 / 136 jobs)
+// 28.0 / 12.2 us, four 512 x 512 (40 / 144) 12.9 / 6.3, six 384 x 384 (36 / 126) 10.2 / 5.2, twelve 768 x 768 (252 / 936)
+// 24.9 / 24.6, forty-eight (1008 / 3744) 76.9 / 92.0.  Finishing calls before (all 128 x 128 and 128 x 256) / now: one
+// 1000 x 2048 738 / 319 us, a layer of width 256 366 / 154, four of width 512 916 / 644, twenty 200 x 200 312 / 141, 4000 x 512
+// 495 / 214; whole CELO2 step on ResNet-50 1.49 / 1.21 ms.
+int ns_tile_edge(long long jobs) { return jobs < 256 ? 64 : kNsTile; }
+
 // Newton-Schulz tables: every 2-D MLP tensor (the fp32 kernels: those whose rows (C) and whose smaller dim are
 // multiples of 4).  `ws_floats` returns the floats of workspace behind off_ns_ws.
 void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long& ws_floats) {
@@ -669,9 +679,13 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
     // part has CUs, each a long reduction: split them along it, up to eight ways, until there are two jobs a CU.
     {
       long long jobs = 0;
-      for (const NsMat& f : L.ns_mats) {
-        const long long nt = (f.m + kNsTile - 1) / kNsTile;
-        jobs += nt * (nt + 1) / 2 * f.n_slabs;
+      for (const int edge : {kNsTile, 64}) {
+        jobs = 0;
+        for (const NsMat& f : L.ns_mats) {
+          const long long nt = (f.m + edge - 1) / edge;
+          jobs += nt * (nt + 1) / 2 * f.n_slabs;
+        }
+        if (ns_tile_edge(jobs) == kNsTile) break;
       }
       if (jobs > 0 && jobs < kNsFewJobs) {
         const int ways = (int)std::min<long long>(8, (kNsFewJobs + jobs - 1) / jobs);
@@ -793,6 +807,19 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
     }
     bt.group0 = (int)L.ns_groups.size();
     bt.n_groups = n_groups;
+    // the tiles of the batch's launches (those of its groups run next to each other)
+    long long gram_jobs = 0, poly_jobs = 0, upd_jobs = 0, upd4_jobs = 0;
+    auto wide_tiles = [&](const NsHfMat& b) { return b.rows_m % 256 == 0 && up(b.m, 256) <= 1.06 * up(b.m, 128); };
+    for (int q = bt.mat0; q < bt.mat0 + bt.n_mats; ++q) {
+      const NsHfMat& b = L.nsb_mats[q];
+      const long long nt = (b.m + kNsTile - 1) / kNsTile, ni = (b.n + kNsTile - 1) / kNsTile;
+      gram_jobs += nt * (nt + 1) / 2 * b.n_slabs;
+      poly_jobs += nt * (nt + 1) / 2;
+      (wide_tiles(b) ? upd4_jobs : upd_jobs) += ni * (wide_tiles(b) ? (b.m + 255) / 256 : nt);
+    }
+    const int gram_edge = ns_tile_edge(gram_jobs), poly_edge = ns_tile_edge(poly_jobs);
+    const bool any_wide = upd4_jobs + upd_jobs >= 256;      // else those of 128 x 256 are cut in two
+    const int upd_edge = ns_tile_edge(any_wide ? upd4_jobs + upd_jobs : 2 * upd4_jobs + upd_jobs);
     for (int g = 0; g < n_groups; ++g) {
       // job runs that read the same operands: per matrix (slab), and finer, per row of tiles, for sets of few matrices
       std::vector<std::pair<int, long long>> gram_units, poly_units, upd_units, upd4_units, gram_rows, poly_rows;
@@ -802,6 +829,9 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
       grp.list0 = (int)L.ns_list.size();
       grp.sitem0 = (int)L.nsb_split_items.size();
       grp.fitem0 = (int)L.ns_flag_items.size();
+      grp.gram_edge = gram_edge;
+      grp.poly_edge = poly_edge;
+      grp.upd_edge = upd_edge;
       for (int q : members[g]) {
         {
           NsHfMat& bw = L.nsb_mats[q];
@@ -815,27 +845,30 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
         L.ns_group_of_tensor[b.tensor] = (int)L.ns_groups.size();
         for (int tr = 0; tr < (b.R + 63) / 64; ++tr)
           for (int tc = 0; tc < (b.C + 63) / 64; ++tc) L.nsb_split_items.push_back(NsTileItem{q, tr, tc});
-        const bool wide_tiles = b.rows_m % 256 == 0 && up(b.m, 256) <= 1.06 * up(b.m, 128);
-        const int nt = (b.m + kNsTile - 1) / kNsTile, n_upper = nt * (nt + 1) / 2;
         // Gram: the tiles of one matrix (of one slab of it) read the same rows of Xs; Poly: the same A
+        auto upper = [&](std::vector<NsItem>& items, std::vector<std::pair<int, long long>>& units,
+                         std::vector<std::pair<int, long long>>& rows, int edge, int k0, int k1, int slab) {
+          const int nt = (b.m + edge - 1) / edge;
+          for (int tm = 0; tm < nt; ++tm) {
+            for (int tn = tm; tn < nt; ++tn) items.push_back(NsItem{q, tm, tn, k0, k1, slab});
+            rows.push_back({nt - tm, (long long)(k1 - k0)});
+          }
+          units.push_back({nt * (nt + 1) / 2, (long long)(k1 - k0)});
+        };
         for (int sl = 0; sl < b.n_slabs; ++sl) {
           const int slab_k = L.ns_mats[q].slab_k;
           const int k0 = b.n_slabs > 1 ? sl * slab_k : 0;
           const int k1 = b.n_slabs > 1 ? up16(std::min(b.n, (sl + 1) * slab_k)) : up16(b.n);
-          for (int tm = 0; tm < nt; ++tm)
-            for (int tn = tm; tn < nt; ++tn) gram.push_back(NsItem{q, tm, tn, k0, k1, b.n_slabs > 1 ? sl : -1});
-          gram_units.push_back({n_upper, (long long)(k1 - k0)});
-          for (int tm = 0; tm < nt; ++tm) gram_rows.push_back({nt - tm, (long long)(k1 - k0)});
+          upper(gram, gram_units, gram_rows, gram_edge, k0, k1, b.n_slabs > 1 ? sl : -1);
         }
-        for (int tm = 0; tm < nt; ++tm)
-          for (int tn = tm; tn < nt; ++tn) poly.push_back(NsItem{q, tm, tn, 0, up16(b.m), -1});
-        poly_units.push_back({n_upper, (long long)up16(b.m)});
-        for (int tm = 0; tm < nt; ++tm) poly_rows.push_back({nt - tm, (long long)up16(b.m)});
+        upper(poly, poly_units, poly_rows, poly_edge, 0, up16(b.m), -1);
         // Update: the tiles of one row block read the same rows of Xl, all of them the same B'
-        const int ni = (b.n + kNsTile - 1) / kNsTile, ntu = wide_tiles ? (b.m + 255) / 256 : nt;
-        std::vector<NsItem>& u = wide_tiles ? upd4 : upd;
-        std::vector<std::pair<int, long long>>& units = wide_tiles ? upd4_units : upd_units;
-        for (int tm = 0; tm < ni; ++tm) {
+        const bool wide = any_wide && wide_tiles(b);
+        const int ei = wide ? kNsTile : upd_edge, ej = wide ? 256 : upd_edge;
+        std::vector<NsItem>& u = wide ? upd4 : upd;
+        std::vector<std::pair<int, long long>>& units = wide ? upd4_units : upd_units;
+        for (int tm = 0; tm < (b.n + ei - 1) / ei; ++tm) {
+          const int ntu = (b.m + ej - 1) / ej;
           for (int tn = 0; tn < ntu; ++tn) u.push_back(NsItem{q, tm, tn, 0, up16(b.m), -1});
           units.push_back({ntu, (long long)up16(b.m)});
         }
@@ -1885,12 +1918,17 @@ int ns_hf_lds_once() {
   std::lock_guard<std::mutex> lock(mu);
   for (int d : done)
     if (d == dev) return 0;
-  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsGram, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2)));
-  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsPoly, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2)));
-  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsProd, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2)));
-  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsProdA, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2)));
-  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsUpdate, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2)));
-  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsUpdate, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(4)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsGram, 2, 2, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 2, 1)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsGram, 1, 1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(1, 1, 4)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsPoly, 2, 2, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 2, 1)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsPoly, 1, 1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(1, 1, 4)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsProd, 2, 2, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 2, 1)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsProd, 1, 1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(1, 1, 4)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsProdA, 2, 2, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 2, 1)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsProdA, 1, 1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(1, 1, 4)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsUpdate, 2, 2, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 2, 1)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsUpdate, 1, 1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(1, 1, 4)));
+  HIP_TRY(hipFuncSetAttribute((const void*)k_ns_hf_gemm<kNsUpdate, 2, 4, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 4, 1)));
   done.push_back(dev);
   return 0;
 }
@@ -2183,16 +2221,18 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
         for (int g = 0; g < n_groups; ++g) {
           const NsGroup& G = L.ns_groups[bt.group0 + g];
           hipStream_t sg = stream_of(g);
-          auto small = [&](auto kern) {
-            if (G.n_poly > 0)
-              hipLaunchKernelGGL(kern, dim3(G.n_poly), dim3(256), hf_gemm_lds(2), sg, bmats, poly + G.poly0, dyn, ns_ws, pw,
-                                 op.par, op.last, op.b, c0, c1, c2, op.pick);
+          auto launch = [&](auto kern, int lds, const NsItem* items, int n) {
+            if (n > 0)
+              hipLaunchKernelGGL(kern, dim3(n), dim3(256), lds, sg, bmats, items, dyn, ns_ws, pw, op.par, op.last, op.b, c0, c1,
+                                 c2, op.pick);
+          };
+          auto by_edge = [&](int edge, auto k128, auto k64, const NsItem* items, int n) {
+            if (edge == 64) launch(k64, hf_gemm_lds(1, 1, 4), items, n);
+            else launch(k128, hf_gemm_lds(2, 2, 1), items, n);
           };
           switch (op.kind) {
             case kOpGram:
-              if (G.n_gram > 0)
-                hipLaunchKernelGGL((k_ns_hf_gemm<kNsGram, 2>), dim3(G.n_gram), dim3(256), hf_gemm_lds(2), sg, bmats,
-                                   gram + G.gram0, dyn, ns_ws, pw, op.par, op.last, op.b, c0, c1, c2, op.pick);
+              by_edge(G.gram_edge, k_ns_hf_gemm<kNsGram, 2, 2, 1>, k_ns_hf_gemm<kNsGram, 1, 1, 4>, gram + G.gram0, G.n_gram);
               if (G.n_split > 0)
                 hipLaunchKernelGGL(k_ns_hf_gram_reduce, dim3(16 * hf_tiles_upper(G.split_max_m), G.n_split), dim3(64), 0, sg, bmats, split + G.split0, dyn, ns_ws, pw, op.pick, op.b.out_scale);
               break;
@@ -2204,16 +2244,18 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
                                    (const float*)chain_part, chain_tau2, chain_flags);
               }
               break;
-            case kOpPoly: small(k_ns_hf_gemm<kNsPoly, 2>); break;
-            case kOpProd: small(k_ns_hf_gemm<kNsProd, 2>); break;
-            case kOpProdA: small(k_ns_hf_gemm<kNsProdA, 2>); break;
+            case kOpPoly:
+              by_edge(G.poly_edge, k_ns_hf_gemm<kNsPoly, 2, 2, 1>, k_ns_hf_gemm<kNsPoly, 1, 1, 4>, poly + G.poly0, G.n_poly);
+              break;
+            case kOpProd:
+              by_edge(G.poly_edge, k_ns_hf_gemm<kNsProd, 2, 2, 1>, k_ns_hf_gemm<kNsProd, 1, 1, 4>, poly + G.poly0, G.n_poly);
+              break;
+            case kOpProdA:
+              by_edge(G.poly_edge, k_ns_hf_gemm<kNsProdA, 2, 2, 1>, k_ns_hf_gemm<kNsProdA, 1, 1, 4>, poly + G.poly0, G.n_poly);
+              break;
             case kOpUpdate:
-              if (G.n_upd4 > 0)
-                hipLaunchKernelGGL((k_ns_hf_gemm<kNsUpdate, 4>), dim3(G.n_upd4), dim3(256), hf_gemm_lds(4), sg, bmats,
-                                   upd4 + G.upd40, dyn, ns_ws, pw, op.par, op.last, op.b, c0, c1, c2, op.pick);
-              if (G.n_upd > 0)
-                hipLaunchKernelGGL((k_ns_hf_gemm<kNsUpdate, 2>), dim3(G.n_upd), dim3(256), hf_gemm_lds(2), sg, bmats,
-                                   upd + G.upd0, dyn, ns_ws, pw, op.par, op.last, op.b, c0, c1, c2, op.pick);
+              launch(k_ns_hf_gemm<kNsUpdate, 2, 4, 1>, hf_gemm_lds(2, 4, 1), upd4 + G.upd40, G.n_upd4);
+              by_edge(G.upd_edge, k_ns_hf_gemm<kNsUpdate, 2, 2, 1>, k_ns_hf_gemm<kNsUpdate, 1, 1, 4>, upd + G.upd0, G.n_upd);
               break;
           }
         }
@@ -2905,7 +2947,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
   const HfPlanes PX{X, rows_x}, PB{B, rows_b};
   if (MODE == 0) {
-    hf_tile_product<WN>(PX, i0, PB, j0, 0, K, lds, acc);
+    hf_tile_product<2, WN>(PX, i0, PB, j0, 0, K, lds, acc);
   } else if (MODE == 4) {
     hf_tile_product_direct<WN>(PX, i0, PB, j0, 0, K, lds, acc);
   } else {
@@ -2965,7 +3007,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
   const HfPlanes PX{X, rows_x}, PB{B, rows_b};
-  hf_tile_product<WN, 8>(PX, i0, PB, j0, 0, K, lds, acc);
+  hf_tile_product<2, WN, 1, 8>(PX, i0, PB, j0, 0, K, lds, acc);
   float sum = 0.0f;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -2990,17 +3032,17 @@ extern "C" int pylo_mi355_matrix_probe(const void* x_planes, int rows_x, const v
   static std::mutex mu;
   {
     std::lock_guard<std::mutex> lock(mu);
-    HIP_TRY(hipFuncSetAttribute((const void*)k_matrix_probe<0>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(4)));
-    HIP_TRY(hipFuncSetAttribute((const void*)k_matrix_probe<1>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(4)));
-    HIP_TRY(hipFuncSetAttribute((const void*)k_matrix_probe<2>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(4)));
+    HIP_TRY(hipFuncSetAttribute((const void*)k_matrix_probe<0>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 4, 1)));
+    HIP_TRY(hipFuncSetAttribute((const void*)k_matrix_probe<1>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 4, 1)));
+    HIP_TRY(hipFuncSetAttribute((const void*)k_matrix_probe<2>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 4, 1)));
     HIP_TRY(hipFuncSetAttribute((const void*)k_matrix_probe_wide, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 512 * kNsRowB));
-    HIP_TRY(hipFuncSetAttribute((const void*)k_matrix_probe<4>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(4)));
+    HIP_TRY(hipFuncSetAttribute((const void*)k_matrix_probe<4>, hipFuncAttributeMaxDynamicSharedMemorySize, hf_gemm_lds(2, 4, 1)));
   }
   const hbits* X = static_cast<const hbits*>(x_planes);
   const hbits* B = static_cast<const hbits*>(b_planes);
-  if (mode == 0) hipLaunchKernelGGL(k_matrix_probe<0>, dim3(grid), dim3(256), hf_gemm_lds(4), s, X, rows_x, B, rows_b, k_steps, out);
-  else if (mode == 1) hipLaunchKernelGGL(k_matrix_probe<1>, dim3(grid), dim3(256), hf_gemm_lds(4), s, X, rows_x, B, rows_b, k_steps, out);
-  else if (mode == 2) hipLaunchKernelGGL(k_matrix_probe<2>, dim3(grid), dim3(256), hf_gemm_lds(4), s, X, rows_x, B, rows_b, k_steps, out);
+  if (mode == 0) hipLaunchKernelGGL(k_matrix_probe<0>, dim3(grid), dim3(256), hf_gemm_lds(2, 4, 1), s, X, rows_x, B, rows_b, k_steps, out);
+  else if (mode == 1) hipLaunchKernelGGL(k_matrix_probe<1>, dim3(grid), dim3(256), hf_gemm_lds(2, 4, 1), s, X, rows_x, B, rows_b, k_steps, out);
+  else if (mode == 2) hipLaunchKernelGGL(k_matrix_probe<2>, dim3(grid), dim3(256), hf_gemm_lds(2, 4, 1), s, X, rows_x, B, rows_b, k_steps, out);
   else if (mode == 3) hipLaunchKernelGGL(k_matrix_probe_wide, dim3(grid / 2), dim3(512), 2 * 512 * kNsRowB, s, X, rows_x, B, rows_b, k_steps, out);
   else hipLaunchKernelGGL(k_matrix_probe<4>, dim3(grid), dim3(256), 2 * 256 * kNsRowB, s, X, rows_x, B, rows_b, k_steps, out);
   HIP_TRY(hipGetLastError());

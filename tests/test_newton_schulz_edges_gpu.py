@@ -27,17 +27,18 @@ def _fp64(x):
 
 
 @pytest.mark.parametrize("part", range(4))
-@pytest.mark.parametrize("batches", [False, True])
-def test_blocks_tiles_and_padding(part, batches, monkeypatch):
-    """Three calls of one plan: random steps, a NaN in every second matrix, random steps again.  The result is held to 2e-4 of its
+@pytest.mark.parametrize("plan_of", ["few", "many", "batches"])
+def test_blocks_tiles_and_padding(part, plan_of, monkeypatch):
+    """Tiles of 64 x 64 (a plan of few tile jobs), of 128 x 128 and 128 x 256 (next to two large matrices), and batches of
+    matrices that share their workspace.  Three calls of one plan: random steps, a NaN in every second matrix, random steps again.  The result is held to 2e-4 of its
     RMS (fp32 products sit at 2e-5 .. 5e-5), the third call's too: a product of padding with a NaN is a NaN, and what of it
     reached the planes' padding would be read by every later call."""
     from pylo_amd import _lib
 
     monkeypatch.setenv("PYLO_MI355_NS_SMALL", "0")
-    if batches:   # the batches of matrices share their workspace one after another
+    if plan_of == "batches":
         monkeypatch.setenv("PYLO_MI355_NS_WORKSPACE_MB", "4")
-    shapes = SHAPES[part::4]
+    shapes = SHAPES[part::4] + ([(2304, 2304)] * 2 if plan_of == "many" else [])
     plan = _lib.Plan(_lib.KIND_CELO2, shapes, [0] * len(shapes), torch.device("cuda:0"))
     gen = torch.Generator(device="cuda").manual_seed(part)
     for call in range(3):
