@@ -628,7 +628,8 @@ __global__ __launch_bounds__(256) void k_ns_hf_chain_sumsq(const NsHfMat* __rest
   const int nt = (mt.m + kNsTile - 1) / kNsTile, wave = it.a & 3;
   int tm = 0, left = it.a >> 2;
   while (left >= nt - tm) left -= nt - tm++;
-  if (left == 0 && wave == 2) {   // the mirror image of wave 1's, which nobody writes
+  // the mirror image of wave 1's, and parts past the matrix: nobody writes them
+  if ((left == 0 && wave == 2) || (tm + left) * kNsTile + (wave & 1) * 64 >= mt.m) {
     if (threadIdx.x == 0) part[mt.fpart0 + it.a] = 0.0f;
     return;
   }
