@@ -281,10 +281,16 @@ bool env_ns_xcd() {
   return !(e && e[0] == '0');
 }
 
-// PYLO_MI355_NS_GROUPS: into how many groups (streams) the matrices of a plan are dealt, 1 to 4; read at plan creation.
+// PYLO_MI355_NS_GROUPS: into how many groups (streams) the matrices of a plan are dealt, 1 to 4; read at plan creation.  Three
+// unless it says otherwise.  A process has four hardware queues here; the runtime gives a new stream one of those that have the
+// fewest streams, and two groups that share one wait for each other.  Streams made in threes land on three queues
+// whatever streams the program has (which is why a plan of two groups makes three as well), and no group rides on the
+// caller's stream, whose queue a group of another plan may share.  Whole ELO-CELO2 step on the GPT-2-small set, the
+// first, second and third plan of a process: three groups 6.02, 6.04, 6.00 ms, four 6.61, 6.00, 6.00, two on two
+// streams 6.09, 6.79, 6.06; with one of three on the caller's stream 6.04 to 6.30.
 int env_ns_groups() {
   const char* e = getenv("PYLO_MI355_NS_GROUPS");
-  const int g = e ? atoi(e) : 4;
+  const int g = e ? atoi(e) : 3;
   return std::max(1, std::min(g, 4));
 }
 
@@ -1375,9 +1381,9 @@ struct PyloPlan {
   int* stale_dev = nullptr;
   hipStream_t side = nullptr;            // the LSTM runs next to the gradient sums on a stream of the plan's own
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  // ELO-CELO2: the Newton-Schulz chains of the groups of matrices after the first run on streams of the plan's own
-  hipStream_t ns_side[3] = {nullptr, nullptr, nullptr};
-  hipEvent_t ns_fork = nullptr, ns_join[3] = {nullptr, nullptr, nullptr};
+  // ELO-CELO2: the Newton-Schulz chains of several groups of matrices run on streams of the plan's own (env_ns_groups)
+  hipStream_t ns_side[4] = {nullptr, nullptr, nullptr, nullptr};
+  hipEvent_t ns_fork = nullptr, ns_join[4] = {nullptr, nullptr, nullptr, nullptr};
   // the per-slice finishing launches next to the matrices' products, where the groups leave a hardware queue free
   hipStream_t slice_side = nullptr;
   hipEvent_t slice_fork = nullptr, slice_join = nullptr;
@@ -1486,15 +1492,15 @@ int pylo_mi355_plan_create(int kind, const PyloTensorShape* shapes, int n_tensor
   }
   size_t ns_streams = 0;
   for (const NsBatch& bt : L.ns_batches) ns_streams = std::max<size_t>(ns_streams, bt.n_groups);
-  for (size_t g = 1; g < ns_streams && e == hipSuccess; ++g) {
-    if (g == 1) e = hipEventCreateWithFlags(&P->ns_fork, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&P->ns_side[g - 1], hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&P->ns_join[g - 1], hipEventDisableTiming);
+  for (size_t g = 0; ns_streams > 1 && g < std::max<size_t>(ns_streams, 3) && e == hipSuccess; ++g) {
+    if (g == 0) e = hipEventCreateWithFlags(&P->ns_fork, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&P->ns_side[g], hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&P->ns_join[g], hipEventDisableTiming);
   }
   bool plan_has_slices = !L.slice_items_w.empty() || !L.slice_items_b.empty();
   for (const auto& v : L.slice_items_l) plan_has_slices = plan_has_slices || !v.empty();
   plan_has_slices = plan_has_slices || !L.sm_mats.empty();   // the small matrices' launches ride on the same stream
-  if (e == hipSuccess && plan_has_slices && ns_streams >= 1 && ns_streams <= 3) {   // main + groups + this one <= 4 queues
+  if (e == hipSuccess && plan_has_slices && ns_streams >= 1 && ns_streams <= 3) {   // groups + this one <= 4 queues
     e = hipStreamCreateWithFlags(&P->slice_side, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&P->slice_fork, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&P->slice_join, hipEventDisableTiming);
@@ -1518,7 +1524,7 @@ int pylo_mi355_plan_destroy(PyloPlan* P) {
   if (P->slice_fork) (void)hipEventDestroy(P->slice_fork);
   if (P->slice_join) (void)hipEventDestroy(P->slice_join);
   if (P->slice_side) (void)hipStreamDestroy(P->slice_side);
-  for (int g = 0; g < 3; ++g) {
+  for (int g = 0; g < 4; ++g) {
     if (P->ns_join[g]) (void)hipEventDestroy(P->ns_join[g]);
     if (P->ns_side[g]) (void)hipStreamDestroy(P->ns_side[g]);
   }
@@ -2096,8 +2102,8 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
     finish_range(s, 0, n_fin, 0, (int)L.fin_units.size(), nullptr, nullptr);
   } else if (L.ns_hf) {
     // The split-fp16 kernels.  Every group of matrices is a chain of its own from the norms of its raw steps to the
-    // update of its parameters, on a stream of its own (the first group on the caller's): the memory-bound ends of
-    // one chain run under the matrix products of the others.
+    // update of its parameters, on a stream of its own where there are several: the memory-bound ends of one chain run
+    // under the matrix products of the others.
     const NsMat* mats = P->at<NsMat>(L.off_ns_mats);
     const NsItem* gram = P->at<NsItem>(L.off_ns_gram);
     const NsItem* poly = P->at<NsItem>(L.off_ns_poly);
@@ -2130,10 +2136,10 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
                            reinterpret_cast<u32x4*>(pw), n16);
       }
       const int n_groups = bt.n_groups;
-      auto stream_of = [&](int g) { return g == 0 ? s : P->ns_side[g - 1]; };
+      auto stream_of = [&](int g) { return n_groups == 1 ? s : P->ns_side[g]; };
       if (n_groups > 1) {
         HIP_TRY(hipEventRecord(P->ns_fork, s));
-        for (int g = 1; g < n_groups; ++g) HIP_TRY(hipStreamWaitEvent(P->ns_side[g - 1], P->ns_fork, 0));
+        for (int g = 0; g < n_groups; ++g) HIP_TRY(hipStreamWaitEvent(P->ns_side[g], P->ns_fork, 0));
       }
       for (int g = 0; g < n_groups; ++g) {
         // ||raw|| per matrix (the finishing pass's sums of squares, taken on the raw steps), then the planes
@@ -2263,9 +2269,9 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
         const NsGroup& G = L.ns_groups[bt.group0 + g];
         finish_range(stream_of(g), G.fin0, G.n_fin, G.unit0, G.n_units, nullptr, nullptr);
       }
-      for (int g = 1; g < n_groups; ++g) {
-        HIP_TRY(hipEventRecord(P->ns_join[g - 1], P->ns_side[g - 1]));
-        HIP_TRY(hipStreamWaitEvent(s, P->ns_join[g - 1], 0));
+      for (int g = 0; n_groups > 1 && g < n_groups; ++g) {
+        HIP_TRY(hipEventRecord(P->ns_join[g], P->ns_side[g]));
+        HIP_TRY(hipStreamWaitEvent(s, P->ns_join[g], 0));
       }
     }
   } else {
