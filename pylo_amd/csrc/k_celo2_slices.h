@@ -6,19 +6,19 @@
 // N-D tensor still span the whole tensor and come from the P0 / V0 passes; everything after that is
 // local to a slice, so one pass does statistics, MLP and the accumulator writes.
 //
-// A slice is walked twice (sum of squares, then apply) by one lane when it is short (conv kernels:
-// 9 .. 32 elements) and by one wave otherwise.  These tensors are small in the models this path
-// serves (patch embeddings, conv kernels, biases); the kernel is written for correctness on any
-// shape, not for the bandwidth roofline.
+// Short slices of tensors with more than two dims (conv kernels: 1 .. 32 elements) are packed, as many whole ones as fit, into a
+// wave of one lane an element (k_celo2_slices_wave).  All others are walked twice (sum of squares, then apply) by k_celo2_slices,
+// by one lane when the slice is short and by one wave otherwise: written for correctness on any shape (patch embeddings, biases).
 #pragma once
 
 #include "k_velo.h"
 
 namespace pylo {
 
-constexpr int kSliceLaneMax = 32;  // slices up to this length are walked by a single lane
-constexpr int kSliceLaneClasses = 4;   // of slice length, for the kernel that stages such slices through LDS
-constexpr int kSliceLaneClassMax[kSliceLaneClasses] = {4, 9, 16, kSliceLaneMax};
+constexpr int kSliceLaneMax = 32;  // slices up to this length are packed into waves, or walked by a single lane
+// launches of k_celo2_slices_wave: slices of one element, of nine (3 x 3), of any other length; and those whose row and
+// column channels are not the same for all slices that meet a vector's entries (slice_runs)
+enum : int { kSliceOne = 0, kSliceNine = 1, kSliceAny = 2, kSliceGather = 3, kSliceWaveClasses = 4 };
 // raw CELO2 MLP block: w_in (30,8) | b_in 8 | w_h (8,8) | b_h 8 | w_out (8,3) | b_out 3, all (in, out)
 constexpr int kC2RawBI = 240, kC2RawWH = 248, kC2RawBH = 312, kC2RawWO = 320, kC2RawBO = 344;
 
@@ -212,163 +212,168 @@ __device__ __forceinline__ float slice_mlp_mfma(const float (&f)[30], const floa
   v4f gb = mfma_w4(wreg[(kC2GrpBH + 1) / 16], 1.0f, zero, (kC2GrpBH + 1) % 16);
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    const float hk = fmaxf(k < 4 ? ha[k] : hb[k - 4], 0.0f);
+    const float hk = relu(k < 4 ? ha[k] : hb[k - 4]);
     ga = mfma_w4(wreg[(kC2GrpWH + 2 * k) / 16], hk, ga, (kC2GrpWH + 2 * k) % 16);
     gb = mfma_w4(wreg[(kC2GrpWH + 2 * k + 1) / 16], hk, gb, (kC2GrpWH + 2 * k + 1) % 16);
   }
   v4f o = mfma_w4(wreg[kC2GrpBO / 16], 1.0f, zero, kC2GrpBO % 16);
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    const float hk = fmaxf(k < 4 ? ga[k] : gb[k - 4], 0.0f);
+    const float hk = relu(k < 4 ? ga[k] : gb[k - 4]);
     o = mfma_w4(wreg[(kC2GrpWO + k) / 16], hk, o, (kC2GrpWO + k) % 16);
   }
   return o[0] * expf(o[1] * exp_mult);
 }
 
-// Short slices of tensors with more than two dims (convolution kernels: 1 .. 32 elements a slice), one lane per
-// slice, 64 consecutive slices per block (one wave).  The wave's slices are contiguous in every array: gradient,
-// parameter and accumulators come in with coalesced loads, through LDS ([element of the slice][slice], pitch 65: the
-// lanes' walks over their own slices are conflict-free), the accumulators are updated there on the first walk, the
-// second walk leaves the raw step in the gradient's place, and everything goes out coalesced.  Every input is read
-// once and every output written once.  A block takes several such groups of 64 slices one after another when the
-// slices are very short (the set-up of a block is some hundreds of instructions, as much as the walk over a few
-// elements).  Item: tensor, first slice of the block.
-constexpr int kSlicePitchF = 65;
-__host__ __device__ constexpr int slice_lane_groups(int S) { return S <= 2 ? 8 : S <= 4 ? 4 : S <= 9 ? 2 : 1; }
-__global__ __launch_bounds__(64) void k_celo2_slices_lane(const TDesc* __restrict__ descs,
-                                                          const PyloTensorArgs* __restrict__ dyn,
-                                                          const Item* __restrict__ items,
-                                                          const float* __restrict__ fac_tab,
-                                                          const Globals* __restrict__ gl, PyloDecays dec,
-                                                          const float* __restrict__ mlp) {
-  extern __shared__ float sl_lds[];
-  constexpr int P = kSlicePitchF;
+// The same where the row and column channels' part of the first layer comes from the term tables (ta, tb: vector 0 with the bias,
+// vector 1): the eighteen channels of an element alone.
+__device__ __forceinline__ float slice_mlp_terms(const float (&f)[kNStat], const float (&s)[kNStat], const v4f (&ta)[2], const v4f (&tb)[2],
+                                                 const float (&wreg)[6], float exp_mult) {
+  const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  v4f ha = ta[0] + tb[0], hb = ta[1] + tb[1];
+#pragma unroll
+  for (int q = 0; q < kNStat; ++q) {
+    const int c = q < 15 ? q : q + 12;
+    const float x = f[q] * s[q];
+    ha = mfma_w4(wreg[(2 * c) / 16], x, ha, (2 * c) % 16);
+    hb = mfma_w4(wreg[(2 * c + 1) / 16], x, hb, (2 * c + 1) % 16);
+  }
+  v4f ga = mfma_w4(wreg[kC2GrpBH / 16], 1.0f, zero, kC2GrpBH % 16);
+  v4f gb = mfma_w4(wreg[(kC2GrpBH + 1) / 16], 1.0f, zero, (kC2GrpBH + 1) % 16);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float hk = relu(k < 4 ? ha[k] : hb[k - 4]);
+    ga = mfma_w4(wreg[(kC2GrpWH + 2 * k) / 16], hk, ga, (kC2GrpWH + 2 * k) % 16);
+    gb = mfma_w4(wreg[(kC2GrpWH + 2 * k + 1) / 16], hk, gb, (kC2GrpWH + 2 * k + 1) % 16);
+  }
+  v4f o = mfma_w4(wreg[kC2GrpBO / 16], 1.0f, zero, kC2GrpBO % 16);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float hk = relu(k < 4 ? ga[k] : gb[k - 4]);
+    o = mfma_w4(wreg[(kC2GrpWO + k) / 16], hk, o, (kC2GrpWO + k) % 16);
+  }
+  return o[0] * expf(o[1] * exp_mult);
+}
+
+// Short slices (1 .. 32 elements) of tensors with more than two dims: a wave takes the 64 / S whole slices that fit it, a
+// lane an element, consecutive in every array, so that all loads and stores are coalesced, every input is read and every
+// output written once, and an element's features are computed once.  The sums over a slice go through the wave's own
+// LDS: f^2 in as [channel][lane], then a lane sums a (slice, channel) at a time -- in the slice's order -- and leaves its
+// normaliser, which the slice's lanes read back.
+// TERMS: a factored vector's entries lie in runs of S that the slices meet whole (slice_runs), so the twelve channels that
+// depend on the row or the column only have one normaliser a run: k_v0b has normalised them and pushed them through the
+// first layer, [entry][8] in the term tables, and 24 of the 89 rank-1 updates of an element's MLP and 18 of its reciprocal
+// roots go.  Else (small tensors whose factored dims are dims of the slice) they are gathered and normalised like the others.
+// What bounds it: instruction issue -- some 370 instructions a trip, 63 of them rank-1 updates and 19 reciprocal roots -- where the
+// bytes would take half the time.  ResNet-50's kernels, a lane walking its slice twice through LDS before / now: 12.1 M
+// elements of 1 x 1 227 / 145 us (3.7 TB/s), 11.3 M of 3 x 3 300 / 161; whole CELO2 step 1.19 / 0.98 ms.
+// Item: tensor, first slice of the block, trips (of 64 / S slices) a wave.  LEN: the slice length, 0: any.
+constexpr int kSliceLd = 65;       // floats per channel of the squares in LDS
+template <int LEN, bool TERMS>
+__global__ __launch_bounds__(kThreads) void k_celo2_slices_wave(const TDesc* __restrict__ descs,
+                                                                const PyloTensorArgs* __restrict__ dyn,
+                                                                const Item* __restrict__ items,
+                                                                const float* __restrict__ fac_tab,
+                                                                const float* __restrict__ term_tab,
+                                                                const Globals* __restrict__ gl, PyloDecays dec,
+                                                                const float* __restrict__ mlp) {
+  constexpr int NC = TERMS ? kNStat : 30, NCP = TERMS ? 20 : 32;   // channels, and the pitch of a slice's normalisers
+  // squares, then the normalisers of at most 32 slices and of the lanes past the last whole one
+  __shared__ float lds[kWaves][LEN == 1 ? 1 : NC * kSliceLd + 33 * NCP];
   const Item it = items[blockIdx.x];
   TDesc d = descs[it.tensor];
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
   set_grad_scale(d, a, gl, it.tensor);
   const EmaConsts e = make_ema(dec);
-  const int S = d.slice_len, lane = threadIdx.x;
-  const long long n = d.n, n_slices = n / S;
-  float* Lg = sl_lds;
-  float* Lp = Lg + S * P;
-  float* Lm0 = Lp + S * P;
-  float* Lm1 = Lm0 + S * P;
-  float* Lm2 = Lm1 + S * P;
-  float* Lr = Lm2 + S * P;
-  // idx / S for idx < 64 * S <= 2048 without the integer division: the half keeps the product 0.5 / S away from
-  // the integers, the rounding of a float product of this size is some 1e-4 at most
+  const int S = LEN ? LEN : d.slice_len, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int spw = 64 / S, per = spw * S, sl = lane / S;
+  const long long n = d.n;
   const float inv_s = 1.0f / (float)S;
+  float* sq = lds[wave];
+  float* nrm = sq + NC * kSliceLd;
+  // the lane's (slice, channel) pairs: its slice, its first channel, and how many channels the wave sums at a time
+  const int pc0 = lane / spw, ps = lane - pc0 * spw, pcs = 64 / spw;
   float wreg[6];
   slice_mlp_weights(mlp, wreg);
-  if (S == 1) {
-    // A slice is an element (1 x 1 kernels): nothing to stage, every lane takes its own element, and the next
-    // group's loads are in flight under this group's arithmetic.  Lanes past the end work on the block's first element
-    // and store nothing.
-    struct In { float g, p, m[3], r; SliceFac fac; };
-    auto fetch = [&](long long idx) {
-      In x;
-      x.g = *(const gfloat*)(a.grad + idx);
-      x.p = *(const gfloat*)(a.param + idx);
-      x.m[0] = *(const gfloat*)(a.mom + idx);
-      x.m[1] = *(const gfloat*)(a.mom + n + idx);
-      x.m[2] = *(const gfloat*)(a.mom + 2 * n + idx);
-      x.r = *(const gfloat*)(a.rms + idx);
-      x.fac = slice_gather_nd(d, a, idx, fac_tab);
-      return x;
-    };
-    const long long b0 = it.a;
-    In cur = fetch(b0 + lane < n ? b0 + lane : b0);
-    for (int grp = 0; grp < slice_lane_groups(1); ++grp) {
-      const long long idx = b0 + 64 * grp + lane;
-      if (b0 + 64 * grp >= n) break;
-      const bool mine = idx < n;
-      const long long nidx = idx + 64;
-      const In nxt = fetch(grp + 1 < slice_lane_groups(1) && nidx < n ? nidx : b0);
-      const float g = cond_grad(cur.g, d.gscale, a.clip_val, d.nan0);
-      float m[3] = {cur.m[0], cur.m[1], cur.m[2]}, rms = cur.r, f[30], sc[30];
+  struct In { float g, p, m[3], r; };
+  auto fetch = [&](long long first, unsigned off) {   // (the wave's first element, the lane's from there)
+    In x;
+    x.g = *(const gfloat*)(a.grad + first + off);
+    x.p = *(const gfloat*)(a.param + first + off);
+    x.m[0] = *(const gfloat*)(a.mom + first + off);
+    x.m[1] = *(const gfloat*)(a.mom + n + first + off);
+    x.m[2] = *(const gfloat*)(a.mom + 2 * n + first + off);
+    x.r = *(const gfloat*)(a.rms + first + off);
+    return x;
+  };
+  // Lanes past the last whole slice of the wave or of the tensor work on the wave's first element and store nothing (the
+  // matrix instructions want the whole wave).
+  long long e0 = ((long long)it.a + (long long)wave * it.b * spw) * S;
+  if (e0 >= n) return;
+  auto mine = [&](long long first) { return lane < per && first + lane < n; };
+  In cur = fetch(e0, mine(e0) ? lane : 0);
+  for (int trip = 0; trip < it.b && e0 < n; ++trip, e0 += per) {
+    const bool live = mine(e0);
+    const unsigned off = live ? lane : 0;
+    const long long idx = e0 + off;
+    const long long next = trip + 1 < it.b && e0 + per < n ? e0 + per : e0;
+    const In nxt = fetch(next, mine(next) ? lane : 0);
+    float f[NC], sc[NC], m[3] = {cur.m[0], cur.m[1], cur.m[2]}, rms = cur.r;
+    const float g = cond_grad(cur.g, d.gscale, a.clip_val, d.nan0);
+    v4f ta[2], tb[2];
+    if constexpr (TERMS) {
+      const unsigned u = (unsigned)idx;
+      const unsigned s0 = (unsigned)d.nd_stride[0], s1 = (unsigned)d.nd_stride[1];
+      const size_t i0 = fd_div(u, d.nd_div_blk[0]) * s0 + (u - fd_div(u, d.nd_div_st[0]) * s0);
+      const size_t i1 = fd_div(u, d.nd_div_blk[1]) * s1 + (u - fd_div(u, d.nd_div_st[1]) * s1);
+      const float4 fa = load_f4(fac_tab + d.fac_off[0] + i0 * 4), fb = load_f4(fac_tab + d.fac_off[1] + i1 * 4);
+      const gv4f* t0 = (const gv4f*)(term_tab + d.term_off[0] + i0 * 8);
+      const gv4f* t1 = (const gv4f*)(term_tab + d.term_off[1] + i1 * 8);
+      ta[0] = t0[0]; ta[1] = t0[1];
+      tb[0] = t1[0]; tb[1] = t1[1];
       ema_update(e, g, m, rms);
-      slice_features_nd(cur.fac, g, cur.p, m, rms, f);
-#pragma unroll
-      for (int c = 0; c < 30; ++c) sc[c] = rsq(1e-9f + f[c] * f[c]);
-      const float step = slice_mlp_mfma(f, sc, wreg, a.exp_mult);
-      if (mine) {
-        *(gfloat*)(a.mom + idx) = m[0];
-        *(gfloat*)(a.mom + n + idx) = m[1];
-        *(gfloat*)(a.mom + 2 * n + idx) = m[2];
-        *(gfloat*)(a.rms + idx) = rms;
-        *(gfloat*)(a.step_out + idx) = step;
-      }
-      cur = nxt;
+      const float rfcf[3] = {fa.x * fb.x, fa.y * fb.y, fa.z * fb.z};
+      lo_features(g, cur.p, m, rms, rfcf, 1e-8f, f);
+    } else {
+      const SliceFac fac = slice_gather_nd(d, a, idx, fac_tab);
+      ema_update(e, g, m, rms);
+      slice_features_nd(fac, g, cur.p, m, rms, f);
     }
-    return;
-  }
-  for (int grp = 0; grp < slice_lane_groups(S); ++grp) {
-    const long long s0 = (long long)it.a + 64 * grp, left = n_slices - s0;
-    if (left <= 0) break;
-    const int live = left < 64 ? (int)left : 64, total = live * S;
-    const long long e0 = s0 * S;
-    for (int idx = lane; idx < total; idx += 64) {
-      const int sl = (int)(((float)idx + 0.5f) * inv_s), pos = (idx - sl * S) * P + sl;
-      const long long gi = e0 + idx;
-      Lg[pos] = cond_grad(*(const gfloat*)(a.grad + gi), d.gscale, a.clip_val, d.nan0);
-      Lp[pos] = *(const gfloat*)(a.param + gi);
-      Lm0[pos] = *(const gfloat*)(a.mom + gi);
-      Lm1[pos] = *(const gfloat*)(a.mom + n + gi);
-      Lm2[pos] = *(const gfloat*)(a.mom + 2 * n + gi);
-      Lr[pos] = *(const gfloat*)(a.rms + gi);
-    }
-    __syncthreads();
-    {
-      // every lane walks a slice (the matrix instructions of the MLP want the whole wave): lanes past the last slice
-      // walk the first one again and write nothing
-      const bool mine = lane < live;
-      const int col = mine ? lane : 0;
-      const long long first = e0 + (long long)col * S;
-      float acc[30], f[30];
+    if constexpr (LEN == 1) {
 #pragma unroll
-      for (int c = 0; c < 30; ++c) acc[c] = 0.0f;
-      SliceFac fac = slice_gather_nd(d, a, first, fac_tab);
-      for (int j = 0; j < S; ++j) {
-        // the next element's loads before this one's arithmetic; the last round fetches the second walk's first
-        const SliceFac nxt = slice_gather_nd(d, a, first + (j + 1 < S ? j + 1 : 0), fac_tab);
-        const int pos = j * P + col;
-        float m[3] = {Lm0[pos], Lm1[pos], Lm2[pos]}, rms = Lr[pos];
-        const float g = Lg[pos];
-        ema_update(e, g, m, rms);
-        if (mine) { Lm0[pos] = m[0]; Lm1[pos] = m[1]; Lm2[pos] = m[2]; Lr[pos] = rms; }
-        slice_features_nd(fac, g, Lp[pos], m, rms, f);
-        fac = nxt;
+      for (int c = 0; c < NC; ++c) sc[c] = rsq(1e-9f + f[c] * f[c]);
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the previous trip's reads are done
 #pragma unroll
-        for (int c = 0; c < 30; ++c) acc[c] = fmaf(f[c], f[c], acc[c]);
-      }
-      float sc[30];
+      for (int c = 0; c < NC; ++c) sq[c * kSliceLd + lane] = f[c] * f[c];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      for (int c = pc0; c < NC && pc0 < pcs; c += pcs) {
+        const float* q = sq + c * kSliceLd + ps * S;
+        float t = 0.0f;
+        if constexpr (LEN != 0) {
 #pragma unroll
-      for (int c = 0; c < 30; ++c) sc[c] = rsq(1e-9f + acc[c] * inv_s);   // the mean by the reciprocal, not thirty divisions
-      for (int j = 0; j < S; ++j) {
-        const int pos = j * P + col;
-        if (S > 1) {   // a slice of one element still has its features from the first walk
-          const SliceFac nxt = slice_gather_nd(d, a, first + (j + 1 < S ? j + 1 : 0), fac_tab);
-          const float m[3] = {Lm0[pos], Lm1[pos], Lm2[pos]};
-          slice_features_nd(fac, Lg[pos], Lp[pos], m, Lr[pos], f);
-          fac = nxt;
+          for (int j = 0; j < LEN; ++j) t += q[j];
+        } else {
+          for (int j = 0; j < S; ++j) t += q[j];
         }
-        const float step = slice_mlp_mfma(f, sc, wreg, a.exp_mult);
-        if (mine) Lg[pos] = step;
+        nrm[ps * NCP + c] = rsq(1e-9f + t * inv_s);   // the mean by the reciprocal
       }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int c = 0; c < NC; ++c) sc[c] = nrm[(lane < per ? sl : 0) * NCP + c];
     }
-    __syncthreads();
-    for (int idx = lane; idx < total; idx += 64) {
-      const int sl = (int)(((float)idx + 0.5f) * inv_s), pos = (idx - sl * S) * P + sl;
-      const long long gi = e0 + idx;
-      *(gfloat*)(a.mom + gi) = Lm0[pos];
-      *(gfloat*)(a.mom + n + gi) = Lm1[pos];
-      *(gfloat*)(a.mom + 2 * n + gi) = Lm2[pos];
-      *(gfloat*)(a.rms + gi) = Lr[pos];
-      *(gfloat*)(a.step_out + gi) = Lg[pos];
+    float step;
+    if constexpr (TERMS) step = slice_mlp_terms(f, sc, ta, tb, wreg, a.exp_mult);
+    else step = slice_mlp_mfma(f, sc, wreg, a.exp_mult);
+    if (live) {
+      *(gfloat*)(a.mom + e0 + off) = m[0];
+      *(gfloat*)(a.mom + n + e0 + off) = m[1];
+      *(gfloat*)(a.mom + 2 * n + e0 + off) = m[2];
+      *(gfloat*)(a.rms + e0 + off) = rms;
+      *(gfloat*)(a.step_out + e0 + off) = step;
     }
-    __syncthreads();   // the next group's loads overwrite what the stores above read
+    cur = nxt;
   }
 }
 

@@ -653,6 +653,28 @@ __global__ __launch_bounds__(kThreads) void k_v0b(const TDesc* __restrict__ desc
       const int st = d.rcm_stride, blk = d.rcm_size * st;
       slice = (i / blk - o_first) * st + i % st;
     }
+    if (d.slice_runs) {   // the channels are normalised over the run of slice_len entries that slices meet (k_celo2_slices_wave)
+      const int S = d.slice_len, r0 = i - i % S;
+      const float inv_s = 1.0f / (float)S;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        float t0 = 0.0f, t1 = 0.0f;
+        for (int j0 = 0; j0 < S; j0 += 9) {   // nine entries are requested before any is added
+          float f[9];
+#pragma unroll
+          for (int j = 0; j < 9; ++j) f[j] = S == 1 ? fpre[q][k] : *(const gfloat*)(fac + (size_t)k * len + r0 + min(j0 + j, S - 1));
+#pragma unroll
+          for (int j = 0; j < 9; ++j) {
+            if (j0 + j >= S) break;
+            const float r = rsq(f[j] + 1e-8f);
+            t0 = fmaf(f[j], f[j], t0);
+            t1 = fmaf(r, r, t1);
+          }
+        }
+        s0[k] = rsq(norm_eps + t0 * inv_s);
+        s1[k] = rsq(norm_eps + t1 * inv_s);
+      }
+    }
     vector_entry(d, is_r, fac, len, i, fpre[q], rcm3, s0, s1, fct, x0, x1, rcm_slices, slice);
     *(float4*)(fac_tab + fac_index(d, which, 0, i)) = make_float4(fct[0], fct[1], fct[2], 0.0f);
     if (w1 != nullptr) vector_terms<H>(d, which, is_r, i, x0, x1, w1, b1 + (size_t)it.tensor * b1_stride, term_tab);

@@ -109,6 +109,7 @@ struct TDesc {
   int adam_indep;          // kModeFlat: AdamW on the tensor's own two moments instead of mom[0] / rms
   int fin_unit0, fin_units;  // ELO-CELO2 finishing pass: the tensor's units (FinUnit)
   int slice_len;           // CELO2, N-D or fewer than two dims: elements per slice of the last two dims (or n)
+  int slice_runs;          // ... short slices, and both vectors lost a dim outside them: their entries lie in runs of slice_len
   int nan0;                // gradients pass through torch.nan_to_num (PYLO_F_NAN_TO_NUM)
   int wd_prestep;          // p -= lr * (step + wd * p) against the pre-step parameter (PYLO_F_WD_PRESTEP)
   int store;               // storage type of the caller's grad / param buffers (kStore*, k_cast.h); 0 = fp32

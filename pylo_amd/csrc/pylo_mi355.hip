@@ -146,10 +146,10 @@ struct Layout {
   long long stage_floats = 0;
   size_t off_dyn_user = 0, off_stage_ofs = 0, off_cast_items = 0, off_stage = 0;
   std::vector<TDesc> descs;
-  std::vector<Item> sl_lane_items;    // ELO-CELO2: blocks of k_celo2_slices_lane, the classes of slice length one after another
-  std::vector<Item> sl_lane_cls[kSliceLaneClasses];
-  int sl_lane_n[kSliceLaneClasses] = {}, sl_lane_lds[kSliceLaneClasses] = {};   // a launch per class: LDS sized for its longest slice
-  size_t off_sl_lane_items = 0;
+  std::vector<Item> sl_wave_items;    // ELO-CELO2: blocks of k_celo2_slices_wave, one class after another
+  std::vector<Item> sl_wave_cls[kSliceWaveClasses];
+  int sl_wave_n[kSliceWaveClasses] = {};
+  size_t off_sl_wave_items = 0;
   std::vector<Item> p0_items, nd_items, sl_items, seg_items, el_items, ap_items, pp_items, ga_items, fin_items, v0a_items, v0b_items;
   std::vector<int> fac_list;
   std::vector<int> dc, dr;
@@ -400,8 +400,8 @@ NsExps ns_plane_exps(float c0, float c1, float c2, int iters) {
   return ex;
 }
 
-// PYLO_MI355_SLICES_LDS=0: the short slices of ELO-CELO2 tensors with more than two dims stay on the kernel that reads
-// them straight from memory, twice (k_celo2_slices); read at plan creation.
+// PYLO_MI355_SLICES_LDS=0: the short slices of ELO-CELO2 tensors with more than two dims stay on the kernel that walks
+// them twice (k_celo2_slices); read at plan creation.
 bool env_slices_lds() {
   const char* e = getenv("PYLO_MI355_SLICES_LDS");
   return !(e && e[0] == '0');
@@ -1032,6 +1032,18 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
   L.split = split > 1;
   L.tensor_norm = (shapes[0].flags & PYLO_F_TENSOR_NORM) != 0;
   L.global_norm = (shapes[0].flags & PYLO_F_GLOBAL_NORM) != 0 || L.tensor_norm;
+  // Short slices (k_celo2_slices_wave): trips a wave, as many as leave sixteen waves a CU and no more than eight
+  // (the set-up of a wave, its weights, costs about as much as a trip).
+  long long slice_elems = 0;
+  for (int t = 0; t < T && kind == PYLO_KIND_CELO2; ++t) {
+    const PyloTensorShape& s = shapes[t];
+    if (s.ndim < 3 || s.ndim > PYLO_MAX_DIMS || s.shape[s.ndim - 2] * s.shape[s.ndim - 1] > kSliceLaneMax) continue;
+    long long n = 1;
+    for (int i = 0; i < s.ndim; ++i) n *= s.shape[i];
+    slice_elems += n;
+  }
+  const int slice_trips = (int)std::max<long long>(1, std::min<long long>(8, slice_elems / (64 * 16 * 256)));
+  auto short_slices = [&](const TDesc& d) { return d.mode == kModeFacND && d.slice_len <= kSliceLaneMax && env_slices_lds(); };
   for (int t = 0; t < T; ++t) {
     const PyloTensorShape& s = shapes[t];
     if (s.ndim < 0 || s.ndim > PYLO_MAX_DIMS) return fail("plan: bad ndim");
@@ -1169,13 +1181,13 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       // one pass per slice of the last two dims (k_celo2_slices): 256 slices a block, or 4
       const long long n_slices = n / d.slice_len, per = d.slice_len <= kSliceLaneMax ? kThreads : kWaves;
       if (n_slices >= (1ll << 31)) return fail("plan: too many slices");
-      if (d.mode == kModeFacND && d.slice_len <= kSliceLaneMax && env_slices_lds()) {
-        // short slices of a tensor with more than two dims: 64 a block, staged through LDS (k_celo2_slices_lane)
-        int cls = 0;
-        while (d.slice_len > kSliceLaneClassMax[cls]) ++cls;
-        for (long long s0 = 0; s0 < n_slices && n > 0; s0 += 64 * slice_lane_groups(d.slice_len))
-          L.sl_lane_cls[cls].push_back(Item{t, (int)s0, 0, 0});
-        L.sl_lane_lds[cls] = std::max(L.sl_lane_lds[cls], (int)sizeof(float) * 6 * d.slice_len * kSlicePitchF);
+      if (short_slices(d)) {
+        // short slices of a tensor with more than two dims: packed into waves (k_celo2_slices_wave)
+        d.slice_runs = d.nd_stride[0] % d.slice_len == 0 && d.nd_stride[1] % d.slice_len == 0;
+        const int cls = !d.slice_runs ? kSliceGather : d.slice_len == 1 ? kSliceOne : d.slice_len == 9 ? kSliceNine : kSliceAny;
+        const long long per_wave = 64 / d.slice_len;
+        for (long long s0 = 0; s0 < n_slices && n > 0; s0 += kWaves * per_wave * slice_trips)
+          L.sl_wave_cls[cls].push_back(Item{t, (int)s0, slice_trips, 0});
       } else
       for (long long s0 = 0; s0 < n_slices && n > 0; s0 += per) L.sl_items.push_back(Item{t, (int)s0, 0, 0});
     } else if (wide && d.C0 % kTileCols == 0) {
@@ -1269,12 +1281,12 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
   L.off_p0_items = take(sizeof(Item) * L.p0_items.size());
   L.off_nd_items = take(sizeof(Item) * L.nd_items.size());
   L.off_sl_items = take(sizeof(Item) * L.sl_items.size());
-  for (int c = 0; c < kSliceLaneClasses; ++c) {
-    L.sl_lane_n[c] = (int)L.sl_lane_cls[c].size();
-    L.sl_lane_items.insert(L.sl_lane_items.end(), L.sl_lane_cls[c].begin(), L.sl_lane_cls[c].end());
-    L.sl_lane_cls[c] = std::vector<Item>();
+  for (int c = 0; c < kSliceWaveClasses; ++c) {
+    L.sl_wave_n[c] = (int)L.sl_wave_cls[c].size();
+    L.sl_wave_items.insert(L.sl_wave_items.end(), L.sl_wave_cls[c].begin(), L.sl_wave_cls[c].end());
+    L.sl_wave_cls[c] = std::vector<Item>();
   }
-  L.off_sl_lane_items = take(sizeof(Item) * L.sl_lane_items.size());
+  L.off_sl_wave_items = take(sizeof(Item) * L.sl_wave_items.size());
   L.off_seg_items = take(sizeof(Item) * L.seg_items.size());
   L.off_segtot = take(sizeof(double) * kStatW * L.seg_items.size());
   L.off_el_items = take(sizeof(Item) * L.el_items.size());
@@ -1432,7 +1444,7 @@ int pylo_mi355_plan_create(int kind, const PyloTensorShape* shapes, int n_tensor
   if (e == hipSuccess) e = up(L.off_cast_items, L.cast_items.data(), sizeof(Item) * L.cast_items.size());
   if (e == hipSuccess) e = up(L.off_nd_items, L.nd_items.data(), sizeof(Item) * L.nd_items.size());
   if (e == hipSuccess) e = up(L.off_sl_items, L.sl_items.data(), sizeof(Item) * L.sl_items.size());
-  if (e == hipSuccess) e = up(L.off_sl_lane_items, L.sl_lane_items.data(), sizeof(Item) * L.sl_lane_items.size());
+  if (e == hipSuccess) e = up(L.off_sl_wave_items, L.sl_wave_items.data(), sizeof(Item) * L.sl_wave_items.size());
   if (e == hipSuccess) e = up(L.off_seg_items, L.seg_items.data(), sizeof(Item) * L.seg_items.size());
   if (e == hipSuccess) e = up(L.off_el_items, L.el_items.data(), sizeof(Item) * L.el_items.size());
   if (e == hipSuccess) e = up(L.off_ap_items, L.ap_items.data(), sizeof(Item) * L.ap_items.size());
@@ -1901,10 +1913,15 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
   }
   if (n_sl > 0)
     hipLaunchKernelGGL(k_celo2_slices, dim3(n_sl), dim3(kThreads), 0, s, descs, dyn, sl_items, fac_tab, gl, dec, mlp);
-  for (int c = 0, at = 0; c < kSliceLaneClasses; at += L.sl_lane_n[c], ++c)
-    if (L.sl_lane_n[c] > 0)
-      hipLaunchKernelGGL(k_celo2_slices_lane, dim3((unsigned)L.sl_lane_n[c]), dim3(64), L.sl_lane_lds[c], s, descs, dyn,
-                         P->at<Item>(L.off_sl_lane_items) + at, fac_tab, gl, dec, mlp);
+  for (int c = 0, at = 0; c < kSliceWaveClasses; at += L.sl_wave_n[c], ++c) {
+    if (L.sl_wave_n[c] == 0) continue;
+    const auto wave = c == kSliceOne    ? k_celo2_slices_wave<1, true>
+                      : c == kSliceNine ? k_celo2_slices_wave<9, true>
+                      : c == kSliceAny  ? k_celo2_slices_wave<0, true>
+                                        : k_celo2_slices_wave<0, false>;
+    hipLaunchKernelGGL(wave, dim3((unsigned)L.sl_wave_n[c]), dim3(kThreads), 0, s, descs, dyn, P->at<Item>(L.off_sl_wave_items) + at,
+                       fac_tab, term_tab, gl, dec, mlp);
+  }
   HIP_TRY(mark());
   mark.done();
   stage_out(P, s, 1);   // only the AdamW tensors were updated
