@@ -1861,10 +1861,16 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
   Marks mark(P, s);
 
   const bool exact_pass = exact_pass_possible(P, args);
+  // Where no tensor is clipped by the global norm nobody reads it: only the matrices' sums are taken, and those of tensors with
+  // more dims, which wait for its scale otherwise, in the same launch.  (Records that are read when the kernels run, as
+  // under capture, may ask for it later.)  CELO2 on ResNet-50, both launches: 124 us, now 54 in one.
+  const bool clips = std::any_of(args, args + P->T, [](const PyloTensorArgs& a) { return a.grad != nullptr && a.clip_norm > 0.0f; }) ||
+                     std::find(P->stage, P->stage + kStageSlots, args) != P->stage + kStageSlots;
+  const int n_tail = clips ? 0 : n_nd;
   HIP_TRY(mark());
-  if (n_p0 > 0)
-    hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 0,
-                       (const Item*)nullptr, n_p0);
+  if (n_p0 + n_tail > 0)
+    hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0 + n_tail), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag,
+                       gl, clips ? 0 : 2, nd_items, n_p0);
   HIP_TRY(mark());
   hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, gsq, flag, n_p0, gl, exact_pass ? 1 : 0,
                      P->at<int>(L.off_sync), 2 * P->T);
@@ -1872,7 +1878,7 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
   if (n_p0 > 0 && exact_pass)
     hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
                        (const Item*)nullptr, n_p0);
-  if (n_nd > 0) hipLaunchKernelGGL(k_p0_nd, dim3(n_nd), dim3(kThreads), 0, s, descs, dyn, nd_items, part, gl);
+  if (n_nd > 0 && clips) hipLaunchKernelGGL(k_p0_nd, dim3(n_nd), dim3(kThreads), 0, s, descs, dyn, nd_items, part, gl);
   HIP_TRY(mark());
   if (n_v0a > 0)
     hipLaunchKernelGGL(k_v0a, dim3(n_v0a), dim3(kV0aThreads), 0, s, descs, dyn, v0a_items, part, gl, dec, v0part);
