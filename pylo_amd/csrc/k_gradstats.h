@@ -316,17 +316,18 @@ __global__ __launch_bounds__(kThreads) void k_p0_nd(const TDesc* __restrict__ de
 // First stage of the per-tensor reduction of the statistics partials, for tensors with thousands
 // of rows: one block adds up kSegRows rows, so that the per-tensor block that follows (one block,
 // hence one CU's bandwidth) reads a few dozen rows instead of thousands.  Fixed order throughout.
-// Item: tensor, first row (relative to the tensor's rows), number of rows.
+// Item: tensor, first row (relative to the tensor's rows), number of rows.  W: doubles a row (kStatW, kNewSumW).
 // =============================================================================================
+template <int W>
 __global__ __launch_bounds__(kThreads) void k_stat_segsum(const TDesc* __restrict__ descs,
                                                           const Item* __restrict__ items,
                                                           const double* __restrict__ stats_part,
                                                           double* __restrict__ seg_tot) {
-  constexpr int G = kThreads / kStatW;  // 6 groups x 40 channels
-  __shared__ double part[G][kStatW];
+  constexpr int G = kThreads / W;  // 6 groups x 40 channels
+  __shared__ double part[G][W];
   const Item it = items[blockIdx.x];
   const int blk0 = descs[it.tensor].blk0 + it.a;
-  const int c = threadIdx.x % kStatW, gI = threadIdx.x / kStatW;
+  const int c = threadIdx.x % W, gI = threadIdx.x / W;
   if (gI < G) {
     double s = 0.0;
     for (int b0 = gI; b0 < it.b; b0 += 16 * G) {
@@ -334,7 +335,7 @@ __global__ __launch_bounds__(kThreads) void k_stat_segsum(const TDesc* __restric
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
         const int b = b0 + q * G;
-        v[q] = b < it.b ? stats_part[(size_t)(blk0 + b) * kStatW + c] : 0.0;
+        v[q] = b < it.b ? stats_part[(size_t)(blk0 + b) * W + c] : 0.0;
       }
 #pragma unroll
       for (int q = 0; q < 16; ++q) s += v[q];
@@ -342,11 +343,11 @@ __global__ __launch_bounds__(kThreads) void k_stat_segsum(const TDesc* __restric
     part[gI][c] = s;
   }
   __syncthreads();
-  if (threadIdx.x < kStatW) {
+  if (threadIdx.x < W) {
     double s = 0.0;
 #pragma unroll
     for (int g2 = 0; g2 < G; ++g2) s += part[g2][threadIdx.x];
-    seg_tot[(size_t)blockIdx.x * kStatW + threadIdx.x] = s;
+    seg_tot[(size_t)blockIdx.x * W + threadIdx.x] = s;
   }
 }
 

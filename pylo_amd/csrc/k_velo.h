@@ -506,6 +506,7 @@ __device__ __forceinline__ float lo_lstm_feature(const TDesc& d, const PyloTenso
 // (VeLO_RNN.py:110-122): relu(mix2 x) and final_mix x for every hidden unit; the maximum over rows and the sum
 // follow in k_velo_mix.  Afterwards the tensor's pivots for the sums its apply pass will take are stored
 // (its accumulators' first elements as they stand now; the apply pass overwrites them while it runs).
+template <int THREADS>
 __device__ __forceinline__ void velo_row_features(const TDesc& d, const PyloTensorArgs& a, int t, int T,
                                                   const double* tot, const float* piv_in, float* __restrict__ piv_out,
                                                   const LossState& ls, const VeloStep& st, float* __restrict__ xfeat,
@@ -524,13 +525,33 @@ __device__ __forceinline__ void velo_row_features(const TDesc& d, const PyloTens
     for (int q = 0; q < 4; ++q) piv_out[(size_t)t * 4 + q] = pv[q];
   }
   if (threadIdx.x < 30) xfeat[(size_t)row * kXW + threadIdx.x] = xs[threadIdx.x];
-  for (int i = threadIdx.x; i < 2 * H; i += kFoldThreads) {
-    const int u = i < H ? i : i - H;
-    const float* w = i < H ? w2t : wft;
-    float acc = i < H ? b2[u] : bf[u];
+  if constexpr (THREADS >= 1024) {
+    for (int i = threadIdx.x; i < 2 * H; i += THREADS) {
+      const int u = i < H ? i : i - H;
+      const float* w = i < H ? w2t : wft;
+      float acc = i < H ? b2[u] : bf[u];
 #pragma unroll
-    for (int k = 0; k < 30; ++k) acc = fmaf(xs[k], w[k * H + u], acc);
-    mixbuf[((size_t)(i < H ? 0 : 1) * T + row) * H + u] = i < H ? fmaxf(acc, 0.0f) : acc;
+      for (int k = 0; k < 30; ++k) acc = fmaf(xs[k], w[k * H + u], acc);
+      mixbuf[((size_t)(i < H ? 0 : 1) * T + row) * H + u] = i < H ? fmaxf(acc, 0.0f) : acc;
+    }
+  } else {   // four units a thread (H is a multiple of 64)
+    for (int i = 4 * threadIdx.x; i < 2 * H; i += 4 * THREADS) {
+      const int u = i < H ? i : i - H;
+      const float* w = (i < H ? w2t : wft) + u;
+      const float4 b = load_f4((i < H ? b2 : bf) + u);
+      float acc[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int k = 0; k < 30; ++k) {
+        const float4 v = load_f4(w + k * H);
+        acc[0] = fmaf(xs[k], v.x, acc[0]);
+        acc[1] = fmaf(xs[k], v.y, acc[1]);
+        acc[2] = fmaf(xs[k], v.z, acc[2]);
+        acc[3] = fmaf(xs[k], v.w, acc[3]);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] = i < H ? fmaxf(acc[q], 0.0f) : acc[q];
+      *(float4*)(mixbuf + ((size_t)(i < H ? 0 : 1) * T + row) * H + u) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    }
   }
 }
 
@@ -572,7 +593,7 @@ __global__ __launch_bounds__(kFoldThreads) void k_lo_reduce(const TDesc* __restr
   }
   __syncthreads();
   if (xfeat == nullptr) return;
-  velo_row_features(d, a, t, T, tot, nullptr, piv_out, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, xs);
+  velo_row_features<kFoldThreads>(d, a, t, T, tot, nullptr, piv_out, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, xs);
 }
 
 // Behind the 2 T counters and flags of `sync` (rounded up to 16 bytes) the workspace holds the guard of the carried
@@ -586,16 +607,20 @@ __device__ __forceinline__ double* velo_guard_sums(int* sync, int T) { return re
 
 // The same from the sums the previous step's apply pass left (rows of kNewSumW doubles per element
 // block, shifted by the tensor's first elements as that pass wrote them, i.e. as they stand now): the
-// LSTM does not wait for this step's statistics pass.
-__global__ __launch_bounds__(kFoldThreads) void k_velo_feat(const TDesc* __restrict__ descs,
-                                                            const PyloTensorArgs* __restrict__ dyn, int T,
-                                                            const double* __restrict__ newsum_part,
-                                                            float* __restrict__ piv, LossState ls, VeloStep st,
-                                                            float* __restrict__ xfeat, int H,
-                                                            const float* __restrict__ w2t, const float* __restrict__ b2,
-                                                            const float* __restrict__ wft, const float* __restrict__ bf,
-                                                            float* __restrict__ mixbuf, int* __restrict__ sync) {
-  constexpr int G = kFoldThreads / kNewSumW;
+// LSTM does not wait for this step's statistics pass.  Tensors of many rows come summed in segments (k_stat_segsum): one
+// block, a tensor's only one, waited 165 us for the 16 000 rows of an embedding of 131 M elements.  Blocks of four waves,
+// four units a thread: next to k_p0, whose blocks take the place of every four waves that end, blocks of sixteen wait.
+// Three thousand tensors and that embedding 387 / 41 us next to k_p0, whole step 2.91 / 2.77 ms; ViT-B/16 80 / 72 us, 1.01 / 1.00 ms
+// (8 us without the gradients streaming past it: what is left is a chain of short dependent loads).
+__global__ __launch_bounds__(kThreads) void k_velo_feat(const TDesc* __restrict__ descs,
+                                                        const PyloTensorArgs* __restrict__ dyn, int T,
+                                                        const double* __restrict__ newsum_part, const double* __restrict__ seg_tot,
+                                                        float* __restrict__ piv, LossState ls, VeloStep st,
+                                                        float* __restrict__ xfeat, int H,
+                                                        const float* __restrict__ w2t, const float* __restrict__ b2,
+                                                        const float* __restrict__ wft, const float* __restrict__ bf,
+                                                        float* __restrict__ mixbuf, int* __restrict__ sync) {
+  constexpr int G = kThreads / kNewSumW;
   __shared__ double part[G][kNewSumW];
   __shared__ double tot[kStatW];
   __shared__ float xs[32];
@@ -605,13 +630,14 @@ __global__ __launch_bounds__(kFoldThreads) void k_velo_feat(const TDesc* __restr
   const int c = threadIdx.x % kNewSumW, gI = threadIdx.x / kNewSumW;
   if (gI < G) {
     double s = 0.0;
-    const double* rows = newsum_part + (size_t)d.blk0 * kNewSumW;
-    for (int b0 = gI; b0 < d.nblk; b0 += 16 * G) {
+    const double* rows = d.nseg > 0 ? seg_tot + (size_t)d.seg0 * kNewSumW : newsum_part + (size_t)d.blk0 * kNewSumW;
+    const int n_rows = d.nseg > 0 ? d.nseg : d.nblk;
+    for (int b0 = gI; b0 < n_rows; b0 += 16 * G) {
       double v[16];
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
         const int b = b0 + q * G;
-        v[q] = b < d.nblk ? rows[(size_t)b * kNewSumW + c] : 0.0;
+        v[q] = b < n_rows ? rows[(size_t)b * kNewSumW + c] : 0.0;
       }
 #pragma unroll
       for (int q = 0; q < 16; ++q) s += v[q];
@@ -630,7 +656,7 @@ __global__ __launch_bounds__(kFoldThreads) void k_velo_feat(const TDesc* __restr
     if (q == 0) velo_guard_sums(sync, T)[t] = s;   // the statistics items of this step hold it against the sum they take themselves
   }
   __syncthreads();
-  velo_row_features(d, a, t, T, tot, nullptr, piv, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, xs);
+  velo_row_features<kThreads>(d, a, t, T, tot, nullptr, piv, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, xs);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -1905,7 +1905,7 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
     const Item* seg_items = P->at<Item>(L.off_seg_items);
     double* seg_tot = P->at<double>(L.off_segtot);
     const int n_seg = (int)L.seg_items.size();
-    if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum, dim3(n_seg), dim3(kThreads), 0, s, descs, seg_items, stats, seg_tot);
+    if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3(n_seg), dim3(kThreads), 0, s, descs, seg_items, stats, seg_tot);
     if (n_fac > 0)
       hipLaunchKernelGGL(k_celo2_fold, dim3(n_fac), dim3(kFoldThreads), 0, s, descs, dyn, fac_list, stats, seg_tot, mlp, wfold,
                          chan_ms);
@@ -2455,7 +2455,11 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
     // previous step's apply items left them.  It runs next to the gradient sums, on the plan's own stream.
     HIP_TRY(hipEventRecord(P->ev_fork, s));
     HIP_TRY(hipStreamWaitEvent(P->side, P->ev_fork, 0));
-    hipLaunchKernelGGL(k_velo_feat, dim3(T), dim3(kFoldThreads), 0, P->side, descs, dyn, T, (const double*)newsum, piv, ls, vs,
+    if (!L.seg_items.empty())
+      hipLaunchKernelGGL(k_stat_segsum<kNewSumW>, dim3((unsigned)L.seg_items.size()), dim3(kThreads), 0, P->side, descs,
+                         P->at<Item>(L.off_seg_items), (const double*)newsum, P->at<double>(L.off_segtot));
+    hipLaunchKernelGGL(k_velo_feat, dim3(T), dim3(kThreads), 0, P->side, descs, dyn, T, (const double*)newsum,
+                       (const double*)P->at<double>(L.off_segtot), piv, ls, vs,
                        xfeat, H, nets->mix2_wt, nets->mix2_b, nets->fmix_wt, nets->fmix_b, mixbuf, P->at<int>(L.off_sync));
     lstm(P->side, nullptr, false);
     HIP_TRY(hipEventRecord(P->ev_join, P->side));
@@ -2490,7 +2494,7 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   const Item* seg_items = P->at<Item>(L.off_seg_items);
   double* seg_tot = P->at<double>(L.off_segtot);
   const int n_seg = (int)L.seg_items.size();
-  if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum, dim3(n_seg), dim3(kThreads), 0, s, descs, seg_items, stats, seg_tot);
+  if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3(n_seg), dim3(kThreads), 0, s, descs, seg_items, stats, seg_tot);
   hipLaunchKernelGGL(k_lo_reduce, dim3(T), dim3(kFoldThreads), 0, s, descs, dyn, T, stats, seg_tot, totals, ls, vs, xfeat,
                      H, nets->mix2_wt, nets->mix2_b, nets->fmix_wt, nets->fmix_b, mixbuf, piv);
   if (n_mx == 0) HIP_TRY(mark());
@@ -2606,7 +2610,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   const Item* seg_items = P->at<Item>(L.off_seg_items);
   double* seg_tot = P->at<double>(L.off_segtot);
   const int n_seg = (int)L.seg_items.size();
-  if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum, dim3(n_seg), dim3(kThreads), 0, s, descs, seg_items, stats, seg_tot);
+  if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3(n_seg), dim3(kThreads), 0, s, descs, seg_items, stats, seg_tot);
   hipLaunchKernelGGL(k_lo_reduce, dim3(T), dim3(kFoldThreads), 0, s, descs, dyn, T, stats, seg_tot, totals, LossState{}, vs,
                      (float*)nullptr, 0, (const float*)nullptr, (const float*)nullptr, (const float*)nullptr,
                      (const float*)nullptr, (float*)nullptr, (float*)nullptr);
