@@ -476,15 +476,16 @@ int ns_small_chunk(int cls) { return cls == 0 ? SmSmall::NB : cls == 1 ? SmMid::
 int ns_small_edge(int cls) { return cls == 0 ? SmSmall::MP : cls == 1 ? SmMid::MP : SmLarge::MP; }
 
 // Which matrices the one-launch kernel takes: a smaller dim of at most 128 (its m x m matrices fit a CU's LDS) and a
-// longer one up to where its few blocks, each walking chunks of the long dim one after another, fall behind tiles on all CUs.
-// Whole steps of a classifier with one n x m matrix in front, small kernel against tiled products:
-//   m = 128: n = 4096 290 / 348 us, 8192 436 / 477, 16384 732 / 487        m = 64: 16384 226 / 419, 32768 341 / 466
-//   m = 32: 16384 206 / 340, 32768 297 / 365, 65536 475 / 410              m = 1: 32768 158 / 306
-// (three thousand odd matrices, the limit of m <= 16 at 1024, 16384, 65536: 3954, 3081, 2792 us)
+// longer one up to where its few blocks, each walking chunks of the long dim one after another, fall behind tiles of 64 x 64
+// on all CUs.  Finishing calls on one matrix, small kernel / tiled products, us:
+//   m = 128: n = 1024 97 / 113, 2048 (two chunks a block) 148 / 115, 8192 348 / 177     m = 100: 1024 88 / 113, 2048 132 / 116
+//   m = 64: 8192 97 / 149, 16384 146 / 156, 32768 240 / 178        m = 32: 8192 99 / 141, 16384 140 / 143, 32768 221 / 163
+//   m = 16: 8192 67 / 135, 16384 92 / 138, 32768 145 / 151
+// (m <= 16 stays to 65536: such matrices come in hundreds, where the blocks that wait for memory are many)
 bool ns_small_takes(int R, int C) {
   const int m = std::min(R, C), n = std::max(R, C);
   if (m > SmLarge::MP) return false;
-  return n <= (m <= 16 ? 65536 : m <= SmMid::MP ? 32768 : 8192);
+  return n <= (m <= 16 ? 65536 : m <= SmMid::MP ? 16384 : 1024);
 }
 
 // Whether a plan's small matrices go aside to their own launches, or with the larger ones through the tiled launches that
