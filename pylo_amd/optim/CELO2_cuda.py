@@ -76,8 +76,9 @@ class CELO2_CUDA(ELO_CELO2_CUDA):
     def _init_state(self, state, p, adam):
         if not adam:
             return super()._init_state(state, p, adam)
-        state["exp_avg"] = torch.zeros_like(p)
-        state["exp_avg_sq"] = torch.zeros_like(p)
+        # float32 whatever the parameter is stored in: what the step reads and writes
+        state["exp_avg"] = torch.zeros(p.shape, device=self.device)
+        state["exp_avg_sq"] = torch.zeros(p.shape, device=self.device)
         state["adam_step"] = 0
 
     # pylo/optim/CELO2_cuda.py:241-251: the counter is per parameter and advances only on steps in

@@ -1,0 +1,40 @@
+"""The state of parameters that are stored in 16 or 64 bits: long enough that a buffer of the wrong type would be left."""
+
+import copy
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.bfloat16, torch.float16, torch.float64]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_celo2_moments_of_stored_vectors(dtype):
+    """Moments and updated parameters of AdamW tensors against a float32 run on the widened values: the arithmetic is the same,
+    so the moments agree bit for bit and the parameters up to the rounding into the storage type."""
+    from pylo_amd import CELO2_CUDA
+    from pylo_amd.models import CELO2MLP
+
+    gen = torch.Generator().manual_seed(5)
+    shapes = [(70001,), (4096,), (301, 64)]
+    init = [(0.05 * torch.randn(s, generator=gen)).to(dtype).cuda() for s in shapes]
+    torch.manual_seed(1)
+    net = CELO2MLP()
+    stored = [torch.nn.Parameter(v.clone()) for v in init]
+    wide = [torch.nn.Parameter(v.float()) for v in init]
+    a, b = ([{"params": ps[:2]}, {"params": ps[2:], "is_embedding": True}] for ps in (stored, wide))
+    oa, ob = CELO2_CUDA(a, lr=1e-3, network=net, hf_key=None), CELO2_CUDA(b, lr=1e-3, network=copy.deepcopy(net), hf_key=None)
+    for t in range(3):
+        for p, q, s in zip(stored, wide, shapes):
+            p.grad = (1e-2 * torch.randn(s, generator=gen)).to(dtype).cuda()
+            q.grad = p.grad.float()
+            q.data.copy_(p.data)
+        oa.step()
+        ob.step()
+        for p, q in zip(stored, wide):
+            for key in ("exp_avg", "exp_avg_sq"):
+                assert oa.state[p][key].dtype == torch.float32
+                assert torch.equal(oa.state[p][key], ob.state[q][key]), (t, key)
+            assert torch.equal(p.data, q.data.to(dtype)), t
