@@ -33,6 +33,25 @@ def store_flag(p: torch.Tensor, who: str) -> int:
         raise TypeError(f"{who}: parameters must be float32, float16, bfloat16 or float64, got {p.dtype}") from None
 
 
+def keep_float32_state(opt, state_dict) -> None:
+    """After ``Optimizer.load_state_dict``, which casts floating state to its parameter's type: the accumulators of parameters
+    that are not stored in float32 as they were saved, in float32, which is what the kernels read and write."""
+    saved_ids = [i for g in state_dict["param_groups"] for i in g["params"]]
+    params = [p for g in opt.param_groups for p in g["params"]]
+    for i, p in zip(saved_ids, params):
+        state = opt.state.get(p)
+        if not state or p.dtype == torch.float32:
+            continue
+        saved = state_dict["state"].get(i, {})
+        for key, t in state.items():
+            if key == "step" or not torch.is_tensor(t) or not t.is_floating_point() or t.dtype == torch.float32:
+                continue
+            was = saved.get(key)
+            if not torch.is_tensor(was) or was.shape != t.shape:
+                was = t
+            state[key] = was.to(device=t.device, dtype=torch.float32)
+
+
 class TensorShape(C.Structure):
     _fields_ = [("ndim", C.c_int32), ("flags", C.c_int32), ("shape", C.c_int64 * MAX_DIMS)]
 

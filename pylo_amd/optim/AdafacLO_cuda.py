@@ -181,6 +181,7 @@ class AdafacLO_CUDA(Optimizer):
 
     def load_state_dict(self, state_dict):
         out = super().load_state_dict(state_dict)
+        _lib.keep_float32_state(self, state_dict)
         if self.capturable and self._plan is not None:
             self._reset_device_steps([(g, p) for g in self.param_groups for p in g["params"]])
         return out

@@ -339,6 +339,7 @@ class ELO_CELO2_CUDA(Optimizer):
     def load_state_dict(self, state_dict):
         self._fast = None
         out = super().load_state_dict(state_dict)
+        _lib.keep_float32_state(self, state_dict)
         if self.capturable and self._plan is not None:
             self._reset_device_steps(self._tensors())
         return out

@@ -18,3 +18,29 @@ def test_celo2_state_is_float32(dtype, adam, shape):
     opt._init_state(state, torch.nn.Parameter(torch.zeros(shape, dtype=dtype)), adam)
     tensors = [t for t in state.values() if torch.is_tensor(t)]
     assert tensors and all(t.dtype == torch.float32 for t in tensors)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_loaded_state_is_float32_and_unrounded(dtype):
+    from pylo_amd import _lib
+
+    def make():
+        p = torch.nn.Parameter(torch.zeros(7, 5, dtype=dtype))
+        q = torch.nn.Parameter(torch.zeros(3, dtype=dtype))
+        return torch.optim.SGD([{"params": [p]}, {"params": [q]}], lr=0.1), p, q
+
+    a, p, q = make()
+    a.state[p].update(mom=torch.randn(3, 7, 5), rms=1e-9 * torch.rand(7, 5), step=torch.tensor(3.0, dtype=torch.float64), adam_step=2)
+    b, p2, q2 = make()
+    sd = a.state_dict()
+    b.load_state_dict(sd)
+    _lib.keep_float32_state(b, sd)
+    assert torch.equal(b.state[p2]["mom"], a.state[p]["mom"]) and b.state[p2]["mom"].dtype == torch.float32
+    assert torch.equal(b.state[p2]["rms"], a.state[p]["rms"]) and b.state[p2]["rms"].dtype == torch.float32
+    assert b.state[p2]["step"].dtype == torch.float64 and b.state[p2]["adam_step"] == 2
+    assert not b.state.get(q2)
+    # accumulators that were saved in the parameter's type are widened
+    sd["state"][0]["mom"] = sd["state"][0]["mom"].to(dtype)
+    b.load_state_dict(sd)
+    _lib.keep_float32_state(b, sd)
+    assert torch.equal(b.state[p2]["mom"], a.state[p]["mom"].to(dtype).float())
