@@ -343,7 +343,7 @@ __device__ __forceinline__ void adafac_apply_tile(const TDesc& d, const PyloTens
                                                   const EmaConsts& e, const float* __restrict__ fac_tab,
                                                   const float* __restrict__ term_tab, const float* wfold_t,
                                                   const float* net, float* xch /* LDS [16][kXPitch] of this wave */) {
-  const TileTask tk(d, task, d.atile_nct, 1);
+  const TileTask tk(d, task, d.atile_nct, 1, d.atile_rows);
   const int lane = threadIdx.x & 63, q = lane >> 4, el = lane & 15;
   // A operands: first layer [b][c'] (inputs 4c'+q), hidden layer [bo][b][r] (input 16b+4q+r)
   float a1[2][4], a2[2][2][4], wo[2][4][2];
@@ -493,8 +493,12 @@ __device__ __forceinline__ void adafac_apply_tile(const TDesc& d, const PyloTens
 // Three v_mfma_f32_32x32x16_f16 per fp32 product leave 18 matrix instructions per row of 64 elements where the
 // fp32 instructions need 96 and three bf16 planes needed 36; the split costs 3.25 vector instructions a value
 // (two conversions and a subtraction per value, a packing conversion per pair and plane) where three bf16
-// planes cost 5.5, in a kernel that is bound by exactly these instructions: splitting the 16 features and the
-// 2 x 16 hidden values a lane holds.
+// planes cost 5.5: splitting the 16 features and the 2 x 16 hidden values a lane holds.
+// What bounds it: power.  On Llama-1.1B the part runs it at 1.9 of 2.4 GHz, and at 1.8 with four waves a SIMD (the column terms
+// in LDS), which took fewer cycles and no less time; scalar instructions and matrix cycles taken out did not show, vector
+// instructions did.  Row terms reach the accumulators by one v_mfma_f32_32x32x2_f32 (terms x ones, exact) instead of 32
+// additions and four 16-byte loads a lane.  18.2 -> 16.3 ms a pass, whole step 23.6 -> 21.7 ms; ResNet-50 740 -> 687 us; every
+// result bit for bit the same.
 //
 // Layouts (lane = 32 half + e): units are the M dimension, elements the N dimension, inputs the K
 // dimension.  A operand: lane holds reduction slots 8 half .. 8 half + 7 of unit e.  B operand: lane holds
@@ -512,12 +516,17 @@ typedef _Float16 ah16x8 __attribute__((ext_vector_type(8)));
 typedef float av16f __attribute__((ext_vector_type(16)));
 typedef unsigned int au32x4 __attribute__((ext_vector_type(4)));
 
-// two values -> one dword of each plane (`a` in the lower halves), by rounding (v_cvt_pk_f16_f32)
+// two values -> one dword of each plane (`a` in the lower halves), by rounding (v_cvt_pk_f16_f32).  What is left is a
+// v_fma_mix_f32, exact like the subtraction it is, that takes the rounded value as the fp16 it is: the compiler makes one of a
+// multiply-add by -1 that it cannot see to be one.  Before, a conversion back and a subtraction: 48 instructions a row of 64
+// elements more (Llama-1.1B, whole step 22.4 / 21.8 ms, ResNet-50 689 / 665 us).
 typedef float af32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 ah16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void hf2_split2(float a, float b, unsigned& h, unsigned& l) {
   const ah16x2 hh = __builtin_convertvector(af32x2{a, b}, ah16x2);
-  const ah16x2 ll = __builtin_convertvector(af32x2{a - (float)hh[0], b - (float)hh[1]}, ah16x2);
+  float neg = -1.0f;
+  asm("" : "+s"(neg));
+  const ah16x2 ll = __builtin_convertvector(af32x2{fmaf((float)hh[0], neg, a), fmaf((float)hh[1], neg, b)}, ah16x2);
   h = __builtin_bit_cast(unsigned, hh);
   l = __builtin_bit_cast(unsigned, ll);
 }
@@ -550,36 +559,82 @@ __device__ __forceinline__ av16f hf2_mfma(const au32x4 (&w)[2], const au32x4 (&x
   return acc;
 }
 
-// Output layer of the two groups of 32 elements a wave holds, from the hidden layer's sums `g2` (D layout): the two outputs
-// of the lane's own element.
-__device__ __forceinline__ void adafac_output(const av16f (&g2)[2], const float (&wo)[16][2], float bo0, float bo1, float& o0,
-                                              float& o1) {
-  float part[2][2];
-#pragma unroll
-  for (int gq = 0; gq < 2; ++gq) {
-    float p0 = 0.0f, p1 = 0.0f;
-#pragma unroll
-    for (int r2 = 0; r2 < 16; ++r2) {
-      const float gv = relu(g2[gq][r2]);
-      p0 = fmaf(gv, wo[r2][0], p0);
-      p1 = fmaf(gv, wo[r2][1], p1);
-    }
-    part[gq][0] = p0;
-    part[gq][1] = p1;
+// acc += (the block's four weights) x v: rows = outputs, v = the lane's own value.  `b` (a constant after unrolling): the block
+// whose weights all eight blocks of a half take, 0 .. 7.
+__device__ __forceinline__ v4f mfma_half_w4(float w, float v, v4f acc, int b) {
+  switch (b & 7) {
+    case 0: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, v, acc, 3, 0, 0);
+    case 1: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, v, acc, 3, 1, 0);
+    case 2: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, v, acc, 3, 2, 0);
+    case 3: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, v, acc, 3, 3, 0);
+    case 4: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, v, acc, 3, 4, 0);
+    case 5: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, v, acc, 3, 5, 0);
+    case 6: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, v, acc, 3, 6, 0);
+    default: return __builtin_amdgcn_mfma_f32_4x4x1f32(w, v, acc, 3, 7, 0);
   }
-  // a lane's element belongs to group `half`; its other 16 units sit 32 lanes away
-  unsigned a0 = __float_as_uint(part[0][0]), b0 = __float_as_uint(part[1][0]);
-  unsigned a1 = __float_as_uint(part[0][1]), b1 = __float_as_uint(part[1][1]);
-  half_swap(a0, b0);
-  half_swap(a1, b1);
-  o0 = (__uint_as_float(a0) + __uint_as_float(b0)) + bo0;
-  o1 = (__uint_as_float(a1) + __uint_as_float(b1)) + bo1;
 }
+
+// Output layer of the two groups of 32 elements a wave holds, from the hidden layer's sums (D layout): the two outputs of
+// the lane's own element, sixteen units added in its own lane and sixteen in the one 32 lanes away.
+// MATRIX: by fp32 matrix instructions whose A operand is two registers of weights (block b of either half of the wave: the four
+// rows, two of them zeros, of the unit that the half's register 8 q + b belongs to), else by fused multiply-adds with 32 registers
+// of them.  The same sums in the same order, and as many cycles.  The walk over convolution kernels takes the first, which leaves
+// it 159 registers, three waves a SIMD, instead of 190, two (ResNet-50, whole step 655 / 669 us); the plain walk the second,
+// at two waves against three (Llama-1.1B 21.05 / 21.3 ms): more waves only lower its clock.
+template <bool MATRIX>
+struct AdafacOut {
+  float w[MATRIX ? 2 : 32], b0, b1;
+
+  __device__ __forceinline__ AdafacOut(const float* net, int lane) {
+    const cfloat* nw = launder(net);
+    b0 = nw[kABO + 0];
+    b1 = nw[kABO + 1];
+    const int half = lane >> 5;
+    if constexpr (MATRIX) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int r = 8 * q + ((lane >> 2) & 7), unit = 8 * (r >> 2) + 4 * half + (r & 3);
+        const float v = *(const gfloat*)(net + kAWO + unit * 2 + (lane & 1));
+        w[q] = (lane & 2) ? 0.0f : v;
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int unit = 8 * (r >> 2) + 4 * half + (r & 3);
+        w[2 * r] = *(const gfloat*)(net + kAWO + unit * 2 + 0);
+        w[2 * r + 1] = *(const gfloat*)(net + kAWO + unit * 2 + 1);
+      }
+    }
+  }
+
+  __device__ __forceinline__ void operator()(const av16f (&g2)[2], float& o0, float& o1) const {
+    v4f part[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int gq = 0; gq < 2; ++gq) {
+        const float gv = relu(g2[gq][r]);
+        if constexpr (MATRIX) {
+          part[gq] = mfma_half_w4(w[r >> 3], gv, part[gq], r);
+        } else {
+          part[gq][0] = fmaf(gv, w[2 * r], part[gq][0]);
+          part[gq][1] = fmaf(gv, w[2 * r + 1], part[gq][1]);
+        }
+      }
+    unsigned p0 = __float_as_uint(part[0][0]), q0 = __float_as_uint(part[1][0]);
+    unsigned p1 = __float_as_uint(part[0][1]), q1 = __float_as_uint(part[1][1]);
+    half_swap(p0, q0);
+    half_swap(p1, q1);
+    o0 = (__uint_as_float(p0) + __uint_as_float(q0)) + b0;
+    o1 = (__uint_as_float(p1) + __uint_as_float(q1)) + b1;
+  }
+};
 
 // Hidden and output layer of the two groups of 32 elements a wave holds, from the first layer's sums `h` (D layout):
 // the two outputs of the lane's own element.
-__device__ __forceinline__ void adafac_hidden_out(const av16f (&h)[2], const au32x4 (&w2)[2][2], const av16f& bh,
-                                                  const float (&wo)[16][2], float bo0, float bo1, float& o0, float& o1) {
+template <class Out>
+__device__ __forceinline__ void adafac_hidden_out(const av16f (&h)[2], const au32x4 (&w2)[2][2], const av16f& bh, const Out& out,
+                                                  float& o0, float& o1) {
   av16f g2[2];
 #pragma unroll
   for (int gq = 0; gq < 2; ++gq) {
@@ -602,7 +657,7 @@ __device__ __forceinline__ void adafac_hidden_out(const av16f (&h)[2], const au3
       g2[gq] = hf2_mfma(w2[s2], hb, g2[gq]);
     }
   }
-  adafac_output(g2, wo, bo0, bo1, o0, o1);
+  out(g2, o0, o1);
 }
 
 // PER: the tensor is an (O, I, k, ..) one walked as the matrix (O, I * P) (TDesc::aper): the vector that is not
@@ -614,7 +669,7 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
                                                      const EmaConsts& e, const float* __restrict__ fac_tab,
                                                      const float* __restrict__ term_tab, const float* wfold_t,
                                                      const float* net) {
-  const TileTask tk(d, task, d.atile_nct, 1);
+  const TileTask tk(d, task, d.atile_nct, 1, d.atile_rows);
   const int lane = threadIdx.x & 63, half = lane >> 5, el = lane & 31;
   // A operands: first layer (unit el, inputs 8 half ..), hidden layer per reduction step s (slot 8 half + 4 q + i:
   // hidden unit 8 (2 s + q) + 4 half + i)
@@ -641,16 +696,12 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
   }
   // what belongs to the units this lane holds in D: hidden bias, output weights
   av16f bh;
-  float wo[16][2];
+  const AdafacOut<PER> out(net, lane);
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int unit = 8 * (r >> 2) + 4 * half + (r & 3);
     bh[r] = *(const gfloat*)(net + kABH + unit);
-    wo[r][0] = *(const gfloat*)(net + kAWO + unit * 2 + 0);
-    wo[r][1] = *(const gfloat*)(net + kAWO + unit * 2 + 1);
   }
-  const cfloat* nw = launder(net);
-  const float bo0 = nw[kABO + 0], bo1 = nw[kABO + 1];
   const float exp_scale = a.exp_mult * 1.44269504088896341f;
   const int cv = PER ? d.aper_col : 1, pv = 1 - cv;   // the vector the column indexes, and the other one
   const int per = PER ? d.aper : 1;
@@ -660,14 +711,16 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
   // offset per lane, immediates per (g, j); row terms likewise from the row's table entry
   const float* tcol = term_tab + pick(d.term_off, cv);
   const unsigned tcol_off = ((tk.col - lane + el) * kAH + 4 * half) * 4u;
-  // row side: byte offsets of the lane's entries relative to the row's first (zero unless PER)
-  unsigned fa_off = 0, trow_off[2] = {4 * half * 4u, 4 * half * 4u};
-  if constexpr (PER) {
-    fa_off = (tk.col % (unsigned)per) * 16u;
+  av16f tb[2];
 #pragma unroll
-    for (int gq = 0; gq < 2; ++gq) trow_off[gq] += ((tk.col - lane + 32 * gq + el) % (unsigned)per) * (kAH * 4u);
-  }
-  const unsigned lo = lane * 4u;
+  for (int gq = 0; gq < 2; ++gq)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float t[4];
+      load_vec_o<4>(tcol + (32 * gq) * kAH + 8 * j, tcol_off, t);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) tb[gq][4 * j + i] = t[i];
+    }
   typedef typename StoredAs<ST>::E E;
   const E* g = reinterpret_cast<const E*>(a.grad) + tk.first;
   E* p = reinterpret_cast<E*>(a.param) + tk.first;
@@ -675,36 +728,54 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
         *m2 = a.mom + 2 * d.n + tk.first, *rms = a.rms + tk.first;
   const float* fr = fac_tab + pick(d.fac_off, pv) + (size_t)tk.r0 * 4 * per;
   const float* tr = term_tab + pick(d.term_off, pv) + (size_t)tk.r0 * kAH * per;
+  // The lane's offsets in the current row: element, and bytes into the row side's tables (PER: of its own column's entries;
+  // else the terms of unit el).  One addition each moves on to the next row; a pointer for each of the streams was advanced by
+  // two scalar instructions and widened by one on the vector pipe.  (A task's elements fit 32-bit byte offsets: atile_rows.)
+  unsigned off = lane, fa_off = 0, trow_off[2] = {el * 4u, 0u};
+  if constexpr (PER) {
+    fa_off = (tk.col % (unsigned)per) * 16u;
+#pragma unroll
+    for (int gq = 0; gq < 2; ++gq)
+      trow_off[gq] = 4 * half * 4u + ((tk.col - lane + 32 * gq + el) % (unsigned)per) * (kAH * 4u);
+  }
   // Everything a row reads from memory.  The loop keeps one row in flight: the loads of row r + 1 are issued
-  // before row r is worked on (a wave shares its SIMD with one other wave only, too few to cover a memory round
+  // before row r is worked on (a wave shares its SIMD with two other waves only, too few to cover a memory round
   // trip per row otherwise).
-  struct RowIn { E g, p; float m0[1], m1[1], m2[1], rms[1], fa[4], ta[PER ? 2 : 1][4][4]; };
-  auto fetch = [&](RowIn& x, long long eo, const float* fr_, const float* tr_) {
-    x.g = load_raw<ST>(g + eo, lane);
-    x.p = load_raw<ST>(p + eo, lane);
-    load_vec_nt<1>(m0 + eo, lo, x.m0);
-    load_vec_nt<1>(m1 + eo, lo, x.m1);
-    load_vec_nt<1>(m2 + eo, lo, x.m2);
-    load_vec_nt<1>(rms + eo, lo, x.rms);
-    if constexpr (PER) load_vec_o<4>(fr_, fa_off, x.fa);
-    else load_uniform<4>(fr_, x.fa);
+  struct RowIn { E g, p; float m0[1], m1[1], m2[1], rms[1], fa[4], ta[PER ? 2 : 1][PER ? 4 : 1][PER ? 4 : 1]; };
+  auto fetch = [&](RowIn& x, unsigned at, int r) {
+    x.g = load_raw<ST>(g, at);
+    x.p = load_raw<ST>(p, at);
+    load_vec_nt<1>(m0, at * 4u, x.m0);
+    load_vec_nt<1>(m1, at * 4u, x.m1);
+    load_vec_nt<1>(m2, at * 4u, x.m2);
+    load_vec_nt<1>(rms, at * 4u, x.rms);
+    if constexpr (PER) {
+      load_vec_o<4>(fr, fa_off, x.fa);
 #pragma unroll
-    for (int gq = 0; gq < (PER ? 2 : 1); ++gq)
+      for (int gq = 0; gq < 2; ++gq)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) load_vec_o<4>(tr_ + 8 * j, trow_off[gq], x.ta[gq][j]);
+        for (int j = 0; j < 4; ++j) load_vec_o<4>(tr + 8 * j, trow_off[gq], x.ta[gq][j]);
+    } else {
+      load_uniform<4>(fr + 4 * r, x.fa);
+      load_vec_o<1>(tr, trow_off[0], x.ta[0][0]);
+    }
   };
   RowIn cur;
-  fetch(cur, 0, fr, tr);
-  for (int r = tk.r0; r < tk.r1; ++r) {
+  fetch(cur, off, 0);
+  const int rows = tk.r1 - tk.r0;
+  for (int r = 0; r < rows; ++r) {
+    // past the last row: the same row again, discarded
+    const bool more = r + 1 < rows;
+    const unsigned step = more ? (unsigned)d.C0 : 0u, here = off, lo = off * 4u;
+    off += step;
+    fa_off += more ? 16u * per : 0u;
+#pragma unroll
+    for (int gq = 0; gq < (PER ? 2 : 1); ++gq) trow_off[gq] += more ? (unsigned)(kAH * 4 * per) : 0u;
     RowIn nxt;
-    {   // past the last row: the same row again, discarded
-      const bool more = r + 1 < tk.r1;
-      fetch(nxt, more ? d.C0 : 0, fr + (more ? 4 * per : 0), tr + (more ? kAH * per : 0));
-    }
+    fetch(nxt, off, more ? r + 1 : r);
     float xg[1] = {widen_raw<ST>(cur.g)}, xp[1] = {widen_raw<ST>(cur.p)}, x0[1] = {cur.m0[0]}, x1[1] = {cur.m1[0]}, x2[1] = {cur.m2[0]},
           xr_[1] = {cur.rms[0]};
     const float (&fa)[4] = cur.fa;
-    const float (&ta)[PER ? 2 : 1][4][4] = cur.ta;
     const float gg = cond_grad(xg[0], d.gscale, a.clip_val, d.nan0);
     float m[3] = {x0[0], x1[0], x2[0]};
     ema_update(e, gg, m, xr_[0]);
@@ -741,22 +812,20 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
     av16f h[2];
 #pragma unroll
     for (int gq = 0; gq < 2; ++gq) {
+      if constexpr (PER) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float tb[4];
-        load_vec_o<4>(tcol + (32 * gq) * kAH + 8 * j, tcol_off, tb);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) h[gq][4 * j + i] = ta[PER ? gq : 0][j][i] + tb[i];
+        for (int i = 0; i < 16; ++i) h[gq][i] = cur.ta[gq][i >> 2][i & 3] + tb[gq][i];
+      } else {
+        // the row's terms, the same for every element: one rank-1 update of the column's (slot 0: terms times one)
+        h[gq] = __builtin_amdgcn_mfma_f32_32x32x2f32(half ? 0.0f : cur.ta[0][0][0], 1.0f, tb[gq], 0, 0, 0);
       }
       h[gq] = hf2_mfma(w1, xb[gq], h[gq]);
     }
     float o0, o1;
-    adafac_hidden_out(h, w2, bh, wo, bo0, bo1, o0, o1);
+    adafac_hidden_out(h, w2, bh, out, o0, o1);
     float pn[1];
     pn[0] = adafac_update(d, a, o0 * __builtin_amdgcn_exp2f(o1 * exp_scale), xp[0]);
-    store_row<1, ST>(p, lane, pn);
-    g += d.C0; p += d.C0; m0 += d.C0; m1 += d.C0; m2 += d.C0; rms += d.C0;
-    fr += 4 * per; tr += kAH * per;
+    store_row<1, ST>(p, here, pn);
     cur = nxt;
   }
 }
@@ -837,17 +906,13 @@ __device__ __forceinline__ void adafac_apply_lin(const TDesc& d, const PyloTenso
     }
   }
   av16f bh, b1;
-  float wo[16][2];
+  const AdafacOut<false> out(net, lane);
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int unit = 8 * (r >> 2) + 4 * half + (r & 3);
     bh[r] = *(const gfloat*)(net + kABH + unit);
-    wo[r][0] = *(const gfloat*)(net + kAWO + unit * 2 + 0);
-    wo[r][1] = *(const gfloat*)(net + kAWO + unit * 2 + 1);
     if constexpr (VEC) b1[r] = *(const gfloat*)(bias_eff + unit);
   }
-  const cfloat* nw = launder(net);
-  const float bo0 = nw[kABO + 0], bo1 = nw[kABO + 1];
   const long long n = d.n;
   const unsigned last = (unsigned)(n - 1);     // n < 2^31
   const unsigned wave0 = (unsigned)base + (threadIdx.x & ~63u);
@@ -967,7 +1032,7 @@ __device__ __forceinline__ void adafac_apply_lin(const TDesc& d, const PyloTenso
         g2[gq] = bf3_mfma(w2[s], xb, g2[gq]);
       }
     float o0, o1;
-    adafac_output(g2, wo, bo0, bo1, o0, o1);
+    out(g2, o0, o1);
     if (w0 + lane <= last)
       *(gfloat*)(a.param + w0 + lane) = adafac_update(d, a, o0 * expf(o1 * a.exp_mult), p);
     cur = nxt;

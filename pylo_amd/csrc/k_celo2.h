@@ -268,14 +268,14 @@ struct TileTask {
   int r0, r1;          // rows
   unsigned col;        // the lane's first column
   long long first;     // element index of (r0, first column of the wave)
-  __device__ __forceinline__ TileTask(const TDesc& d, int task, int nct, int V) {
+  __device__ __forceinline__ TileTask(const TDesc& d, int task, int nct, int V, int rows) {
     const int ct = task % nct, rr = task / nct;
-    r0 = rr * d.tile_rows;
-    r1 = r0 + d.tile_rows < d.R0 ? r0 + d.tile_rows : d.R0;
+    r0 = rr * rows;
+    r1 = r0 + rows < d.R0 ? r0 + rows : d.R0;
     col = (unsigned)ct * (64 * V) + (threadIdx.x & 63) * V;
     first = (long long)r0 * d.C0 + (long long)ct * (64 * V);
   }
-  __device__ __forceinline__ TileTask(const TDesc& d, int task) : TileTask(d, task, d.tile_nct, kTileV) {}
+  __device__ __forceinline__ TileTask(const TDesc& d, int task) : TileTask(d, task, d.tile_nct, kTileV, d.tile_rows) {}
 };
 
 // Statistics of one wave task: the column factors stay in registers, the row factors arrive through

@@ -18,6 +18,7 @@ constexpr int kElemIters = 8;   // an element chunk is kThreads * vec * TDesc::i
 constexpr int kTileV = 2;       // column-resident walk: a wave owns 64 * kTileV columns ...
 constexpr int kTileCols = 64 * kTileV;
 constexpr int kTileRows = 16;   // ... and walks TDesc::tile_rows of them, at most this many
+constexpr int kApplyRowsMax = 64;   // the same of AdafacLO's apply pass, TDesc::atile_rows
 constexpr int kNStat = 18;      // feature channels that vary per element (the other 12 are
                                 // functions of the row or of the column only)
 constexpr int kV0aEnt = 64;     // vector entries per k_v0a block
@@ -99,8 +100,8 @@ struct TDesc {
   // element block a holds tasks 4a .. 4a+3.  tile_nct == 0: linear chunks instead.
   int tile_nct, tile_ntask, tile_rows;
   // AdafacLO's apply pass walks one column per lane (its 32-wide MLP leaves no registers for two):
-  // same scheme with 64 columns per wave task; apply block a holds tasks 4a .. 4a+3.
-  int atile_nct, atile_ntask;
+  // same scheme with 64 columns and atile_rows rows per wave task; apply block a holds tasks 4a .. 4a+3.
+  int atile_nct, atile_ntask, atile_rows;
   // ... and an (O, I, k, ..) tensor whose factored dims are the two leading ones is walked the same way as the
   // matrix (O, I * P), P = product of the trailing dims: one vector is indexed by the matrix column, the other by
   // (row, column mod P).  aper = P (0: not walked so), aper_col = which vector the column indexes; R0 / C0 hold

@@ -1031,6 +1031,12 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
   }
   const int split = split_for(total_elems);
   L.split = split > 1;
+  // Rows of a wave task of AdafacLO's walks: a wave's set-up (weights split into planes, column terms, three dependent loads
+  // before the first row) costs about as much as a row, so rows are doubled up to 64 while 16384 tasks, five rounds of what
+  // runs at once, are left.  Whole steps, 16 / 32 / 64 rows: 22 M elements 505 / 505 / 520 us, 86 M 1769 / 1741 / 1733, 124 M
+  // 2476 / 2418 / 2404, 355 M 6872 / 6700 / 6611.
+  int apply_rows = tile_rows_for(kind, split);
+  while (apply_rows >= kTileRows && apply_rows < kApplyRowsMax && total_elems >= 16384ll * 64 * 2 * apply_rows) apply_rows *= 2;
   L.tensor_norm = (shapes[0].flags & PYLO_F_TENSOR_NORM) != 0;
   L.global_norm = (shapes[0].flags & PYLO_F_GLOBAL_NORM) != 0 || L.tensor_norm;
   // Short slices (k_celo2_slices_wave): trips a wave, as many as leave sixteen waves a CU and no more than eight
@@ -1227,8 +1233,9 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       }
       if ((wide && d.C0 % 64 == 0) || periodic) {
         d.atile_nct = d.C0 / 64;
-        if (d.tile_rows == 0) d.tile_rows = tile_rows_for(kind, split);
-        d.atile_ntask = d.atile_nct * ((d.R0 + d.tile_rows - 1) / d.tile_rows);
+        // (the walk's offsets inside a task are 32-bit byte offsets)
+        d.atile_rows = (int)std::max<long long>(1, std::min<long long>(apply_rows, (1ll << 30) / d.C0));
+        d.atile_ntask = d.atile_nct * ((d.R0 + d.atile_rows - 1) / d.atile_rows);
         for (int b = 0; b * 4 < d.atile_ntask; ++b) (periodic ? L.pp_items : L.ap_items).push_back(Item{t, b, 0, 0});
       } else {
         lin_tensors.push_back(t);
