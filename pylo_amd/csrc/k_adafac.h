@@ -730,7 +730,8 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
   const float* tr = term_tab + pick(d.term_off, pv) + (size_t)tk.r0 * kAH * per;
   // The lane's offsets in the current row: element, and bytes into the row side's tables (PER: of its own column's entries;
   // else the terms of unit el).  One addition each moves on to the next row; a pointer for each of the streams was advanced by
-  // two scalar instructions and widened by one on the vector pipe.  (A task's elements fit 32-bit byte offsets: atile_rows.)
+  // two scalar instructions and widened by one on the vector pipe.  (atile_rows keeps a task's elements and, PER, its rows' terms
+  // within 32 bits.)
   unsigned off = lane, fa_off = 0, trow_off[2] = {el * 4u, 0u};
   if constexpr (PER) {
     fa_off = (tk.col % (unsigned)per) * 16u;

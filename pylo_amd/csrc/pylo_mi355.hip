@@ -1233,8 +1233,12 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       }
       if ((wide && d.C0 % 64 == 0) || periodic) {
         d.atile_nct = d.C0 / 64;
-        // (the walk's offsets inside a task are 32-bit byte offsets)
-        d.atile_rows = (int)std::max<long long>(1, std::min<long long>(apply_rows, (1ll << 30) / d.C0));
+        // The walk's offsets inside a task are 32-bit byte offsets: 4 C0 a row into the tensor, and, where the row side has an
+        // entry per column mod P, 128 P a row into its first-layer terms, the larger ones for I < 32.  (P, the product of up to
+        // six dims none of which exceeds the two leading ones, stays below 2^24 in a tensor of 2^31 elements: one row always fits.)
+        long long rows_max = (1ll << 30) / d.C0;
+        if (periodic) rows_max = std::min<long long>(rows_max, (1ll << 31) / ((long long)sizeof(float) * kAH * d.aper));
+        d.atile_rows = (int)std::max<long long>(1, std::min<long long>(apply_rows, rows_max));
         d.atile_ntask = d.atile_nct * ((d.R0 + d.atile_rows - 1) / d.atile_rows);
         for (int b = 0; b * 4 < d.atile_ntask; ++b) (periodic ? L.pp_items : L.ap_items).push_back(Item{t, b, 0, 0});
       } else {
