@@ -74,7 +74,7 @@ __device__ __forceinline__ void adafac_stats_tile(const TDesc& d, const PyloTens
   const float* f1 = fac_tab + d.fac_off[1];
   float fb[V][4];
 #pragma unroll
-  for (int v = 0; v < V; ++v) load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
+  for (int v = 0; v < V; ++v) load_vec_o<4>(f1 + (size_t)tk.wcol * 4 + v * 4, (threadIdx.x & 63) * (V * 16u), fb[v]);
   const unsigned le = (threadIdx.x & 63) * V, lo = le * 4u;
   typedef typename StoredAs<ST>::E E;
   const E *g = reinterpret_cast<const E*>(a.grad) + tk.first, *p = reinterpret_cast<const E*>(a.param) + tk.first;
@@ -369,10 +369,10 @@ __device__ __forceinline__ void adafac_apply_tile(const TDesc& d, const PyloTens
   const float bo0 = nw[kABO + 0], bo1 = nw[kABO + 1];
   const float exp_scale = a.exp_mult * 1.44269504088896341f;
   float fb[4];
-  load_vec_o<4>(fac_tab + d.fac_off[1], tk.col * 16u, fb);
+  load_vec_o<4>(fac_tab + d.fac_off[1] + (size_t)tk.wcol * 4, lane * 16u, fb);
   // column terms of element (16 g + el), units 16 b + 4 q ..: one voffset, immediates per (g, b)
-  const float* tcol = term_tab + d.term_off[1];
-  const unsigned tcol_off = ((tk.col - lane + el) * kAH + 4 * q) * 4u;
+  const float* tcol = term_tab + d.term_off[1] + (size_t)tk.wcol * kAH;
+  const unsigned tcol_off = (el * kAH + 4 * q) * 4u;
   const unsigned trow_off = 4 * q * 4u;
   const unsigned lo = lane * 4u;
   float* xw = xch + lane;                 // feature c of this lane's element goes to xch[c][lane]
@@ -706,11 +706,11 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
   const int cv = PER ? d.aper_col : 1, pv = 1 - cv;   // the vector the column indexes, and the other one
   const int per = PER ? d.aper : 1;
   float fb[4];
-  load_vec_o<4>(fac_tab + pick(d.fac_off, cv), tk.col * 16u, fb);
+  load_vec_o<4>(fac_tab + pick(d.fac_off, cv) + (size_t)tk.wcol * 4, lane * 16u, fb);
   // column terms of element e of group g (column: the wave's first + 32 g + e), units 8 j + 4 half ..: one
   // offset per lane, immediates per (g, j); row terms likewise from the row's table entry
-  const float* tcol = term_tab + pick(d.term_off, cv);
-  const unsigned tcol_off = ((tk.col - lane + el) * kAH + 4 * half) * 4u;
+  const float* tcol = term_tab + pick(d.term_off, cv) + (size_t)tk.wcol * kAH;
+  const unsigned tcol_off = (el * kAH + 4 * half) * 4u;
   av16f tb[2];
 #pragma unroll
   for (int gq = 0; gq < 2; ++gq)
@@ -737,7 +737,7 @@ __device__ __forceinline__ void adafac_apply_tile_hf(const TDesc& d, const PyloT
     fa_off = (tk.col % (unsigned)per) * 16u;
 #pragma unroll
     for (int gq = 0; gq < 2; ++gq)
-      trow_off[gq] = 4 * half * 4u + ((tk.col - lane + 32 * gq + el) % (unsigned)per) * (kAH * 4u);
+      trow_off[gq] = 4 * half * 4u + ((tk.wcol + 32 * gq + el) % (unsigned)per) * (kAH * 4u);
   }
   // Everything a row reads from memory.  The loop keeps one row in flight: the loads of row r + 1 are issued
   // before row r is worked on (a wave shares its SIMD with two other waves only, too few to cover a memory round
@@ -970,8 +970,8 @@ __device__ __forceinline__ void adafac_apply_lin(const TDesc& d, const PyloTenso
 #pragma unroll
       for (int gq = 0; gq < 2; ++gq) entries(min(w0 + 32 * gq + el, last), i0[gq], i1[gq]);
       float fa[4], fb[4];
-      load_vec_o<4>(fac_tab + d.fac_off[0], (half ? i0[1] : i0[0]) * 16u, fa);
-      load_vec_o<4>(fac_tab + d.fac_off[1], (half ? i1[1] : i1[0]) * 16u, fb);
+      load_vec<4>(fac_tab + d.fac_off[0] + (size_t)(half ? i0[1] : i0[0]) * 4, fa);
+      load_vec<4>(fac_tab + d.fac_off[1] + (size_t)(half ? i1[1] : i1[0]) * 4, fb);
 #pragma unroll
       for (int gq = 0; gq < 2; ++gq) {
         const float* t0 = term_tab + d.term_off[0] + (size_t)i0[gq] * kAH + 4 * half;

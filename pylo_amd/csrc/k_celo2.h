@@ -202,11 +202,12 @@ struct ChunkPtrs {
   }
 };
 
-// eight consecutive floats of row i of a table with eight floats per row
+// eight consecutive floats of row i of a table with eight floats per row (64-bit addresses: from 2^27 rows on the table is longer
+// than 4 GB)
 __device__ __forceinline__ void load_row8(const float* tab, unsigned i, float (&t)[8]) {
   float lo[4], hi[4];
-  load_vec_o<4>(tab, i * 32u, lo);
-  load_vec_o<4>(tab + 4, i * 32u, hi);
+  load_vec<4>(tab + (size_t)i * 8, lo);
+  load_vec<4>(tab + (size_t)i * 8 + 4, hi);
 #pragma unroll
   for (int j = 0; j < 4; ++j) { t[j] = lo[j]; t[4 + j] = hi[j]; }
 }
@@ -227,11 +228,11 @@ __device__ __forceinline__ void load_elems_at(const TDesc& d, const PyloTensorAr
   x.i0 = (int)i0;
   x.i1 = (int)i1;
   float fa[4];
-  load_vec_o<4>(f0, i0 * 16u, fa);
+  load_vec<4>(f0 + (size_t)i0 * 4, fa);
 #pragma unroll
   for (int v = 0; v < V; ++v) {
     float fb[4];
-    load_vec_o<4>(f1 + v * 4, i1 * 16u, fb);
+    load_vec<4>(f1 + (size_t)i1 * 4 + v * 4, fb);
     x.g[v] = clampf(x.g[v] * scale, a.clip_val);
     x.m[v][0] = m0[v]; x.m[v][1] = m1[v]; x.m[v][2] = m2[v];
     x.rfcf[v][0] = fa[0] * fb[0];
@@ -263,16 +264,18 @@ __device__ __forceinline__ void celo2_stats_chunk(const TDesc& d, const PyloTens
   }
 }
 
-// Geometry of one wave task of the column-resident walk: V columns per lane, nct column tiles.
+// Geometry of one wave task of the column-resident walk: V columns per lane, nct column tiles.  Tables with an entry a column are
+// addressed from the entry of the first column on: a byte offset to a column itself passes 32 bits from 2^25 columns (AdafacLO) on.
 struct TileTask {
   int r0, r1;          // rows
-  unsigned col;        // the lane's first column
+  unsigned wcol, col;  // the wave's and the lane's first column
   long long first;     // element index of (r0, first column of the wave)
   __device__ __forceinline__ TileTask(const TDesc& d, int task, int nct, int V, int rows) {
     const int ct = task % nct, rr = task / nct;
     r0 = rr * rows;
     r1 = r0 + rows < d.R0 ? r0 + rows : d.R0;
-    col = (unsigned)ct * (64 * V) + (threadIdx.x & 63) * V;
+    wcol = (unsigned)ct * (64 * V);
+    col = wcol + (threadIdx.x & 63) * V;
     first = (long long)r0 * d.C0 + (long long)ct * (64 * V);
   }
   __device__ __forceinline__ TileTask(const TDesc& d, int task) : TileTask(d, task, d.tile_nct, kTileV, d.tile_rows) {}
@@ -291,7 +294,7 @@ __device__ __forceinline__ void celo2_stats_tile(const TDesc& d, const PyloTenso
   const TileTask tk(d, task);
   float fb[V][4];
 #pragma unroll
-  for (int v = 0; v < V; ++v) load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
+  for (int v = 0; v < V; ++v) load_vec_o<4>(f1 + (size_t)tk.wcol * 4 + v * 4, (threadIdx.x & 63) * (V * 16u), fb[v]);
   const unsigned le = (threadIdx.x & 63) * V, lo = le * 4u;
   typedef typename StoredAs<ST>::E E;
   const E *g = reinterpret_cast<const E*>(a.grad) + tk.first, *p = reinterpret_cast<const E*>(a.param) + tk.first;
@@ -687,8 +690,8 @@ __device__ __forceinline__ void celo2_apply_tile(const TDesc& d, const PyloTenso
   float fb[V][4], tb[V][8];
 #pragma unroll
   for (int v = 0; v < V; ++v) {
-    load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
-    load_row8(t1 + v * 8, tk.col, tb[v]);
+    load_vec_o<4>(f1 + (size_t)tk.wcol * 4 + v * 4, lane * (V * 16u), fb[v]);
+    load_row8(t1 + (size_t)tk.wcol * 8 + v * 8, lane * V, tb[v]);
   }
   const unsigned le = lane * V, lo = le * 4u;
   typedef typename StoredAs<ST>::E E;

@@ -211,7 +211,7 @@ __device__ __forceinline__ void velo_stats_tile(const TDesc& d, const PyloTensor
   const float* f1 = fac_tab + d.fac_off[1];
   float fb[V][4];
 #pragma unroll
-  for (int v = 0; v < V; ++v) load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
+  for (int v = 0; v < V; ++v) load_vec_o<4>(f1 + (size_t)tk.wcol * 4 + v * 4, (threadIdx.x & 63) * (V * 16u), fb[v]);
   const unsigned le = (threadIdx.x & 63) * V, lo = le * 4u;
   typedef typename StoredAs<ST>::E E;
   const E *g = reinterpret_cast<const E*>(a.grad) + tk.first, *p = reinterpret_cast<const E*>(a.param) + tk.first;
@@ -1050,8 +1050,8 @@ __device__ __forceinline__ void velo_apply_tile(const TDesc& d, const PyloTensor
   float fb[V][4], tb[V][4];
 #pragma unroll
   for (int v = 0; v < V; ++v) {
-    load_vec_o<4>(f1 + v * 4, tk.col * 16u, fb[v]);
-    load_vec_o<4>(t1 + v * 4, tk.col * 16u, tb[v]);
+    load_vec_o<4>(f1 + (size_t)tk.wcol * 4 + v * 4, lane * (V * 16u), fb[v]);
+    load_vec_o<4>(t1 + (size_t)tk.wcol * 4 + v * 4, lane * (V * 16u), tb[v]);
   }
   const unsigned le = lane * V, lo = le * 4u;
   typedef typename StoredAs<ST>::E E;
