@@ -35,7 +35,8 @@ def store_flag(p: torch.Tensor, who: str) -> int:
 
 def keep_float32_state(opt, state_dict) -> None:
     """After ``Optimizer.load_state_dict``, which casts floating state to its parameter's type: the accumulators of parameters
-    that are not stored in float32 as they were saved, in float32, which is what the kernels read and write."""
+    that are not stored in float32 as they were saved, in float32, which is what the kernels read and write.  Copies: steps write
+    them in place, and the dict and the optimizer it came from keep theirs."""
     saved_ids = [i for g in state_dict["param_groups"] for i in g["params"]]
     params = [p for g in opt.param_groups for p in g["params"]]
     for i, p in zip(saved_ids, params):
@@ -49,7 +50,7 @@ def keep_float32_state(opt, state_dict) -> None:
             was = saved.get(key)
             if not torch.is_tensor(was) or was.shape != t.shape:
                 was = t
-            state[key] = was.to(device=t.device, dtype=torch.float32)
+            state[key] = was.detach().to(device=t.device, dtype=torch.float32, copy=True)
 
 
 class TensorShape(C.Structure):

@@ -44,3 +44,27 @@ def test_loaded_state_is_float32_and_unrounded(dtype):
     b.load_state_dict(sd)
     _lib.keep_float32_state(b, sd)
     assert torch.equal(b.state[p2]["mom"], a.state[p]["mom"].to(dtype).float())
+
+
+@pytest.mark.parametrize("dtype", [t for t in DTYPES if t != torch.float32])
+def test_loaded_state_is_a_copy(dtype):
+    """Steps write accumulators in place: neither the dict nor the optimizer that it came from may see it, and a second load
+    from the same dict starts where the first did."""
+    from pylo_amd import _lib
+
+    def make():
+        p = torch.nn.Parameter(torch.zeros(7, 5, dtype=dtype))
+        return torch.optim.SGD([p], lr=0.1), p
+
+    a, p = make()
+    a.state[p].update(mom=torch.randn(3, 7, 5), rms=torch.rand(7, 5), step=3)
+    kept = {k: v.clone() for k, v in a.state[p].items() if torch.is_tensor(v)}
+    sd = a.state_dict()
+    for _ in range(2):
+        b, q = make()
+        b.load_state_dict(sd)
+        _lib.keep_float32_state(b, sd)
+        for k, v in kept.items():
+            assert torch.equal(b.state[q][k], v)
+            b.state[q][k].add_(1.0)
+            assert torch.equal(a.state[p][k], v) and torch.equal(sd["state"][0][k], v)
