@@ -53,6 +53,19 @@ def keep_float32_state(opt, state_dict) -> None:
             state[key] = was.detach().to(device=t.device, dtype=torch.float32, copy=True)
 
 
+def load_float32_state(opt, load, state_dict):
+    """``load(state_dict)`` (``Optimizer.load_state_dict``) with ``keep_float32_state`` between its hooks: on the dict that the
+    hooks before it leave, and before those after it see the state."""
+    read = []
+    before = opt.register_load_state_dict_pre_hook(lambda _, sd: read.append(sd))
+    after = opt.register_load_state_dict_post_hook(lambda o: keep_float32_state(o, read[0]), prepend=True)
+    try:
+        return load(state_dict)
+    finally:
+        before.remove()
+        after.remove()
+
+
 class TensorShape(C.Structure):
     _fields_ = [("ndim", C.c_int32), ("flags", C.c_int32), ("shape", C.c_int64 * MAX_DIMS)]
 

@@ -180,8 +180,7 @@ class AdafacLO_CUDA(Optimizer):
         return super().state_dict()
 
     def load_state_dict(self, state_dict):
-        out = super().load_state_dict(state_dict)
-        _lib.keep_float32_state(self, state_dict)
+        out = _lib.load_float32_state(self, super().load_state_dict, state_dict)
         if self.capturable and self._plan is not None:
             self._reset_device_steps([(g, p) for g in self.param_groups for p in g["params"]])
         return out

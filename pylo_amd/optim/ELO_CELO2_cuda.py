@@ -338,8 +338,7 @@ class ELO_CELO2_CUDA(Optimizer):
     # the per-group scalars are refreshed, which keeps the host ahead of a ~1.7 ms GPU step.
     def load_state_dict(self, state_dict):
         self._fast = None
-        out = super().load_state_dict(state_dict)
-        _lib.keep_float32_state(self, state_dict)
+        out = _lib.load_float32_state(self, super().load_state_dict, state_dict)
         if self.capturable and self._plan is not None:
             self._reset_device_steps(self._tensors())
         return out

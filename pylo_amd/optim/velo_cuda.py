@@ -224,8 +224,7 @@ class VeLO_CUDA(Optimizer):
         loss_buffer = state_dict.pop("loss_buffer")
         lstm_hidden_state = state_dict.pop("lstm_hidden_state")
         num_steps = state_dict.pop("num_steps")
-        super().load_state_dict(state_dict)
-        _lib.keep_float32_state(self, state_dict)
+        _lib.load_float32_state(self, super().load_state_dict, state_dict)
         self.loss_buffer = {k: (v.to(self.device) if torch.is_tensor(v) else v) for k, v in loss_buffer.items()}
         self.lstm_hidden_state = tuple(t.to(self.device).contiguous() for t in lstm_hidden_state)
         self.num_steps = num_steps

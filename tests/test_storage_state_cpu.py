@@ -68,3 +68,34 @@ def test_loaded_state_is_a_copy(dtype):
             assert torch.equal(b.state[q][k], v)
             b.state[q][k].add_(1.0)
             assert torch.equal(a.state[p][k], v) and torch.equal(sd["state"][0][k], v)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_hooks_of_loading_are_heard(dtype):
+    """What a hook before the load puts into the dict, or returns in its place, is what is loaded; what one after it does to the
+    state stays."""
+    from pylo_amd import AdafacLO_CUDA
+
+    def make():
+        opt = object.__new__(AdafacLO_CUDA)
+        p = torch.nn.Parameter(torch.zeros(7, 5, dtype=dtype))
+        torch.optim.Optimizer.__init__(opt, [p], {"lr": 0.1})
+        opt.capturable = False
+        opt.sync_step_counters = lambda: None
+        return opt, p
+
+    a, p = make()
+    a.state[p].update(mom=torch.randn(3, 7, 5), rms=torch.rand(7, 5), step=3)
+    b, q = make()
+
+    def doubled(_, sd):
+        return {**sd, "state": {0: {**sd["state"][0], "mom": 2.0 * sd["state"][0]["mom"]}}}
+
+    def cleared(opt):
+        opt.state[q]["rms"].zero_()
+
+    b.register_load_state_dict_pre_hook(doubled)
+    b.register_load_state_dict_post_hook(cleared)
+    b.load_state_dict(a.state_dict())
+    assert torch.equal(b.state[q]["mom"], 2.0 * a.state[p]["mom"])
+    assert b.state[q]["rms"].dtype == torch.float32 and not b.state[q]["rms"].any()
