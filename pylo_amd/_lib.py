@@ -36,21 +36,23 @@ def store_flag(p: torch.Tensor, who: str) -> int:
 def keep_float32_state(opt, state_dict) -> None:
     """After ``Optimizer.load_state_dict``, which casts floating state to its parameter's type: the accumulators of parameters
     that are not stored in float32 as they were saved, in float32, which is what the kernels read and write.  Copies: steps write
-    them in place, and the dict and the optimizer it came from keep theirs."""
+    them in place, and the dict and the optimizer it came from keep theirs.  One copy of a tensor that the state names twice."""
     saved_ids = [i for g in state_dict["param_groups"] for i in g["params"]]
     params = [p for g in opt.param_groups for p in g["params"]]
     for i, p in zip(saved_ids, params):
         state = opt.state.get(p)
         if not state or p.dtype == torch.float32:
             continue
-        saved = state_dict["state"].get(i, {})
+        saved, copies = state_dict["state"].get(i, {}), {}
         for key, t in state.items():
             if key == "step" or not torch.is_tensor(t) or not t.is_floating_point() or t.dtype == torch.float32:
                 continue
             was = saved.get(key)
             if not torch.is_tensor(was) or was.shape != t.shape:
                 was = t
-            state[key] = was.detach().to(device=t.device, dtype=torch.float32, copy=True)
+            if id(was) not in copies:
+                copies[id(was)] = was.detach().to(device=t.device, dtype=torch.float32, copy=True)
+            state[key] = copies[id(was)]
 
 
 def load_float32_state(opt, load, state_dict):

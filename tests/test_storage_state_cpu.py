@@ -71,6 +71,21 @@ def test_loaded_state_is_a_copy(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_tensors_of_two_names_stay_one(dtype):
+    """AdafacLO keeps the second moments of a vector under two names."""
+    from pylo_amd import _lib
+
+    p, q = (torch.nn.Parameter(torch.zeros(7, 5, dtype=dtype)) for _ in range(2))
+    a, b = torch.optim.SGD([p], lr=0.1), torch.optim.SGD([q], lr=0.1)
+    a.state[p].update(mom=torch.randn(3, 7, 5), rms=torch.rand(7, 5))
+    a.state[p]["exp_avg"] = a.state[p]["mom"]
+    sd = a.state_dict()
+    b.load_state_dict(sd)
+    _lib.keep_float32_state(b, sd)
+    assert b.state[q]["exp_avg"] is b.state[q]["mom"] and b.state[q]["rms"] is not b.state[q]["mom"]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_hooks_of_loading_are_heard(dtype):
     """What a hook before the load puts into the dict, or returns in its place, is what is loaded; what one after it does to the
     state stays."""
