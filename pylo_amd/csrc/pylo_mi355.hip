@@ -458,12 +458,13 @@ double ns_tiled_work(int m, int n) {
 
 // Into how many groups (streams) the matrices of a plan are dealt: as many as have eight of its matrices each, those that
 // go aside to k_ns_small counted (which launch takes them says nothing about the others), and 55 G of work each.  Below that a
-// group's launches are bound by their number, and more streams only add to it.  Whole steps, 1 / 2 / 3 groups (one
-// decoder layer of width 256, 384, 512, 1024: 1.3, 4.3, 10, 82 G; two embeddings of 4000 rows: 2.6, 6, 11, 50 G):
-//   width 256, 12 layers (18 G) 856 / 903 / 957 us      384, 8 layers (43 G) 1294 / 1293 / 1331, 12 (60 G) 1667 / 1593 / 1648
-//   512, 4 layers (52 G) 1244 / 1291 / 1331, 6 (72 G) 1691 / 1621 / 1633, 8 (93 G) 2057 / 1896 / 1945, 12 (133 G) 2551 / 2446 / 2405
-//   1024, 2 layers (210 G) 2799 / 2547 / 2542, 3 layers 3367 / 3103 / 3091 us
-//   64 of 256 x 256 (11 G) 533 / 588 us, four streams 664; 500 of 200 x 200 (88 G) 1817 / 1643 / four 1676
+// group's launches are bound by their number, and more streams only add to it.  Whole steps, 1 / 2 / 3 groups (with two
+// embeddings of 4000 rows):
+//   width 256, 4, 12 layers (9, 21 G) 408 / 480 / 492 us, 668 / 691 / 718      384, 8 (47 G) 1101 / 1108 / 1151, 12 (68 G)
+//   1404 / 1391 / 1456      512, 4 (60 G) 1086 / 1136 / 1229, 6 (84 G) 1435 / 1425 / 1439, 8 (109 G) 1774 / 1721 / 1778, 12 (157 G)
+//   2514 / 2438 / 2403      768, 2 (110 G) 1586 / 1583 / 1669, 4 (192 G) 2481 / 2341 / 2307      1024, 2 (247 G, fourteen matrices)
+//   2648 / 2471 / 2489, 3 (344 G) 3397 / 3325 / 3336, 8 (830 G) 7773 / 7436 / 7425
+//   64 of 256 x 256 (11 G) 383 / 385 / 459, 40 of 512 x 512 (56 G) 883 / 918 / 951, 500 of 200 x 200 (88 G) 1664 / 1541 / 1544
 int ns_group_count(int mats, double work) {
   return (int)std::min<double>(std::min(env_ns_groups(), std::max(mats / 8, 1)), 1.0 + std::floor(work / 55e9));
 }
@@ -477,15 +478,35 @@ int ns_small_edge(int cls) { return cls == 0 ? SmSmall::MP : cls == 1 ? SmMid::M
 
 // Which matrices the one-launch kernel takes: a smaller dim of at most 128 (its m x m matrices fit a CU's LDS) and a
 // longer one up to where its few blocks, each walking chunks of the long dim one after another, fall behind tiles of 64 x 64
-// on all CUs.  Finishing calls on one matrix, small kernel / tiled products, us:
-//   m = 128: n = 1024 97 / 113, 2048 (two chunks a block) 148 / 115, 8192 348 / 177     m = 100: 1024 88 / 113, 2048 132 / 116
-//   m = 64: 8192 97 / 149, 16384 146 / 156, 32768 240 / 178        m = 32: 8192 99 / 141, 16384 140 / 143, 32768 221 / 163
-//   m = 16: 8192 67 / 135, 16384 92 / 138, 32768 145 / 151
-// (m <= 16 stays to 65536: such matrices come in hundreds, where the blocks that wait for memory are many)
-bool ns_small_takes(int R, int C) {
+// on all CUs.  Where that is depends on how many a plan has: few long ones leave CUs idle that tiles would use, sixteen and
+// more fill them either way and need half the launches here.  The line for few: 24576 for m of 49 to 64, for m > 64 1024 at
+// m = 128, 2147 at 100, 5753 at 72, and n / 30 times that in a plan of n > 30 matrices with m > 64, whose launch the long ones
+// end under; `many[c]`: the plan has four of the former (c = 0) or sixteen of the latter (c = 1) beyond it.
+// Whole steps on matrices of m x n, here / by tiles, us:
+//   m = 128, 1, 8, 16, 32, 64 of them: n = 1100 197 / 180, 224 / 215, 249 / 250, 272 / 304, 479 / 447      4096 282 / 199,
+//     344 / 292, 469 / 447, 535 / 623, 899 / 1089      8192 440 / 253, 610 / 475, 781 / 716, 916 / 1075, 1719 / 2032
+//   m = 96: 2048 175 / 169, 213 / 220, 244 / 271, 296 / 374, 466 / 579      8192 374 / 252, 467 / 409, 680 / 664, 814 / 964,
+//     1490 / 1834
+//   m = 72: 3000 177 / 181, 212 / 240, 246 / 285, 305 / 412, 504 / 668      6000 257 / 211, 299 / 288, 387 / 436, 516 / 645,
+//     1092 / 1157
+//   m = 64, 1, 4, 16, 64 of them: 16384 213 / 232, 258 / 314, 737 / 786, 1974 / 2457      32768 317 / 284, 446 / 497, 1219 / 1453,
+//     4028 / 4528
+//   m = 48: 24000 229 / 248, 286 / 342, 823 / 874, 2573 / 2806      32768 267 / 271, 358 / 418, 1043 / 1299, 3110 / 3748
+//   m = 32: 16384 178 / 217, 228 / 273, 668 / 531, 1418 / 1586      32768 247 / 250, 309 / 327, 893 / 996, 2331 / 2811
+//   decoders of width 128 with two embeddings: 12 layers (74 matrices) 2000 239 / 266, 4000 324 / 291; 24 (146) 2000 287 / 345,
+//     4000 374 / 402, 8000 549 / 472; 40 (242) 4000 424 / 559, 8000 571 / 688
+// (m <= 16 to 65536: finishing calls on one matrix 67 / 135 at 8192, 145 / 151 at 32768)
+struct NsSmallRule {
+  double stretch = 1.0;
+  bool many[2] = {true, true};
+};
+bool ns_small_long(int m, int n, const NsSmallRule& r) {
+  return m > SmMid::MP ? (double)m * m * m * n > r.stretch * (1ll << 31) : m > 48 && n > 24576;
+}
+bool ns_small_takes(int R, int C, const NsSmallRule& r) {
   const int m = std::min(R, C), n = std::max(R, C);
-  if (m > SmLarge::MP) return false;
-  return n <= (m <= 16 ? 65536 : m <= SmMid::MP ? 16384 : 1024);
+  if (m > SmLarge::MP || n > (m <= 16 ? 65536 : m <= SmMid::MP ? 32768 : 8192)) return false;
+  return !ns_small_long(m, n, r) || r.many[m > SmMid::MP];
 }
 
 // Whether a plan's small matrices go aside to their own launches, or with the larger ones through the tiled launches that
@@ -493,14 +514,14 @@ bool ns_small_takes(int R, int C) {
 // a block; in the tiled launches they are a few more tiles, free while the launches leave CUs idle.  So they stay with larger
 // matrices that are one group, if these are less than 22 G of work (or the small one is alone) and the small ones add
 // no more than 512 update tiles, two a CU.  Whole steps, tiled / aside:
-//   classifier 784 -> 1024 -> 1024 -> 10 (17 G) 978 / 1013 us, 784 -> 384 -> 384 -> 10 477 / 508, 784 -> 2048 (x 4) -> 10
-//     (280 G, one small) 3144 / 3171
-//   one 512 x 512 (1.4 G) and 8, 32, 64 of 16 x 1024 564 / 580, 582 / 643, 652 / 708
-//   decoder of width 256 with k, v of 32, 1, 4, 12 layers 530 / 543, 576 / 583, 858 / 867; width 384, 48, 1 layer 643 / 677
-//   four 1024 x 1024 (44 G) and 8, 16, 64 of 16 x 1024 1118 / 1092, 1144 / 1107, 1458 / 1202
-//   two 1024 x 1024 (22 G) and 4, 16 of 64 x 2000 979 / 956, 1026 / 1013
-//   decoder of width 512 with k, v of 64 (32 G) 994 / 987, 8 layers (93 G, two groups) 1896 / 1877
-//   three thousand odd tensors (1720 small matrices) 4.35 / 2.79 ms
+//   classifier 784 -> 1024 -> 1024 -> 10 (19 G) 442 / 468 us, 784 -> 384 -> 384 -> 10 250 / 269, 784 -> 2048 (x 4) -> 10
+//     (373 G, one small) 3103 / 3135
+//   one 512 x 512 (1.4 G) and 8, 32, 64 of 16 x 1024 262 / 283, 346 / 353, 389 / 413
+//   decoder of width 256 with k, v of 32, 1, 4, 12 layers (4, 7, 17 G) 293 / 317, 379 / 412, 642 / 610; width 384, 48, 1 layer 404 / 430
+//   four 1024 x 1024 (45 G) and 8, 16, 64 of 16 x 1024 715 / 753, 756 / 791, 937 / 888
+//   two 1024 x 1024 (23 G) and 4, 16 of 64 x 2000 467 / 478, 613 / 548
+//   decoder of width 512 with k, v of 64, 2 layers (30 G) 727 / 723, 8 (86 G, two groups) 1496 / 1480
+//   decoder of width 1024 with k, v of 128, 1, 2 layers (127, 202 G) 1648 / 1634, 2230 / 2205
 bool ns_small_aside(int n_large, double work_large, int n_small, long long small_tiles) {
   if (n_large == 0 || small_tiles > 512 || ns_group_count(n_large + n_small, work_large) > 1) return true;
   return n_small > 1 && work_large >= 22e9;
@@ -609,14 +630,23 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
   int R = 0, C = 0, n_sl = 0;
   // Chains of other lengths than pairs and singles, where the environment asks for them, are the tiled products' only.
   const char* chains = getenv("PYLO_MI355_NS_CHAINS");
+  NsSmallRule rule;
   bool small = L.ns_hf && env_ns_small() && !(chains && chains[0]) && !ns_adaptive();
   if (small) {
-    int n_large = 0, n_small = 0;
+    int n_large = 0, n_small = 0, n_cls = 0, n_long[2] = {0, 0};
     double work = 0.0;
     long long tiles = 0;
+    for (int t = 0; t < T; ++t)
+      if (matrices(t, R, C, n_sl) && std::min(R, C) > SmMid::MP && ns_small_takes(R, C, rule)) n_cls += n_sl;
+    rule.stretch = std::max(1.0, n_cls / 30.0);
+    for (int t = 0; t < T; ++t)
+      if (matrices(t, R, C, n_sl) && ns_small_takes(R, C, rule) && ns_small_long(std::min(R, C), std::max(R, C), rule))
+        n_long[std::min(R, C) > SmMid::MP] += n_sl;
+    rule.many[0] = n_long[0] >= 4;
+    rule.many[1] = n_long[1] >= 16;
     for (int t = 0; t < T; ++t) {
       if (!matrices(t, R, C, n_sl)) continue;
-      if (ns_small_takes(R, C)) {
+      if (ns_small_takes(R, C, rule)) {
         n_small += n_sl;
         tiles += (long long)n_sl * ((std::max(R, C) + kNsTile - 1) / kNsTile);
       } else {
@@ -628,7 +658,7 @@ void build_ns_tables(Layout& L, const PyloTensorShape* shapes, int T, long long&
   }
   for (int t = 0; t < T; ++t) {
     if (!matrices(t, R, C, n_sl)) continue;
-    if (small && ns_small_takes(R, C)) {
+    if (small && ns_small_takes(R, C, rule)) {
       L.small_of_tensor[t] = (long long)R * C % 4 == 0 ? 2 : 1;
       for (int sl = 0; sl < n_sl; ++sl) {
         NsSmall b{};

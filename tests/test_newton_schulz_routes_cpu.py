@@ -70,3 +70,32 @@ def test_long_thin_matrices_keep_their_class(longs):
     """Next to one 100 x 100 their blocks and partial sums are those that they have without it (64 x 32^2 floats, twice; the
     largest class would give them 8 x 128^2)."""
     assert _bytes(longs + [(100, 100)]) - _bytes(longs) <= _bytes([(100, 100)])
+
+
+# long matrices with a smaller dim above 32: few of them go to tiles, many stay with the one-launch kernel
+@pytest.mark.parametrize("shape,few,many", [((128, 2048), 15, 16), ((4096, 100), 1, 16), ((72, 8192), 15, 200),
+                                            ((64, 32768), 3, 4), ((25000, 49), 1, 64)])
+def test_long_matrices_go_to_tiles_while_they_are_few(shape, few, many, monkeypatch):
+    monkeypatch.delenv("PYLO_MI355_NS_SMALL", raising=False)
+    default = [_bytes([shape] * c) for c in (few, many)]
+    monkeypatch.setenv("PYLO_MI355_NS_SMALL", "0")
+    tiled = [_bytes([shape] * c) for c in (few, many)]
+    assert default[0] == tiled[0] and default[1] != tiled[1]
+
+
+def test_long_matrices_end_under_the_launch_of_many_others(monkeypatch):
+    """One of 2000 x 128 next to eight and to eighty of 128 x 128: as the other launch and this one need, apart or together."""
+    monkeypatch.delenv("PYLO_MI355_NS_SMALL", raising=False)
+    few, many = ([(128, 128)] * c for c in (8, 80))
+    alone = _bytes([(2000, 128)])
+    together = 2 * 8 * 128 * 128 * 4              # its partial sums: eight blocks
+    assert _bytes(few + [(2000, 128)]) - _bytes(few) > 0.9 * alone
+    assert abs(_bytes(many + [(2000, 128)]) - _bytes(many) - together) < 0.9 * (alone - together)
+
+
+@pytest.mark.parametrize("shape", [(128, 1024), (72, 5700), (100, 2100), (64, 24000), (48, 32768), (17, 30000), (16, 65536)])
+def test_others_never_do(shape, monkeypatch):
+    monkeypatch.delenv("PYLO_MI355_NS_SMALL", raising=False)
+    default = _bytes([shape])
+    monkeypatch.setenv("PYLO_MI355_NS_SMALL", "0")
+    assert default != _bytes([shape])
