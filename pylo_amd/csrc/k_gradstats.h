@@ -518,9 +518,10 @@ __device__ __forceinline__ void vector_terms(const TDesc& d, int which, bool is_
 // writes the factor tables and, when first-layer weights are given (shared by all tensors), the
 // per-row / per-column MLP terms: the 12 feature channels that depend on the row or on the column
 // only are normalised and pushed through the first layer once per row / column instead of once
-// per element.  The bias goes into the terms of vector 0.
+// per element.  The bias goes into the terms of vector 0.  RUNS: plans with such slices (TDesc::slice_runs); the loop over
+// a run costs the launch of every other plan 1 us of its 5 to 7 where it is compiled in.
 // =============================================================================================
-template <int H>
+template <int H, bool RUNS = false>
 __global__ __launch_bounds__(kThreads) void k_v0b(const TDesc* __restrict__ descs,
                                                   const PyloTensorArgs* __restrict__ dyn,
                                                   const Item* __restrict__ items,
@@ -668,7 +669,7 @@ __global__ __launch_bounds__(kThreads) void k_v0b(const TDesc* __restrict__ desc
       const int st = d.rcm_stride, blk = d.rcm_size * st;
       slice = (i / blk - o_first) * st + i % st;
     }
-    if (d.slice_runs) {   // the channels are normalised over the run of slice_len entries that slices meet (k_celo2_slices_wave)
+    if (RUNS && d.slice_runs) {   // the channels are normalised over the run of slice_len entries that slices meet (k_celo2_slices_wave)
       const int S = d.slice_len, r0 = i - i % S;
       const float inv_s = 1.0f / (float)S;
 #pragma unroll

@@ -149,6 +149,7 @@ struct Layout {
   std::vector<Item> sl_wave_items;    // ELO-CELO2: blocks of k_celo2_slices_wave, one class after another
   std::vector<Item> sl_wave_cls[kSliceWaveClasses];
   int sl_wave_n[kSliceWaveClasses] = {};
+  bool slice_runs = false;            // some tensor's (TDesc::slice_runs)
   size_t off_sl_wave_items = 0;
   std::vector<Item> p0_items, nd_items, sl_items, seg_items, el_items, ap_items, pp_items, ga_items, fin_items, v0a_items, v0b_items;
   std::vector<int> fac_list;
@@ -1221,6 +1222,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       if (short_slices(d)) {
         // short slices of a tensor with more than two dims: packed into waves (k_celo2_slices_wave)
         d.slice_runs = d.nd_stride[0] % d.slice_len == 0 && d.nd_stride[1] % d.slice_len == 0;
+        L.slice_runs = L.slice_runs || d.slice_runs;
         const int cls = !d.slice_runs ? kSliceGather : d.slice_len == 1 ? kSliceOne : d.slice_len == 9 ? kSliceNine : kSliceAny;
         const long long per_wave = 64 / d.slice_len;
         for (long long s0 = 0; s0 < n_slices && n > 0; s0 += kWaves * per_wave * slice_trips)
@@ -1925,8 +1927,9 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
   if (n_v0a > 0)
     hipLaunchKernelGGL(k_v0a, dim3(n_v0a), dim3(kV0aThreads), 0, s, descs, dyn, v0a_items, part, gl, dec, v0part);
   HIP_TRY(mark());
+  const auto v0b = L.slice_runs ? k_v0b<8, true> : k_v0b<8>;
   if (n_v0b > 0)
-    hipLaunchKernelGGL(k_v0b<8>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, v0part, 1e-9f, mlp,
+    hipLaunchKernelGGL(v0b, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, v0part, 1e-9f, mlp,
                        mlp + 240, 0, fac_tab, term_tab, bscale);
   HIP_TRY(mark());
   const int n_mx = (int)L.mx_items.size();
