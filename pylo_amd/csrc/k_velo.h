@@ -127,6 +127,7 @@ __device__ __forceinline__ void lstm_pivots(const TDesc& d, const PyloTensorArgs
 // kernel that formed the LSTM's inputs, since the apply pass overwrites them while it runs) and the
 // tensor's first gradient element; they are wave-uniform and live in scalar registers.
 constexpr int kNewSumW = 10;    // doubles per row of those partial sums (9 used)
+constexpr int kFeatWide = 512;  // blocks of k_p0 and of k_velo_feat together up to which the latter's have sixteen waves
 struct NewSums {
   float v[9];
   float piv[4];
@@ -608,11 +609,14 @@ __device__ __forceinline__ double* velo_guard_sums(int* sync, int T) { return re
 // The same from the sums the previous step's apply pass left (rows of kNewSumW doubles per element
 // block, shifted by the tensor's first elements as that pass wrote them, i.e. as they stand now): the
 // LSTM does not wait for this step's statistics pass.  Tensors of many rows come summed in segments (k_stat_segsum): one
-// block, a tensor's only one, waited 165 us for the 16 000 rows of an embedding of 131 M elements.  Blocks of four waves,
-// four units a thread: next to k_p0, whose blocks take the place of every four waves that end, blocks of sixteen wait.
-// Three thousand tensors and that embedding 387 / 41 us next to k_p0, whole step 2.91 / 2.77 ms; ViT-B/16 80 / 72 us, 1.01 / 1.00 ms
-// (8 us without the gradients streaming past it: what is left is a chain of short dependent loads).
-__global__ __launch_bounds__(kThreads) void k_velo_feat(const TDesc* __restrict__ descs,
+// block, a tensor's only one, waited 165 us for the 16 000 rows of an embedding of 131 M elements.  Blocks of four waves
+// take four units a thread: next to k_p0, whose blocks take the place of every four waves that end, blocks of sixteen wait.
+// Three thousand tensors and an embedding 387 / 41 us next to k_p0; ViT-B/16 80 / 72 us (8 us without the gradients streaming
+// past it: what is left is a chain of short dependent loads).  Where k_p0 leaves room the shorter chain of a unit a thread is
+// worth more, 11.6 / 8.6 us: whole steps, four / sixteen waves, 0.6 M elements 108 / 106 us, 1.4 M 119 / 116, 4.4 M (280 blocks) 157 / 155,
+// 10.0 M (630) 247 / 252, 12.5 M 226 / 231, 89 M 1030 / 1037, a thousand tensors of 1 M 632 / 637 (kFeatWide).
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_velo_feat(const TDesc* __restrict__ descs,
                                                         const PyloTensorArgs* __restrict__ dyn, int T,
                                                         const double* __restrict__ newsum_part, const double* __restrict__ seg_tot,
                                                         float* __restrict__ piv, LossState ls, VeloStep st,
@@ -620,7 +624,7 @@ __global__ __launch_bounds__(kThreads) void k_velo_feat(const TDesc* __restrict_
                                                         const float* __restrict__ w2t, const float* __restrict__ b2,
                                                         const float* __restrict__ wft, const float* __restrict__ bf,
                                                         float* __restrict__ mixbuf, int* __restrict__ sync) {
-  constexpr int G = kThreads / kNewSumW;
+  constexpr int G = THREADS / kNewSumW;
   __shared__ double part[G][kNewSumW];
   __shared__ double tot[kStatW];
   __shared__ float xs[32];
@@ -656,7 +660,7 @@ __global__ __launch_bounds__(kThreads) void k_velo_feat(const TDesc* __restrict_
     if (q == 0) velo_guard_sums(sync, T)[t] = s;   // the statistics items of this step hold it against the sum they take themselves
   }
   __syncthreads();
-  velo_row_features<kThreads>(d, a, t, T, tot, nullptr, piv, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, xs);
+  velo_row_features<THREADS>(d, a, t, T, tot, nullptr, piv, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, xs);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -2503,7 +2503,9 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
     if (!L.seg_items.empty())
       hipLaunchKernelGGL(k_stat_segsum<kNewSumW>, dim3((unsigned)L.seg_items.size()), dim3(kThreads), 0, P->side, descs,
                          P->at<Item>(L.off_seg_items), (const double*)newsum, P->at<double>(L.off_segtot));
-    hipLaunchKernelGGL(k_velo_feat, dim3(T), dim3(kThreads), 0, P->side, descs, dyn, T, (const double*)newsum,
+    const bool wide_feat = n_p0 + n_nd + T <= kFeatWide;
+    hipLaunchKernelGGL(wide_feat ? k_velo_feat<kFoldThreads> : k_velo_feat<kThreads>, dim3(T), dim3(wide_feat ? kFoldThreads : kThreads),
+                       0, P->side, descs, dyn, T, (const double*)newsum,
                        (const double*)P->at<double>(L.off_segtot), piv, ls, vs,
                        xfeat, H, nets->mix2_wt, nets->mix2_b, nets->fmix_wt, nets->fmix_b, mixbuf, P->at<int>(L.off_sync));
     lstm(P->side, nullptr, false);
