@@ -18,8 +18,8 @@
 // starting values through sigma -> sigma p(sigma^2), ns_plane_exps): X and A = X X^T stay below 1.5, B' = p(A)
 // below c0, products of k such B' below c0^k.  Every kind of matrix gets the power of two that puts its bound at
 // 12 000 .. 24 000; a product's accumulators are scaled back by the reciprocal of its operands' scales (exact) and
-// what it writes is scaled by its own.  A value outside its bound -- there should be none -- is clamped, not made
-// an infinity.
+// what it writes is scaled by its own.  A value outside its bound -- there should be none -- is not clamped: it
+// becomes an infinity and then a NaN, which stays visible.
 //
 // Operands therefore live as *planes*: two fp16 matrices (h, l) with the reduction index contiguous,
 // written by the kernel that produces the matrix (never converted inside a product's main loop).
@@ -239,8 +239,8 @@ __device__ __forceinline__ void hf_tile_product(const HfPlanes& P1, int i0, cons
 // lane's fragment of a row is 16 consecutive bytes of the planes): only the second operand goes through LDS, 48 KB
 // of LDS traffic a step and block instead of 73.  128 rows of P1 (by 256 threads), 64 WN rows of P2; LDS: two
 // stages of 64 WN x 64 bytes.  Benchmark instrumentation only (pylo_mi355_matrix_probe, mode 4): the bare loop is
-// 8 - 12 % faster this way on one large operand, the update product inside whole steps (four groups of matrices on
-// four streams) 2.5 % slower.
+// 8 - 12 % faster this way on one large operand, the update product inside whole steps 2.5 % slower (with four groups of matrices
+// on four streams).
 template <int WN>
 __device__ __forceinline__ void hf_tile_product_direct(const HfPlanes& P1, int i0, const HfPlanes& P2, int j0, int k0, int k1,
                                                        PYLO_LDS char* lds, v16f (&acc)[2][WN]) {

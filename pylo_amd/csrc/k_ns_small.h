@@ -29,9 +29,9 @@
 // kSpinLimit polls a block gives up and leaves NaN in its part of the parameter.
 // Measured: the kernel is a chain on one CU -- on 128 x 784 (seven blocks, 92 us) five products of an m x m pair phase
 // take 13.7 us of which the matrix instructions are 1.3 us each, a meeting with its partial sums 8.5 us, a Gram or
-// update product 3 us.  Whole ELO-CELO2 steps with it and with the tiled products: classifier 784 -> 128 -> 128 -> 10
-// 148 / 311 us, transformers of width 96 and 128 with twelve layers and 4000 x width embeddings 266 / 568 and 331 / 569 us,
-// three thousand odd matrices 2.79 / 3.95 ms.
+// update product 3 us.  Whole ELO-CELO2 steps with it and with the tiled products alone: classifiers 784 -> 128 -> 128 -> 10
+// 148 / 181 us, 784 -> 64 (x 4) -> 10 103 / 178, transformers of width 96 and 128 with twelve layers and two 4000 x width
+// embeddings 267 / 272 and 302 / 301 us, three thousand odd tensors 2.74 / 4.07 ms.
 #pragma once
 
 #include "k_ns_hf.h"

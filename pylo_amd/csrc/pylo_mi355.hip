@@ -451,7 +451,7 @@ bool env_ns_small() {
 // The products of an m x n matrix in the unit of the rules below: five iterations in pairs are three Gram products on
 // the upper blocks, three updates and eleven m x m products.
 double ns_work(int m, int n) { return (double)m * m * (4.6 * n + 5.9 * m); }
-// ... as the tiled launches do it, in whole tiles (a thousand 130 x 130, 176 G and not 23: 1917 us on four streams, 2145 on one)
+// ... as the tiled launches do it, in whole tiles (a thousand 130 x 130, 176 G and not 23: 2000 us on two streams, 2177 on one)
 double ns_tiled_work(int m, int n) {
   auto up = [](int x) { return (x + kNsTile - 1) / kNsTile * kNsTile; };
   return ns_work(up(m), up(n));
