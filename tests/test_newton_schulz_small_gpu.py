@@ -16,6 +16,8 @@ SETS = {
     "up to 32": [(1, 1), (1, 7), (7, 1), (31, 33), (32, 32), (5, 128), (129, 5), (32, 1025), (3000, 17), (1, 30000), (16, 65536), (17, 32769)],
     "up to 64": [(33, 33), (33, 128), (129, 40), (64, 64), (64, 2048), (4099, 37), (37, 8191), (32768, 33)],
     "past the limits": [(65537, 5), (32769, 33), (8193, 96), (70, 8200)],       # the tiled products', with no small ones
+    "four long ones": [(64, 32768), (25000, 49), (63, 24577), (30001, 64)],     # one to three of these are the tiled products'
+    "sixteen long ones": [(128, 8192), (8192, 127), (1025, 128), (128, 4099), (2148, 100), (5754, 72), (7820, 65), (3000, 96)] * 2,
     "beside a higher class": [(16, 65536), (64, 8192), (65, 65), (3, 9)],       # lifted, and too long to be
     "beside larger ones": [(10, 512), (512, 300), (100, 300), (31, 33)],        # in the larger ones' launches
     "up to 128": [(65, 65), (65, 128), (129, 100), (128, 128), (784, 128), (128, 4096), (1027, 127), (96, 257), (8193, 80)],
