@@ -1,4 +1,5 @@
-// Newton-Schulz, normaliser and update of small matrices in one launch: a block (or a few) per matrix.
+// Newton-Schulz, normaliser and update of small matrices (a smaller dim m of 33 to 128, and thinner ones lifted to their launch;
+// k_ns_thin.h has the others) in one launch: a block (or a few) per matrix.
 //
 // The tiled products (k_ns_hf.h) are one launch per product for all matrices of a plan: sixteen dependent launches of
 // 128 x 128 tiles with whole 128-row operands in memory.  A matrix whose smaller dim m is at most 128 pads that to several
@@ -10,7 +11,7 @@
 // ns_plane_exps, three v_mfma_f32_32x32x16_f16 per fp32 product, fp32 accumulation; iterations in pairs that share
 // one Gram product and one update (T = A B', A' = B' T, B'' = p(A'), Q = B'' B', X'' = Q X).
 //
-// Layout.  MT = m rounded up to 32 over 32 (1, 2 or 4); MT / RT x MT waves, each owning the 32 x 32 tiles (tr0 + i, tc), i <
+// Layout.  MT = m rounded up to 32 over 32 (2 or 4); MT / RT x MT waves, each owning the 32 x 32 tiles (tr0 + i, tc), i <
 // RT, of every m x m matrix and the tiles (tr0 + i, tc + MT j), j < J, of a chunk of NB = 32 MT J columns of X (m x n, n
 // the longer dim, whatever way the tensor stores it), all as fp32 accumulators: register r of a lane is row 8 (r / 4) + 4 (lane / 32)
 // + r % 4, its column is lane % 32.  Planes in LDS, the reduction index contiguous, rows padded by 16 bytes so that
@@ -24,14 +25,14 @@
 // (norm, three Gram products, RMS), leaving their partial sums in the workspace and adding all of them in slab order.
 // Blocks wait for blocks of their own matrix only.  The wait ends: a block draws its place in the item table when it
 // starts, so that of all matrices with a block running at most one still has blocks to start -- as many as wait in
-// it, at most 64, 32 or 8 by class of the 2048, 512 or 256 that the chip holds (kSlabsMax), so that the launches that four
+// it, at most 32 or 8 by class of the 512 or 256 that the chip holds (kSlabsMax), so that the launches that four
 // hardware queues can run at once never fill it with them; all others have their blocks running, end, and make room.  After
 // kSpinLimit polls a block gives up and leaves NaN in its part of the parameter.
 // Measured: the kernel is a chain on one CU -- on 128 x 784 (seven blocks, 92 us) five products of an m x m pair phase
 // take 13.7 us of which the matrix instructions are 1.3 us each, a meeting with its partial sums 8.5 us, a Gram or
 // update product 3 us.  Whole ELO-CELO2 steps with it and with the tiled products alone: classifiers 784 -> 128 -> 128 -> 10
 // 148 / 181 us, 784 -> 64 (x 4) -> 10 103 / 178, transformers of width 96 and 128 with twelve layers and two 4000 x width
-// embeddings 267 / 272 and 302 / 301 us, three thousand odd tensors 2.74 / 4.07 ms.
+// embeddings 267 / 272 and 302 / 301 us.
 #pragma once
 
 #include "k_ns_hf.h"
@@ -45,6 +46,7 @@ struct NsSmall {
   long long elem_off;    // elements from the tensor's first
   long long part;        // floats into the partial-sum workspace: 2 x slabs x (32 MT)^2, slabs > 1 only
   int sums, sync;        // its 2 x slabs doubles and two counters (zero between calls)
+  int fold;              // k_ns_thin: 2^fold columns side by side
 };
 struct NsSmallItem { int mat, slab; };
 
@@ -302,7 +304,7 @@ __global__ __launch_bounds__(64 * (MT / RT) * MT) void k_ns_small(
       if (threadIdx.x == 0) coh_store_wait(o + it.slab, t);
       ++meets;
       if (good) good = sm_meet(sync + q.sync, meets * q.slabs, &s_flag);
-      t = wave_sum(lane < q.slabs ? coh_load(o + lane) : 0.0);   // at most 64 slabs; the same tree in every wave of every block
+      t = wave_sum(lane < q.slabs ? coh_load(o + lane) : 0.0);   // at most 32 slabs; the same tree in every wave of every block
     }
     return t;
   };

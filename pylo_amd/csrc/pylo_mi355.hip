@@ -32,6 +32,7 @@
 #include "k_ns.h"
 #include "k_ns_hf.h"
 #include "k_ns_small.h"
+#include "k_ns_thin.h"
 #include "k_slice_finish.h"
 #include "k_cast.h"
 #include "pylo_common.h"
@@ -88,7 +89,7 @@ struct NsGroup {
 // One batch of matrices: those whose operand planes share the plane workspace at one time.
 struct NsBatch { int mat0, n_mats, group0, n_groups; long long plane_elems; };
 
-constexpr int kNsSmallClasses = 3;
+constexpr int kNsSmallClasses = 4;
 struct Layout {
   std::vector<Item> mx_items;   // ELO-CELO2: statistics and apply items in slab order (k_celo2_elem)
   bool split = false;           // element blocks smaller than 8192 elements (split_for)
@@ -118,8 +119,8 @@ struct Layout {
   int slice_lds_l[kSliceLaneSets] = {}, slice_lds_w = 0, slice_lds_b = 0;
   size_t off_slice_mats = 0, off_slice_items_l[kSliceLaneSets] = {}, off_slice_items_w = 0, off_slice_items_b = 0;
   int ns_max_m = 0;
-  // Newton-Schulz: matrices that one launch takes from the raw step to the parameter (k_ns_small.h), by class (m up to
-  // 32, 64, 128)
+  // Newton-Schulz: matrices that one launch takes from the raw step to the parameter (k_ns_thin.h, k_ns_small.h), by class (m up to
+  // 16, 32, 64, 128)
   std::vector<NsSmall> sm_mats;
   std::vector<NsSmallItem> sm_items[kNsSmallClasses];
   std::vector<char> small_of_tensor;  // per tensor: its matrices are in sm_mats (2: they are multiples of four elements long)
@@ -470,12 +471,13 @@ int ns_group_count(int mats, double work) {
   return (int)std::min<double>(std::min(env_ns_groups(), std::max(mats / 8, 1)), 1.0 + std::floor(work / 55e9));
 }
 
-using SmSmall = SmDims<1, 1, 2>;
 using SmMid = SmDims<2, 1, 2>;
 using SmLarge = SmDims<4, 2, 1>;
-int ns_small_class(int m) { return m <= SmSmall::MP ? 0 : m <= SmMid::MP ? 1 : 2; }
-int ns_small_chunk(int cls) { return cls == 0 ? SmSmall::NB : cls == 1 ? SmMid::NB : SmLarge::NB; }
-int ns_small_edge(int cls) { return cls == 0 ? SmSmall::MP : cls == 1 ? SmMid::MP : SmLarge::MP; }
+// 0, 1: k_ns_thin<1>, <2>; 2, 3: k_ns_small<2, 1, 2>, <4, 2, 1>
+int ns_small_class(int m) { return m <= ThinDims<1>::MP ? 0 : m <= ThinDims<2>::MP ? 1 : m <= SmMid::MP ? 2 : 3; }
+int ns_small_chunk(int cls) { return cls < 2 ? kThinChunk : cls == 2 ? SmMid::NB : SmLarge::NB; }
+// floats of partial sums that a block of a matrix of several leaves: G in fp64, or A in fp32 twice
+int ns_small_part(int cls) { return cls == 0 ? ThinDims<1>::NT * 512 : cls == 1 ? ThinDims<2>::NT * 512 : 2 * (cls == 2 ? SmMid::MP * SmMid::MP : SmLarge::MP * SmLarge::MP); }
 
 // Which matrices the one-launch kernel takes: a smaller dim of at most 128 (its m x m matrices fit a CU's LDS) and a
 // longer one up to where its few blocks, each walking chunks of the long dim one after another, fall behind tiles of 64 x 64
@@ -493,10 +495,12 @@ int ns_small_edge(int cls) { return cls == 0 ? SmSmall::MP : cls == 1 ? SmMid::M
 //   m = 64, 1, 4, 16, 64 of them: 16384 213 / 232, 258 / 314, 737 / 786, 1974 / 2457      32768 317 / 284, 446 / 497, 1219 / 1453,
 //     4028 / 4528
 //   m = 48: 24000 229 / 248, 286 / 342, 823 / 874, 2573 / 2806      32768 267 / 271, 358 / 418, 1043 / 1299, 3110 / 3748
-//   m = 32: 16384 178 / 217, 228 / 273, 668 / 531, 1418 / 1586      32768 247 / 250, 309 / 327, 893 / 996, 2331 / 2811
+//   m = 32 (k_ns_thin, no line below its limits): 1024 98 / 172, 99 / 173, 102 / 174, 125 / 236      16384 106 / 209, 138 / 257,
+//     327 / 491, 764 / 1404      32768 135 / 235, 192 / 310, 538 / 929, 1441 / 2471
+//   m = 16, 1, 16 of them: 8192 89 / 185, 131 / 264      32768 99 / 220, 347 / 719      65536 127 / 242, 550 / 1160
+//   m = 4: 65536 97 / 228, 264 / 934
 //   decoders of width 128 with two embeddings: 12 layers (74 matrices) 2000 239 / 266, 4000 324 / 291; 24 (146) 2000 287 / 345,
 //     4000 374 / 402, 8000 549 / 472; 40 (242) 4000 424 / 559, 8000 571 / 688
-// (m <= 16 to 65536: finishing calls on one matrix 67 / 135 at 8192, 145 / 151 at 32768)
 struct NsSmallRule {
   double stretch = 1.0;
   bool many[2] = {true, true};
@@ -530,11 +534,13 @@ bool ns_small_aside(int n_large, double work_large, int n_small, long long small
 
 // Slabs (blocks) of each small matrix and the items of the launches.
 void build_small_items(Layout& L) {
-  // what a launch of the class holds at a time on 256 CUs (LDS), and the most blocks one matrix may have waiting
-  // (k_ns_small.h)
-  constexpr int kHolds[kNsSmallClasses] = {2048, 512, 256}, kSlabsMax[kNsSmallClasses] = {64, 32, 8};
+  // how many blocks a launch of the class is cut into at most -- what 256 CUs hold at a time (LDS), for the thin ones fewer: every
+  // block of a matrix goes through its m x m products (sixteen of 17 x 32768, blocks up to 256 / 512 / 1024: 164 / 128 / 161 us,
+  // three hundred of 32 x 1024 124 / 98 / 121) -- and the most blocks one matrix may have waiting (k_ns_small.h)
+  constexpr int kHolds[kNsSmallClasses] = {1024, 512, 512, 256}, kSlabsMax[kNsSmallClasses] = {64, 64, 32, 8};
+  constexpr int kChunksMin[kNsSmallClasses] = {8, 4, 1, 1};   // what a block takes before a matrix is cut
   auto cls_of = [](const NsSmall& b) { return ns_small_class(b.m); };
-  int lift[kNsSmallClasses] = {0, 1, 2};
+  int lift[kNsSmallClasses] = {0, 1, 2, 3};
   // A plan with few small matrices takes them in the class of the largest, one launch: the small ones end under it,
   // unless the fewer and larger blocks of that class walk more than eight chunks each, what its own longest matrix walks
   // (a chunk is 15 to 25 us of a block's chain).  Whole steps, a class of 65 x 65 or 100 x 100 next to others, lifted /
@@ -557,7 +563,11 @@ void build_small_items(Layout& L) {
   for (int cls = 0; cls < kNsSmallClasses; ++cls) {
     std::vector<int> of;
     const int nb = ns_small_chunk(cls);
-    auto chunks = [&](int q) { return (L.sm_mats[q].n + nb - 1) / nb; };
+    if (cls == 0)
+      for (int q = 0; q < (int)L.sm_mats.size(); ++q)
+        if (lift[cls_of(L.sm_mats[q])] == 0)
+          for (NsSmall& b = L.sm_mats[q]; (2 << b.fold) * b.m <= ThinDims<1>::MP;) ++b.fold;
+    auto chunks = [&](int q) { return (L.sm_mats[q].n + (nb << L.sm_mats[q].fold) - 1) / (nb << L.sm_mats[q].fold); };
     long long total = 0;
     for (int q = 0; q < (int)L.sm_mats.size(); ++q)
       if (lift[cls_of(L.sm_mats[q])] == cls) {
@@ -565,7 +575,7 @@ void build_small_items(Layout& L) {
         total += chunks(q);
       }
     // one slab a chunk while no more blocks are started than twice what runs at once, longer ones when there are more
-    const int per = (int)std::max<long long>(1, total / kHolds[cls]);
+    const int per = (int)std::max<long long>(kChunksMin[cls], total / kHolds[cls]);
     for (int q : of) {
       NsSmall& b = L.sm_mats[q];
       const int c = chunks(q);
@@ -575,7 +585,7 @@ void build_small_items(Layout& L) {
       b.chunks = (c + b.slabs - 1) / b.slabs;      // even slabs
       b.slabs = (c + b.chunks - 1) / b.chunks;
       b.part = L.sm_part_floats;
-      L.sm_part_floats += 2ll * b.slabs * ns_small_edge(cls) * ns_small_edge(cls);
+      L.sm_part_floats += (long long)b.slabs * ns_small_part(cls);
       b.sums = L.sm_sums;
       L.sm_sums += 2 * b.slabs;
       b.sync = L.sm_sync;
@@ -2034,7 +2044,6 @@ int small_lds_once() {
     if (d == dev) return 0;
   HIP_TRY(hipFuncSetAttribute((const void*)(k_ns_small<4, 2, 1>), hipFuncAttributeMaxDynamicSharedMemorySize, SmLarge::kLds));
   HIP_TRY(hipFuncSetAttribute((const void*)(k_ns_small<2, 1, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, SmMid::kLds));
-  HIP_TRY(hipFuncSetAttribute((const void*)(k_ns_small<1, 1, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, SmSmall::kLds));
   done.push_back(dev);
   return 0;
 }
@@ -2068,9 +2077,17 @@ int enqueue_small(PyloPlan* P, hipStream_t s, const TDesc* descs, const PyloTens
                          P->at<double>(L.off_sm_sums), P->at<int>(L.off_sm_sync), st, orth,
                          L.sm_meets[cls] ? P->at<int>(L.off_sm_sync) + L.sm_ticket0 + cls : (int*)nullptr);
   };
-  launch(k_ns_small<4, 2, 1>, 2, SmLarge::kThr, SmLarge::kLds);
-  launch(k_ns_small<2, 1, 2>, 1, SmMid::kThr, SmMid::kLds);
-  launch(k_ns_small<1, 1, 2>, 0, SmSmall::kThr, SmSmall::kLds);
+  const ThinStep thin{st.c0, st.c1, st.c2, ns_eps, ns_iters};
+  auto launch_thin = [&](auto kern, int cls, int lds) {
+    if (!L.sm_items[cls].empty())
+      hipLaunchKernelGGL(kern, dim3((unsigned)L.sm_items[cls].size()), dim3(kThreads), lds, s, P->at<NsSmall>(L.off_sm_mats),
+                         P->at<NsSmallItem>(L.off_sm_items[cls]), descs, dyn, P->at<float>(L.off_sm_part), P->at<int>(L.off_sm_sync),
+                         thin, orth, L.sm_meets[cls] ? P->at<int>(L.off_sm_sync) + L.sm_ticket0 + cls : (int*)nullptr);
+  };
+  launch(k_ns_small<4, 2, 1>, 3, SmLarge::kThr, SmLarge::kLds);
+  launch(k_ns_small<2, 1, 2>, 2, SmMid::kThr, SmMid::kLds);
+  launch_thin(k_ns_thin<2>, 1, ThinDims<2>::kLds);
+  launch_thin(k_ns_thin<1>, 0, ThinDims<1>::kLds);
   return 0;
 }
 
