@@ -399,7 +399,7 @@ __global__ __launch_bounds__(kThreads) void k_celo2_stats(const TDesc* __restric
   if (a.grad == nullptr) return;
   if (!celo2_stats_block<false, TYPED>(d, a, it, fac_tab, gl, dec, red)) return;
   if (threadIdx.x < kNStat)
-    stats_part[(size_t)blockIdx.x * kStatW + stat_channel(threadIdx.x)] = stats_block_total(red, threadIdx.x);
+    stats_part[(size_t)it.b * kStatW + stat_channel(threadIdx.x)] = stats_block_total(red, threadIdx.x);
 }
 
 // Per factored tensor: s_c = rsqrt(1e-9 + mean f_c^2) folded into the first-layer rows of the 18

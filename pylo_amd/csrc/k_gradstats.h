@@ -316,7 +316,7 @@ __global__ __launch_bounds__(kThreads) void k_p0_nd(const TDesc* __restrict__ de
 // First stage of the per-tensor reduction of the statistics partials, for tensors with thousands
 // of rows: one block adds up kSegRows rows, so that the per-tensor block that follows (one block,
 // hence one CU's bandwidth) reads a few dozen rows instead of thousands.  Fixed order throughout.
-// Item: tensor, first row (relative to the tensor's rows), number of rows.  W: doubles a row (kStatW, kNewSumW).
+// Item: tensor, first row (relative to the tensor's rows), number of rows, row of the result.  W: doubles a row (kStatW, kNewSumW).
 // =============================================================================================
 template <int W>
 __global__ __launch_bounds__(kThreads) void k_stat_segsum(const TDesc* __restrict__ descs,
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(kThreads) void k_stat_segsum(const TDesc* __restric
     double s = 0.0;
 #pragma unroll
     for (int g2 = 0; g2 < G; ++g2) s += part[g2][threadIdx.x];
-    seg_tot[(size_t)blockIdx.x * W + threadIdx.x] = s;
+    seg_tot[(size_t)it.c * W + threadIdx.x] = s;
   }
 }
 

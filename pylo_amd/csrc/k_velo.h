@@ -394,7 +394,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) v
   velo_stats_block<true, false, TYPED>(d, a, it, fac_tab, dec, red);
   if (threadIdx.x < 38) {
     const int c = threadIdx.x;
-    stats_part[(size_t)blockIdx.x * kStatW + c] =
+    stats_part[(size_t)it.b * kStatW + c] =
         ((double)red[0][c] + (double)red[1][c]) + ((double)red[2][c] + (double)red[3][c]);
   }
 }
@@ -1232,7 +1232,75 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   const TDesc d = elem_desc<SPLIT>(descs + it.tensor);
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
-  velo_apply_block<TYPED>(d, a, it, fac_tab, term_tab, dec, wfold, piv, newsum_part, (int)blockIdx.x, false, red);
+  velo_apply_block<TYPED>(d, a, it, fac_tab, term_tab, dec, wfold, piv, newsum_part, it.b, false, red);
+}
+
+// A tensor's channel sums (n_rows rows, added in order) and the folded block from them, its MLP in wmix, param_scale and lr_mult.
+// COH: the rows were written by other blocks of the running kernel and the block is for such (see coh_store_wait).
+template <bool COH>
+__device__ __forceinline__ void velo_fold_tensor(const TDesc& d, int t, const double* __restrict__ rows, int n_rows,
+                                                 const float* __restrict__ wmix, float* __restrict__ wfold, int* __restrict__ sync,
+                                                 int n_tensors) {
+  __shared__ double part[kThreads / 30][30];
+  __shared__ float sc[30];
+  constexpr int G = kThreads / 30;
+  const int c = threadIdx.x % 30, gI = threadIdx.x / 30;
+  if (gI < G) {
+    double s = 0.0;
+    for (int b0 = gI; b0 < n_rows; b0 += 16 * G) {
+      double v[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        const int b = b0 + q * G;
+        v[q] = b >= n_rows ? 0.0 : COH ? coh_load(rows + (size_t)b * kStatW + c) : rows[(size_t)b * kStatW + c];
+      }
+#pragma unroll
+      for (int q = 0; q < 16; ++q) s += v[q];
+    }
+    part[gI][c] = s;
+  }
+  __syncthreads();
+  __shared__ float pscale_s;
+  if (threadIdx.x < 30) {
+    double s = 0.0;
+    for (int g2 = 0; g2 < G; ++g2) s += part[g2][threadIdx.x];
+    const double n = (double)(d.n > 0 ? d.n : 1);
+    sc[threadIdx.x] = rsq(1e-5f + (float)(s / n));
+    if (threadIdx.x == 2) {   // channel 2 is the parameter
+      // The LSTM of this step was fed the sum of p^2 that the previous step's apply items carried over; `s` is
+      // the same sum over the parameter as it stands now.  They differ (beyond the rounding of two summation
+      // orders) only if somebody else wrote the parameter in between without the plan being told: the
+      // tensor's step is poisoned (a NaN param_scale multiplies it) and the plan's flag raised rather than a
+      // step taken on stale statistics.  The flag is pinned host memory (a system-scope store of 1 + tensor).
+      // Both addresses are found behind the counters of `sync` rather than passed as arguments: k_velo_elem's
+      // scalar registers are spilled as it is, and three more live arguments cost its hot loops 7 %.
+      const double carried = velo_guard_sums(sync, n_tensors)[t];
+      const bool ok = fabs(s - carried) <= 1e-3 * fmax(fabs(s), fabs(carried));
+      pscale_s = ok ? sqrtf((float)(s / n) + 1e-9f) : __builtin_nanf("");
+      if (!ok) __hip_atomic_store(velo_guard_flag(sync, n_tensors), t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+  }
+  __syncthreads();
+  const float* wm = wmix + (size_t)t * 160;
+  if (threadIdx.x < kVFold) {
+    const float v = velo_fold_entry(d, wm, sc, pscale_s, wm[kVBank], threadIdx.x);
+    float* o = wfold + (size_t)t * kVFold + threadIdx.x;
+    if constexpr (COH) coh_store_wait(o, v);
+    else *o = v;
+  }
+}
+
+// The folded blocks of tensors whose statistics were a launch of their own, one block per tensor.
+__global__ __launch_bounds__(kThreads) void k_velo_fold(const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn,
+                                                        const int* __restrict__ list, const double* __restrict__ stats_part,
+                                                        const double* __restrict__ seg_tot, const float* __restrict__ wmix,
+                                                        float* __restrict__ wfold, int* __restrict__ sync, int n_tensors) {
+  const int t = list[blockIdx.x];
+  const TDesc d = descs[t];
+  if (dyn[t].grad == nullptr) return;
+  int n_rows;
+  const double* rows = stat_rows(d, stats_part, seg_tot, n_rows);
+  velo_fold_tensor<false>(d, t, rows, n_rows, wmix, wfold, sync, n_tensors);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1256,8 +1324,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                                                         double* __restrict__ newsum_part, int* __restrict__ sync,
                                                         int n_tensors) {
   __shared__ float red[kWaves][38];
-  __shared__ double part[kThreads / 30][30];
-  __shared__ float sc[30];
   __shared__ int s_flag;
   const Item it = items[blockIdx.x];
   const TDesc d = elem_desc<SPLIT>(descs + it.tensor);
@@ -1307,50 +1373,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     s_flag = __hip_atomic_fetch_add(sync + it.tensor, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == d.nblk - 1;
   __syncthreads();
   if (!s_flag) return;
-  // the tensor's last statistics block: channel sums in row order, then the folded block
-  constexpr int G = kThreads / 30;
-  const int c = threadIdx.x % 30, gI = threadIdx.x / 30;
-  if (gI < G) {
-    const double* rows = stats_part + (size_t)d.blk0 * kStatW;
-    double s = 0.0;
-    for (int b0 = gI; b0 < d.nblk; b0 += 16 * G) {
-      double v[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int b = b0 + q * G;
-        v[q] = b < d.nblk ? coh_load(rows + (size_t)b * kStatW + c) : 0.0;
-      }
-#pragma unroll
-      for (int q = 0; q < 16; ++q) s += v[q];
-    }
-    part[gI][c] = s;
-  }
-  __syncthreads();
-  __shared__ float pscale_s;
-  if (threadIdx.x < 30) {
-    double s = 0.0;
-    for (int g2 = 0; g2 < G; ++g2) s += part[g2][threadIdx.x];
-    const double n = (double)(d.n > 0 ? d.n : 1);
-    sc[threadIdx.x] = rsq(1e-5f + (float)(s / n));
-    if (threadIdx.x == 2) {   // channel 2 is the parameter
-      // The LSTM of this step was fed the sum of p^2 that the previous step's apply items carried over; `s` is
-      // the same sum over the parameter as it stands now.  They differ (beyond the rounding of two summation
-      // orders) only if somebody else wrote the parameter in between without the plan being told: the
-      // tensor's step is poisoned (a NaN param_scale multiplies it) and the plan's flag raised rather than a
-      // step taken on stale statistics.  The flag is pinned host memory (a system-scope store of 1 + tensor).
-      // Both addresses are found behind the counters of `sync` rather than passed as arguments: the kernel's
-      // scalar registers are spilled as it is, and three more live arguments cost its hot loops 7 %.
-      const double carried = velo_guard_sums(sync, n_tensors)[it.tensor];
-      const bool ok = fabs(s - carried) <= 1e-3 * fmax(fabs(s), fabs(carried));
-      pscale_s = ok ? sqrtf((float)(s / n) + 1e-9f) : __builtin_nanf("");
-      if (!ok) __hip_atomic_store(velo_guard_flag(sync, n_tensors), it.tensor + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-  }
-  __syncthreads();
-  const float* wm = wmix + (size_t)it.tensor * 160;
-  if (threadIdx.x < kVFold)
-    coh_store_wait(wfold + (size_t)it.tensor * kVFold + threadIdx.x,
-                   velo_fold_entry(d, wm, sc, pscale_s, wm[kVBank], threadIdx.x));
+  velo_fold_tensor<true>(d, it.tensor, stats_part + (size_t)d.blk0 * kStatW, d.nblk, wmix, wfold, sync, n_tensors);
   __syncthreads();   // every folded weight has been performed
   if (threadIdx.x == 0) __hip_atomic_store(sync + n_tensors + it.tensor, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -91,9 +91,13 @@ struct NsBatch { int mat0, n_mats, group0, n_groups; long long plane_elems; };
 
 constexpr int kNsSmallClasses = 4;
 struct Layout {
-  std::vector<Item> mx_items;   // ELO-CELO2: statistics and apply items in slab order (k_celo2_elem)
+  std::vector<Item> mx_items;   // ELO-CELO2, VeLO: statistics and apply items in slab order (k_celo2_elem, k_velo_elem)
+  bool fused = false;           // ... whatever tensors are in them
+  // ... and the streamed tensors: their blocks, the same last to first, the segments of their rows of sums, and the tensors
+  std::vector<Item> big_items, big_apply, big_seg;
+  std::vector<int> big_list;
   bool split = false;           // element blocks smaller than 8192 elements (split_for)
-  size_t off_mx_items = 0, off_sync = 0;
+  size_t off_mx_items = 0, off_big_items = 0, off_big_apply = 0, off_big_seg = 0, off_big_list = 0, off_sync = 0;
   size_t off_newsum = 0, off_piv = 0, off_wmix = 0;   // VeLO: sums carried to the next step, pivots, un-folded MLPs
   // ELO-CELO2: Newton-Schulz on the 2-D tensors (k_ns.h)
   std::vector<NsMat> ns_mats;
@@ -223,9 +227,10 @@ int tile_rows_for(int kind, int split) {
 }
 
 // Items of k_celo2_elem.  Slabs are runs of whole tensors, last tensors first (their gradients are what
-// k_p0 read last).  A tensor too large to stay cached is streamed: its statistics items are cut into
-// slab-sized pieces (so that the apply items of the slabs before it keep their place two pieces behind),
-// and its apply items follow its last piece, last item first: they start on what was read last.
+// k_p0 read last).  A tensor too large to stay cached gains nothing from one launch and pays for the hand-over in every block (the
+// memory-side round trips of its sums, of the flag and of the weights): its statistics are a launch of the plain kernel in
+// front of this one and its apply items one behind it, last item first, since they start on what was read last.  VeLO on one tensor of
+// 131 M elements 1704 / 1519 us.
 void build_elem_items(Layout& L, int T, int kind) {
   struct Piece { int st0, st1, ap0, ap1; bool keep; };   // statistics items [st0, st1); apply items [ap0, ap1) or none
   const long long cap = env_slab_elems(), keep_max = env_keep_elems();
@@ -241,15 +246,15 @@ void build_elem_items(Layout& L, int T, int kind) {
   for (int t = T - 1; t >= 0; --t) {
     const TDesc& d = L.descs[t];
     if (d.nblk == 0) continue;
-    if (d.n > keep_max) {
-      close();
-      const long long per_item = std::max<long long>(d.n / d.nblk, 1);
-      const int step = (int)std::max<long long>(cap / per_item, 1);
-      for (int i = d.blk0; i < d.blk0 + d.nblk; i += step) {
-        const int e = std::min(i + step, d.blk0 + d.nblk);
-        const bool last = e == d.blk0 + d.nblk;
-        pieces.push_back(Piece{i, e, last ? d.blk0 : 0, last ? d.blk0 + d.nblk : 0, false});
-      }
+    if (d.n > keep_max) close();   // a run of items has no gaps
+    if (d.n > keep_max && d.mode != kModeFlat) {
+      L.big_list.push_back(t);
+      for (int i = d.blk0; i < d.blk0 + d.nblk; ++i) L.big_items.push_back(L.el_items[i]);
+      for (int i = d.seg0; i < d.seg0 + d.nseg; ++i) L.big_seg.push_back(L.seg_items[i]);
+      continue;
+    }
+    if (d.n > keep_max) {   // AdamW: finished by what would be its statistics items, which nobody waits for
+      pieces.push_back(Piece{d.blk0, d.blk0 + d.nblk, 0, 0, false});
       continue;
     }
     if (elems > 0 && elems + d.n > cap) close();
@@ -258,9 +263,10 @@ void build_elem_items(Layout& L, int T, int kind) {
     elems += d.n;
   }
   close();
+  L.fused = true;
+  L.big_apply.assign(L.big_items.rbegin(), L.big_items.rend());
   const int np = (int)pieces.size(), depth = env_slab_depth(kind);
   auto push = [&](int i0, int i1, bool apply, bool keep) {
-    const int n0 = (int)L.mx_items.size();
     for (int i = i0; i < i1; ++i) {
       Item it = L.el_items[i];
       if (apply && L.descs[it.tensor].mode == kModeFlat) continue;   // AdamW tensors are finished by their statistics items
@@ -268,7 +274,6 @@ void build_elem_items(Layout& L, int T, int kind) {
       it.c = apply ? kElemApply : (keep ? kElemKeep : 0);
       L.mx_items.push_back(it);
     }
-    if (apply && !keep) std::reverse(L.mx_items.begin() + n0, L.mx_items.end());
   };
   for (int k = 0; k < np + depth; ++k) {
     if (k < np) push(pieces[k].st0, pieces[k].st1, false, pieces[k].keep);
@@ -1252,7 +1257,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
     d.nblk = (int)L.el_items.size() - d.blk0;
     if (d.nblk > kSegMin) {  // two-stage reduction of the statistics partials (k_stat_segsum)
       d.seg0 = (int)L.seg_items.size();
-      for (int r = 0; r < d.nblk; r += kSegRows) L.seg_items.push_back(Item{t, r, std::min(kSegRows, d.nblk - r), 0});
+      for (int r = 0; r < d.nblk; r += kSegRows) L.seg_items.push_back(Item{t, r, std::min(kSegRows, d.nblk - r), (int)L.seg_items.size()});
       d.nseg = (int)L.seg_items.size() - d.seg0;
     }
     // blocks of AdafacLO's apply pass: one column per lane where the tensor allows it (ap_items,
@@ -1299,6 +1304,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
     const long long chunk = L.lin_matrix ? (long long)kThreads * trips : (long long)kThreads * L.descs[t].vec * kElemIters;
     for (long long c = 0; c * chunk < L.descs[t].n; ++c) L.ga_items.push_back(Item{t, (int)c, L.lin_matrix ? trips : 0, 0});
   }
+  for (int i = 0; i < (int)L.el_items.size(); ++i) L.el_items[i].b = i;   // rows of the partial sums
   if (kind == PYLO_KIND_CELO2 || kind == PYLO_KIND_VELO) build_elem_items(L, T, kind);
   long long ns_floats = 0;
   if (kind == PYLO_KIND_CELO2) {
@@ -1377,6 +1383,10 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
   L.off_canon = take(kind == PYLO_KIND_VELO ? sizeof(float) * kVCanon * (size_t)T : 0);
   L.off_frac = take(kind == PYLO_KIND_VELO ? sizeof(float) * 9 * PYLO_MAX_GROUPS : 0);
   L.off_mx_items = take(sizeof(Item) * L.mx_items.size());
+  L.off_big_items = take(sizeof(Item) * L.big_items.size());
+  L.off_big_apply = take(sizeof(Item) * L.big_apply.size());
+  L.off_big_seg = take(sizeof(Item) * L.big_seg.size());
+  L.off_big_list = take(sizeof(int) * L.big_list.size());
   // (VeLO: behind the counters, the guard of the carried sums: flag address, padding, T doubles -- k_velo.h)
   L.off_sync = take(sizeof(int) * (size_t)((2 * T + 3) & ~3) + (kind == PYLO_KIND_VELO ? 16 + sizeof(double) * (size_t)T : 0));
   L.off_newsum = take(kind == PYLO_KIND_VELO ? sizeof(double) * kNewSumW * L.el_items.size() : 0);
@@ -1510,6 +1520,10 @@ int pylo_mi355_plan_create(int kind, const PyloTensorShape* shapes, int n_tensor
   if (e == hipSuccess) e = up(L.off_v0a_items, L.v0a_items.data(), sizeof(Item) * L.v0a_items.size());
   if (e == hipSuccess) e = up(L.off_v0b_items, L.v0b_items.data(), sizeof(Item) * L.v0b_items.size());
   if (e == hipSuccess) e = up(L.off_mx_items, L.mx_items.data(), sizeof(Item) * L.mx_items.size());
+  if (e == hipSuccess) e = up(L.off_big_items, L.big_items.data(), sizeof(Item) * L.big_items.size());
+  if (e == hipSuccess) e = up(L.off_big_apply, L.big_apply.data(), sizeof(Item) * L.big_apply.size());
+  if (e == hipSuccess) e = up(L.off_big_seg, L.big_seg.data(), sizeof(Item) * L.big_seg.size());
+  if (e == hipSuccess) e = up(L.off_big_list, L.big_list.data(), sizeof(int) * L.big_list.size());
   if (e == hipSuccess) e = up(L.off_ns_mats, L.ns_mats.data(), sizeof(NsMat) * L.ns_mats.size());
   if (e == hipSuccess) e = up(L.off_ns_gram, L.ns_gram.data(), sizeof(NsItem) * L.ns_gram.size());
   if (e == hipSuccess) e = up(L.off_ns_poly, L.ns_poly.data(), sizeof(NsItem) * L.ns_poly.size());
@@ -1551,7 +1565,7 @@ int pylo_mi355_plan_create(int kind, const PyloTensorShape* shapes, int n_tensor
       if (e == hipSuccess) e = hipStreamSynchronize(s);
     }
   }
-  if (e == hipSuccess && kind == PYLO_KIND_VELO && !P->L.mx_items.empty()) {
+  if (e == hipSuccess && kind == PYLO_KIND_VELO && P->L.fused) {
     e = hipStreamCreateWithFlags(&P->side, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&P->ev_fork, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&P->ev_join, hipEventDisableTiming);
@@ -1616,9 +1630,9 @@ static const char* kAdafacLaunches[] = {"k_p0(sums)", "k_p0_nd", "k_v0a", "k_ada
 
 int pylo_mi355_plan_num_launches(const PyloPlan* P) {
   if (!P) return -1;
-  const int n_celo2 = P->L.mx_items.empty() ? (int)(sizeof(kCelo2Launches) / sizeof(kCelo2Launches[0]))
+  const int n_celo2 = !P->L.fused ? (int)(sizeof(kCelo2Launches) / sizeof(kCelo2Launches[0]))
                                             : (int)(sizeof(kCelo2FusedLaunches) / sizeof(kCelo2FusedLaunches[0]));
-  const int n_velo = P->L.mx_items.empty() ? (int)(sizeof(kVeloLaunches) / sizeof(kVeloLaunches[0]))
+  const int n_velo = !P->L.fused ? (int)(sizeof(kVeloLaunches) / sizeof(kVeloLaunches[0]))
                                            : (int)(sizeof(kVeloFusedLaunches) / sizeof(kVeloFusedLaunches[0]));
   constexpr int n_adafac = sizeof(kAdafacLaunches) / sizeof(kAdafacLaunches[0]);
   return P->kind == PYLO_KIND_CELO2 ? n_celo2 : P->kind == PYLO_KIND_VELO ? n_velo : P->kind == PYLO_KIND_ADAFAC ? n_adafac : -1;
@@ -1626,8 +1640,8 @@ int pylo_mi355_plan_num_launches(const PyloPlan* P) {
 
 const char* pylo_mi355_plan_launch_name(const PyloPlan* P, int launch) {
   if (!P || launch < 0 || launch >= pylo_mi355_plan_num_launches(P)) return "";
-  return P->kind == PYLO_KIND_CELO2 ? (P->L.mx_items.empty() ? kCelo2Launches[launch] : kCelo2FusedLaunches[launch])
-         : P->kind == PYLO_KIND_VELO ? (P->L.mx_items.empty() ? kVeloLaunches[launch] : kVeloFusedLaunches[launch])
+  return P->kind == PYLO_KIND_CELO2 ? (!P->L.fused ? kCelo2Launches[launch] : kCelo2FusedLaunches[launch])
+         : P->kind == PYLO_KIND_VELO ? (!P->L.fused ? kVeloLaunches[launch] : kVeloFusedLaunches[launch])
                                      : kAdafacLaunches[launch];
 }
 
@@ -1862,7 +1876,7 @@ struct Marks {  // per-launch HIP events when timing is on
     const bool timed = P->timing && P->t_steps < P->t_steps_max;
     ev = timed ? &P->tev[(size_t)P->t_steps * P->t_per_step] : nullptr;
   }
-  hipError_t operator()() { return ev ? hipEventRecord(ev[mark++], s) : hipSuccess; }
+  hipError_t operator()(bool skip = false) { return ev && !skip ? hipEventRecord(ev[mark++], s) : hipSuccess; }
   void done() { if (ev) P->t_steps++; }
 };
 
@@ -1942,35 +1956,43 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
     hipLaunchKernelGGL(v0b, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, v0part, 1e-9f, mlp,
                        mlp + 240, 0, fac_tab, term_tab, bscale);
   HIP_TRY(mark());
-  const int n_mx = (int)L.mx_items.size();
-  if (n_mx > 0) {
+  auto apply_items = [&](const Item* items, int n) {   // the apply pass as a launch of its own
+    const auto apply = in_place                ? (L.split ? k_celo2_apply<true, true, true> : k_celo2_apply<true, true, false>)
+                       : P->mlp_on_matrix_pipe ? (L.split ? k_celo2_apply<true, false, true> : k_celo2_apply<true, false, false>)
+                                               : (L.split ? k_celo2_apply<false, false, true> : k_celo2_apply<false, false, false>);
+    hipLaunchKernelGGL(apply, dim3(n), dim3(kThreads), 0, s, descs, dyn, items, fac_tab, term_tab, gl, dec, wfold);
+  };
+  const auto stats_pass = variant(in_place, L.split, k_celo2_stats<false, false>, k_celo2_stats<false, true>,
+                                  k_celo2_stats<true, false>, k_celo2_stats<true, true>);
+  // statistics and folded weights of n_fac tensors as launches of their own
+  auto stats_items = [&](const Item* items, int n, const Item* seg, int n_seg, const int* list, int n_fac) {
+    double* seg_tot = P->at<double>(L.off_segtot);
+    if (n > 0) hipLaunchKernelGGL(stats_pass, dim3(n), dim3(kThreads), 0, s, descs, dyn, items, fac_tab, gl, dec, stats);
+    HIP_TRY(mark(L.fused));
+    if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3(n_seg), dim3(kThreads), 0, s, descs, seg, stats, seg_tot);
+    if (n_fac > 0)
+      hipLaunchKernelGGL(k_celo2_fold, dim3(n_fac), dim3(kFoldThreads), 0, s, descs, dyn, list, stats, seg_tot, mlp, wfold, chan_ms);
+    HIP_TRY(mark(L.fused));
+    return 0;
+  };
+  const int n_mx = (int)L.mx_items.size(), n_big = (int)L.big_items.size();
+  if (L.fused) {
+    if (n_big > 0)
+      if (int rc = stats_items(P->at<Item>(L.off_big_items), n_big, P->at<Item>(L.off_big_seg), (int)L.big_seg.size(),
+                               P->at<int>(L.off_big_list), (int)L.big_list.size())) return rc;
     const Item* mx_items = P->at<Item>(L.off_mx_items);
     int* sync = P->at<int>(L.off_sync);
     const auto elem = in_place              ? (L.split ? k_celo2_elem<true, true, true> : k_celo2_elem<true, false, true>)
                       : P->mlp_on_matrix_pipe ? (L.split ? k_celo2_elem<true, true> : k_celo2_elem<true, false>)
                                               : (L.split ? k_celo2_elem<false, true> : k_celo2_elem<false, false>);
-    hipLaunchKernelGGL(elem, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, mx_items, fac_tab, term_tab, gl, dec, mlp,
-                       wfold, chan_ms, stats, sync, P->T);
+    if (n_mx > 0)
+      hipLaunchKernelGGL(elem, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, mx_items, fac_tab, term_tab, gl, dec, mlp,
+                         wfold, chan_ms, stats, sync, P->T);
+    if (n_big > 0) apply_items(P->at<Item>(L.off_big_apply), n_big);
     HIP_TRY(mark());
   } else {
-    const auto stats_pass = variant(in_place, L.split, k_celo2_stats<false, false>, k_celo2_stats<false, true>,
-                                    k_celo2_stats<true, false>, k_celo2_stats<true, true>);
-    if (n_el > 0) hipLaunchKernelGGL(stats_pass, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, gl, dec, stats);
-    HIP_TRY(mark());
-    const Item* seg_items = P->at<Item>(L.off_seg_items);
-    double* seg_tot = P->at<double>(L.off_segtot);
-    const int n_seg = (int)L.seg_items.size();
-    if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3(n_seg), dim3(kThreads), 0, s, descs, seg_items, stats, seg_tot);
-    if (n_fac > 0)
-      hipLaunchKernelGGL(k_celo2_fold, dim3(n_fac), dim3(kFoldThreads), 0, s, descs, dyn, fac_list, stats, seg_tot, mlp, wfold,
-                         chan_ms);
-    HIP_TRY(mark());
-    if (n_el > 0) {
-      const auto apply = in_place                ? (L.split ? k_celo2_apply<true, true, true> : k_celo2_apply<true, true, false>)
-                         : P->mlp_on_matrix_pipe ? (L.split ? k_celo2_apply<true, false, true> : k_celo2_apply<true, false, false>)
-                                                 : (L.split ? k_celo2_apply<false, false, true> : k_celo2_apply<false, false, false>);
-      hipLaunchKernelGGL(apply, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, term_tab, gl, dec, wfold);
-    }
+    if (int rc = stats_items(el_items, n_el, P->at<Item>(L.off_seg_items), (int)L.seg_items.size(), fac_list, n_fac)) return rc;
+    if (n_el > 0) apply_items(el_items, n_el);
   }
   if (n_sl > 0)
     hipLaunchKernelGGL(k_celo2_slices, dim3(n_sl), dim3(kThreads), 0, s, descs, dyn, sl_items, fac_tab, gl, dec, mlp);
@@ -2512,7 +2534,7 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   };
   const int n_mx = (int)L.mx_items.size();
   HIP_TRY(mark());
-  if (n_mx > 0 && P->stats_carried) {
+  if (L.fused && P->stats_carried) {
     // The LSTM's inputs are sums over the parameters and accumulators as they stand before the step: the
     // previous step's apply items left them.  It runs next to the gradient sums, on the plan's own stream.
     HIP_TRY(hipEventRecord(P->ev_fork, s));
@@ -2534,9 +2556,24 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
     if (n_v0b > 0)
       hipLaunchKernelGGL(k_terms<4>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, bscale, canon, kVCanon, term_tab);
     HIP_TRY(mark());
+    const unsigned n_big = (unsigned)L.big_items.size();
+    if (n_big > 0) {
+      hipLaunchKernelGGL((L.split ? k_velo_stats<false, true> : k_velo_stats<false, false>), dim3(n_big), dim3(kThreads), 0, s, descs, dyn, P->at<Item>(L.off_big_items), fac_tab,
+                         dec, stats);
+      if (!L.big_seg.empty())
+        hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3((unsigned)L.big_seg.size()), dim3(kThreads), 0, s, descs,
+                           P->at<Item>(L.off_big_seg), (const double*)stats, P->at<double>(L.off_segtot));
+      hipLaunchKernelGGL(k_velo_fold, dim3((unsigned)L.big_list.size()), dim3(kThreads), 0, s, descs, dyn, P->at<int>(L.off_big_list),
+                         (const double*)stats, (const double*)P->at<double>(L.off_segtot), (const float*)wmix, wfold,
+                         P->at<int>(L.off_sync), T);
+    }
     const auto elem = L.split ? k_velo_elem<true> : k_velo_elem<false>;
-    hipLaunchKernelGGL(elem, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, P->at<Item>(L.off_mx_items), fac_tab, term_tab,
-                       dec, (const float*)wmix, wfold, stats, (const float*)piv, newsum, P->at<int>(L.off_sync), T);
+    if (n_mx > 0)
+      hipLaunchKernelGGL(elem, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, P->at<Item>(L.off_mx_items), fac_tab, term_tab,
+                         dec, (const float*)wmix, wfold, stats, (const float*)piv, newsum, P->at<int>(L.off_sync), T);
+    if (n_big > 0)
+      hipLaunchKernelGGL((L.split ? k_velo_apply<false, true> : k_velo_apply<false, false>), dim3(n_big), dim3(kThreads), 0, s, descs, dyn, P->at<Item>(L.off_big_apply), fac_tab,
+                         term_tab, dec, (const float*)wfold, (const float*)piv, newsum);
     HIP_TRY(mark());
     mark.done();
     stage_out(P, s, 0);
@@ -2547,22 +2584,22 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   // invalidated, and every step with PYLO_MI355_SLAB_ELEMS=0.
   gradient_sums();
   HIP_TRY(mark());
-  if (n_mx == 0) HIP_TRY(mark());
+  HIP_TRY(mark(L.fused));
   if (int rc = factor_tables()) return rc;
   const auto stats_pass = variant(typed, L.split, k_velo_stats<false, false>, k_velo_stats<false, true>, k_velo_stats<true, false>,
                                   k_velo_stats<true, true>);
   const auto apply_pass = variant(typed, L.split, k_velo_apply<false, false>, k_velo_apply<false, true>, k_velo_apply<true, false>,
                                   k_velo_apply<true, true>);
   if (n_el > 0) hipLaunchKernelGGL(stats_pass, dim3(n_el), dim3(kThreads), 0, s, descs, dyn, el_items, fac_tab, dec, stats);
-  if (n_mx == 0) HIP_TRY(mark());
+  HIP_TRY(mark(L.fused));
   const Item* seg_items = P->at<Item>(L.off_seg_items);
   double* seg_tot = P->at<double>(L.off_segtot);
   const int n_seg = (int)L.seg_items.size();
   if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3(n_seg), dim3(kThreads), 0, s, descs, seg_items, stats, seg_tot);
   hipLaunchKernelGGL(k_lo_reduce, dim3(T), dim3(kFoldThreads), 0, s, descs, dyn, T, stats, seg_tot, totals, ls, vs, xfeat,
                      H, nets->mix2_wt, nets->mix2_b, nets->fmix_wt, nets->fmix_b, mixbuf, piv);
-  if (n_mx == 0) HIP_TRY(mark());
-  lstm(s, totals, n_mx == 0);   // the LSTM's launches have intervals of their own only in the launch list without k_velo_elem
+  HIP_TRY(mark(L.fused));
+  lstm(s, totals, !L.fused);   // the LSTM's launches have intervals of their own only in the launch list without k_velo_elem
   if (n_v0b > 0)
     hipLaunchKernelGGL(k_terms<4>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, bscale, canon, kVCanon, term_tab);
   HIP_TRY(mark());
@@ -2573,7 +2610,7 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   mark.done();
   stage_out(P, s, 0);
   HIP_TRY(hipGetLastError());
-  P->stats_carried = n_mx > 0;
+  P->stats_carried = L.fused;
   return 0;
 }
 
