@@ -20,6 +20,7 @@ constexpr int kVCanon = 128;   // per-tensor un-scaled first layer (30,4) + bias
 constexpr int kVBank = 159;    // floats per bank entry: W_in (4,30) | b_in 4 | W_h (4,4) | b_h 4 | W_out (3,4) | b_out 3
 constexpr int kXW = 32;        // row pitch of the LSTM input features (30 used)
 constexpr int kGateBT = 8;     // tensors per k_velo_gates block
+constexpr int kManyRows = 768; // tensors from which the LSTM's products are k_velo_gates_many's and its heads four rows a block
 
 struct LossState {             // by-value kernel argument: the caller's loss accumulators (PyloVeloStep)
   float* means;
@@ -815,6 +816,123 @@ __global__ __launch_bounds__(kThreads) void k_velo_gates(const float* __restrict
   }
 }
 
+// The same for many tensors, as fp32 matrix products (v_mfma_f32_32x32x2_f32): a block takes 64 tensors x 32 units (128 gate columns), its
+// four waves 32 tensors x 64 columns each.  The gate columns are the M side, so that the four gates of a unit are consecutive
+// accumulators of a lane (row 8 (r / 4) + 4 (lane / 32) + r % 4: unit 2 (r / 4) + lane / 32, gate r % 4) and the cell is worked out
+// where they are.  16 inputs a stage through LDS, the next stage's loads in flight; rows padded by 32 floats, so that the two inputs
+// of an instruction come from different halves of the banks.  Sums as in k_velo_gates: 64 inputs, then the sixteen of them.
+// Bound by the fp32 matrix pipe: 12.6 GFLOP at 3001 tensors, 80 us at its peak.  k_velo_gates reads the weights again for every
+// eight tensors.  By themselves, that one / this: 256 tensors 24 us, 512 42 / 59, 1024 80 / 62, 2000 152 / 103; next to k_p0 at 3001
+// 383 / 187.  (k_velo_heads, a row / four rows a block: 512 19 / 21 us, 1024 43 / 49, 2000 85 / 59.)
+constexpr int kGateM = 64, kGateMU = 32, kGateMK = 16;   // tensors and units a block, inputs a stage
+__global__ __launch_bounds__(kThreads) void k_velo_gates_many(const float* __restrict__ xT, int T, int Tpad, int H,
+                                                              const float* __restrict__ wt /*(2H, H, 4)*/, const float* __restrict__ b /*4H*/,
+                                                              float* __restrict__ h_state, float* __restrict__ c_state) {
+  constexpr int PX = kGateM + 32, PW = 4 * kGateMU + 32, PC = kGateMU + 1;
+  constexpr int kStage = kGateMK * (PX + PW);
+  static_assert(2 * kGateM * PC <= 2 * kStage, "the cell states take the stages' place");
+  __shared__ __attribute__((aligned(16))) float lds[2 * kStage];
+  const int n_ub = H / kGateMU;
+  int ub, rb;
+  if (n_ub % 8 == 0) {   // as k_velo_gates: the blocks of an XCD share their units' weights
+    const int per = n_ub / 8, xcd = blockIdx.x % 8, j = blockIdx.x / 8;
+    ub = xcd * per + j % per;
+    rb = j / per;
+  } else {
+    ub = blockIdx.x % n_ub;
+    rb = blockIdx.x / n_ub;
+  }
+  const int u0 = ub * kGateMU, r0 = rb * kGateM;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int el = lane & 31, half = lane >> 5, wr = (wave & 1) * 32, wc = (wave >> 1) * 64;
+  const int K2 = 2 * H;
+  // a stage: 16 x 64 inputs (a 16-byte piece a thread) and 16 x 128 weights (two); Tpad is a multiple of eight
+  constexpr int NX = kGateMK * kGateM / 4 / kThreads, NW = kGateMK * kGateMU / kThreads;
+  float4 px[NX], pw[NW];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int q = 0; q < NX; ++q) {
+      const int i = q * kThreads + threadIdx.x, k = i / 16, c = i % 16 * 4;
+      px[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (r0 + c < Tpad) px[q] = load_f4(xT + (size_t)(k0 + k) * Tpad + r0 + c);
+    }
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+      const int i = q * kThreads + threadIdx.x, k = i / 32, c = i % 32 * 4;
+      pw[q] = load_f4(wt + ((size_t)(k0 + k) * H + u0) * 4 + c);
+    }
+  };
+  auto stage = [&](float* to) {
+#pragma unroll
+    for (int q = 0; q < NX; ++q) {
+      const int i = q * kThreads + threadIdx.x;
+      *(float4*)(to + i / 16 * PX + i % 16 * 4) = px[q];
+    }
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+      const int i = q * kThreads + threadIdx.x;
+      *(float4*)(to + kGateMK * PX + i / 32 * PW + i % 32 * 4) = pw[q];
+    }
+  };
+  typedef float f32x16 __attribute__((ext_vector_type(16)));
+  f32x16 sum[2], acc[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sum[t][i] = acc[t][i] = 0.0f;
+  fetch(0);
+  for (int k0 = 0, u = 0; k0 < K2; k0 += kGateMK, u ^= 1) {
+    float* const at = lds + u * kStage;
+    stage(at);
+    __syncthreads();     // the other stage's readers are past it: a wave is at most one barrier behind
+    if (k0 + kGateMK < K2) fetch(k0 + kGateMK);
+    const float *x = at + half * PX + wr + el, *w = at + kGateMK * PX + half * PW + wc + el;
+#pragma unroll
+    for (int k = 0; k < kGateMK; k += 2) {
+      const float xv = x[k * PX];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[k * PW + 32 * t], xv, acc[t], 0, 0, 0);
+    }
+    if ((k0 & 63) == 64 - kGateMK) {   // 64 inputs (K2 is a multiple of 128)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          sum[t][i] += acc[t][i];
+          acc[t][i] = 0.0f;
+        }
+    }
+  }
+  __syncthreads();
+  // cell states [tensor][unit], in and out through LDS
+  float (*cs)[PC] = reinterpret_cast<float (*)[PC]>(lds);
+  float (*hs)[PC] = reinterpret_cast<float (*)[PC]>(lds + kGateM * PC);
+  for (int i = threadIdx.x; i < kGateM * kGateMU; i += kThreads) {
+    const int t = i / kGateMU, j = i % kGateMU;
+    cs[t][j] = r0 + t < T ? c_state[(size_t)(r0 + t) * H + u0 + j] : 0.0f;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int j = wc / 4 + 8 * t + 2 * q + half;
+      float gate[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) gate[g] = b[g * H + u0 + j] + sum[t][4 * q + g];
+      const float c_new = sigmoidf_(gate[2] + 1.0f) * cs[wr + el][j] + sigmoidf_(gate[0]) * tanhf(gate[1]);
+      cs[wr + el][j] = c_new;
+      hs[wr + el][j] = sigmoidf_(gate[3]) * tanhf(c_new);
+    }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kGateM * kGateMU; i += kThreads) {
+    const int t = i / kGateMU, j = i % kGateMU;
+    if (r0 + t >= T) continue;
+    c_state[(size_t)(r0 + t) * H + u0 + j] = cs[t][j];
+    h_state[(size_t)(r0 + t) * H + u0 + j] = hs[t][j];
+  }
+}
+
 // Entry i of a tensor's folded weight block (layout at the top of this file) from its un-scaled MLP `wm`
 // (a bank entry's layout, kVBank floats), the channel normalisers sc[30], param_scale and lr_mult.
 // Entries the layout leaves unused read as zero.
@@ -836,11 +954,13 @@ __device__ __forceinline__ float velo_fold_entry(const TDesc& d, const float* wm
   return 0.0f;
 }
 
-// One block per tensor row r: controls = h Wc^T + bc, lr_mult = h.wlr + blr, the tensor's MLP =
+// R tensor rows a block (four where there are many: a block reads 0.7 MB of weights; in blocks of four waves there, which find a place
+// next to launches that fill the chip where blocks of sixteen wait: next to k_velo_stats on a streamed tensor 524 us and 102; by themselves 1024 tensors 24 and 49, 2000 55 and 59), each: controls = h Wc^T + bc, lr_mult = h.wlr + blr, the tensor's MLP =
 // 100 * mean_i(control_i * bank_i) (VeLO_MLP.py:92-126), then the weight blocks the element
 // kernels read: un-scaled first layer for k_terms, and the folded block (first-layer rows scaled
 // by rsqrt(1e-5 + mean f_c^2), param_scale = sqrt(mean p^2 + 1e-9), lr_mult).
-__global__ __launch_bounds__(kFoldThreads) void k_velo_heads(const TDesc* __restrict__ descs, int T, int H, int K,
+template <int R, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_velo_heads(const TDesc* __restrict__ descs, int T, int H, int K,
                                                              const float* __restrict__ h_state,
                                                              const float* __restrict__ wct /*(H,K)*/,
                                                              const float* __restrict__ bc, const float* __restrict__ wlr,
@@ -858,60 +978,68 @@ __global__ __launch_bounds__(kFoldThreads) void k_velo_heads(const TDesc* __rest
   // into four slices that run side by side and are added in a fixed order; eight loads are issued
   // before the first is used, since a block is bound by the bytes it keeps in flight.
   constexpr int kSl = 4;
-  extern __shared__ float smem[];  // hs[H] | ctrl[K] | wm[160] | sc[32] | red[16] | part[kSl][max(K,160)]
-  float* hs = smem;
-  float* ctrl = hs + H;
-  float* wm = ctrl + K;
-  float* sc = wm + 160;
-  float* red = sc + 32;
-  float* part = red + 16;
+  extern __shared__ float smem[];  // R times: hs[H] | ctrl[K] | wm[160] | sc[32] | red[16] | part[kSl][max(K,160)]
+  float* hs = smem;                 // [R][H] ...
+  float* ctrl = hs + R * H;
+  float* wm = ctrl + R * K;
+  float* sc = wm + R * 160;
+  float* red = sc + R * 32;
+  float* part = red + R * 16;       // [kSl][R][pitch]
   const int pitch = K > 160 ? K : 160;
-  const int r = blockIdx.x;
-  const int t = T - 1 - r;
-  const TDesc d = descs[t];
-  for (int u = threadIdx.x; u < H; u += kFoldThreads) hs[u] = h_state[(size_t)r * H + u];
+  const int row0 = blockIdx.x * R;
+#pragma unroll
+  for (int q = 0; q < R; ++q)       // rows past the last: the last one again, not written
+    for (int u = threadIdx.x; u < H; u += THREADS) hs[q * H + u] = h_state[(size_t)min(row0 + q, T - 1) * H + u];
   __syncthreads();
-  for (int i = threadIdx.x; i < K * kSl; i += kFoldThreads) {
+  for (int i = threadIdx.x; i < K * kSl; i += THREADS) {
     const int j = i % K, sl = i / K;
     const int u0 = sl * (H / kSl), u1 = u0 + H / kSl;  // H is a multiple of 64
-    float acc = 0.0f;
+    float acc[R] = {};
     for (int u = u0; u < u1; u += 8) {
       float w[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) w[q] = wct[(size_t)(u + q) * K + j];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) acc = fmaf(hs[u + q], w[q], acc);
+      for (int q = 0; q < 8; ++q)
+#pragma unroll
+        for (int p = 0; p < R; ++p) acc[p] = fmaf(hs[p * H + u + q], w[q], acc[p]);
     }
-    part[sl * pitch + j] = acc;
+#pragma unroll
+    for (int p = 0; p < R; ++p) part[(sl * R + p) * pitch + j] = acc[p];
   }
-  {
+#pragma unroll
+  for (int p = 0; p < R; ++p) {
     float s = 0.0f;
-    for (int u = threadIdx.x; u < H; u += kFoldThreads) s = fmaf(hs[u], wlr[u], s);
+    for (int u = threadIdx.x; u < H; u += THREADS) s = fmaf(hs[p * H + u], wlr[u], s);
     s = wave_sum(s);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    if ((threadIdx.x & 63) == 0) red[p * 16 + (threadIdx.x >> 6)] = s;
   }
-  if (threadIdx.x < 30 && totals != nullptr) {
-    const double n = (double)(d.n > 0 ? d.n : 1);
-    sc[threadIdx.x] = rsq(1e-5f + (float)(totals[(size_t)t * kStatW + threadIdx.x] / n));
+  if (threadIdx.x < 32 * R && (threadIdx.x & 31) < 30 && totals != nullptr) {
+    const int t = max(T - 1 - row0 - (int)(threadIdx.x >> 5), 0);
+    const double n = (double)(descs[t].n > 0 ? descs[t].n : 1);
+    sc[threadIdx.x] = rsq(1e-5f + (float)(totals[(size_t)t * kStatW + (threadIdx.x & 31)] / n));
   }
   __syncthreads();
-  for (int j = threadIdx.x; j < K; j += kFoldThreads) {
-    const float acc = bc[j] + ((part[j] + part[pitch + j]) + (part[2 * pitch + j] + part[3 * pitch + j]));
-    ctrl[j] = acc;
-    if (controls_out != nullptr) controls_out[(size_t)r * K + j] = acc;
+  for (int i = threadIdx.x; i < R * K; i += THREADS) {
+    const int p = i / K, j = i % K;
+    const float* o = part + p * pitch + j;
+    const float acc = bc[j] + ((o[0] + o[R * pitch]) + (o[2 * R * pitch] + o[3 * R * pitch]));
+    ctrl[i] = acc;
+    if (controls_out != nullptr && row0 + p < T) controls_out[(size_t)(row0 + p) * K + j] = acc;
   }
-  float lr_mult = blr[0];
-  {
+  float lr_mult[R];
+#pragma unroll
+  for (int p = 0; p < R; ++p) {
     float s = 0.0f;
 #pragma unroll
-    for (int w = 0; w < kFoldThreads / 64; ++w) s += red[w];
-    lr_mult += s;
+    for (int w = 0; w < THREADS / 64; ++w) s += red[p * 16 + w];
+    lr_mult[p] = blr[0] + s;
   }
   __syncthreads();
   const int Kq = (K + kSl - 1) / kSl;
-  for (int i = threadIdx.x; i < 160 * kSl; i += kFoldThreads) {
+  for (int i = threadIdx.x; i < 160 * kSl; i += THREADS) {
     const int q = i % 160, sl = i / 160;
-    float acc = 0.0f;
+    float acc[R] = {};
     if (q < kVBank) {
       const int i0 = sl * Kq, i1 = min(K, i0 + Kq);
       int c = i0;
@@ -920,31 +1048,46 @@ __global__ __launch_bounds__(kFoldThreads) void k_velo_heads(const TDesc* __rest
 #pragma unroll
         for (int e = 0; e < 8; ++e) b8[e] = bank[(size_t)(c + e) * kVBank + q];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc = fmaf(ctrl[c + e], b8[e], acc);
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int p = 0; p < R; ++p) acc[p] = fmaf(ctrl[p * K + c + e], b8[e], acc[p]);
       }
-      for (; c < i1; ++c) acc = fmaf(ctrl[c], bank[(size_t)c * kVBank + q], acc);
+      for (; c < i1; ++c)
+#pragma unroll
+        for (int p = 0; p < R; ++p) acc[p] = fmaf(ctrl[p * K + c], bank[(size_t)c * kVBank + q], acc[p]);
     }
-    part[sl * pitch + q] = acc;
+#pragma unroll
+    for (int p = 0; p < R; ++p) part[(sl * R + p) * pitch + q] = acc[p];
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < kVBank; q += kFoldThreads) {
-    const float acc = (part[q] + part[pitch + q]) + (part[2 * pitch + q] + part[3 * pitch + q]);
-    wm[q] = (acc / (float)K) * 100.0f;
+  for (int i = threadIdx.x; i < R * 160; i += THREADS) {
+    const int p = i / 160, q = i % 160;
+    if (q >= kVBank) continue;
+    const float* o = part + p * pitch + q;
+    const float acc = (o[0] + o[R * pitch]) + (o[2 * R * pitch] + o[3 * R * pitch]);
+    wm[i] = (acc / (float)K) * 100.0f;
   }
   __syncthreads();
-  float* cn = canon + (size_t)t * kVCanon;
-  for (int i = threadIdx.x; i < 124; i += kFoldThreads) cn[i] = i < 120 ? wm[(i % 4) * 30 + i / 4] : wm[i];
-  if (threadIdx.x == 0 && lr_mult_out != nullptr) lr_mult_out[r] = lr_mult;
-  if (totals == nullptr) {
-    float* o = wmix + (size_t)t * 160;
-    for (int i = threadIdx.x; i < 160; i += kFoldThreads) o[i] = i < kVBank ? wm[i] : lr_mult;
-    return;
-  }
-  const double n = (double)(d.n > 0 ? d.n : 1);
-  const float pscale = sqrtf((float)(totals[(size_t)t * kStatW + 2] / n) + 1e-9f);
-  for (int i = threadIdx.x; i < kVFold; i += kFoldThreads) {
-    const float v = velo_fold_entry(d, wm, sc, pscale, lr_mult, i);
-    if (i < kVLR + 1) wfold[(size_t)t * kVFold + i] = v;
+#pragma unroll
+  for (int p = 0; p < R; ++p) {
+    const int t = T - 1 - row0 - p;
+    if (t < 0) break;
+    const float* wp = wm + p * 160;
+    float* cn = canon + (size_t)t * kVCanon;
+    for (int i = threadIdx.x; i < 124; i += THREADS) cn[i] = i < 120 ? wp[(i % 4) * 30 + i / 4] : wp[i];
+    if (threadIdx.x == 0 && lr_mult_out != nullptr) lr_mult_out[row0 + p] = lr_mult[p];
+    if (totals == nullptr) {
+      float* o = wmix + (size_t)t * 160;
+      for (int i = threadIdx.x; i < 160; i += THREADS) o[i] = i < kVBank ? wp[i] : lr_mult[p];
+      continue;
+    }
+    const TDesc d = descs[t];
+    const double n = (double)(d.n > 0 ? d.n : 1);
+    const float pscale = sqrtf((float)(totals[(size_t)t * kStatW + 2] / n) + 1e-9f);
+    for (int i = threadIdx.x; i < kVFold; i += THREADS) {
+      const float v = velo_fold_entry(d, wp, sc + p * 32, pscale, lr_mult[p], i);
+      if (i < kVLR + 1) wfold[(size_t)t * kVFold + i] = v;
+    }
   }
 }
 

@@ -2506,10 +2506,18 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
     hipLaunchKernelGGL(k_velo_mix, dim3(H / 64, L.Tpad / kGateBT), dim3(kThreads), 0, q, (const float*)mixbuf, T, L.Tpad, H,
                        (const float*)pmax, n_chunks, step->lstm_h, xT, ls);
     if (timed) (void)mark();
-    hipLaunchKernelGGL(k_velo_gates, dim3((L.Tpad / kGateBT) * (H / kGateU)), dim3(kThreads), 0, q, xT, T, L.Tpad, H,
-                       nets->lstm_wt, nets->lstm_b, step->lstm_h, step->lstm_c);
+    const bool many = T >= kManyRows;
+    if (many)
+      hipLaunchKernelGGL(k_velo_gates_many, dim3((T + kGateM - 1) / kGateM * (H / kGateMU)), dim3(kThreads), 0, q, xT, T, L.Tpad, H,
+                         nets->lstm_wt, nets->lstm_b, step->lstm_h, step->lstm_c);
+    else
+      hipLaunchKernelGGL(k_velo_gates, dim3((L.Tpad / kGateBT) * (H / kGateU)), dim3(kThreads), 0, q, xT, T, L.Tpad, H,
+                         nets->lstm_wt, nets->lstm_b, step->lstm_h, step->lstm_c);
     if (timed) (void)mark();
-    hipLaunchKernelGGL(k_velo_heads, dim3(T), dim3(kFoldThreads), heads_lds, q, descs, T, H, K, step->lstm_h,
+    const bool rows4 = many && 4 * heads_lds <= 64 * 1024;
+    hipLaunchKernelGGL((rows4 ? k_velo_heads<4, kThreads> : k_velo_heads<1, kFoldThreads>), dim3(rows4 ? (T + 3) / 4 : T),
+                       dim3(rows4 ? kThreads : kFoldThreads),
+                       rows4 ? 4 * heads_lds : heads_lds, q, descs, T, H, K, step->lstm_h,
                        nets->ctrl_wt, nets->ctrl_b, nets->lr_w, nets->lr_b, nets->bank, tot, canon, wfold,
                        step->controls_out, step->lr_mult_out, wmix);
     if (timed) (void)mark();
@@ -2552,21 +2560,22 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
     gradient_sums();
     HIP_TRY(mark());
     if (int rc = factor_tables()) return rc;
+    // the streamed tensors' statistics need nothing from the LSTM either: its launches have this one to run under as well
+    const unsigned n_big = (unsigned)L.big_items.size();
+    if (n_big > 0)
+      hipLaunchKernelGGL((L.split ? k_velo_stats<false, true> : k_velo_stats<false, false>), dim3(n_big), dim3(kThreads), 0, s, descs, dyn,
+                         P->at<Item>(L.off_big_items), fac_tab, dec, stats);
     HIP_TRY(hipStreamWaitEvent(s, P->ev_join, 0));
     if (n_v0b > 0)
       hipLaunchKernelGGL(k_terms<4>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, bscale, canon, kVCanon, term_tab);
     HIP_TRY(mark());
-    const unsigned n_big = (unsigned)L.big_items.size();
-    if (n_big > 0) {
-      hipLaunchKernelGGL((L.split ? k_velo_stats<false, true> : k_velo_stats<false, false>), dim3(n_big), dim3(kThreads), 0, s, descs, dyn, P->at<Item>(L.off_big_items), fac_tab,
-                         dec, stats);
-      if (!L.big_seg.empty())
-        hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3((unsigned)L.big_seg.size()), dim3(kThreads), 0, s, descs,
-                           P->at<Item>(L.off_big_seg), (const double*)stats, P->at<double>(L.off_segtot));
+    if (!L.big_seg.empty())
+      hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3((unsigned)L.big_seg.size()), dim3(kThreads), 0, s, descs,
+                         P->at<Item>(L.off_big_seg), (const double*)stats, P->at<double>(L.off_segtot));
+    if (n_big > 0)
       hipLaunchKernelGGL(k_velo_fold, dim3((unsigned)L.big_list.size()), dim3(kThreads), 0, s, descs, dyn, P->at<int>(L.off_big_list),
                          (const double*)stats, (const double*)P->at<double>(L.off_segtot), (const float*)wmix, wfold,
                          P->at<int>(L.off_sync), T);
-    }
     const auto elem = L.split ? k_velo_elem<true> : k_velo_elem<false>;
     if (n_mx > 0)
       hipLaunchKernelGGL(elem, dim3(n_mx), dim3(kThreads), 0, s, descs, dyn, P->at<Item>(L.off_mx_items), fac_tab, term_tab,
