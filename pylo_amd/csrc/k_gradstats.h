@@ -17,6 +17,19 @@ __device__ __forceinline__ float abs_or_inf(float x, int nan0) {
   return (nan0 && ax != ax) ? __builtin_inff() : ax;
 }
 
+// The block's sums of at most kP0Thin rows (columns) out of what its waves' 16-lane groups left: [wave][four of them][group][which].
+__device__ __forceinline__ void p0_thin_total(const float* lds_row, int n, float* __restrict__ out) {
+  const int j = threadIdx.x;
+  if (j >= n) return;
+  float s = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const float* t = lds_row + (w * (kP0Rows / 16) + j / 4) * 16 + j % 4;
+    s += (t[0] + t[4]) + (t[8] + t[12]);
+  }
+  out[j] = s;
+}
+
 // ST: storage type of the gradient (k_cast.h).
 template <int V, bool exact, int ST = kStoreF32>
 __device__ __forceinline__ void p0_factored(const TDesc& d, const typename StoredAs<ST>::E* g, int strip, int cb,
@@ -96,6 +109,97 @@ __device__ __forceinline__ void p0_factored(const TDesc& d, const typename Store
     const float* t = lds_row + ((w * (kP0Rows / 16) + q / 4) * 4) * 4 + (q % 4);
     rowpart[(size_t)cb * R0 + r0 + j] = (t[0] + t[4]) + (t[8] + t[12]);
   }
+}
+
+// Matrices of at most kP0Thin rows: a tile is all of them times kP0Long columns, four columns a thread (V = 4: next to each other,
+// V = 1: kThreads apart), whose sums it has to itself.  Tiles of 128 x 256 have one row of work in four waves on a 1 x n matrix:
+// three thousand odd tensors and an embedding took 46900 blocks, now 24200: 183 / 133 us.
+template <int V, bool exact>
+__device__ __forceinline__ void p0_wide(const TDesc& d, const float* g, int cb, float scale, float clipv, int nan0,
+                                        float* __restrict__ rowpart, float* __restrict__ colpart, float* lds_row, float& gsq, float& amax) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int C0 = d.C0, R0 = d.R0, c = cb * kP0Long + (int)threadIdx.x * V;
+  float col[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int rb = 0; rb < kP0Thin; rb += 4) {
+    if (rb >= R0) break;
+    float x[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float* row = g + (size_t)min(rb + u, R0 - 1) * C0;
+      if constexpr (V == 4) {
+        load_vec<4>(row + min(c, C0 - 4), x[u]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[u][j] = *(const gfloat*)(row + min(c + j * kThreads, C0 - 1));
+      }
+    }
+    float rs[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      float sq[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const bool live = rb + u < R0 && (V == 4 ? c : c + j * kThreads) < C0;
+        const float raw = live ? x[u][j] : 0.0f;
+        amax = fmaxf(amax, abs_or_inf(raw, nan0));
+        if (exact) gsq = fmaf(raw, raw, gsq);
+        const float y = exact ? cond_grad(raw, scale, clipv, nan0) : raw;
+        sq[j] = y * y;
+        col[j] += sq[j];
+      }
+      rs[u] = (sq[0] + sq[1]) + (sq[2] + sq[3]);
+      if (!exact) gsq += rs[u];
+    }
+    const float tot = reduce4_rows16(rs[0], rs[1], rs[2], rs[3]);
+    if ((lane & 12) == 0) lds_row[((wave * (kP0Rows / 16) + rb / 4) * 4 + (lane >> 4)) * 4 + (lane & 3)] = tot;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int cc = V == 4 ? c + j : c + j * kThreads;
+    if (cc < C0) colpart[cc] = col[j];
+  }
+  __syncthreads();
+  p0_thin_total(lds_row, R0, rowpart + (size_t)cb * R0);
+}
+
+// ... and of at most kP0Thin columns: kP0Long rows, four a thread, whose sums it has to itself.
+template <bool exact>
+__device__ __forceinline__ void p0_tall(const TDesc& d, const float* g, int strip, float scale, float clipv, int nan0,
+                                        float* __restrict__ rowpart, float* __restrict__ colpart, float* lds_row, float& gsq, float& amax) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int C0 = d.C0, R0 = d.R0, r = strip * kP0Long + (int)threadIdx.x;
+  float rs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int cb = 0; cb < kP0Thin; cb += 4) {
+    if (cb >= C0) break;
+    float x[4][4], col[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        x[j][u] = *(const gfloat*)(g + (size_t)min(r + j * kThreads, R0 - 1) * C0 + min(cb + u, C0 - 1));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float raw = r + j * kThreads < R0 && cb + u < C0 ? x[j][u] : 0.0f;
+        amax = fmaxf(amax, abs_or_inf(raw, nan0));
+        if (exact) gsq = fmaf(raw, raw, gsq);
+        const float y = exact ? cond_grad(raw, scale, clipv, nan0) : raw, sq = y * y;
+        col[u] += sq;
+        rs[j] += sq;
+      }
+    const float tot = reduce4_rows16(col[0], col[1], col[2], col[3]);
+    if ((lane & 12) == 0) lds_row[((wave * (kP0Rows / 16) + cb / 4) * 4 + (lane >> 4)) * 4 + (lane & 3)] = tot;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (r + j * kThreads < R0) rowpart[r + j * kThreads] = rs[j];
+    if (!exact) gsq += rs[j];
+  }
+  __syncthreads();
+  p0_thin_total(lds_row, C0, colpart + (size_t)strip * C0);
 }
 
 template <int V>
@@ -203,6 +307,19 @@ __global__ __launch_bounds__(kThreads) void k_p0(const TDesc* __restrict__ descs
         else if (d.store == kStoreBF16) p0_factored<4, false, kStoreBF16>(d, g16, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
         else if (exact) p0_factored<4, true, kStoreF16>(d, g16, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
         else p0_factored<4, false, kStoreF16>(d, g16, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
+      } else if (d.p0_thin == 1) {
+        auto wide = [&](auto v, auto ex) {
+          p0_wide<decltype(v)::value, decltype(ex)::value>(d, a.grad, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_row, gsq, amax);
+        };
+        using one = std::integral_constant<int, 1>;
+        using four = std::integral_constant<int, 4>;
+        if (d.vec == 4 && exact) wide(four{}, std::true_type{});
+        else if (d.vec == 4) wide(four{}, std::false_type{});
+        else if (exact) wide(one{}, std::true_type{});
+        else wide(one{}, std::false_type{});
+      } else if (d.p0_thin == 2) {
+        if (exact) p0_tall<true>(d, a.grad, it.a, scale, a.clip_val, d.nan0, p0r, p0c, lds_row, gsq, amax);
+        else p0_tall<false>(d, a.grad, it.a, scale, a.clip_val, d.nan0, p0r, p0c, lds_row, gsq, amax);
       } else if (d.vec == 4 && exact) p0_factored<4, true>(d, a.grad, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
       else if (d.vec == 4) p0_factored<4, false>(d, a.grad, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
       else if (exact) p0_factored<1, true>(d, a.grad, it.a, it.b, scale, a.clip_val, d.nan0, p0r, p0c, lds_col, lds_row, gsq, amax);
@@ -352,7 +469,7 @@ __global__ __launch_bounds__(kThreads) void k_stat_segsum(const TDesc* __restric
 }
 
 // =============================================================================================
-// V0a: one block per 64 entries of a statistics vector.  Finishes the sums of g^2 over the
+// V0a: one block per 64 entries of a statistics vector (Item::c: 256, a thread an entry).  Finishes the sums of g^2 over the
 // partials, advances the three Adafactor accumulators (ELO_CELO2_naive.py:152-160) and leaves
 // per-block partial sums of  f, f^2, rsqrt(f+1e-8)^2  per decay.
 // =============================================================================================
@@ -373,8 +490,58 @@ __global__ __launch_bounds__(kV0aThreads) void k_v0a(const TDesc* __restrict__ d
   const int npart = pick(d.npart, which);
   const float* pp = part + pick(d.part_off, which);
   const int e = threadIdx.x & 63, grp = threadIdx.x >> 6;
-  const int i = it.a * kV0aEnt + e;
   const int k = grp;  // after the sums: waves 0..2 take one decay each
+  if (it.c) {         // many blocks, few partial sums an entry: three thousand odd tensors took 39800 blocks,
+                      // 87 us, now 12500, 33
+    static_assert(kV0aWide == kV0aThreads, "a thread an entry");
+    const bool is_r = (which == 0) == (d.vec0_is_r != 0);
+    float* fac = is_r ? a.fac_r : a.fac_c;
+    constexpr int Q = kV0aWide / 64;
+    float old[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int i = it.a * kV0aWide + q * 64 + e;
+      old[q] = k < 3 && i < len ? *(const gfloat*)(fac + (size_t)k * len + i) : 0.0f;
+    }
+    double s2 = 1.0;
+    if (a.clip_norm > 0.0f && gl->flag == 0 && d.mode == kModeFac2D) {
+      const float sc = grad_scale(d, a, gl, it.tensor);
+      s2 = (double)sc * (double)sc;
+    }
+    const int own = min(it.a * kV0aWide + (int)threadIdx.x, len - 1);
+    float p[kV0aParts];
+#pragma unroll
+    for (int q = 0; q < kV0aParts; ++q) p[q] = q < npart ? *(const gfloat*)(pp + (size_t)q * len + own) : 0.0f;
+    double S = 0.0;
+#pragma unroll
+    for (int q = 0; q < kV0aParts; ++q) S += (double)p[q];
+    lds[grp][e] = S;
+    __syncthreads();
+    if (k >= 3) return;
+    const double by = s2 / (double)pick(d.sumlen, which);
+    const float beta = dec.beta_fac[k];
+    double s_f = 0.0, s_ff = 0.0, s_rr = 0.0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const int i = it.a * kV0aWide + q * 64 + e;
+      if (i >= len) break;
+      const float f = beta * old[q] + (1.0f - beta) * ((float)(by * lds[q][e]) + 1e-30f);
+      fac[(size_t)k * len + i] = f;
+      const float rq = rsq(f + 1e-8f);
+      s_f += (double)f;
+      s_ff += (double)f * (double)f;
+      s_rr += (double)rq * (double)rq;
+    }
+    s_f = wave_sum(s_f);
+    s_ff = wave_sum(s_ff);
+    s_rr = wave_sum(s_rr);
+    if (e == 0) {
+      double* o = v0part + (size_t)blockIdx.x * kNV0 + k * 3;
+      o[0] = s_f; o[1] = s_ff; o[2] = s_rr;
+    }
+    return;
+  }
+  const int i = it.a * kV0aEnt + e;
   // everything the second half needs from memory is requested before the partial sums are read, so that
   // the block pays one memory round trip instead of two (kernels start with cold caches)
   const bool is_r = (which == 0) == (d.vec0_is_r != 0);

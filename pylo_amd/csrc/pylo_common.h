@@ -14,6 +14,8 @@ namespace pylo {
 constexpr int kThreads = 256;   // 4 waves of 64 lanes
 constexpr int kWaves = 4;
 constexpr int kP0Rows = 128;    // rows of one row/column-sum tile; tile columns = 64 * vec
+constexpr int kP0Thin = 16;     // rows (columns) up to which a matrix is summed in tiles of all its rows (columns) ...
+constexpr int kP0Long = 4 * kThreads;   // ... and this many columns (rows), four a thread
 constexpr int kElemIters = 8;   // an element chunk is kThreads * vec * TDesc::iters elements, iters <= kElemIters
 constexpr int kTileV = 2;       // column-resident walk: a wave owns 64 * kTileV columns ...
 constexpr int kTileCols = 64 * kTileV;
@@ -21,7 +23,9 @@ constexpr int kTileRows = 16;   // ... and walks TDesc::tile_rows of them, at mo
 constexpr int kApplyRowsMax = 64;   // the same of AdafacLO's apply pass, TDesc::atile_rows
 constexpr int kNStat = 18;      // feature channels that vary per element (the other 12 are
                                 // functions of the row or of the column only)
-constexpr int kV0aEnt = 64;     // vector entries per k_v0a block
+constexpr int kV0aEnt = 64;     // vector entries per k_v0a block ...
+constexpr int kV0aWide = 256;   // ... and where a plan has many blocks and an entry at most kV0aParts partial sums
+constexpr int kV0aParts = 8;
 constexpr int kV0bEnt = 1024;   // vector entries per k_v0b block
 constexpr int kNV0 = 9;         // partial sums per k_v0a block
 constexpr int kV0aThreads = 256;   // groups of 64 lanes share the partial rows of 64 entries
@@ -87,6 +91,7 @@ struct TDesc {
   int rcm_size;     // N-D: size of the 2nd-largest dim and its stride inside the row vector; row_col_mean
   int rcm_stride;   //      is the mean over that axis, one value per slice (2-D: one value per tensor)
   int n_strips, n_colblk;
+  int p0_thin;      // tiles of the row / column sums: 0 kP0Rows x 64 vec; 1 all rows x kP0Long; 2 kP0Long x all columns
   int blk0, nblk;   // range of element-chunk blocks (rows of the statistics partials)
   int seg0, nseg;   // tensors with many rows: their rows are first summed in segments of kSegRows (k_stat_segsum)
   int fac_slot;     // index among factored tensors, -1 otherwise

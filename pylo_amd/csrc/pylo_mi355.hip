@@ -1068,6 +1068,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
   L.dr.assign(T, -1);
   long long part = 0, fac = 0, term = 0;
   std::vector<int> lin_tensors;   // AdafacLO: tensors of the linear apply pass
+  long long v0a_blocks = 0;
   const int H = L.H;
   long long total_elems = 0;
   for (int t = 0; t < T; ++t) {
@@ -1169,8 +1170,12 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
         d.vec0_is_r = (edr == 1) ? 1 : 0;  // vector 0 (indexed by dim 0) results from summing over dim 1
         d.len[0] = d.R0; d.len[1] = d.C0;
         d.sumlen[0] = d.C0; d.sumlen[1] = d.R0;
-        d.n_strips = (d.R0 + kP0Rows - 1) / kP0Rows;
-        d.n_colblk = (d.C0 + 64 * d.vec - 1) / (64 * d.vec);
+        // (16-bit gradients that k_p0 reads itself are taken in the usual tiles)
+        const bool typed16 = d.store == kStoreF16 || d.store == kStoreBF16;
+        d.p0_thin = typed16 ? 0 : d.R0 <= kP0Thin && d.C0 > 64 * d.vec ? 1 : d.C0 <= kP0Thin && d.R0 > kP0Rows ? 2 : 0;
+        const int tile_r = d.p0_thin == 2 ? kP0Long : kP0Rows, tile_c = d.p0_thin == 1 ? kP0Long : 64 * d.vec;
+        d.n_strips = (d.R0 + tile_r - 1) / tile_r;
+        d.n_colblk = (d.C0 + tile_c - 1) / tile_c;
         d.npart[0] = d.n_colblk; d.npart[1] = d.n_strips;
         d.nd_div_blk[0] = make_fastdiv((unsigned)std::max(d.C0, 1));   // element -> row (k_adafac_apply_lin)
       } else {
@@ -1205,9 +1210,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
         d.fac_slot = (int)L.fac_list.size();
         L.fac_list.push_back(t);
         for (int w = 0; w < 2; ++w) {
-          d.v0a_first[w] = (int)L.v0a_items.size();
-          for (int c = 0; c * kV0aEnt < d.len[w]; ++c) L.v0a_items.push_back(Item{t, c, w, 0});
-          d.v0a_n[w] = (int)L.v0a_items.size() - d.v0a_first[w];
+          v0a_blocks += (d.len[w] + kV0aEnt - 1) / kV0aEnt;
           for (int c = 0; c * kV0bEnt < d.len[w]; ++c) L.v0b_items.push_back(Item{t, c, w, 0});
           if (d.mode == kModeFacND)
             for (int c = 0; c * kV0aEnt < d.len[w]; ++c)
@@ -1291,6 +1294,17 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
       } else {
         lin_tensors.push_back(t);
       }
+    }
+  }
+  // Blocks of k_v0a: four times the entries where there are more of them than the chip holds at a time (2048)
+  for (int t : L.fac_list) {
+    TDesc& d = L.descs[t];
+    for (int w = 0; w < 2; ++w) {
+      const bool wide = v0a_blocks > 4096 && d.npart[w] <= kV0aParts && d.len[w] > kV0aEnt;
+      const int ent = wide ? kV0aWide : kV0aEnt;
+      d.v0a_first[w] = (int)L.v0a_items.size();
+      for (int c = 0; c * ent < d.len[w]; ++c) L.v0a_items.push_back(Item{t, c, w, wide ? 1 : 0});
+      d.v0a_n[w] = (int)L.v0a_items.size() - d.v0a_first[w];
     }
   }
   // Blocks of AdafacLO's linear apply pass: on the matrix pipe Item::b trips of 256 elements each, as many as leave
