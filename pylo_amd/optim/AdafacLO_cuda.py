@@ -12,6 +12,7 @@ from __future__ import annotations
 
 from typing import Optional, Union
 
+import numpy as np
 import torch
 from torch.optim import Optimizer
 
@@ -42,6 +43,7 @@ class AdafacLO_CUDA(Optimizer):
     # ``state_dict()`` / ``sync_step_counters()`` only.  The reference has no such mode.
     capturable = False
     _dev_steps = None
+    _fast = None         # what a step needs when nothing but values has changed since the one before (_unchanged)
 
     def __init__(
         self,
@@ -180,6 +182,7 @@ class AdafacLO_CUDA(Optimizer):
         return super().state_dict()
 
     def load_state_dict(self, state_dict):
+        self._fast = None
         out = _lib.load_float32_state(self, super().load_state_dict, state_dict)
         if self.capturable and self._plan is not None:
             self._reset_device_steps([(g, p) for g in self.param_groups for p in g["params"]])
@@ -199,8 +202,76 @@ class AdafacLO_CUDA(Optimizer):
         return dict(lr=group["lr"], weight_decay=group["weight_decay"], exp_mult=self.exp_mult,
                     step_mult=self.step_mult, clip_norm=0.0 if mx is None else float(mx))
 
+    # Three microseconds of Python a tensor for its row of the argument table, and one for its counter, were the whole step on a
+    # convolutional network of 161 tensors (host 673 us, its kernels 660).  After a step in which every parameter had a dense
+    # contiguous gradient the rows are kept; the counters, one 0-dim tensor a parameter, are moved side by side into one
+    # buffer, in place, and advanced together.
+    def _keep_rows(self, tensors):
+        index = {id(g): i for i, g in enumerate(self.param_groups)}
+        counters = torch.tensor([float(self.state[p]["step"]) for _, p in tensors], dtype=torch.float64)
+        keys = ("exp_avg", "exp_avg_sq", "exp_avg_sq_r", "exp_avg_sq_c", "step")
+        records = []
+        for i, (_, p) in enumerate(tensors):
+            state = self.state[p]
+            t = state["step"]
+            if not torch.is_tensor(t) or t.dtype != torch.float64 or t.device.type != "cpu" or t.dim() != 0:
+                return None
+            t.set_(counters.untyped_storage(), i, ())
+            kept = tuple(state[k] for k in keys)
+            records.append((p, p.shape, p.dtype, state, kept, tuple(x.data_ptr() for x in kept)))
+        return dict(key=self._plan_key, flags=self._plan_key[0], n_state=len(self.state), records=records, counters=counters,
+                    values=counters.numpy(), scalars=None, gidx=np.asarray([index[id(g)] for g, _ in tensors], dtype=np.int64))
+
+    def _unchanged(self, fast):
+        """Gradient and parameter addresses if nothing but values has changed since the step that made ``fast``, else None."""
+        if (fast["key"] is not self._plan_key or fast["flags"] != self._PLAN_FLAGS | self._norm_flags()
+                or len(self.state) != fast["n_state"]):
+            return None
+        strided = torch.strided
+        params = [p for group in self.param_groups for p in group["params"]]
+        records = fast["records"]
+        if len(params) != len(records):
+            return None
+        grads, addresses = [], []
+        for p, (old, shape, dtype, state, kept, at) in zip(params, records):
+            g = p.grad
+            if (p is not old or g is None or p.dtype is not dtype or g.dtype is not dtype or p.shape != shape
+                    or g.layout is not strided or not g.is_contiguous()):
+                return None
+            m, v, fr, fc, t = kept
+            if (state.get("exp_avg") is not m or state.get("exp_avg_sq") is not v or state.get("exp_avg_sq_r") is not fr
+                    or state.get("exp_avg_sq_c") is not fc or state.get("step") is not t
+                    or at != (m.data_ptr(), v.data_ptr(), fr.data_ptr(), fc.data_ptr(), t.data_ptr())):
+                return None
+            grads.append(g.data_ptr())
+            addresses.append(p.data_ptr())
+        return grads, addresses
+
+    def _step_fast(self, fast, found):
+        plan, values = self._plan, fast["values"]
+        args = plan.args
+        args["grad"], args["param"] = found
+        scalars = [{k: float(v) for k, v in self._scalars(g).items()} for g in self.param_groups]
+        if scalars != fast["scalars"]:
+            for k in scalars[0]:
+                args[k] = np.asarray([sc[k] for sc in scalars], dtype=np.float64)[fast["gidx"]]
+            fast["scalars"] = scalars
+        step_fed = float(values[0])
+        if not (values == step_fed).all():       # the library reads each parameter's own counter
+            args["bc1"] = values
+            step_fed = -1.0
+        fast["counters"].add_(1.0)
+        with torch.cuda.device(self.device):
+            plan.adafac_step(self._decays, self._net, step_fed, torch.cuda.current_stream(self.device).cuda_stream)
+
     @torch.no_grad()
     def step(self, loss=None):
+        if self._fast is not None and not self.capturable:
+            found = self._unchanged(self._fast)
+            if found is not None:
+                self._step_fast(self._fast, found)
+                return loss
+            self._fast = None
         tensors = [(g, p) for g in self.param_groups for p in g["params"]]
         self._ensure_plan(tensors)
         plan = self._plan
@@ -258,5 +329,7 @@ class AdafacLO_CUDA(Optimizer):
         with torch.cuda.device(self.device):
             plan.adafac_step(self._decays, self._net, step_fed, torch.cuda.current_stream(self.device).cuda_stream,
                              args=table)
+        if not self.capturable and not keep and all(p.grad is not None for _, p in tensors):
+            self._fast = self._keep_rows(tensors)
         del keep
         return loss
