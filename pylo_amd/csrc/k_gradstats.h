@@ -266,31 +266,29 @@ __device__ __forceinline__ void p0_nd_block(const TDesc* __restrict__ descs, con
 // pass 2: pass 0 where no tensor is clipped by the global norm: blocks that only add to it leave a zero.
 // TYPED: plans with tensors whose 16-bit gradient is read here (TDesc::direct; their rows are multiples of 128).
 template <bool TYPED, bool SPLIT>
-__global__ __launch_bounds__(kThreads) void k_p0(const TDesc* __restrict__ descs,
-                                                 const PyloTensorArgs* __restrict__ dyn,
-                                                 const Item* __restrict__ items, float* __restrict__ part,
-                                                 double* __restrict__ gsq_part, int* __restrict__ flag_part,
-                                                 const Globals* __restrict__ gl, int pass,
-                                                 const Item* __restrict__ nd_items, int n_main) {
+__device__ __forceinline__ void p0_block(int block, const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn,
+                                         const Item* __restrict__ items, float* __restrict__ part,
+                                         double* __restrict__ gsq_part, int* __restrict__ flag_part,
+                                         const Globals* __restrict__ gl, int pass, const Item* __restrict__ nd_items, int n_main) {
   __shared__ float lds_col[kWaves * 256];
   __shared__ float lds_row[kWaves * (kP0Rows / 16) * 16];
   __shared__ float lds_red[kWaves];
   __shared__ int lds_flag[kWaves];
   // blocks past the main items: the N-D tensors' sums, when the launcher appended them (it does when
   // no tensor is clipped by the global norm, which they would have to wait for)
-  if ((int)blockIdx.x >= n_main) {
-    p0_nd_block(descs, dyn, nd_items[blockIdx.x - n_main], part, gl, lds_col);
+  if (block >= n_main) {
+    p0_nd_block(descs, dyn, nd_items[block - n_main], part, gl, lds_col);
     return;
   }
-  const Item it = items[blockIdx.x];
+  const Item it = items[block];
   const TDesc d = elem_desc<SPLIT>(descs + it.tensor);
   const PyloTensorArgs a = dyn[it.tensor];
   const bool clip_on = a.clip_norm > 0.0f;
   if (pass == 1 && (!clip_on || d.mode != kModeFac2D || gl->flag == 0)) return;
   if (pass == 2 && d.mode != kModeFac2D) {
     if (threadIdx.x == 0) {
-      gsq_part[blockIdx.x] = 0.0;
-      flag_part[blockIdx.x] = 0;
+      gsq_part[block] = 0.0;
+      flag_part[block] = 0;
     }
     return;
   }
@@ -337,9 +335,19 @@ __global__ __launch_bounds__(kThreads) void k_p0(const TDesc* __restrict__ descs
   if (lane == 0) { lds_red[wave] = gsq; lds_flag[wave] = flag; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    gsq_part[blockIdx.x] = ((double)lds_red[0] + (double)lds_red[1]) + ((double)lds_red[2] + (double)lds_red[3]);
-    flag_part[blockIdx.x] = (clip_on && (lds_flag[0] | lds_flag[1] | lds_flag[2] | lds_flag[3])) ? 1 : 0;
+    gsq_part[block] = ((double)lds_red[0] + (double)lds_red[1]) + ((double)lds_red[2] + (double)lds_red[3]);
+    flag_part[block] = (clip_on && (lds_flag[0] | lds_flag[1] | lds_flag[2] | lds_flag[3])) ? 1 : 0;
   }
+}
+
+template <bool TYPED, bool SPLIT>
+__global__ __launch_bounds__(kThreads) void k_p0(const TDesc* __restrict__ descs,
+                                                 const PyloTensorArgs* __restrict__ dyn,
+                                                 const Item* __restrict__ items, float* __restrict__ part,
+                                                 double* __restrict__ gsq_part, int* __restrict__ flag_part,
+                                                 const Globals* __restrict__ gl, int pass,
+                                                 const Item* __restrict__ nd_items, int n_main) {
+  p0_block<TYPED, SPLIT>((int)blockIdx.x, descs, dyn, items, part, gsq_part, flag_part, gl, pass, nd_items, n_main);
 }
 
 // use_flags == 0: the caller has shown that no element can exceed its clamp after scaling (the scaled
@@ -473,15 +481,12 @@ __global__ __launch_bounds__(kThreads) void k_stat_segsum(const TDesc* __restric
 // partials, advances the three Adafactor accumulators (ELO_CELO2_naive.py:152-160) and leaves
 // per-block partial sums of  f, f^2, rsqrt(f+1e-8)^2  per decay.
 // =============================================================================================
-__global__ __launch_bounds__(kV0aThreads) void k_v0a(const TDesc* __restrict__ descs,
-                                                  const PyloTensorArgs* __restrict__ dyn,
-                                                  const Item* __restrict__ items,
-                                                  const float* __restrict__ part,
-                                                  const Globals* __restrict__ gl, PyloDecays dec,
-                                                  double* __restrict__ v0part) {
+__device__ __forceinline__ void v0a_block(int block, const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn,
+                                          const Item* __restrict__ items, const float* __restrict__ part,
+                                          const Globals* __restrict__ gl, const PyloDecays& dec, double* __restrict__ v0part) {
   constexpr int G = kV0aThreads / 64;
   __shared__ double lds[G][kV0aEnt];
-  const Item it = items[blockIdx.x];
+  const Item it = items[block];
   const TDesc d = descs[it.tensor];
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
@@ -536,7 +541,7 @@ __global__ __launch_bounds__(kV0aThreads) void k_v0a(const TDesc* __restrict__ d
     s_ff = wave_sum(s_ff);
     s_rr = wave_sum(s_rr);
     if (e == 0) {
-      double* o = v0part + (size_t)blockIdx.x * kNV0 + k * 3;
+      double* o = v0part + (size_t)block * kNV0 + k * 3;
       o[0] = s_f; o[1] = s_ff; o[2] = s_rr;
     }
     return;
@@ -581,9 +586,18 @@ __global__ __launch_bounds__(kV0aThreads) void k_v0a(const TDesc* __restrict__ d
   s_ff = wave_sum(s_ff);
   s_rr = wave_sum(s_rr);
   if (e == 0) {
-    double* o = v0part + (size_t)blockIdx.x * kNV0 + k * 3;
+    double* o = v0part + (size_t)block * kNV0 + k * 3;
     o[0] = s_f; o[1] = s_ff; o[2] = s_rr;
   }
+}
+
+__global__ __launch_bounds__(kV0aThreads) void k_v0a(const TDesc* __restrict__ descs,
+                                                  const PyloTensorArgs* __restrict__ dyn,
+                                                  const Item* __restrict__ items,
+                                                  const float* __restrict__ part,
+                                                  const Globals* __restrict__ gl, PyloDecays dec,
+                                                  double* __restrict__ v0part) {
+  v0a_block((int)blockIdx.x, descs, dyn, items, part, gl, dec, v0part);
 }
 
 // Where entry i of vector `which` of tensor d lives in the factor / term tables.
@@ -688,19 +702,15 @@ __device__ __forceinline__ void vector_terms(const TDesc& d, int which, bool is_
 // per element.  The bias goes into the terms of vector 0.  RUNS: plans with such slices (TDesc::slice_runs); the loop over
 // a run costs the launch of every other plan 1 us of its 5 to 7 where it is compiled in.
 // =============================================================================================
-template <int H, bool RUNS = false>
-__global__ __launch_bounds__(kThreads) void k_v0b(const TDesc* __restrict__ descs,
-                                                  const PyloTensorArgs* __restrict__ dyn,
-                                                  const Item* __restrict__ items,
-                                                  const double* __restrict__ v0part, float norm_eps,
-                                                  const float* __restrict__ w1, const float* __restrict__ b1,
-                                                  int b1_stride /* floats between the tensors' biases, 0: shared */,
-                                                  float* __restrict__ fac_tab, float* __restrict__ term_tab,
-                                                  BScale* __restrict__ bscale) {
+template <int H, bool RUNS>
+__device__ __forceinline__ void v0b_block(int block, const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn,
+                                          const Item* __restrict__ items, const double* __restrict__ v0part, float norm_eps,
+                                          const float* __restrict__ w1, const float* __restrict__ b1, int b1_stride,
+                                          float* __restrict__ fac_tab, float* __restrict__ term_tab, BScale* __restrict__ bscale) {
   constexpr int G = 14;  // 14 groups x 18 (vector, slot) pairs = 252 threads
   __shared__ double red[G][2 * kNV0];
   __shared__ double tot[2 * kNV0];
-  const Item it = items[blockIdx.x];
+  const Item it = items[block];
   const TDesc d = descs[it.tensor];
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
@@ -862,6 +872,18 @@ __global__ __launch_bounds__(kThreads) void k_v0b(const TDesc* __restrict__ desc
     *(float4*)(fac_tab + fac_index(d, which, 0, i)) = make_float4(fct[0], fct[1], fct[2], 0.0f);
     if (w1 != nullptr) vector_terms<H>(d, which, is_r, i, x0, x1, w1, b1 + (size_t)it.tensor * b1_stride, term_tab);
   }
+}
+
+template <int H, bool RUNS = false>
+__global__ __launch_bounds__(kThreads) void k_v0b(const TDesc* __restrict__ descs,
+                                                  const PyloTensorArgs* __restrict__ dyn,
+                                                  const Item* __restrict__ items,
+                                                  const double* __restrict__ v0part, float norm_eps,
+                                                  const float* __restrict__ w1, const float* __restrict__ b1,
+                                                  int b1_stride /* floats between the tensors' biases, 0: shared */,
+                                                  float* __restrict__ fac_tab, float* __restrict__ term_tab,
+                                                  BScale* __restrict__ bscale) {
+  v0b_block<H, RUNS>((int)blockIdx.x, descs, dyn, items, v0part, norm_eps, w1, b1, b1_stride, fac_tab, term_tab, bscale);
 }
 
 // First-layer terms with per-tensor weights that only exist after k_v0b has run (VeLO: the LSTM

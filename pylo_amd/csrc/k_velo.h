@@ -128,7 +128,7 @@ __device__ __forceinline__ void lstm_pivots(const TDesc& d, const PyloTensorArgs
 // kernel that formed the LSTM's inputs, since the apply pass overwrites them while it runs) and the
 // tensor's first gradient element; they are wave-uniform and live in scalar registers.
 constexpr int kNewSumW = 10;    // doubles per row of those partial sums (9 used)
-constexpr int kFeatWide = 512;  // blocks of k_p0 and of k_velo_feat together up to which the latter's have sixteen waves
+constexpr int kVeloPaired = 448;   // blocks of k_p0 and k_velo_feat up to which both chains share launches (k_velo_p0_feat)
 struct NewSums {
   float v[9];
   float piv[4];
@@ -613,23 +613,19 @@ __device__ __forceinline__ double* velo_guard_sums(int* sync, int T) { return re
 // block, a tensor's only one, waited 165 us for the 16 000 rows of an embedding of 131 M elements.  Blocks of four waves
 // take four units a thread: next to k_p0, whose blocks take the place of every four waves that end, blocks of sixteen wait.
 // Three thousand tensors and an embedding 387 / 41 us next to k_p0; ViT-B/16 80 / 72 us (8 us without the gradients streaming
-// past it: what is left is a chain of short dependent loads).  Where k_p0 leaves room the shorter chain of a unit a thread is
-// worth more, 11.6 / 8.6 us: whole steps, four / sixteen waves, 0.6 M elements 108 / 106 us, 1.4 M 119 / 116, 4.4 M (280 blocks) 157 / 155,
-// 10.0 M (630) 247 / 252, 12.5 M 226 / 231, 89 M 1030 / 1037, a thousand tensors of 1 M 632 / 637 (kFeatWide).
+// past it: what is left is a chain of short dependent loads).  Blocks of sixteen with a unit a thread are the shorter chain where
+// nothing streams past them, 8.6 us for 11.6: k_velo_p0_feat.
 template <int THREADS>
-__global__ __launch_bounds__(THREADS) void k_velo_feat(const TDesc* __restrict__ descs,
-                                                        const PyloTensorArgs* __restrict__ dyn, int T,
-                                                        const double* __restrict__ newsum_part, const double* __restrict__ seg_tot,
-                                                        float* __restrict__ piv, LossState ls, VeloStep st,
-                                                        float* __restrict__ xfeat, int H,
-                                                        const float* __restrict__ w2t, const float* __restrict__ b2,
-                                                        const float* __restrict__ wft, const float* __restrict__ bf,
-                                                        float* __restrict__ mixbuf, int* __restrict__ sync) {
+__device__ __forceinline__ void velo_feat_block(int t, const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, int T,
+                                                const double* __restrict__ newsum_part, const double* __restrict__ seg_tot,
+                                                float* __restrict__ piv, const LossState& ls, const VeloStep& st,
+                                                float* __restrict__ xfeat, int H, const float* __restrict__ w2t,
+                                                const float* __restrict__ b2, const float* __restrict__ wft,
+                                                const float* __restrict__ bf, float* __restrict__ mixbuf, int* __restrict__ sync) {
   constexpr int G = THREADS / kNewSumW;
   __shared__ double part[G][kNewSumW];
   __shared__ double tot[kStatW];
   __shared__ float xs[32];
-  const int t = blockIdx.x;
   const TDesc d = descs[t];
   const PyloTensorArgs a = dyn[t];
   const int c = threadIdx.x % kNewSumW, gI = threadIdx.x / kNewSumW;
@@ -664,6 +660,17 @@ __global__ __launch_bounds__(THREADS) void k_velo_feat(const TDesc* __restrict__
   velo_row_features<THREADS>(d, a, t, T, tot, nullptr, piv, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, xs);
 }
 
+__global__ __launch_bounds__(kThreads) void k_velo_feat(const TDesc* __restrict__ descs,
+                                                        const PyloTensorArgs* __restrict__ dyn, int T,
+                                                        const double* __restrict__ newsum_part, const double* __restrict__ seg_tot,
+                                                        float* __restrict__ piv, LossState ls, VeloStep st,
+                                                        float* __restrict__ xfeat, int H,
+                                                        const float* __restrict__ w2t, const float* __restrict__ b2,
+                                                        const float* __restrict__ wft, const float* __restrict__ bf,
+                                                        float* __restrict__ mixbuf, int* __restrict__ sync) {
+  velo_feat_block<kThreads>((int)blockIdx.x, descs, dyn, T, newsum_part, seg_tot, piv, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, sync);
+}
+
 // ---------------------------------------------------------------------------------------------
 // LSTM (VeLO_RNN.py:43-66,110-135).  All weights are pre-transposed to (in, out) by the host.
 // Rows are in the reference's order r = T-1-t.
@@ -695,23 +702,22 @@ __global__ __launch_bounds__(kThreads) void k_velo_colmax(const float* __restric
 // products are in mixbuf (written by k_lo_reduce).  Block (x, y): 64 hidden units (one per lane) and
 // the 8 rows 8y .. 8y+7, two per wave; the maximum over all rows is taken by every block itself, or
 // from the per-chunk maxima of k_velo_colmax when there are many rows.
-__global__ __launch_bounds__(kThreads) void k_velo_mix(const float* __restrict__ mixbuf, int T, int Tpad, int H,
-                                                       const float* __restrict__ pmax, int n_chunks,
-                                                       const float* __restrict__ h_state, float* __restrict__ xT,
-                                                       LossState ls) {
+__device__ __forceinline__ void velo_mix_block(int bx, int by, const float* __restrict__ mixbuf, int T, int Tpad, int H,
+                                               const float* __restrict__ pmax, int n_chunks, const float* __restrict__ h_state,
+                                               float* __restrict__ xT, const LossState& ls) {
   __shared__ float mx_s[kWaves][64];
   // every block of k_lo_reduce has read the loss accumulators by now: one block advances them
-  if (blockIdx.x == 0 && blockIdx.y == 0) {
+  if (bx == 0 && by == 0) {
     __shared__ float cor_s[10], rmin_s[10], feat_s[9];
     loss_step(ls.means, ls.running_min, ls.decays, ls.iteration, ls.loss, true, cor_s, rmin_s, feat_s);
   }
   const int lane = threadIdx.x & 63, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int u = blockIdx.x * 64 + lane;  // H is a multiple of 64
+  const int u = bx * 64 + lane;  // H is a multiple of 64
   const float* fm = mixbuf + (size_t)T * H;
   const float v = pmax != nullptr ? mix_colmax(pmax, 0, n_chunks, H, u, mx_s) : mix_colmax(mixbuf, 0, T, H, u, mx_s);
 #pragma unroll
   for (int q = 0; q < kGateBT / kWaves; ++q) {
-    const int r = blockIdx.y * kGateBT + q * kWaves + grp;  // < Tpad
+    const int r = by * kGateBT + q * kWaves + grp;  // < Tpad
     float acc = 0.0f, hv = 0.0f;
     if (r < T) {
       acc = fm[(size_t)r * H + u] + v;
@@ -720,6 +726,13 @@ __global__ __launch_bounds__(kThreads) void k_velo_mix(const float* __restrict__
     xT[(size_t)u * Tpad + r] = acc;
     xT[(size_t)(H + u) * Tpad + r] = hv;
   }
+}
+
+__global__ __launch_bounds__(kThreads) void k_velo_mix(const float* __restrict__ mixbuf, int T, int Tpad, int H,
+                                                       const float* __restrict__ pmax, int n_chunks,
+                                                       const float* __restrict__ h_state, float* __restrict__ xT,
+                                                       LossState ls) {
+  velo_mix_block((int)blockIdx.x, (int)blockIdx.y, mixbuf, T, Tpad, H, pmax, n_chunks, h_state, xT, ls);
 }
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
@@ -734,10 +747,9 @@ __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf
 // loop.  Blocks are numbered so that the blocks one XCD receives (block id modulo 8) share their
 // unit blocks: each XCD's L2 then holds its 1/8 of the 8 MB weight matrix instead of all of it.
 constexpr int kGateU = 16, kGateS = 16;
-__global__ __launch_bounds__(kThreads) void k_velo_gates(const float* __restrict__ xT, int T, int Tpad, int H,
-                                                         const float* __restrict__ wt /*(2H, H, 4)*/,
-                                                         const float* __restrict__ b /*4H*/,
-                                                         float* __restrict__ h_state, float* __restrict__ c_state) {
+__device__ __forceinline__ void velo_gates_block(int block, const float* __restrict__ xT, int T, int Tpad, int H,
+                                                 const float* __restrict__ wt /*(2H, H, 4)*/, const float* __restrict__ b /*4H*/,
+                                                 float* __restrict__ h_state, float* __restrict__ c_state) {
   // x tile [2H][8] during the loop (2H <= 2048: 64 KB would not fit, so it is staged in two halves),
   // then the partial sums [kGateS][4 * kGateBT][kGateU]
   constexpr int kHalf = 1024;
@@ -749,12 +761,12 @@ __global__ __launch_bounds__(kThreads) void k_velo_gates(const float* __restrict
   const int n_ub = H / kGateU;
   int ub, rb;
   if (n_ub % 8 == 0) {
-    const int per = n_ub / 8, xcd = blockIdx.x % 8, j = blockIdx.x / 8;
+    const int per = n_ub / 8, xcd = block % 8, j = block / 8;
     ub = xcd * per + j % per;
     rb = j / per;
   } else {
-    ub = blockIdx.x % n_ub;
-    rb = blockIdx.x / n_ub;
+    ub = block % n_ub;
+    rb = block / n_ub;
   }
   const int u = ub * kGateU + ul;
   const int r0 = rb * kGateBT;
@@ -814,6 +826,54 @@ __global__ __launch_bounds__(kThreads) void k_velo_gates(const float* __restrict
     c_state[(size_t)r * H + u] = c_new;
     h_state[(size_t)r * H + u] = sigmoidf_(gate[3]) * tanhf(c_new);
   }
+}
+
+__global__ __launch_bounds__(kThreads) void k_velo_gates(const float* __restrict__ xT, int T, int Tpad, int H,
+                                                         const float* __restrict__ wt /*(2H, H, 4)*/,
+                                                         const float* __restrict__ b /*4H*/,
+                                                         float* __restrict__ h_state, float* __restrict__ c_state) {
+  velo_gates_block((int)blockIdx.x, xT, T, Tpad, H, wt, b, h_state, c_state);
+}
+
+// Plans of few blocks: what needs the gradients and what needs the LSTM, two chains of short launches that meet in k_terms, as
+// three launches of both on the caller's stream.  Such a step is bound by its launches: on a second stream the LSTM's chain took
+// four of its own, two events and two waits for them, 78 us of host time a step where these take 24, and the GPU stood still between
+// dependent launches of 4 to 12 us.  Where k_p0 streams for longer than the LSTM's chain takes, that chain is better hidden under
+// it on a stream of its own (kVeloPaired).  Whole steps, apart / paired: MLP of width 32 91 / 58 us, 128 89 / 65, 1024 122 / 105,
+// ViT of 12 layers and width 64 165 / 131, 192 (400 blocks) 167 / 145, 256 (455) 197 / 192, 320 291 / 295, of 7 of 384 (610) 226 / 226,
+// 12 of 384 (970) 325 / 337; ResNet-50 of width 32 218 / 189, 40 237 / 242, 64 464 / 514; 250 tensors 315 / 258.
+template <bool SPLIT>
+__global__ __launch_bounds__(kFoldThreads) void k_velo_p0_feat(
+    const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const Item* __restrict__ items, float* __restrict__ part,
+    double* __restrict__ gsq_part, int* __restrict__ flag_part, const Globals* __restrict__ gl, const Item* __restrict__ nd_items,
+    int n_main, int T, const double* __restrict__ newsum_part, const double* __restrict__ seg_tot, float* __restrict__ piv, LossState ls,
+    VeloStep st, float* __restrict__ xfeat, int H, const float* __restrict__ w2t, const float* __restrict__ b2,
+    const float* __restrict__ wft, const float* __restrict__ bf, float* __restrict__ mixbuf, int* __restrict__ sync) {
+  const int block = (int)blockIdx.x;
+  if (block < T)
+    velo_feat_block<kFoldThreads>(block, descs, dyn, T, newsum_part, seg_tot, piv, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, sync);
+  else if (threadIdx.x < kThreads)   // whole waves: the others' end, a barrier counts those that are left
+    p0_block<false, SPLIT>(block - T, descs, dyn, items, part, gsq_part, flag_part, gl, 0, nd_items, n_main);
+}
+
+__global__ __launch_bounds__(kThreads) void k_velo_v0a_mix(
+    const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const Item* __restrict__ items, const float* __restrict__ part,
+    const Globals* __restrict__ gl, PyloDecays dec, double* __restrict__ v0part, const float* __restrict__ mixbuf, int T, int Tpad, int H,
+    const float* __restrict__ h_state, float* __restrict__ xT, LossState ls) {
+  static_assert(kV0aThreads == kThreads, "one block size");
+  const int block = (int)blockIdx.x, nx = H / 64, n_mix = nx * (Tpad / kGateBT);
+  if (block < n_mix) velo_mix_block(block % nx, block / nx, mixbuf, T, Tpad, H, nullptr, 1, h_state, xT, ls);
+  else v0a_block(block - n_mix, descs, dyn, items, part, gl, dec, v0part);
+}
+
+__global__ __launch_bounds__(kThreads) void k_velo_v0b_gates(
+    const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const Item* __restrict__ items,
+    const double* __restrict__ v0part, float* __restrict__ fac_tab, float* __restrict__ term_tab, BScale* __restrict__ bscale,
+    const float* __restrict__ xT, int T, int Tpad, int H, const float* __restrict__ wt, const float* __restrict__ b,
+    float* __restrict__ h_state, float* __restrict__ c_state) {
+  const int block = (int)blockIdx.x, n_gates = Tpad / kGateBT * (H / kGateU);
+  if (block < n_gates) velo_gates_block(block, xT, T, Tpad, H, wt, b, h_state, c_state);
+  else v0b_block<4, false>(block - n_gates, descs, dyn, items, v0part, 1e-5f, nullptr, nullptr, 0, fac_tab, term_tab, bscale);
 }
 
 // The same for many tensors, as fp32 matrix products (v_mfma_f32_32x32x2_f32): a block takes 64 tensors x 32 units (128 gate columns), its
@@ -954,9 +1014,10 @@ __device__ __forceinline__ float velo_fold_entry(const TDesc& d, const float* wm
   return 0.0f;
 }
 
-// R tensor rows a block (four where there are many: a block reads 0.7 MB of weights; in blocks of four waves there, which find a place
-// next to launches that fill the chip where blocks of sixteen wait: next to k_velo_stats on a streamed tensor 524 us and 102; by themselves 1024 tensors 24 and 49, 2000 55 and 59), each: controls = h Wc^T + bc, lr_mult = h.wlr + blr, the tensor's MLP =
-// 100 * mean_i(control_i * bank_i) (VeLO_MLP.py:92-126), then the weight blocks the element
+// R tensor rows a block: four where there are many, since a block reads 0.7 MB of weights; in blocks of four waves there, which
+// find a place next to launches that fill the chip where blocks of sixteen wait (next to k_velo_stats on a streamed tensor 524
+// us and 102; by themselves 1024 tensors 24 and 49, 2000 55 and 59).  Each row: controls = h Wc^T + bc, lr_mult = h.wlr + blr,
+// the tensor's MLP = 100 * mean_i(control_i * bank_i) (VeLO_MLP.py:92-126), then the weight blocks the element
 // kernels read: un-scaled first layer for k_terms, and the folded block (first-layer rows scaled
 // by rsqrt(1e-5 + mean f_c^2), param_scale = sqrt(mean p^2 + 1e-9), lr_mult).
 template <int R, int THREADS>

@@ -2513,6 +2513,14 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   const int n_chunks = (T + kMixRows - 1) / kMixRows;
   float* pmax = n_chunks > 1 ? P->at<float>(L.off_pmax) : nullptr;
   const size_t heads_lds = sizeof(float) * (H + K + 160 + 32 + 16 + 4 * (size_t)std::max(K, 160));
+  auto heads = [&](hipStream_t q, const double* tot, bool many) {
+    const bool rows4 = many && 4 * heads_lds <= 64 * 1024;
+    hipLaunchKernelGGL((rows4 ? k_velo_heads<4, kThreads> : k_velo_heads<1, kFoldThreads>), dim3(rows4 ? (T + 3) / 4 : T),
+                       dim3(rows4 ? kThreads : kFoldThreads),
+                       rows4 ? 4 * heads_lds : heads_lds, q, descs, T, H, K, step->lstm_h,
+                       nets->ctrl_wt, nets->ctrl_b, nets->lr_w, nets->lr_b, nets->bank, tot, canon, wfold,
+                       step->controls_out, step->lr_mult_out, wmix);
+  };
   // The LSTM from the tensors' 30 input features on: input mixing across tensors, cell, heads.
   auto lstm = [&](hipStream_t q, const double* tot, bool timed) {
     if (pmax != nullptr)
@@ -2528,12 +2536,7 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
       hipLaunchKernelGGL(k_velo_gates, dim3((L.Tpad / kGateBT) * (H / kGateU)), dim3(kThreads), 0, q, xT, T, L.Tpad, H,
                          nets->lstm_wt, nets->lstm_b, step->lstm_h, step->lstm_c);
     if (timed) (void)mark();
-    const bool rows4 = many && 4 * heads_lds <= 64 * 1024;
-    hipLaunchKernelGGL((rows4 ? k_velo_heads<4, kThreads> : k_velo_heads<1, kFoldThreads>), dim3(rows4 ? (T + 3) / 4 : T),
-                       dim3(rows4 ? kThreads : kFoldThreads),
-                       rows4 ? 4 * heads_lds : heads_lds, q, descs, T, H, K, step->lstm_h,
-                       nets->ctrl_wt, nets->ctrl_b, nets->lr_w, nets->lr_b, nets->bank, tot, canon, wfold,
-                       step->controls_out, step->lr_mult_out, wmix);
+    heads(q, tot, many);
     if (timed) (void)mark();
   };
   // clip_norm is 0 for VeLO tensors: k_p0 clamps directly; its norm / flag outputs are not used
@@ -2558,28 +2561,46 @@ extern "C" int pylo_mi355_velo_step(PyloPlan* P, const PyloTensorArgs* args, con
   HIP_TRY(mark());
   if (L.fused && P->stats_carried) {
     // The LSTM's inputs are sums over the parameters and accumulators as they stand before the step: the
-    // previous step's apply items left them.  It runs next to the gradient sums, on the plan's own stream.
-    HIP_TRY(hipEventRecord(P->ev_fork, s));
-    HIP_TRY(hipStreamWaitEvent(P->side, P->ev_fork, 0));
-    if (!L.seg_items.empty())
-      hipLaunchKernelGGL(k_stat_segsum<kNewSumW>, dim3((unsigned)L.seg_items.size()), dim3(kThreads), 0, P->side, descs,
-                         P->at<Item>(L.off_seg_items), (const double*)newsum, P->at<double>(L.off_segtot));
-    const bool wide_feat = n_p0 + n_nd + T <= kFeatWide;
-    hipLaunchKernelGGL(wide_feat ? k_velo_feat<kFoldThreads> : k_velo_feat<kThreads>, dim3(T), dim3(wide_feat ? kFoldThreads : kThreads),
-                       0, P->side, descs, dyn, T, (const double*)newsum,
-                       (const double*)P->at<double>(L.off_segtot), piv, ls, vs,
-                       xfeat, H, nets->mix2_wt, nets->mix2_b, nets->fmix_wt, nets->fmix_b, mixbuf, P->at<int>(L.off_sync));
-    lstm(P->side, nullptr, false);
-    HIP_TRY(hipEventRecord(P->ev_join, P->side));
-    gradient_sums();
-    HIP_TRY(mark());
-    if (int rc = factor_tables()) return rc;
-    // the streamed tensors' statistics need nothing from the LSTM either: its launches have this one to run under as well
+    // previous step's apply items left them.  It runs next to the gradient sums, on the plan's own stream or, where there are
+    // few blocks, in the launches of the caller's.
     const unsigned n_big = (unsigned)L.big_items.size();
-    if (n_big > 0)
-      hipLaunchKernelGGL((L.split ? k_velo_stats<false, true> : k_velo_stats<false, false>), dim3(n_big), dim3(kThreads), 0, s, descs, dyn,
-                         P->at<Item>(L.off_big_items), fac_tab, dec, stats);
-    HIP_TRY(hipStreamWaitEvent(s, P->ev_join, 0));
+    const bool paired = n_p0 + n_nd + T <= kVeloPaired && T <= kMixRows && n_big == 0;
+    const hipStream_t q = paired ? s : P->side;
+    if (!paired) {
+      HIP_TRY(hipEventRecord(P->ev_fork, s));
+      HIP_TRY(hipStreamWaitEvent(q, P->ev_fork, 0));
+    }
+    if (!L.seg_items.empty())
+      hipLaunchKernelGGL(k_stat_segsum<kNewSumW>, dim3((unsigned)L.seg_items.size()), dim3(kThreads), 0, q, descs,
+                         P->at<Item>(L.off_seg_items), (const double*)newsum, P->at<double>(L.off_segtot));
+    if (paired) {
+      const int n_mix = (H / 64) * (L.Tpad / kGateBT), n_gates = (L.Tpad / kGateBT) * (H / kGateU);
+      hipLaunchKernelGGL((L.split ? k_velo_p0_feat<true> : k_velo_p0_feat<false>), dim3(T + n_p0 + n_nd), dim3(kFoldThreads), 0, s, descs, dyn,
+                         p0_items, part, gsq, flag, gl, nd_items, n_p0, T, (const double*)newsum, (const double*)P->at<double>(L.off_segtot),
+                         piv, ls, vs, xfeat, H, nets->mix2_wt, nets->mix2_b, nets->fmix_wt, nets->fmix_b, mixbuf, P->at<int>(L.off_sync));
+      HIP_TRY(mark());
+      hipLaunchKernelGGL(k_velo_v0a_mix, dim3(n_mix + n_v0a), dim3(kThreads), 0, s, descs, dyn, v0a_items, part, gl, dec, v0part,
+                         (const float*)mixbuf, T, L.Tpad, H, step->lstm_h, xT, ls);
+      HIP_TRY(mark());
+      hipLaunchKernelGGL(k_velo_v0b_gates, dim3(n_gates + n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, v0part, fac_tab, term_tab,
+                         bscale, xT, T, L.Tpad, H, nets->lstm_wt, nets->lstm_b, step->lstm_h, step->lstm_c);
+      heads(s, nullptr, false);
+      HIP_TRY(mark());
+    } else {
+      hipLaunchKernelGGL(k_velo_feat, dim3(T), dim3(kThreads), 0, P->side, descs, dyn, T, (const double*)newsum,
+                         (const double*)P->at<double>(L.off_segtot), piv, ls, vs,
+                         xfeat, H, nets->mix2_wt, nets->mix2_b, nets->fmix_wt, nets->fmix_b, mixbuf, P->at<int>(L.off_sync));
+      lstm(P->side, nullptr, false);
+      HIP_TRY(hipEventRecord(P->ev_join, P->side));
+      gradient_sums();
+      HIP_TRY(mark());
+      if (int rc = factor_tables()) return rc;
+      // the streamed tensors' statistics need nothing from the LSTM either: its launches have this one to run under as well
+      if (n_big > 0)
+        hipLaunchKernelGGL((L.split ? k_velo_stats<false, true> : k_velo_stats<false, false>), dim3(n_big), dim3(kThreads), 0, s, descs, dyn,
+                           P->at<Item>(L.off_big_items), fac_tab, dec, stats);
+      HIP_TRY(hipStreamWaitEvent(s, P->ev_join, 0));
+    }
     if (n_v0b > 0)
       hipLaunchKernelGGL(k_terms<4>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, bscale, canon, kVCanon, term_tab);
     HIP_TRY(mark());
