@@ -26,18 +26,34 @@ __host__ __device__ constexpr bool adafac_channel(int c) { return c != 1 && c !=
 // b_eff = b1 + w_time^T tanh(step / ts - 1)   (AdafacLO_naive.py:81-87,226)
 // One block per tensor: `step` >= 0 is the counter of every tensor, a negative `step` takes each
 // tensor's own counter from its argument record (bc1; AdafacLO_cuda.py:304-305,400 keeps one per parameter).
-__global__ __launch_bounds__(64) void k_adafac_bias(const float* __restrict__ net, float step,
-                                                    const PyloTensorArgs* __restrict__ dyn,
-                                                    float* __restrict__ bias_all) {
+__device__ __forceinline__ void adafac_bias_block(int t, const float* __restrict__ net, float step,
+                                                  const PyloTensorArgs* __restrict__ dyn, float* __restrict__ bias_all) {
   const float ts[11] = {1.f, 3.f, 10.f, 30.f, 100.f, 300.f, 1000.f, 3000.f, 10000.f, 30000.f, 100000.f};
   const int j = threadIdx.x;
   if (j >= kAH) return;
-  if (step < 0.0f) step = dyn[blockIdx.x].bc1;
-  float* bias_eff = bias_all + (size_t)blockIdx.x * kAH;
+  if (step < 0.0f) step = dyn[t].bc1;
+  float* bias_eff = bias_all + (size_t)t * kAH;
   float acc = net[kAB1 + j];
 #pragma unroll
   for (int q = 0; q < 11; ++q) acc = fmaf(tanhf(step / ts[q] - 1.0f), net[kAWT + q * kAH + j], acc);
   bias_eff[j] = acc;
+}
+
+// k_v0a and, in the blocks behind its own, the tensors' biases, which nothing before k_v0b asks for.  NORM: and k_gnorm.  The
+// step of a small network is its launches: MLP 784-128-128-10 under ELO took twelve, 3 us of host time each and 4 to 8 us of the
+// GPU, now eight (this one, the norm, the fold, both apply passes).
+template <bool NORM>
+__global__ __launch_bounds__(kThreads) void k_adafac_v0a(const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn,
+                                                         const Item* __restrict__ items, int n_items, const float* __restrict__ part,
+                                                         NormArgs na, Globals* __restrict__ gl, PyloDecays dec,
+                                                         double* __restrict__ v0part, const float* __restrict__ net, float step,
+                                                         float* __restrict__ bias_all) {
+  __shared__ Globals own;
+  if constexpr (NORM) own_norm(na, gl, &own);
+  const int block = (int)blockIdx.x;
+  if (block >= n_items) adafac_bias_block(block - n_items, net, step, dyn, bias_all);
+  else if constexpr (NORM) v0a_block(block, descs, dyn, items, part, &own, dec, v0part);
+  else v0a_block(block, descs, dyn, items, part, gl, dec, v0part);
 }
 
 template <int V, bool ND>
@@ -175,22 +191,39 @@ __global__ __launch_bounds__(kThreads) void k_adafac_stats(const TDesc* __restri
   }
 }
 
-// Per tensor: first-layer rows scaled by rsqrt(1e-5 + mean f_c^2) (AdafacLO_naive.py:90-92,301).
-__global__ __launch_bounds__(kThreads) void k_adafac_fold(const TDesc* __restrict__ descs,
-                                                          const PyloTensorArgs* __restrict__ dyn,
-                                                          const double* __restrict__ totals,
-                                                          const float* __restrict__ net, float* __restrict__ wfold) {
+// Per tensor: the sums of its blocks, and first-layer rows scaled by rsqrt(1e-5 + mean f_c^2) (AdafacLO_naive.py:90-92,301).
+__global__ __launch_bounds__(kFoldThreads) void k_adafac_fold(const TDesc* __restrict__ descs,
+                                                              const PyloTensorArgs* __restrict__ dyn,
+                                                              const double* __restrict__ stats_part,
+                                                              const double* __restrict__ seg_tot,
+                                                              const float* __restrict__ net, float* __restrict__ wfold) {
+  constexpr int G = kFoldThreads / kStatW;  // 25 groups x 40 sums = 1000 threads
+  __shared__ double part[G][kStatW];
   __shared__ float sc[32];
   const int t = blockIdx.x;
   const TDesc d = descs[t];
   if (dyn[t].grad == nullptr) return;
+  const int c = threadIdx.x % kStatW, gI = threadIdx.x / kStatW;
+  if (gI < G) {
+    double s = 0.0;
+    if (c < 30) {
+      int n_rows;
+      const double* rows = stat_rows(d, stats_part, seg_tot, n_rows);
+#pragma unroll 16
+      for (int b = gI; b < n_rows; b += G) s += rows[(size_t)b * kStatW + c];
+    }
+    part[gI][c] = s;
+  }
+  __syncthreads();
   if (threadIdx.x < 30) {
+    double s = 0.0;
+    for (int g2 = 0; g2 < G; ++g2) s += part[g2][threadIdx.x];
     const double n = (double)(d.n > 0 ? d.n : 1);
-    sc[threadIdx.x] = rsq(1e-5f + (float)(totals[(size_t)t * kStatW + threadIdx.x] / n));
+    sc[threadIdx.x] = rsq(1e-5f + (float)(s / n));
   }
   __syncthreads();
   float* w = wfold + (size_t)t * kAFold;
-  for (int i = threadIdx.x; i < 30 * kAH; i += kThreads) w[i] = net[kAW1 + i] * sc[i / kAH];
+  for (int i = threadIdx.x; i < 30 * kAH; i += kFoldThreads) w[i] = net[kAW1 + i] * sc[i / kAH];
   if (threadIdx.x < 32) w[30 * kAH + threadIdx.x] = threadIdx.x < 30 ? sc[threadIdx.x] : 0.0f;
 }
 
@@ -1040,12 +1073,10 @@ __device__ __forceinline__ void adafac_apply_lin(const TDesc& d, const PyloTenso
   }
 }
 
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_adafac_apply_lin(
-    const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const Item* __restrict__ items,
-    const float* __restrict__ fac_tab, const float* __restrict__ term_tab, PyloDecays dec,
-    const float* __restrict__ wfold, const float* __restrict__ net, const float* __restrict__ bias_eff,
-    const Globals* __restrict__ gl) {
-  const Item it = items[blockIdx.x];
+__device__ __forceinline__ void adafac_lin_block(
+    const Item& it, const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const float* __restrict__ fac_tab,
+    const float* __restrict__ term_tab, const PyloDecays& dec, const float* __restrict__ wfold, const float* __restrict__ net,
+    const float* __restrict__ bias_eff, const Globals* __restrict__ gl) {
   TDesc d = descs[it.tensor];
   const PyloTensorArgs a = dyn[it.tensor];
   if (a.grad == nullptr) return;
@@ -1057,6 +1088,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   if (d.mode == kModeFac2D) adafac_apply_lin<kModeFac2D>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
   else if (d.mode == kModeFacND) adafac_apply_lin<kModeFacND>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
   else adafac_apply_lin<kModeVec>(d, a, base, it.b, e, dec, fac_tab, term_tab, w, net, be);
+}
+
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_adafac_apply_lin(
+    const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const Item* __restrict__ items,
+    const float* __restrict__ fac_tab, const float* __restrict__ term_tab, PyloDecays dec,
+    const float* __restrict__ wfold, const float* __restrict__ net, const float* __restrict__ bias_eff,
+    const Globals* __restrict__ gl) {
+  adafac_lin_block(items[blockIdx.x], descs, dyn, fac_tab, term_tab, dec, wfold, net, bias_eff, gl);
 }
 
 __global__ __launch_bounds__(kThreads) void k_adafac_apply(const TDesc* __restrict__ descs,
@@ -1111,6 +1150,27 @@ void k_adafac_apply_tile(const TDesc* __restrict__ descs, const PyloTensorArgs* 
       adafac_apply_tile_hf<PER, kStoreF32>(d, a, task, make_ema(dec), fac_tab, term_tab, w, net);
   } else
     adafac_apply_tile(d, a, task, make_ema(dec), fac_tab, term_tab, wfold + (size_t)it.tensor * kAFold, net, xch[wave]);
+}
+
+// Both walks of a plan of fp32 tensors in one launch, blocks of the tiles first: where all of them find a place at once the two
+// launches ran one after the other for nothing.  (Larger plans: each walk compiled by itself.)
+constexpr int kApplyTogether = 512;   // two blocks a CU
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_adafac_apply_both(
+    const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const Item* __restrict__ tiles, int n_tiles,
+    const Item* __restrict__ lines, const float* __restrict__ fac_tab, const float* __restrict__ term_tab, PyloDecays dec,
+    const float* __restrict__ wfold, const float* __restrict__ net, const float* __restrict__ bias_eff, const Globals* __restrict__ gl) {
+  const int block = (int)blockIdx.x;
+  if (block >= n_tiles) {
+    adafac_lin_block(lines[block - n_tiles], descs, dyn, fac_tab, term_tab, dec, wfold, net, bias_eff, gl);
+    return;
+  }
+  const Item it = tiles[block];
+  TDesc d = descs[it.tensor];
+  const PyloTensorArgs a = dyn[it.tensor];
+  const int task = it.a * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (a.grad == nullptr || task >= d.atile_ntask) return;
+  set_grad_scale(d, a, gl, it.tensor);
+  adafac_apply_tile_hf<false, kStoreF32>(d, a, task, make_ema(dec), fac_tab, term_tab, wfold + (size_t)it.tensor * kAFold, net);
 }
 
 }  // namespace pylo

@@ -350,16 +350,13 @@ __global__ __launch_bounds__(kThreads) void k_p0(const TDesc* __restrict__ descs
   p0_block<TYPED, SPLIT>((int)blockIdx.x, descs, dyn, items, part, gsq_part, flag_part, gl, pass, nd_items, n_main);
 }
 
-// use_flags == 0: the caller has shown that no element can exceed its clamp after scaling (the scaled
+// The global norm and the flag of the exact pass, from all blocks' partials in a fixed order: to `to` by thread 0, in
+// LDS or memory.  use_flags == 0: the caller has shown that no element can exceed its clamp after scaling (the scaled
 // gradient is bounded by clip_norm), so the exact pass never runs and the flags are ignored.
-__global__ __launch_bounds__(kThreads) void k_gnorm(const double* __restrict__ gsq_part,
-                                                    const int* __restrict__ flag_part, int nblk,
-                                                    Globals* __restrict__ gl, int use_flags,
-                                                    int* __restrict__ sync, int n_sync) {
+__device__ __forceinline__ void gnorm_block(const double* __restrict__ gsq_part, const int* __restrict__ flag_part, int nblk,
+                                            int use_flags, Globals* to) {
   __shared__ double red[kWaves];
   __shared__ int fred[kWaves];
-  // the counters and flags of the fused element pass that follows (k_celo2_elem) start at zero
-  for (int i = threadIdx.x; i < n_sync; i += kThreads) sync[i] = 0;
   double s = 0.0;
   int f = 0;
   // sixteen partials are fetched before the first is added: the one block is bound by load latency
@@ -380,9 +377,50 @@ __global__ __launch_bounds__(kThreads) void k_gnorm(const double* __restrict__ g
   if ((threadIdx.x & 63) == 0) { red[threadIdx.x >> 6] = s; fred[threadIdx.x >> 6] = f; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    gl->gnorm = (float)sqrt((red[0] + red[1]) + (red[2] + red[3]));
-    gl->flag = use_flags ? (fred[0] | fred[1] | fred[2] | fred[3]) : 0;
+    to->gnorm = (float)sqrt((red[0] + red[1]) + (red[2] + red[3]));
+    to->flag = use_flags ? (fred[0] | fred[1] | fred[2] | fred[3]) : 0;
   }
+}
+
+// What a launch behind k_p0 needs to work the norm out for itself.  `sync`: counters and flags of the fused element pass that
+// follows (k_celo2_elem), which start at zero.
+struct NormArgs {
+  const double* gsq_part;
+  const int* flag_part;
+  int nblk, use_flags;
+  int* sync;
+  int n_sync;
+};
+
+__global__ __launch_bounds__(kThreads) void k_gnorm(NormArgs na, Globals* __restrict__ gl) {
+  for (int i = threadIdx.x; i < na.n_sync; i += kThreads) na.sync[i] = 0;
+  gnorm_block(na.gsq_part, na.flag_part, na.nblk, na.use_flags, gl);
+}
+
+// Where k_p0 had few blocks, every block of the launch behind it adds their partials up for itself -- the same sum in the same
+// order -- and one leaves the result for the launches that follow: a launch of one block and the gap behind it, 4 to 8 us of a
+// step of 60 to 150, for 1 us of loads that hit L2.  (kNormBlocks: two partials a thread; at 512 blocks of k_p0 3 MB for all.)
+constexpr int kNormBlocks = 512;
+__device__ __forceinline__ void own_norm(const NormArgs& na, Globals* __restrict__ gl, Globals* own) {
+  gnorm_block(na.gsq_part, na.flag_part, na.nblk, na.use_flags, own);
+  __syncthreads();
+  if (blockIdx.x != 0) return;
+  for (int i = threadIdx.x; i < na.n_sync; i += kThreads) na.sync[i] = 0;
+  if (threadIdx.x == 0) {
+    gl->gnorm = own->gnorm;
+    gl->flag = own->flag;
+  }
+}
+
+// k_gnorm and the exact pass
+template <bool TYPED, bool SPLIT>
+__global__ __launch_bounds__(kThreads) void k_gnorm_p0(const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn,
+                                                       const Item* __restrict__ items, float* __restrict__ part, NormArgs na,
+                                                       Globals* __restrict__ gl) {
+  __shared__ Globals own;
+  own_norm(na, gl, &own);
+  if (own.flag == 0) return;
+  p0_block<TYPED, SPLIT>((int)blockIdx.x, descs, dyn, items, part, nullptr, nullptr, &own, 1, nullptr, na.nblk);
 }
 
 // Per-tensor norm clipping (PYLO_F_TENSOR_NORM; AdafacLO_naive.py:199-200 calls torch.nn.utils.clip_grad_norm_
@@ -598,6 +636,16 @@ __global__ __launch_bounds__(kV0aThreads) void k_v0a(const TDesc* __restrict__ d
                                                   const Globals* __restrict__ gl, PyloDecays dec,
                                                   double* __restrict__ v0part) {
   v0a_block((int)blockIdx.x, descs, dyn, items, part, gl, dec, v0part);
+}
+
+// k_gnorm and k_v0a
+__global__ __launch_bounds__(kThreads) void k_gnorm_v0a(const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn,
+                                                        const Item* __restrict__ items, const float* __restrict__ part, NormArgs na,
+                                                        Globals* __restrict__ gl, PyloDecays dec, double* __restrict__ v0part) {
+  static_assert(kV0aThreads == kThreads, "one block size");
+  __shared__ Globals own;
+  own_norm(na, gl, &own);
+  v0a_block((int)blockIdx.x, descs, dyn, items, part, &own, dec, v0part);
 }
 
 // Where entry i of vector `which` of tensor d lives in the factor / term tables.

@@ -594,7 +594,6 @@ __global__ __launch_bounds__(kFoldThreads) void k_lo_reduce(const TDesc* __restr
     totals[(size_t)t * kStatW + threadIdx.x] = s;
   }
   __syncthreads();
-  if (xfeat == nullptr) return;
   velo_row_features<kFoldThreads>(d, a, t, T, tot, nullptr, piv_out, ls, st, xfeat, H, w2t, b2, wft, bf, mixbuf, xs);
 }
 

@@ -1639,8 +1639,8 @@ static const char* kVeloLaunches[] = {"k_p0(sums)", "k_p0_nd", "k_v0a", "k_v0b",
                                       "k_velo_apply"};
 
 static const char* kVeloFusedLaunches[] = {"k_p0(sums) | LSTM", "k_v0a", "k_v0b", "k_terms", "k_velo_elem"};
-static const char* kAdafacLaunches[] = {"k_p0(sums)", "k_p0_nd", "k_v0a", "k_adafac_bias", "k_v0b", "k_adafac_stats",
-                                        "k_lo_reduce", "k_adafac_fold", "k_adafac_apply"};
+static const char* kAdafacLaunches[] = {"k_p0(sums)", "k_p0_nd", "k_adafac_v0a", "k_v0b", "k_adafac_stats",
+                                        "k_adafac_fold", "k_adafac_apply"};
 
 int pylo_mi355_plan_num_launches(const PyloPlan* P) {
   if (!P) return -1;
@@ -1904,6 +1904,9 @@ F variant(bool typed, bool split, F plain, F split_only, F typed_only, F both) {
 inline auto p0_kernel(bool typed, bool split) {
   return variant(typed, split, k_p0<false, false>, k_p0<false, true>, k_p0<true, false>, k_p0<true, true>);
 }
+inline auto norm_p0_kernel(bool typed, bool split) {
+  return variant(typed, split, k_gnorm_p0<false, false>, k_gnorm_p0<false, true>, k_gnorm_p0<true, false>, k_gnorm_p0<true, true>);
+}
 
 extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, const PyloDecays* decays,
                                      const float* mlp, void* stream) {
@@ -1954,15 +1957,21 @@ extern "C" int pylo_mi355_celo2_step(PyloPlan* P, const PyloTensorArgs* args, co
     hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0 + n_tail), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag,
                        gl, clips ? 0 : 2, nd_items, n_p0);
   HIP_TRY(mark());
-  hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, gsq, flag, n_p0, gl, exact_pass ? 1 : 0,
-                     P->at<int>(L.off_sync), 2 * P->T);
+  const NormArgs na{gsq, flag, n_p0, exact_pass ? 1 : 0, P->at<int>(L.off_sync), 2 * P->T};
+  const bool few = n_p0 > 0 && n_p0 <= kNormBlocks, norm_p0 = few && exact_pass;
+  const bool norm_v0a = few && !exact_pass && n_v0a > 0 && !(n_nd > 0 && clips);
+  if (!norm_p0 && !norm_v0a) hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, na, gl);
   HIP_TRY(mark());
-  if (n_p0 > 0 && exact_pass)
+  if (norm_p0)
+    hipLaunchKernelGGL(norm_p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, na, gl);
+  else if (n_p0 > 0 && exact_pass)
     hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
                        (const Item*)nullptr, n_p0);
   if (n_nd > 0 && clips) hipLaunchKernelGGL(k_p0_nd, dim3(n_nd), dim3(kThreads), 0, s, descs, dyn, nd_items, part, gl);
   HIP_TRY(mark());
-  if (n_v0a > 0)
+  if (norm_v0a)
+    hipLaunchKernelGGL(k_gnorm_v0a, dim3(n_v0a), dim3(kThreads), 0, s, descs, dyn, v0a_items, part, na, gl, dec, v0part);
+  else if (n_v0a > 0)
     hipLaunchKernelGGL(k_v0a, dim3(n_v0a), dim3(kV0aThreads), 0, s, descs, dyn, v0a_items, part, gl, dec, v0part);
   HIP_TRY(mark());
   const auto v0b = L.slice_runs ? k_v0b<8, true> : k_v0b<8>;
@@ -2697,14 +2706,11 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   BScale* bscale = P->at<BScale>(L.off_bscale);
   double* stats = P->at<double>(L.off_stats);
   float* wfold = P->at<float>(L.off_wfold);
-  double* totals = P->at<double>(L.off_totals);
   float* bias_eff = P->at<float>(L.off_xfeat);  // [T][32]; the LSTM feature buffer is unused by this kind
   const int n_p0 = (int)L.p0_items.size(), n_nd = (int)L.nd_items.size(), n_el = (int)L.el_items.size();
   const int n_v0a = (int)L.v0a_items.size(), n_v0b = (int)L.v0b_items.size();
   const int T = P->T;
   const PyloDecays dec = *decays;
-  VeloStep vs;
-  std::memset(&vs, 0, sizeof(vs));
   const bool in_place = L.in_place;   // tensors of 16-bit storage without staging (the fp16 matrix instructions' walk only)
   Marks mark(P, s);
 
@@ -2727,20 +2733,27 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   if (clips && L.tensor_norm) {
     // every tensor against its own norm (AdafacLO_naive.py:199-200): no clamp on such tensors, no exact pass
     hipLaunchKernelGGL(k_tnorm, dim3(T), dim3(kThreads), 0, s, descs, dyn, gsq, gl, P->at<float>(L.off_tscale));
-  } else if (clips) {
-    const bool exact_pass = exact_pass_possible(P, args);
-    hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, gsq, flag, n_p0, gl, exact_pass ? 1 : 0, (int*)nullptr, 0);
-    if (n_p0 > 0 && exact_pass)
-      hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
-                         (const Item*)nullptr, n_p0);
+  }
+  NormArgs na{gsq, flag, n_p0, 0, nullptr, 0};
+  bool norm_v0a = false;
+  if (clips && !L.tensor_norm) {
+    const bool exact_pass = exact_pass_possible(P, args), few = n_p0 > 0 && n_p0 <= kNormBlocks;
+    na.use_flags = exact_pass ? 1 : 0;
+    norm_v0a = few && !exact_pass && n_nd == 0;
+    if (few && exact_pass) {
+      hipLaunchKernelGGL(norm_p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, na, gl);
+    } else if (!norm_v0a) {
+      hipLaunchKernelGGL(k_gnorm, dim3(1), dim3(kThreads), 0, s, na, gl);
+      if (n_p0 > 0 && exact_pass)
+        hipLaunchKernelGGL(p0_kernel(in_place, L.split), dim3(n_p0), dim3(kThreads), 0, s, descs, dyn, p0_items, part, gsq, flag, gl, 1,
+                           (const Item*)nullptr, n_p0);
+    }
   }
   HIP_TRY(mark());
   if (n_nd > 0 && clips) hipLaunchKernelGGL(k_p0_nd, dim3(n_nd), dim3(kThreads), 0, s, descs, dyn, nd_items, part, gl);
   HIP_TRY(mark());
-  if (n_v0a > 0)
-    hipLaunchKernelGGL(k_v0a, dim3(n_v0a), dim3(kV0aThreads), 0, s, descs, dyn, v0a_items, part, gl, dec, v0part);
-  HIP_TRY(mark());
-  hipLaunchKernelGGL(k_adafac_bias, dim3(T), dim3(64), 0, s, net, P->dsteps.counters ? -1.0f : step, dyn, bias_eff);
+  hipLaunchKernelGGL((norm_v0a ? k_adafac_v0a<true> : k_adafac_v0a<false>), dim3(n_v0a + T), dim3(kThreads), 0, s, descs, dyn, v0a_items,
+                     n_v0a, part, na, gl, dec, v0part, net, P->dsteps.counters ? -1.0f : step, bias_eff);
   HIP_TRY(mark());
   if (n_v0b > 0)
     hipLaunchKernelGGL(k_v0b<kAH>, dim3(n_v0b), dim3(kThreads), 0, s, descs, dyn, v0b_items, v0part, 1e-5f,
@@ -2756,17 +2769,17 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   double* seg_tot = P->at<double>(L.off_segtot);
   const int n_seg = (int)L.seg_items.size();
   if (n_seg > 0) hipLaunchKernelGGL(k_stat_segsum<kStatW>, dim3(n_seg), dim3(kThreads), 0, s, descs, seg_items, stats, seg_tot);
-  hipLaunchKernelGGL(k_lo_reduce, dim3(T), dim3(kFoldThreads), 0, s, descs, dyn, T, stats, seg_tot, totals, LossState{}, vs,
-                     (float*)nullptr, 0, (const float*)nullptr, (const float*)nullptr, (const float*)nullptr,
-                     (const float*)nullptr, (float*)nullptr, (float*)nullptr);
-  HIP_TRY(mark());
-  hipLaunchKernelGGL(k_adafac_fold, dim3(T), dim3(kThreads), 0, s, descs, dyn, totals, net, wfold);
+  hipLaunchKernelGGL(k_adafac_fold, dim3(T), dim3(kFoldThreads), 0, s, descs, dyn, stats, seg_tot, net, wfold);
   HIP_TRY(mark());
   const Item* ap_items = P->at<Item>(L.off_ap_items);
   const Item* ga_items = P->at<Item>(L.off_ga_items);
   const Item* pp_items = P->at<Item>(L.off_pp_items);
   const int n_ap = (int)L.ap_items.size(), n_ga = (int)L.ga_items.size(), n_pp = (int)L.pp_items.size();
-  if (n_ga > 0 && L.lin_matrix)
+  const bool both = n_ga > 0 && n_ap > 0 && n_ga + n_ap <= kApplyTogether && L.lin_matrix && P->adafac_hf && !in_place;
+  if (both)
+    hipLaunchKernelGGL(k_adafac_apply_both, dim3(n_ap + n_ga), dim3(kThreads), 0, s, descs, dyn, ap_items, n_ap, ga_items, fac_tab, term_tab,
+                       dec, wfold, net, (const float*)bias_eff, gl);
+  else if (n_ga > 0 && L.lin_matrix)
     hipLaunchKernelGGL(k_adafac_apply_lin, dim3(n_ga), dim3(kThreads), 0, s, descs, dyn, ga_items, fac_tab, term_tab, dec,
                        wfold, net, (const float*)bias_eff, gl);
   else if (n_ga > 0)
@@ -2775,7 +2788,7 @@ extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, c
   if (n_pp > 0)
     hipLaunchKernelGGL((k_adafac_apply_tile<true, true>), dim3(n_pp), dim3(kThreads), 0, s, descs, dyn, pp_items, fac_tab,
                        term_tab, dec, wfold, net, gl);
-  if (n_ap > 0) {
+  if (n_ap > 0 && !both) {
     const auto apply = in_place       ? k_adafac_apply_tile<true, false, true>
                        : P->adafac_hf ? k_adafac_apply_tile<true, false, false>
                                       : k_adafac_apply_tile<false, false, false>;
