@@ -1476,6 +1476,8 @@ struct PyloPlan {
   hipEvent_t ns_fork = nullptr, ns_join[4] = {nullptr, nullptr, nullptr, nullptr};
   // the per-slice finishing launches next to the matrices' products, where the groups leave a hardware queue free
   hipStream_t slice_side = nullptr;
+  hipStream_t small_side = nullptr;   // two of the small matrices' classes (enqueue_small)
+  hipEvent_t small_fork = nullptr, small_join = nullptr;
   hipEvent_t slice_fork = nullptr, slice_join = nullptr;
 
   template <class Tp>
@@ -1599,6 +1601,13 @@ int pylo_mi355_plan_create(int kind, const PyloTensorShape* shapes, int n_tensor
     if (e == hipSuccess) e = hipEventCreateWithFlags(&P->slice_fork, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&P->slice_join, hipEventDisableTiming);
   }
+  // the small matrices' classes on two streams (enqueue_small), with the caller's and slice_side three
+  const bool small_a = !L.sm_items[0].empty() || !L.sm_items[3].empty(), small_b = !L.sm_items[1].empty() || !L.sm_items[2].empty();
+  if (e == hipSuccess && small_a && small_b && ns_streams <= 1) {
+    e = hipStreamCreateWithFlags(&P->small_side, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&P->small_fork, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&P->small_join, hipEventDisableTiming);
+  }
   if (e != hipSuccess) {
     pylo_mi355_plan_destroy(P);
     return fail(std::string("plan_create: ") + hipGetErrorString(e));
@@ -1618,6 +1627,9 @@ int pylo_mi355_plan_destroy(PyloPlan* P) {
   if (P->slice_fork) (void)hipEventDestroy(P->slice_fork);
   if (P->slice_join) (void)hipEventDestroy(P->slice_join);
   if (P->slice_side) (void)hipStreamDestroy(P->slice_side);
+  if (P->small_side) (void)hipStreamDestroy(P->small_side);
+  if (P->small_fork) (void)hipEventDestroy(P->small_fork);
+  if (P->small_join) (void)hipEventDestroy(P->small_join);
   for (int g = 0; g < 4; ++g) {
     if (P->ns_join[g]) (void)hipEventDestroy(P->ns_join[g]);
     if (P->ns_side[g]) (void)hipStreamDestroy(P->ns_side[g]);
@@ -2093,7 +2105,9 @@ int small_lds_once() {
   return 0;
 }
 
-// The launches of the small matrices (k_ns_small.h): one per class, largest first.
+// The launches of the small matrices (k_ns_small.h): one per class, largest first.  A class is a launch of chains that leaves
+// most of the chip idle (three thousand matrices: 102, 120, 50 and 71 us one after the other, 345 us next to 235 of tiled products): where
+// the groups of tiled products have left a queue, the middle two run on a stream of their own, which the caller joins.
 int enqueue_small(PyloPlan* P, hipStream_t s, const TDesc* descs, const PyloTensorArgs* dyn, const float* coeffs, int ns_iters,
                   float ns_eps) {
   const Layout& L = P->L;
@@ -2115,7 +2129,11 @@ int enqueue_small(PyloPlan* P, hipStream_t s, const TDesc* descs, const PyloTens
     if (*std::max_element(chains.begin(), chains.end()) == 1) st.n_pairs = 0;
     st.n_chains = ns_iters - st.n_pairs;
   }
-  auto launch = [&](auto kern, int cls, int threads, int lds) {
+  if (P->small_side != nullptr) {
+    HIP_TRY(hipEventRecord(P->small_fork, s));
+    HIP_TRY(hipStreamWaitEvent(P->small_side, P->small_fork, 0));
+  }
+  auto launch = [&](auto kern, int cls, int threads, int lds, hipStream_t s) {
     if (!L.sm_items[cls].empty())
       hipLaunchKernelGGL(kern, dim3((unsigned)L.sm_items[cls].size()), dim3(threads), lds, s, P->at<NsSmall>(L.off_sm_mats),
                          P->at<NsSmallItem>(L.off_sm_items[cls]), descs, dyn, P->at<float>(L.off_sm_part),
@@ -2123,16 +2141,18 @@ int enqueue_small(PyloPlan* P, hipStream_t s, const TDesc* descs, const PyloTens
                          L.sm_meets[cls] ? P->at<int>(L.off_sm_sync) + L.sm_ticket0 + cls : (int*)nullptr);
   };
   const ThinStep thin{st.c0, st.c1, st.c2, ns_eps, ns_iters};
-  auto launch_thin = [&](auto kern, int cls, int lds) {
+  auto launch_thin = [&](auto kern, int cls, int lds, hipStream_t s) {
     if (!L.sm_items[cls].empty())
       hipLaunchKernelGGL(kern, dim3((unsigned)L.sm_items[cls].size()), dim3(kThreads), lds, s, P->at<NsSmall>(L.off_sm_mats),
                          P->at<NsSmallItem>(L.off_sm_items[cls]), descs, dyn, P->at<float>(L.off_sm_part), P->at<int>(L.off_sm_sync),
                          thin, orth, L.sm_meets[cls] ? P->at<int>(L.off_sm_sync) + L.sm_ticket0 + cls : (int*)nullptr);
   };
-  launch(k_ns_small<4, 2, 1>, 3, SmLarge::kThr, SmLarge::kLds);
-  launch(k_ns_small<2, 1, 2>, 2, SmMid::kThr, SmMid::kLds);
-  launch_thin(k_ns_thin<2>, 1, ThinDims<2>::kLds);
-  launch_thin(k_ns_thin<1>, 0, ThinDims<1>::kLds);
+  const hipStream_t mid = P->small_side != nullptr ? P->small_side : s;
+  launch(k_ns_small<4, 2, 1>, 3, SmLarge::kThr, SmLarge::kLds, s);
+  launch(k_ns_small<2, 1, 2>, 2, SmMid::kThr, SmMid::kLds, mid);
+  launch_thin(k_ns_thin<2>, 1, ThinDims<2>::kLds, mid);
+  launch_thin(k_ns_thin<1>, 0, ThinDims<1>::kLds, s);
+  if (P->small_side != nullptr) HIP_TRY(hipEventRecord(P->small_join, P->small_side));
   return 0;
 }
 
@@ -2216,6 +2236,7 @@ int finish_impl(PyloPlan* P, const PyloTensorArgs* args, const float* coeffs, in
       hipLaunchKernelGGL(k_celo2_slice_finish<true>, dim3((unsigned)L.slice_items_b.size()), dim3(256), L.slice_lds_b, s,
                          smats, P->at<Item>(L.off_slice_items_b), descs, dyn, orth_call, ns_iters, ns_eps, c0, c1, c2);
   }
+  if (any_small && P->small_side != nullptr) HIP_TRY(hipStreamWaitEvent(slices_aside ? P->slice_side : s, P->small_join, 0));
   if (slices_aside) HIP_TRY(hipEventRecord(P->slice_join, P->slice_side));
   if (n_fin == 0) {
     HIP_TRY(hipGetLastError());
