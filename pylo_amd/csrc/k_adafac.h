@@ -40,8 +40,8 @@ __device__ __forceinline__ void adafac_bias_block(int t, const float* __restrict
 }
 
 // k_v0a and, in the blocks behind its own, the tensors' biases, which nothing before k_v0b asks for.  NORM: and k_gnorm.  The
-// step of a small network is its launches: MLP 784-128-128-10 under ELO took twelve, 3 us of host time each and 4 to 8 us of the
-// GPU, now eight (this one, the norm, the fold, both apply passes).
+// step of a small network is its launches: MLP 784-128-128-10 under ELO took eleven, 3 us of host time each and 4 to 8 us of the
+// GPU, now seven (this one, the norm, the fold, both apply passes).
 template <bool NORM>
 __global__ __launch_bounds__(kThreads) void k_adafac_v0a(const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn,
                                                          const Item* __restrict__ items, int n_items, const float* __restrict__ part,
