@@ -2,8 +2,13 @@
 //
 // With A = X X^T every iterate is a polynomial of A times X, so the five iterations need X twice only: once for A, once for
 // Q X.  In fp32 that loses the small singular directions -- the chained A inherits the rounding of the first one, which the
-// polynomial amplifies by c0^2 an iteration (k_ns_hf.h) -- in fp64 it does not: products of fp32 values are exact, A is off by
-// 1e-16 of its largest eigenvalue and five iterations leave 1e-10 of a direction.  And on m x m matrices of at most two
+// polynomial amplifies by c0^2 an iteration (k_ns_hf.h) -- in fp64 a run of a few does not: products of fp32 values are exact, A is
+// off by 1e-16 of its largest eigenvalue, and five iterations leave 1e-10 of a direction.  What of it is not symmetric grows faster,
+// 23-fold an iteration (the products take a matrix for its transpose): six iterations are the most that the usual coefficients
+// allow.  More are taken in runs (thin_runs, RUNS) that each form the Gram matrix again, from X in fp32.  Every matrix of a run is a
+// multiple of the identity and the rest (B = c0 I + P, Q = q0 I + M), the multiple applied by itself: equal rows of X stay equal to
+// the bit, as in the formula, and leave no difference for later runs to amplify.  32 x 500 of ones, off by (of the RMS) at 8, 12,
+// 20 iterations: one run 2e-6, 6, NaN; runs of six 1e-7 at most; the formula in fp32 1e-5.  And on m x m matrices of at most two
 // tiles of v_mfma_f64_16x16x4_f64 a side the fp64 pipe is fast enough.  So a block takes a slab of columns through
 //   G += X X^T (fp32 values widened);  [the blocks of a matrix meet once and add their G in slab order]
 //   A = G / (sqrt(tr G) + eps)^2;  B = c2 A A + c1 A + c0 I,  Q <- B Q,  A <- B A B  (every block for itself)
@@ -40,16 +45,18 @@ struct ThinDims {
 };
 constexpr int kThinChunk = 64;         // columns of a chunk (NsSmall::chunks): a group of each of the four waves
 
+// A launch takes a run of iterations: all of them, or where they are too many for one Gram matrix (thin_runs) the first, the
+// next, ..., the last (RUNS).  Runs but the last leave X <- Q X in place, rounded to fp32, runs but the first start from it as it is.
 struct ThinStep {
   double c0, c1, c2, eps;
-  int iters;
+  int iters, first, last;
 };
 
 // A matrix has at most 32 x 65536 elements: 32-bit offsets.
 __device__ __forceinline__ float thin_at(const float* p, int i) { return *(const gfloat*)((const gchar*)p + (unsigned)i * 4u); }
 __device__ __forceinline__ void thin_put(float* p, int i, float v) { *(gfloat*)((gchar*)p + (unsigned)i * 4u) = v; }
 
-template <int MT>
+template <int MT, bool RUNS>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 1 ? 5 : 4))) void k_ns_thin(
     const NsSmall* __restrict__ mats, const NsSmallItem* __restrict__ items, const TDesc* __restrict__ descs,
     const PyloTensorArgs* __restrict__ dyn, float* __restrict__ part, int* __restrict__ sync, ThinStep st, int orth_call,
@@ -90,6 +97,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
     return tall ? u * m + row : row * n + u * nv;
   };
   const bool orth = orth_call && (a.flags & kArgOrthogonalize);
+  const bool first = !RUNS || st.first, last_run = !RUNS || st.last;
+  if (!orth && !last_run) return;
   bool good = true;
 
   // ---- G over the block's columns.  Lane: row 16 t + lo; the four columns of slot hi are neighbours where a row's entries
@@ -213,7 +222,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
   const double tr = wave_sum(lane < D::MP ? s0[lane * D::PD + lane] : 0.0);   // rows past m are zero
 
   // ---- the m x m matrices.  Wave w < MT^2 owns tile (w / MT, w % MT).
-  double ss = tr, xs = 1.0;
+  double ss = tr, xs = 1.0, q0 = 1.0;
   if (orth) {
     const int ti = wave / MT, tj = wave % MT;
     const bool own = wave < MT * MT;
@@ -228,7 +237,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
 #pragma unroll
       for (int r = 0; r < 4; ++r) p[(16 * ti + 4 * r + hi) * D::PD + 16 * tj + lo] = d[r];
     };
-    xs = 1.0 / (sqrt(tr) + st.eps);
+    if (first) xs = 1.0 / (sqrt(tr) + st.eps);
     v4d A, A0, Q;
     if (own) {
 #pragma unroll
@@ -240,21 +249,29 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
     __syncthreads();
     for (int i = 0; i < st.iters; ++i) {
       const bool last = i == st.iters - 1;
-      v4d B, T;
+      v4d B, T;                              // RUNS: P, and M in Q's place
       if (own) {
         B = prod(s0, s0);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int row = 16 * ti + 4 * r + hi, col = 16 * tj + lo;
-          B[r] = st.c2 * B[r] + st.c1 * A[r] + (row == col && row < m ? st.c0 : 0.0);
+          B[r] = st.c2 * B[r] + st.c1 * A[r] + (!RUNS && row == col && row < m ? st.c0 : 0.0);
         }
         put(s1, B);
       }
       __syncthreads();
       if (own) {
-        Q = i > 0 ? prod(s1, s2) : B;        // B Q
+        Q = i > 0 ? RUNS ? prod(s2, s1) : prod(s1, s2) : B;        // B Q
         if (!last) T = prod(s0, s1);         // A B
+        if constexpr (RUNS) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (i > 0) Q[r] += st.c0 * s2[(16 * ti + 4 * r + hi) * D::PD + 16 * tj + lo] + q0 * B[r];
+            if (!last) T[r] += st.c0 * A[r];
+          }
+        }
       }
+      if constexpr (RUNS) q0 *= st.c0;
       __syncthreads();
       if (own) {
         put(s2, Q);
@@ -262,7 +279,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
       }
       __syncthreads();
       if (!last) {
-        if (own) A = prod(s1, s0);           // B A B
+        if (own) {                           // B A B
+          A = RUNS ? prod(s0, s1) : prod(s1, s0);
+          if constexpr (RUNS) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) A[r] += st.c0 * T[r];
+          }
+        }
         __syncthreads();
         if (own) put(s0, A);
         __syncthreads();
@@ -275,12 +298,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
     if (own) {
       const v4d t = prod(s2, s0);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) s += t[r] * Q[r];
+      for (int r = 0; r < 4; ++r) {
+        if constexpr (RUNS) s += (t[r] + q0 * A0[r]) * (16 * ti + 4 * r + hi == 16 * tj + lo ? Q[r] + q0 : Q[r]);
+        else s += t[r] * Q[r];
+      }
     }
     s = wave_sum(s);
     if (lane == 0) red[wave] = s;
     __syncthreads();
     ss = (red[0] + red[1]) + (red[2] + red[3]);
+    if (RUNS && !good) xs = __builtin_nan("");
   }
   // ---- step = X * rsqrt(1e-9 + mean X^2) * rmsmult; p <- p - lr (step + wd p)
   const float rm = a.step_mult, wd = a.weight_decay, nlr = -a.lr;
@@ -362,11 +389,22 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
         for (int r = 0; r < 4; ++r) {
           int idx;
           w[t][r] = 0.0f;
-          if (place(c, t, r, idx)) w[t][r] = store == 0 ? thin_at(pb, idx) : load_stored(a.param, q.elem_off + idx, store);
+          if (last_run && place(c, t, r, idx)) w[t][r] = store == 0 ? thin_at(pb, idx) : load_stored(a.param, q.elem_off + idx, store);
         }
       v4d d[MT];
 #pragma unroll
       for (int t = 0; t < MT; ++t) d[t] = v4d{0.0, 0.0, 0.0, 0.0};
+      if constexpr (RUNS) {
+#pragma unroll
+        for (int s = 0; s < K; ++s) {
+          const double y = (double)x[s];
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            const double e = 16 * t + lo == slot(s) ? q0 * xs : 0.0;
+            d[t] = tall ? __builtin_amdgcn_mfma_f64_16x16x4f64(y, e, d[t], 0, 0, 0) : __builtin_amdgcn_mfma_f64_16x16x4f64(e, y, d[t], 0, 0, 0);
+          }
+        }
+      }
 #pragma unroll
       for (int s = 0; s < K; ++s) {
         const double y = (double)x[s];
@@ -384,6 +422,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MT == 
           const float v = (float)d[t][r];
           const float p = fmaf(nlr, (v * sc) * rm + wd * w[t][r], w[t][r]);
           thin_put(x0, idx, v);
+          if (!last_run) continue;
           if (store == 0) thin_put(pb, idx, p);
           else store_stored(a.param, q.elem_off + idx, store, p);
         }

@@ -1478,6 +1478,9 @@ struct PyloPlan {
   hipStream_t slice_side = nullptr;
   hipStream_t small_side = nullptr;   // two of the small matrices' classes (enqueue_small)
   hipEvent_t small_fork = nullptr, small_join = nullptr;
+  float thin_c[3] = {};               // what thin_run (thin_runs) was worked out for
+  int thin_iters = 0;
+  std::vector<int> thin_run;
   hipEvent_t slice_fork = nullptr, slice_join = nullptr;
 
   template <class Tp>
@@ -2091,6 +2094,43 @@ __global__ __launch_bounds__(256) void k_ns_zero(u32x4* __restrict__ p, size_t n
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n16; i += (size_t)gridDim.x * 256) p[i] = u32x4{0u, 0u, 0u, 0u};
 }
 
+// The iterations as runs that k_ns_thin takes from one Gram matrix each.  An entry of A (of the largest eigenvalue `top`) is off by 2^-52
+// of that; an iteration multiplies what is off between two eigenvectors of eigenvalues a, b by at most `grow`, in the kernel's own
+// order of operands (B = p(A A^T), T = A B^T, A <- T B^T), and B is off by B' times it.  A run ends before that is 2^-27 of B.
+// With the usual coefficients grow is 23: runs of six.  (Errors at six and seven, eight, nine iterations of a run, 32 x 500 of ones: the last
+// rounding, 4e-8, 2e-6, 5e-5.)
+std::vector<int> thin_runs(double c0, double c1, double c2, int iters) {
+  constexpr int N = 32;
+  std::vector<int> runs{0};
+  double top = 1.0, err = 0x1p-52;
+  for (int i = 0; i < iters; ++i) {
+    double b_max = 0.0, db_max = 0.0, next = 0.0, grow = 0.0;
+    for (int k = 0; k <= N; ++k) {
+      const double a = top * k / N, B = c0 + a * (c1 + a * c2);
+      b_max = std::max(b_max, std::fabs(B));
+      db_max = std::max(db_max, std::fabs(c1 + 2.0 * a * c2));
+      next = std::max(next, a * B * B);
+      for (int l = 0; l <= N; ++l) {
+        const double b = top * l / N, Bb = c0 + b * (c1 + b * c2);
+        double row = 0.0;   // what A'_ab takes from A_ab and A_ba
+        for (int q = 0; q < 2; ++q) {
+          const double x = 1 - q, y = q, p21 = c2 * (a * y + b * x) + c1 * y;
+          row += std::fabs(a * B * p21 + (a * p21 + x * Bb) * Bb);
+        }
+        grow = std::max(grow, row);
+      }
+    }
+    if (runs.back() > 0 && !(err * db_max <= 0x1p-27 * b_max)) {
+      runs.push_back(0);
+      err = 0x1p-52 * std::max(top, 1.0);
+    }
+    ++runs.back();
+    top = next;
+    err = err * grow + 0x1p-52 * std::max(top, 1.0);
+  }
+  return runs;
+}
+
 int small_lds_once() {
   static std::mutex mu;
   static std::vector<int> done;
@@ -2140,18 +2180,27 @@ int enqueue_small(PyloPlan* P, hipStream_t s, const TDesc* descs, const PyloTens
                          P->at<double>(L.off_sm_sums), P->at<int>(L.off_sm_sync), st, orth,
                          L.sm_meets[cls] ? P->at<int>(L.off_sm_sync) + L.sm_ticket0 + cls : (int*)nullptr);
   };
-  const ThinStep thin{st.c0, st.c1, st.c2, ns_eps, ns_iters};
+  if (orth && (P->thin_c[0] != coeffs[0] || P->thin_c[1] != coeffs[1] || P->thin_c[2] != coeffs[2] || P->thin_iters != ns_iters)) {
+    std::copy(coeffs, coeffs + 3, P->thin_c);
+    P->thin_iters = ns_iters;
+    P->thin_run = thin_runs(coeffs[0], coeffs[1], coeffs[2], ns_iters);
+  }
   auto launch_thin = [&](auto kern, int cls, int lds, hipStream_t s) {
-    if (!L.sm_items[cls].empty())
+    if (L.sm_items[cls].empty()) return;
+    const size_t n_runs = orth ? P->thin_run.size() : 1;
+    for (size_t r = 0; r < n_runs; ++r) {
+      const ThinStep thin{st.c0, st.c1, st.c2, ns_eps, orth ? P->thin_run[r] : 0, r == 0, r + 1 == n_runs};
       hipLaunchKernelGGL(kern, dim3((unsigned)L.sm_items[cls].size()), dim3(kThreads), lds, s, P->at<NsSmall>(L.off_sm_mats),
                          P->at<NsSmallItem>(L.off_sm_items[cls]), descs, dyn, P->at<float>(L.off_sm_part), P->at<int>(L.off_sm_sync),
                          thin, orth, L.sm_meets[cls] ? P->at<int>(L.off_sm_sync) + L.sm_ticket0 + cls : (int*)nullptr);
+    }
   };
   const hipStream_t mid = P->small_side != nullptr ? P->small_side : s;
   launch(k_ns_small<4, 2, 1>, 3, SmLarge::kThr, SmLarge::kLds, s);
   launch(k_ns_small<2, 1, 2>, 2, SmMid::kThr, SmMid::kLds, mid);
-  launch_thin(k_ns_thin<2>, 1, ThinDims<2>::kLds, mid);
-  launch_thin(k_ns_thin<1>, 0, ThinDims<1>::kLds, s);
+  const bool runs = orth && P->thin_run.size() > 1;
+  launch_thin(runs ? k_ns_thin<2, true> : k_ns_thin<2, false>, 1, ThinDims<2>::kLds, mid);
+  launch_thin(runs ? k_ns_thin<1, true> : k_ns_thin<1, false>, 0, ThinDims<1>::kLds, s);
   if (P->small_side != nullptr) HIP_TRY(hipEventRecord(P->small_join, P->small_side));
   return 0;
 }

@@ -32,6 +32,42 @@ def test_thin_matrices_against_fp64(tall, iters):
         assert off <= 1e-9, (tuple(x.shape), off)
 
 
+def _deficient(kind, m, n, gen):
+    x = torch.randn((m, n), generator=gen, device="cuda")
+    if kind == "constant":
+        x = torch.full((m, n), 0.01, device="cuda")
+    elif kind == "rank 1":
+        x = torch.randn((m, 1), generator=gen, device="cuda") * torch.randn((1, n), generator=gen, device="cuda")
+    elif kind == "twin rows":
+        x[1::2] = x[0::2][: m // 2].clone()
+    return x
+
+
+@pytest.mark.parametrize("iters", [6, 7, 8, 12, 20])
+@pytest.mark.parametrize("tall", [False, True])
+def test_iterations_beyond_one_run(tall, iters):
+    """More iterations than one Gram matrix in fp64 is good for, on matrices with and without a null space, folded, cut, and neither.
+    Bound on the error's RMS over the result's: runs round X to fp32 where the formula in fp32 rounds X, A and A A after every
+    iteration, so a quarter of that formula's error, and eight roundings of the result where that one is small."""
+    gen = torch.Generator(device="cuda").manual_seed(iters)
+    sizes = [(1, 65536), (4, 300), (4, 20011), (8, 64), (16, 16), (16, 40000), (17, 64), (32, 500), (32, 32768)]
+    kinds = [(k, m, n) for m, n in sizes for k in ("gaussian", "constant", "rank 1", "twin rows")]
+    mats = [_deficient(k, m, n, gen) for k, m, n in kinds]
+    mats = [x.t().contiguous() for x in mats] if tall else mats
+    for kind, x, got in zip(kinds, mats, _orthogonalise_direct(mats, iters)):
+        want = _reference_direct(x, iters, coeffs=COEFFS)
+        y = (x.t() if tall else x).cpu()
+        y = y / (y.double().norm().float() + 1e-8)
+        for _ in range(iters):
+            a = y @ y.t()
+            y = COEFFS[0] * y + (COEFFS[1] * a + COEFFS[2] * (a @ a)) @ y
+        y = (y / y.double().pow(2).mean().sqrt().float()).double()
+        y = (y.t() if tall else y).to(want.device)
+        off = float((got.double() - want).pow(2).mean().sqrt())
+        fp32 = float((y - want).pow(2).mean().sqrt())
+        assert off <= 8 * 2.0 ** -24 + fp32 / 4, (kind, off, fp32)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_normalise_only_and_storage(dtype):
     """Without the flag the step is applied as it stands; parameters in their own type; each at rel 6 x 2^-24 plus its spacing."""
