@@ -10,6 +10,7 @@ reduces the decay axis instead, AdafacLO_cuda.py:342-343), and 1-D tensors use
 
 from __future__ import annotations
 
+import operator
 from typing import Optional, Union
 
 import numpy as np
@@ -210,41 +211,48 @@ class AdafacLO_CUDA(Optimizer):
         index = {id(g): i for i, g in enumerate(self.param_groups)}
         counters = torch.tensor([float(self.state[p]["step"]) for _, p in tensors], dtype=torch.float64)
         keys = ("exp_avg", "exp_avg_sq", "exp_avg_sq_r", "exp_avg_sq_c", "step")
-        records = []
+        steps, at = [], []
         for i, (_, p) in enumerate(tensors):
             state = self.state[p]
             t = state["step"]
             if not torch.is_tensor(t) or t.dtype != torch.float64 or t.device.type != "cpu" or t.dim() != 0:
                 return None
             t.set_(counters.untyped_storage(), i, ())
-            kept = tuple(state[k] for k in keys)
-            records.append((p, p.shape, p.dtype, state, kept, tuple(x.data_ptr() for x in kept)))
-        return dict(key=self._plan_key, flags=self._plan_key[0], n_state=len(self.state), records=records, counters=counters,
+            steps.append(t)
+            at.append(tuple(state[k].data_ptr() for k in keys))
+        return dict(key=self._plan_key, flags=self._plan_key[0], steps=steps, at=at, counters=counters,
                     values=counters.numpy(), scalars=None, gidx=np.asarray([index[id(g)] for g, _ in tensors], dtype=np.int64))
 
     def _unchanged(self, fast):
-        """Gradient and parameter addresses if nothing but values has changed since the step that made ``fast``, else None."""
-        if (fast["key"] is not self._plan_key or fast["flags"] != self._PLAN_FLAGS | self._norm_flags()
-                or len(self.state) != fast["n_state"]):
+        """Gradient and parameter addresses if nothing but values has changed since the step that made ``fast``, else None.  The
+        state is the one that ``self.state`` has for each parameter now; only addresses of it are kept, so that a program that
+        replaces accumulators to free them does."""
+        if fast["key"] is not self._plan_key or fast["flags"] != self._PLAN_FLAGS | self._norm_flags():
             return None
         strided = torch.strided
         params = [p for group in self.param_groups for p in group["params"]]
-        records = fast["records"]
-        if len(params) != len(records):
+        if len(params) != len(fast["at"]):
             return None
+        # (a look-up by parameter costs as much as the rest of the walk: not where the states are in the parameters' order)
+        if len(self.state) == len(params) and all(map(operator.is_, self.state, params)):
+            states = self.state.values()
+        else:
+            states = [self.state.get(p) for p in params]
         grads, addresses = [], []
-        for p, (old, shape, dtype, state, kept, at) in zip(params, records):
-            g = p.grad
-            if (p is not old or g is None or p.dtype is not dtype or g.dtype is not dtype or p.shape != shape
-                    or g.layout is not strided or not g.is_contiguous()):
-                return None
-            m, v, fr, fc, t = kept
-            if (state.get("exp_avg") is not m or state.get("exp_avg_sq") is not v or state.get("exp_avg_sq_r") is not fr
-                    or state.get("exp_avg_sq_c") is not fc or state.get("step") is not t
-                    or at != (m.data_ptr(), v.data_ptr(), fr.data_ptr(), fc.data_ptr(), t.data_ptr())):
-                return None
-            grads.append(g.data_ptr())
-            addresses.append(p.data_ptr())
+        try:
+            for p, state, (shape, dtype), t, at in zip(params, states, fast["key"][1:], fast["steps"], fast["at"]):
+                g = p.grad
+                if (g is None or p.dtype is not dtype or g.dtype is not dtype or p.shape != shape or g.layout is not strided
+                        or not g.is_contiguous()):
+                    return None
+                if state["step"] is not t or at != (
+                        state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(), state["exp_avg_sq_r"].data_ptr(),
+                        state["exp_avg_sq_c"].data_ptr(), t.data_ptr()):
+                    return None
+                grads.append(g.data_ptr())
+                addresses.append(p.data_ptr())
+        except (KeyError, TypeError, AttributeError):    # no state, or one without a tensor that it should have
+            return None
         return grads, addresses
 
     def _step_fast(self, fast, found):
