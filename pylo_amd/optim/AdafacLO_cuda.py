@@ -208,7 +208,7 @@ class AdafacLO_CUDA(Optimizer):
     # contiguous gradient the rows are kept; the counters, one 0-dim tensor a parameter, are moved side by side into one
     # buffer, in place, and advanced together.
     def _keep_rows(self, tensors):
-        index = {id(g): i for i, g in enumerate(self.param_groups)}
+        sizes = [len(g["params"]) for g in self.param_groups]
         counters = torch.tensor([float(self.state[p]["step"]) for _, p in tensors], dtype=torch.float64)
         keys = ("exp_avg", "exp_avg_sq", "exp_avg_sq_r", "exp_avg_sq_c", "step")
         steps, at = [], []
@@ -221,7 +221,7 @@ class AdafacLO_CUDA(Optimizer):
             steps.append(t)
             at.append(tuple(state[k].data_ptr() for k in keys))
         return dict(key=self._plan_key, flags=self._plan_key[0], steps=steps, at=at, counters=counters,
-                    values=counters.numpy(), scalars=None, gidx=np.asarray([index[id(g)] for g, _ in tensors], dtype=np.int64))
+                    values=counters.numpy(), scalars=None, sizes=sizes, gidx=np.repeat(np.arange(len(sizes)), sizes))
 
     def _unchanged(self, fast):
         """Gradient and parameter addresses if nothing but values has changed since the step that made ``fast``, else None.  The
@@ -229,10 +229,10 @@ class AdafacLO_CUDA(Optimizer):
         replaces accumulators to free them does."""
         if fast["key"] is not self._plan_key or fast["flags"] != self._PLAN_FLAGS | self._norm_flags():
             return None
+        if [len(group["params"]) for group in self.param_groups] != fast["sizes"]:    # a parameter's group, by its place
+            return None
         strided = torch.strided
         params = [p for group in self.param_groups for p in group["params"]]
-        if len(params) != len(fast["at"]):
-            return None
         # (a look-up by parameter costs as much as the rest of the walk: not where the states are in the parameters' order)
         if len(self.state) == len(params) and all(map(operator.is_, self.state, params)):
             states = self.state.values()

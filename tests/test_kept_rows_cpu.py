@@ -130,6 +130,23 @@ def _copied(opt, i):
     opt.state[_params(opt)[i]] = copy.deepcopy(opt.state[_params(opt)[i]])
 
 
+def _move(opt):
+    a, b = opt.param_groups[:2]
+    b["params"].insert(0, a["params"].pop())
+
+
+def _split(opt):
+    g = opt.param_groups[0]
+    tail, g["params"] = g["params"][1:], g["params"][:1]
+    opt.add_param_group(dict({k: v for k, v in g.items() if k != "params"}, params=tail, lr=0.125))
+    opt.param_groups.insert(1, opt.param_groups.pop())
+
+
+def _merge(opt):
+    opt.param_groups[0]["params"] += opt.param_groups[1]["params"]
+    del opt.param_groups[1]
+
+
 def _swapped(opt):
     st, (p, q) = opt.state, _params(opt)[:2]
     st[p], st[q] = st[q], st[p]
@@ -140,6 +157,9 @@ EVENTS = {
     "one state copied": lambda opt: _copied(opt, 1),
     "every state copied": lambda opt: [_copied(opt, i) for i in range(len(SHAPES))],
     "two states swapped": _swapped,
+    "moved between groups": _move,
+    "group split": _split,
+    "groups merged": _merge,
     "learning rate": lambda opt: opt.param_groups[1].update(lr=0.0625),
 }
 FAMILIES = ["adafac", "elo"]
