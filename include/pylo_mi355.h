@@ -355,6 +355,10 @@ int pylo_mi355_plan_statistics_stale(const PyloPlan* plan);
 int pylo_mi355_adafac_step(PyloPlan* plan, const PyloTensorArgs* args, const PyloDecays* decays,
                            const float* net, float step, void* stream);
 
+/* Adds one to each of `n` counters in host memory, one after the other, and leaves what each was in `before`: the step counters
+ * of n tensors, which the reference keeps as one float64 scalar per parameter (AdafacLO_cuda.py:304-305,400). */
+int pylo_mi355_advance_counters(double* const* counters, int n, double* before);
+
 /* ---- Single-tensor calls with the argument lists of the reference's extension functions ------------
  * For callers that keep the reference's per-tensor loop (its optimizer classes update the accumulators
  * and form row_factor / col_factor with tensor operations, then call one function per tensor).  All

@@ -143,6 +143,7 @@ def load():
                                          C.POINTER(VeloStep), C.c_void_p]
     lib.pylo_mi355_adafac_step.argtypes = [C.c_void_p, C.c_void_p, C.POINTER(Decays), C.c_void_p, C.c_float,
                                            C.c_void_p]
+    lib.pylo_mi355_advance_counters.argtypes = [C.c_void_p, C.c_int, C.c_void_p]
     lib.pylo_mi355_plan_invalidate_statistics.argtypes = [C.c_void_p]
     lib.pylo_mi355_plan_statistics_stale.argtypes = [C.c_void_p]
     lib.pylo_mi355_plan_arg_table.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_void_p)]
@@ -156,6 +157,11 @@ def load():
 def check(rc: int, what: str) -> None:
     if rc != 0:
         raise RuntimeError(f"{what}: {load().pylo_mi355_last_error().decode()}")
+
+
+def advance_counters(addresses: int, n: int, before: int) -> None:
+    """Adds one to the float64 scalars at the `n` addresses that lie at `addresses`; what they were goes to `before`."""
+    check(load().pylo_mi355_advance_counters(addresses, n, before), "advance_counters")
 
 
 def make_shapes(shapes: Sequence[Sequence[int]], flags: Sequence[int]):

@@ -2749,6 +2749,15 @@ extern "C" int pylo_mi355_plan_statistics_stale(const PyloPlan* P) {
   return *static_cast<const volatile int*>(P->stale_host);
 }
 
+extern "C" int pylo_mi355_advance_counters(double* const* counters, int n, double* before) {
+  if (n < 0 || (n > 0 && (!counters || !before))) return fail("advance_counters: null argument");
+  for (int i = 0; i < n; ++i) {
+    before[i] = *counters[i];
+    *counters[i] = before[i] + 1.0;
+  }
+  return 0;
+}
+
 extern "C" int pylo_mi355_adafac_step(PyloPlan* P, const PyloTensorArgs* args, const PyloDecays* decays,
                                       const float* net, float step, void* stream) {
   if (!P || !args || !decays || !net) return fail("adafac_step: null argument");

@@ -205,23 +205,19 @@ class AdafacLO_CUDA(Optimizer):
 
     # Three microseconds of Python a tensor for its row of the argument table, and one for its counter, were the whole step on a
     # convolutional network of 161 tensors (host 673 us, its kernels 660).  After a step in which every parameter had a dense
-    # contiguous gradient the rows are kept; the counters, one 0-dim tensor a parameter, are moved side by side into one
-    # buffer, in place, and advanced together.
+    # contiguous gradient the rows are kept; the counters, one 0-dim tensor a parameter, stay where they are and are advanced by
+    # one call.
     def _keep_rows(self, tensors):
+        steps = [self.state[p]["step"] for _, p in tensors]
+        if not all(torch.is_tensor(t) and t.dtype == torch.float64 and t.device.type == "cpu" and t.dim() == 0 for t in steps):
+            return None
         sizes = [len(g["params"]) for g in self.param_groups]
-        counters = torch.tensor([float(self.state[p]["step"]) for _, p in tensors], dtype=torch.float64)
         keys = ("exp_avg", "exp_avg_sq", "exp_avg_sq_r", "exp_avg_sq_c", "step")
-        steps, at = [], []
-        for i, (_, p) in enumerate(tensors):
-            state = self.state[p]
-            t = state["step"]
-            if not torch.is_tensor(t) or t.dtype != torch.float64 or t.device.type != "cpu" or t.dim() != 0:
-                return None
-            t.set_(counters.untyped_storage(), i, ())
-            steps.append(t)
-            at.append(tuple(state[k].data_ptr() for k in keys))
-        return dict(key=self._plan_key, flags=self._plan_key[0], steps=steps, at=at, counters=counters,
-                    values=counters.numpy(), scalars=None, sizes=sizes, gidx=np.repeat(np.arange(len(sizes)), sizes))
+        at = [tuple(self.state[p][k].data_ptr() for k in keys) for _, p in tensors]
+        counters, values = np.asarray([a[-1] for a in at], dtype=np.uint64), np.zeros(len(at))
+        return dict(key=self._plan_key, flags=self._plan_key[0], steps=steps, at=at, counters=counters, values=values,
+                    advance=(counters.ctypes.data, len(at), values.ctypes.data), scalars=None, sizes=sizes,
+                    gidx=np.repeat(np.arange(len(sizes)), sizes))
 
     def _unchanged(self, fast):
         """Gradient and parameter addresses if nothing but values has changed since the step that made ``fast``, else None.  The
@@ -264,11 +260,11 @@ class AdafacLO_CUDA(Optimizer):
             for k in scalars[0]:
                 args[k] = np.asarray([sc[k] for sc in scalars], dtype=np.float64)[fast["gidx"]]
             fast["scalars"] = scalars
+        _lib.advance_counters(*fast["advance"])
         step_fed = float(values[0])
         if not (values == step_fed).all():       # the library reads each parameter's own counter
             args["bc1"] = values
             step_fed = -1.0
-        fast["counters"].add_(1.0)
         with torch.cuda.device(self.device):
             plan.adafac_step(self._decays, self._net, step_fed, torch.cuda.current_stream(self.device).cuda_stream)
 

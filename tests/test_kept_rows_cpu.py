@@ -192,6 +192,44 @@ def test_replaced_accumulators_are_freed(family):
 
 
 @pytest.mark.parametrize("family", ["adafac", "elo"])
+def test_counters_stay_where_they_are(family):
+    """Views, and what shares a counter's memory, follow it; two parameters that share one advance it twice a step."""
+    opt = _make(family)
+    _step(family, opt)
+    opt.state[_params(opt)[4]]["step"] = torch.tensor(7.0, dtype=torch.float64).share_memory_()
+    steps = [opt.state[p]["step"] for p in _params(opt)]
+    views = [(t.detach(), t.numpy(), t.data_ptr()) for t in steps]
+    for _ in range(3):
+        _step(family, opt)
+    assert opt._fast is not None
+    for i, (t, (view, array, at)) in enumerate(zip(steps, views)):
+        want = 10.0 if i == 4 else 4.0
+        assert opt.state[_params(opt)[i]]["step"] is t and t.data_ptr() == at
+        assert float(t) == float(view) == float(array) == want and t.untyped_storage().nbytes() == 8, i
+    assert steps[4].is_shared()
+    opt.state[_params(opt)[0]]["step"] = steps[3]
+    for n in range(1, 4):
+        for p in _params(opt):
+            p.grad = torch.randn(p.shape)
+        opt.step()
+        assert float(steps[3]) == 4.0 + 2 * n
+        assert opt._plan.tables[-1]["bc1"][0] == 2.0 + 2 * n and opt._plan.tables[-1]["bc1"][3] == 3.0 + 2 * n
+
+
+@pytest.mark.parametrize("odd", [2.0, torch.tensor(2.0)], ids=["number", "float32"])
+def test_counters_of_another_kind(odd):
+    """... are taken as before, and the others' are left alone."""
+    opt = _make("adafac")
+    _step("adafac", opt)
+    opt.state[_params(opt)[3]]["step"] = odd
+    at = [opt.state[p]["step"].data_ptr() for p in _params(opt)[:3]]
+    for _ in range(3):
+        _step("adafac", opt)
+    assert opt._fast is None and float(opt.state[_params(opt)[3]]["step"]) == 5.0
+    assert at == [opt.state[p]["step"].data_ptr() for p in _params(opt)[:3]]
+
+
+@pytest.mark.parametrize("family", ["adafac", "elo"])
 def test_cleared_states_start_again(family):
     opt = _make(family)
     for _ in range(3):
