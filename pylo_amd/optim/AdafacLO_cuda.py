@@ -270,8 +270,8 @@ class AdafacLO_CUDA(Optimizer):
 
     @torch.no_grad()
     def step(self, loss=None):
-        if self._fast is not None and not self.capturable:
-            found = self._unchanged(self._fast)
+        if self._fast is not None:
+            found = None if self.capturable else self._unchanged(self._fast)
             if found is not None:
                 self._step_fast(self._fast, found)
                 return loss

@@ -230,6 +230,19 @@ def test_counters_of_another_kind(odd):
 
 
 @pytest.mark.parametrize("family", ["adafac", "elo"])
+def test_rows_do_not_outlive_a_capturable_step(family, monkeypatch):
+    """... which fills the table anew: the groups' scalars in it are those of that step."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    opt = _make(family)
+    for _ in range(3):
+        _step(family, opt)
+    opt.capturable, opt.param_groups[0]["lr"] = True, 0.1
+    opt.step()
+    opt.capturable, opt.param_groups[0]["lr"] = False, 0.5
+    _step(family, opt)
+
+
+@pytest.mark.parametrize("family", ["adafac", "elo"])
 def test_cleared_states_start_again(family):
     opt = _make(family)
     for _ in range(3):
