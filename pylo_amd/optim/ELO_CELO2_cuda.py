@@ -527,6 +527,16 @@ class ELO_CELO2_CUDA(Optimizer):
             self._plan.celo2_orthogonalize_finish(fin, self.ns_coeffs, self.ns_iters, self.ns_eps,
                                                   torch.cuda.current_stream(self.device).cuda_stream)
 
+    def _raw_parts(self, tensors):
+        """The buffers of raw steps with the tensors in them; a copy for each group where a tensor has moved to another since the
+        plan was made (recorded graphs hold the plan and its buffers, so neither is made anew for that)."""
+        for buf, idx in self._raw_groups:
+            members = {}
+            for j, i in enumerate(idx):
+                members.setdefault(id(tensors[i][0]), []).append(j)
+            for js in members.values():
+                yield (buf, idx) if len(members) == 1 else (buf[js], [idx[j] for j in js])
+
     def _finish_step(self, tensors):
         if getattr(self, "_fast", None) is not None and self._fast_taken:
             ff = getattr(self, "_fin_fast", None)
@@ -540,7 +550,7 @@ class ELO_CELO2_CUDA(Optimizer):
         fin["flags"] = 0
         lib_ns = self._lib_ns
         keep, any_fin = [], False   # post-Newton-Schulz matrices must outlive the launch
-        for buf, idx in self._raw_groups:
+        for buf, idx in self._raw_parts(tensors):
             group = tensors[idx[0]][0]
             ps = [tensors[i][1] for i in idx]
             # a tensor that sits this step out keeps its row out of the table (its raw step is stale or unset; the

@@ -158,6 +158,7 @@ EVENTS = {
     "every state copied": lambda opt: [_copied(opt, i) for i in range(len(SHAPES))],
     "two states swapped": _swapped,
     "moved between groups": _move,
+    "matrices moved": lambda opt: [_move(opt) for _ in range(2)],
     "group split": _split,
     "groups merged": _merge,
     "learning rate": lambda opt: opt.param_groups[1].update(lr=0.0625),
@@ -240,6 +241,19 @@ def test_rows_do_not_outlive_a_capturable_step(family, monkeypatch):
     opt.step()
     opt.capturable, opt.param_groups[0]["lr"] = False, 0.5
     _step(family, opt)
+
+
+@pytest.mark.parametrize("event", ["matrices moved", "group split", "groups merged"])
+@pytest.mark.parametrize("family", ["elo_celo2", "celo2"])
+def test_groups_change_without_kept_rows(family, event):
+    """Raw steps of one shape share a buffer that is finished group by group, whatever group each tensor is in now."""
+    opt = _make(family)
+    for _ in range(2):
+        _step(family, opt)
+    EVENTS[event](opt)
+    for _ in range(2):
+        opt._fast = None
+        _step(family, opt)
 
 
 @pytest.mark.parametrize("family", ["adafac", "elo"])
