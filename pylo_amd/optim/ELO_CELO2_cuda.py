@@ -18,6 +18,7 @@ from __future__ import annotations
 
 from typing import Optional
 
+import operator
 import os
 
 import numpy as np
@@ -360,12 +361,24 @@ class ELO_CELO2_CUDA(Optimizer):
                 np.where(adam, per_group(lambda g: 1.0 - beta2 ** g["step"]), 0.0))
 
     def _fused_step_fast(self, fast):
-        grads = [p.grad for p in fast["params"]]
-        for g in grads:     # a dense gradient has its parameter's dtype (torch enforces it on assignment)
-            if g is None or g.layout is not torch.strided or not g.is_contiguous():
-                return None
+        # the same parameters of the same shapes and types in the same groups, each with the state it had
         groups = self.param_groups
-        if len(groups) != fast["n_groups"] or len(self.state) != fast["n_state"]:
+        params = [p for g in groups for p in g["params"]]
+        if ([len(g["params"]) for g in groups] != fast["sizes"] or not all(map(operator.is_, groups, fast["groups"]))
+                or len(self.state) != len(fast["states"]) or not all(map(operator.is_, self.state, fast["owners"]))
+                or not all(map(operator.is_, self.state.values(), fast["states"]))):
+            return None
+        if ([p.shape for p in params] != fast["shapes"] or [p.dtype for p in params] != fast["dtypes"]
+                or not all(map(operator.is_, params, fast["params"]))):
+            return None
+        # a dense gradient has its parameter's dtype (torch enforces it on assignment); no gradient, or one that is not
+        # dense, has no address
+        grads = [p.grad for p in params]
+        try:
+            if not all(map(torch.Tensor.is_contiguous, grads)):
+                return None
+            grad_at, param_at = (np.fromiter(map(torch.Tensor.data_ptr, ts), np.uint64, len(ts)) for ts in (grads, params))
+        except (TypeError, RuntimeError):
             return None
         for st, key, t in fast["alive"]:
             if st.get(key) is not t:      # a state tensor was replaced: the cached pointers are stale
@@ -381,8 +394,7 @@ class ELO_CELO2_CUDA(Optimizer):
             return np.asarray([fn(g) for g in groups], dtype=np.float64)[gidx]
 
         args = self._plan.args
-        args["grad"] = [g.data_ptr() for g in grads]
-        args["param"] = [p.data_ptr() for p in fast["params"]]
+        args["grad"], args["param"] = grad_at, param_at
         args["clip_norm"] = per_group(lambda g: g["clip_norm"] if g["clip_grad"] else 0.0)
         args["clip_val"] = per_group(lambda g: g["grad_clip_val"])
         args["exp_mult"] = per_group(lambda g: g["exp_mult"])
@@ -460,8 +472,10 @@ class ELO_CELO2_CUDA(Optimizer):
                 items = [(k, t) for k, t in state.items() if torch.is_tensor(t) and t.dim() > 0]
                 return items if len(tensors) <= _WATCH_ALL else items[:1]
             alive = [(self.state[p], k, t) for _, p, _a in tensors for k, t in watched(self.state[p])]
-            self._fast = dict(tensors=tensors, params=[p for _, p, _a in tensors], n_groups=len(self.param_groups),
-                              n_state=len(self.state), alive=alive,
+            self._fast = dict(tensors=tensors, params=[p for _, p, _a in tensors], groups=list(self.param_groups),
+                              sizes=[len(g["params"]) for g in self.param_groups], owners=list(self.state),
+                              states=list(self.state.values()), shapes=[p.shape for _, p, _a in tensors],
+                              dtypes=[p.dtype for _, p, _a in tensors], alive=alive,
                               routing=[(g["use_adamw_for_1d"], g["is_embedding"]) for g in self.param_groups],
                               gidx=np.asarray([index[id(g)] for g, _p, _a in tensors], dtype=np.int64),
                               adam=np.asarray([a for _g, _p, a in tensors], dtype=bool))

@@ -163,7 +163,7 @@ EVENTS = {
     "groups merged": _merge,
     "learning rate": lambda opt: opt.param_groups[1].update(lr=0.0625),
 }
-FAMILIES = ["adafac", "elo"]
+FAMILIES = ["adafac", "elo", "elo_celo2", "celo2"]
 
 
 @pytest.mark.parametrize("event", EVENTS)
@@ -256,7 +256,7 @@ def test_groups_change_without_kept_rows(family, event):
         _step(family, opt)
 
 
-@pytest.mark.parametrize("family", ["adafac", "elo"])
+@pytest.mark.parametrize("family", FAMILIES)
 def test_cleared_states_start_again(family):
     opt = _make(family)
     for _ in range(3):
@@ -267,6 +267,16 @@ def test_cleared_states_start_again(family):
         _step(family, opt)
     key = "exp_avg_sq" if family in ("adafac", "elo") else "rms"
     assert key in opt.state[_params(opt)[1]]
+
+
+@pytest.mark.parametrize("family", ["elo_celo2", "celo2"])
+def test_another_group_in_its_place(family):
+    opt = _make(family)
+    for _ in range(3):
+        _step(family, opt)
+    opt.param_groups[1] = dict(opt.param_groups[1], lr=0.0625, param_scale_mult=True)
+    for _ in range(2):
+        _step(family, opt)
 
 
 @pytest.mark.parametrize("family", FAMILIES)
