@@ -163,7 +163,7 @@ EVENTS = {
     "groups merged": _merge,
     "learning rate": lambda opt: opt.param_groups[1].update(lr=0.0625),
 }
-FAMILIES = ["adafac", "elo", "elo_celo2", "celo2"]
+FAMILIES = ["adafac", "elo", "velo", "elo_celo2", "celo2"]
 
 
 @pytest.mark.parametrize("event", EVENTS)
@@ -256,7 +256,54 @@ def test_groups_change_without_kept_rows(family, event):
         _step(family, opt)
 
 
+def test_velo_frozen_parameters_do_not_hide_a_move():
+    """Frozen parameters have no row: the groups' lists keep their lengths while a row goes from one group to the other."""
+    opt = _make("velo")
+    a, b = opt.param_groups
+    frozen = [_Param(torch.zeros(2)).requires_grad_(False) for _ in range(2)]
+    a["params"].append(frozen[0])
+    b["params"].append(frozen[1])
+    rows = [p for p in _params(opt) if p.requires_grad]
+
+    def step():
+        for p in rows:
+            p.grad = torch.randn(p.shape)
+        opt.step(torch.tensor(1.0))
+        table = opt._plan.tables[-1]
+        assert [p.data_ptr() for p in rows] == table["param"].tolist()
+        assert [gi for gi, g in enumerate(opt.param_groups) for p in g["params"] if p.requires_grad] == table["group"].tolist()
+
+    for _ in range(3):
+        step()
+    assert opt._fast is not None
+    b["params"].insert(0, a["params"].pop(2))
+    a["params"].append(b["params"].pop())
+    for _ in range(2):
+        step()
+
+
 @pytest.mark.parametrize("family", FAMILIES)
+def test_sparse_gradients_are_refused(family):
+    opt = _make(family)
+    for _ in range(3):
+        _step(family, opt)
+    n, p = len(opt._plan.tables), _params(opt)[4]
+    p.grad = torch.eye(7, 3).to_sparse()
+    with pytest.raises((RuntimeError, TypeError), match="[Ss]parse|dense"):
+        opt.step(torch.tensor(1.0))
+    assert len(opt._plan.tables) == n
+    p.grad = None
+    if family == "velo":
+        with pytest.raises(RuntimeError, match="needs a gradient"):
+            opt.step(torch.tensor(1.0))
+    else:
+        opt.step()
+        assert opt._plan.tables[-1]["grad"][4] == 0
+    for _ in range(3):
+        _step(family, opt)
+
+
+@pytest.mark.parametrize("family", ["adafac", "elo", "elo_celo2", "celo2"])
 def test_cleared_states_start_again(family):
     opt = _make(family)
     for _ in range(3):
