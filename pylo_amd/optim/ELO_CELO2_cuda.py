@@ -361,15 +361,16 @@ class ELO_CELO2_CUDA(Optimizer):
                 np.where(adam, per_group(lambda g: 1.0 - beta2 ** g["step"]), 0.0))
 
     def _fused_step_fast(self, fast):
-        # the same parameters of the same shapes and types in the same groups, each with the state it had
+        # the same parameters in the same groups, each with the state it had and of the size that this was made for (a shape
+        # costs twice what a size does; float16 and bfloat16 are of one size)
         groups = self.param_groups
         params = [p for g in groups for p in g["params"]]
         if ([len(g["params"]) for g in groups] != fast["sizes"] or not all(map(operator.is_, groups, fast["groups"]))
                 or len(self.state) != len(fast["states"]) or not all(map(operator.is_, self.state, fast["owners"]))
                 or not all(map(operator.is_, self.state.values(), fast["states"]))):
             return None
-        if ([p.shape for p in params] != fast["shapes"] or [p.dtype for p in params] != fast["dtypes"]
-                or not all(map(operator.is_, params, fast["params"]))):
+        if ([p.nbytes for p in params] != fast["nbytes"] or not all(map(operator.is_, params, fast["params"]))
+                or (fast["dtypes"] is not None and [p.dtype for p in params] != fast["dtypes"])):
             return None
         # a dense gradient has its parameter's dtype (torch enforces it on assignment); no gradient, or one that is not
         # dense, has no address
@@ -472,10 +473,11 @@ class ELO_CELO2_CUDA(Optimizer):
                 items = [(k, t) for k, t in state.items() if torch.is_tensor(t) and t.dim() > 0]
                 return items if len(tensors) <= _WATCH_ALL else items[:1]
             alive = [(self.state[p], k, t) for _, p, _a in tensors for k, t in watched(self.state[p])]
+            dtypes = [p.dtype for _, p, _a in tensors]
             self._fast = dict(tensors=tensors, params=[p for _, p, _a in tensors], groups=list(self.param_groups),
                               sizes=[len(g["params"]) for g in self.param_groups], owners=list(self.state),
-                              states=list(self.state.values()), shapes=[p.shape for _, p, _a in tensors],
-                              dtypes=[p.dtype for _, p, _a in tensors], alive=alive,
+                              states=list(self.state.values()), nbytes=[p.nbytes for _, p, _a in tensors],
+                              dtypes=dtypes if any(t.itemsize == 2 for t in dtypes) else None, alive=alive,
                               routing=[(g["use_adamw_for_1d"], g["is_embedding"]) for g in self.param_groups],
                               gidx=np.asarray([index[id(g)] for g, _p, _a in tensors], dtype=np.int64),
                               adam=np.asarray([a for _g, _p, a in tensors], dtype=bool))

@@ -350,3 +350,19 @@ def test_a_parameter_of_another_size(family):
     p.data = torch.randn(2, 5)
     _step(family, opt)
     assert opt._plan is not plan
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+def test_parameters_of_another_type(family):
+    opt = _make(family)
+    for old, new in ((torch.float32, torch.bfloat16), (torch.bfloat16, torch.float16), (torch.float16, torch.float32)):
+        for dtype in (old, old, old, new):
+            for p in _params(opt):
+                p.grad = None
+                p.data = p.data.to(dtype)
+            before, plan = [float(opt.state[p].get("step", 0)) if p in opt.state else 0.0 for p in _params(opt)], opt._plan
+            for p in _params(opt):
+                p.grad = torch.randn(p.shape, dtype=dtype)
+            opt.step(torch.tensor(1.0))
+            _check(family, opt, before)
+            assert (opt._plan is not plan) == (plan is None or dtype is new)
