@@ -18,16 +18,22 @@ __device__ __forceinline__ float abs_or_inf(float x, int nan0) {
 }
 
 // The block's sums of at most kP0Thin rows (columns) out of what its waves' 16-lane groups left: [wave][four of them][group][which].
+// In double and as two floats (n apart), the sum and what its rounding left, for k_v0a to add up: a sum of kP0Long values goes
+// through fewer fp32 roundings than the usual tiles' of 64 or 256.  The sums that a thread has to itself are added in pairs.  Means of
+// g^2, RMS error against fp64 in 2^-24, usual tiles / these: 16 x 4096 rows 0.65 / 0.63, columns 0.86 / 0.82; 7 x 333 rows 0.74 / 0.69, columns
+// 0.97 / 0.92; 4096 x 16 rows 0.82 / 0.82, columns 0.66 / 0.65.  (In fp32 to the end, one after the other: 1.16 of sixteen, 0.98 of 333.)
 __device__ __forceinline__ void p0_thin_total(const float* lds_row, int n, float* __restrict__ out) {
   const int j = threadIdx.x;
   if (j >= n) return;
-  float s = 0.0f;
+  double s = 0.0;
 #pragma unroll
   for (int w = 0; w < kWaves; ++w) {
     const float* t = lds_row + (w * (kP0Rows / 16) + j / 4) * 16 + j % 4;
-    s += (t[0] + t[4]) + (t[8] + t[12]);
+    s += ((double)t[0] + (double)t[4]) + ((double)t[8] + (double)t[12]);
   }
-  out[j] = s;
+  const float hi = (float)s;
+  out[j] = hi;
+  out[n + j] = fabsf(hi) < __builtin_inff() ? (float)(s - (double)hi) : 0.0f;
 }
 
 // ST: storage type of the gradient (k_cast.h).
@@ -119,7 +125,7 @@ __device__ __forceinline__ void p0_wide(const TDesc& d, const float* g, int cb, 
                                         float* __restrict__ rowpart, float* __restrict__ colpart, float* lds_row, float& gsq, float& amax) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int C0 = d.C0, R0 = d.R0, c = cb * kP0Long + (int)threadIdx.x * V;
-  float col[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  float col[4][kP0Thin / 4] = {};
 #pragma unroll
   for (int rb = 0; rb < kP0Thin; rb += 4) {
     if (rb >= R0) break;
@@ -134,10 +140,9 @@ __device__ __forceinline__ void p0_wide(const TDesc& d, const float* g, int cb, 
         for (int j = 0; j < 4; ++j) x[u][j] = *(const gfloat*)(row + min(c + j * kThreads, C0 - 1));
       }
     }
-    float rs[4];
+    float rs[4], sq[4][4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      float sq[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const bool live = rb + u < R0 && (V == 4 ? c : c + j * kThreads) < C0;
@@ -145,22 +150,23 @@ __device__ __forceinline__ void p0_wide(const TDesc& d, const float* g, int cb, 
         amax = fmaxf(amax, abs_or_inf(raw, nan0));
         if (exact) gsq = fmaf(raw, raw, gsq);
         const float y = exact ? cond_grad(raw, scale, clipv, nan0) : raw;
-        sq[j] = y * y;
-        col[j] += sq[j];
+        sq[u][j] = y * y;
       }
-      rs[u] = (sq[0] + sq[1]) + (sq[2] + sq[3]);
+      rs[u] = (sq[u][0] + sq[u][1]) + (sq[u][2] + sq[u][3]);
       if (!exact) gsq += rs[u];
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) col[j][rb / 4] = (sq[0][j] + sq[1][j]) + (sq[2][j] + sq[3][j]);
     const float tot = reduce4_rows16(rs[0], rs[1], rs[2], rs[3]);
     if ((lane & 12) == 0) lds_row[((wave * (kP0Rows / 16) + rb / 4) * 4 + (lane >> 4)) * 4 + (lane & 3)] = tot;
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int cc = V == 4 ? c + j : c + j * kThreads;
-    if (cc < C0) colpart[cc] = col[j];
+    if (cc < C0) colpart[cc] = (col[j][0] + col[j][1]) + (col[j][2] + col[j][3]);
   }
   __syncthreads();
-  p0_thin_total(lds_row, R0, rowpart + (size_t)cb * R0);
+  p0_thin_total(lds_row, R0, rowpart + (size_t)cb * 2 * R0);
 }
 
 // ... and of at most kP0Thin columns: kP0Long rows, four a thread, whose sums it has to itself.
@@ -169,7 +175,7 @@ __device__ __forceinline__ void p0_tall(const TDesc& d, const float* g, int stri
                                         float* __restrict__ rowpart, float* __restrict__ colpart, float* lds_row, float& gsq, float& amax) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int C0 = d.C0, R0 = d.R0, r = strip * kP0Long + (int)threadIdx.x;
-  float rs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  float rs[4][kP0Thin / 4] = {};
 #pragma unroll
   for (int cb = 0; cb < kP0Thin; cb += 4) {
     if (cb >= C0) break;
@@ -180,26 +186,30 @@ __device__ __forceinline__ void p0_tall(const TDesc& d, const float* g, int stri
       for (int u = 0; u < 4; ++u)
         x[j][u] = *(const gfloat*)(g + (size_t)min(r + j * kThreads, R0 - 1) * C0 + min(cb + u, C0 - 1));
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      float sq[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const float raw = r + j * kThreads < R0 && cb + u < C0 ? x[j][u] : 0.0f;
         amax = fmaxf(amax, abs_or_inf(raw, nan0));
         if (exact) gsq = fmaf(raw, raw, gsq);
-        const float y = exact ? cond_grad(raw, scale, clipv, nan0) : raw, sq = y * y;
-        col[u] += sq;
-        rs[j] += sq;
+        const float y = exact ? cond_grad(raw, scale, clipv, nan0) : raw;
+        sq[u] = y * y;
+        col[u] += sq[u];
       }
+      rs[j][cb / 4] = (sq[0] + sq[1]) + (sq[2] + sq[3]);
+    }
     const float tot = reduce4_rows16(col[0], col[1], col[2], col[3]);
     if ((lane & 12) == 0) lds_row[((wave * (kP0Rows / 16) + cb / 4) * 4 + (lane >> 4)) * 4 + (lane & 3)] = tot;
   }
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    if (r + j * kThreads < R0) rowpart[r + j * kThreads] = rs[j];
-    if (!exact) gsq += rs[j];
+    const float t = (rs[j][0] + rs[j][1]) + (rs[j][2] + rs[j][3]);
+    if (r + j * kThreads < R0) rowpart[r + j * kThreads] = t;
+    if (!exact) gsq += t;
   }
   __syncthreads();
-  p0_thin_total(lds_row, C0, colpart + (size_t)strip * C0);
+  p0_thin_total(lds_row, C0, colpart + (size_t)strip * 2 * C0);
 }
 
 template <int V>

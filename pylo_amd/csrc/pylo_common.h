@@ -83,7 +83,7 @@ struct TDesc {
   int vec0_is_r;    // vector 0 carries fac_r / row_factor (else fac_c / col_factor)
   int len[2];       // entries of vector 0 / 1
   int sumlen[2];    // elements summed into one entry
-  int npart[2];     // partial rows to add up per entry (2-D: column blocks / strips; N-D: 1)
+  int npart[2];     // partial rows to add up per entry (2-D: column blocks / strips, two each where p0_thin sums along them; N-D: 1)
   int pitch[2];     // len rounded up to 4
   int nd_size[2];   // N-D: size and stride of the dim removed from vector 0 / 1;
   int nd_stride[2]; //      entry = (idx / (size*stride)) * stride + idx % stride

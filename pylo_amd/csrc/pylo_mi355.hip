@@ -1176,7 +1176,7 @@ int build_layout(int kind, const PyloTensorShape* shapes, int T, Layout& L, int 
         const int tile_r = d.p0_thin == 2 ? kP0Long : kP0Rows, tile_c = d.p0_thin == 1 ? kP0Long : 64 * d.vec;
         d.n_strips = (d.R0 + tile_r - 1) / tile_r;
         d.n_colblk = (d.C0 + tile_c - 1) / tile_c;
-        d.npart[0] = d.n_colblk; d.npart[1] = d.n_strips;
+        d.npart[0] = d.n_colblk * (d.p0_thin == 1 ? 2 : 1); d.npart[1] = d.n_strips * (d.p0_thin == 2 ? 2 : 1);   // p0_thin_total: two
         d.nd_div_blk[0] = make_fastdiv((unsigned)std::max(d.C0, 1));   // element -> row (k_adafac_apply_lin)
       } else {
         d.vec = 1;

@@ -74,3 +74,49 @@ def test_velo(shapes):
         opt.step(torch.tensor(1.5 - 0.2 * t, device="cuda"))
         for i, p in enumerate(gpu):
             assert max_err(p, cpu[i], REL, ABS) <= 1.0, (t, shapes[i])
+
+
+def _own(m):
+    """Sizes of the partial sums that a thread adds m <= 16 squares up in: fours in pairs, then the fours in pairs."""
+    fours = [min(4, m - i) for i in range(0, m, 4)]
+    sizes = [k for f in fours for k in ([2] * (f > 1) + [2] * (f > 3) + [f] * (f > 2))]
+    return sizes + [sum(fours[i:i + 2]) for i in (0, 2) if len(fours) > i + 1] + [m] * (len(fours) > 2)
+
+
+def _bound(n, sizes):
+    """RMS of the relative error, in 2^-24, of a mean of n squares of normal numbers that is then multiplied by a weight: a rounding
+    has an RMS of 0.425 (values spread over their logarithm), two of them on the result, one on each square (fourth moment 3), one
+    on each partial sum of k squares, whose share of the whole has the second moment (k / n)^2 (1 + 2 / k) / (1 + 2 / n)."""
+    return 0.425 * (2 + 3 / n + sum((k / n) ** 2 * (1 + 2 / k) / (1 + 2 / n) for k in sizes)) ** 0.5
+
+
+@pytest.mark.parametrize("m,n", [(16, 1024), (16, 4096), (7, 333), (13, 5001), (3, 1030)])
+@pytest.mark.parametrize("tall", [False, True])
+def test_means_of_squares(tall, m, n):
+    """fac_r and fac_c after one step from zero, (1 - decay) times the means of g^2, against fp64: no more roundings than sums in
+    pairs have.  Sums over the long side are fp32 up to 64 squares and double from there on."""
+    from pylo_amd import ELO_CELO2_CUDA
+    from pylo_amd.models import CELO2MLP
+
+    torch.manual_seed(0)
+    gen = torch.Generator(device="cuda").manual_seed(m * n)
+    params = [torch.nn.Parameter(torch.randn((n, m) if tall else (m, n), generator=gen, device="cuda")) for _ in range(120)]
+    for p in params:
+        p.grad = torch.randn(p.shape, generator=gen, device="cuda") * 2.0 ** torch.rand(1, generator=gen, device="cuda")
+    opt = ELO_CELO2_CUDA(params, network=CELO2MLP(), hf_key=None, clip_grad=False, orthogonalize=False)
+    opt.step()
+    err = {0: [], 1: []}
+    for p in params:
+        for key in ("fac_r", "fac_c"):
+            fac = opt.state[p][key].double()
+            dim = 1 if fac.shape[1] == 1 else 2              # summed over
+            want = (p.grad.double() ** 2).mean(dim - 1, keepdim=True) * (1 - opt.beta_fac.float()).double().view(3, 1, 1)
+            rel = (fac - want) / want
+            assert float(rel.abs().max()) <= 8 * 2.0 ** -24
+            err[int((dim == 1) == tall)].append(float(rel.pow(2).mean()))
+    long_sizes = [k for k in (2, 4, 8, 16, 32, 64) for _ in range(n // k)]
+    for over_long, bound in ((1, _bound(n, long_sizes)), (0, _bound(m, _own(m)))):
+        e = err[over_long]
+        got = (sum(e) / len(e)) ** 0.5 * 2 ** 24
+        print(over_long, got, bound)
+        assert got <= 1.1 * bound, (over_long, got, bound)      # a tenth: from 360 sums (m = 3) on
