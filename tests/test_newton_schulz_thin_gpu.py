@@ -68,6 +68,40 @@ def test_iterations_beyond_one_run(tall, iters):
         assert off <= 8 * 2.0 ** -24 + fp32 / 4, (kind, off, fp32)
 
 
+@pytest.mark.parametrize("iters", [5, 8])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_nan_and_infinity_stay_in_their_matrix(bad, iters):
+    """... and reach every element of it, as in the formula; in folded and cut matrices, in the first and the last column."""
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    shapes = [(1, 3000), (3000, 1), (4, 20011), (9, 40), (16, 65536), (32, 257), (4097, 31), (32, 32768), (32, 32)]
+    mats = [torch.randn(s, generator=gen, device="cuda") for s in shapes]
+    clean = _orthogonalise_direct(mats, iters)
+    hit = mats[0::2]
+    for i, x in enumerate(hit):
+        x.view(-1)[0 if i % 2 else -1] = bad
+    for i, (was, now) in enumerate(zip(clean, _orthogonalise_direct(mats, iters))):
+        assert torch.isfinite(was).all()
+        assert torch.isnan(now).all() if i % 2 == 0 else torch.equal(was, now), shapes[i]
+
+
+def test_all_classes_next_to_slices_and_one_group_of_tiles():
+    """Small matrices of every class on two streams, next to slices of tensors with more dims and to larger matrices of one group:
+    three streams beside the caller's, twice over the same buffers, against the formula in fp64."""
+    from test_slice_finish_gpu import _formula
+
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    shapes = [(1024, 1024)] * 2 + [(40, 3, 3, 3), (7, 16, 16), (2, 64, 128), (5, 4, 1, 1)]
+    for i in range(20):
+        shapes += [(16 - i % 4, 700 + i), (900 + i, 17 + i % 15), (33 + i, 800), (700, 65 + 3 * i)]
+    mats = [torch.randn(s, generator=gen, device="cuda") for s in shapes]
+    first, second = _orthogonalise_direct(mats), _orthogonalise_direct(mats)
+    for x, y, z in zip(mats, first, second):
+        assert torch.equal(y, z), tuple(x.shape)
+        off = float((y.double() - _formula(x, 5)).abs().max())      # the result has unit RMS
+        # larger matrices: the level that their own tests hold them to on Gaussian input
+        assert off <= (2e-4 if min(x.shape[-2:]) > 32 else 2e-5), (tuple(x.shape), off)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_normalise_only_and_storage(dtype):
     """Without the flag the step is applied as it stands; parameters in their own type; each at rel 6 x 2^-24 plus its spacing."""

@@ -13,6 +13,7 @@ from golden_io import max_err
 pytestmark = pytest.mark.gpu
 
 REL, ABS = 1e-5, 1e-6
+FAC = 2e-6      # accumulators after three steps: at most eleven roundings of 2^-24 each
 EDGES = [(1, 65), (1, 257), (16, 260), (16, 1025), (17, 300), (2, 4100), (129, 1), (128, 16), (1025, 16), (1030, 17), (2050, 7), (1, 1)]
 MANY = [(3, 65536), (2, 65540), (65600, 2), (4, 65537), (66000, 1), (5, 777)]
 
@@ -49,6 +50,8 @@ def test_elo_celo2(shapes, clip):
         opt.step()
         for i, (p, r) in enumerate(zip(gpu, ref)):
             assert max_err(p, r, REL, ABS) <= 1.0, (t, shapes[i])
+            for key in ("fac_r", "fac_c"):
+                assert max_err(opt.state[p][key], orc.state[i][key], FAC, 1e-30) <= 1.0, (t, shapes[i], key)
 
 
 @pytest.mark.parametrize("shapes", [EDGES, MANY], ids=["edges", "many"])
@@ -74,6 +77,44 @@ def test_velo(shapes):
         opt.step(torch.tensor(1.5 - 0.2 * t, device="cuda"))
         for i, p in enumerate(gpu):
             assert max_err(p, cpu[i], REL, ABS) <= 1.0, (t, shapes[i])
+            for key in ("fac_vec_row", "fac_vec_col"):
+                assert max_err(opt.state[p][key], orc.state[i][key], REL, 1e-30) <= 1.0, (t, shapes[i], key)
+
+
+@pytest.mark.parametrize("clip", [True, False])
+def test_elo_with_nan_and_infinity(clip):
+    """NaNs become zeros before they are squared (the exact pass, which they ask for); with clipping a NaN makes the global norm one and
+    the scale 1, an infinity makes the scale 0."""
+    from oracle import pylo_oracle as O
+    from pylo_amd import ELO_CUDA
+    from pylo_amd.models import MetaMLP
+
+    torch.manual_seed(9)
+    net = MetaMLP(39, 32, 1)
+    gen = torch.Generator().manual_seed(30)
+    cpu = [torch.randn(s, generator=gen) * 0.3 for s in EDGES]
+    gpu = [torch.nn.Parameter(v.clone().cuda()) for v in cpu]
+    cfg = dict(lr=1e-2, clip_grad=clip, clip_norm=3.0)
+    orc = O.EloOracle(cpu, net.state_dict(), **cfg)
+    opt = ELO_CUDA(gpu, network=copy.deepcopy(net), hf_key=None, **cfg)
+    for t in range(4):
+        grads = [torch.randn(s, generator=gen) for s in EDGES]
+        if t == 1:
+            for g in grads[:-1]:
+                g.view(-1)[[0, g.numel() // 2, g.numel() - 1]] = float("nan")
+        if t == 2 and clip:
+            grads[1].view(-1)[256] = float("inf")
+            grads[8][1024, 15] = -float("inf")
+        for p, g in zip(gpu, grads):
+            p.grad = g.cuda()
+        orc.step(grads)
+        opt.step()
+        for i, p in enumerate(gpu):
+            st, so = opt.state[p], orc.state[i]
+            assert max_err(p, cpu[i], REL, ABS) <= 1.0, (t, EDGES[i])
+            for key, was in (("exp_avg_sq_r", "exp_avg_sq_r"), ("exp_avg_sq_c", "exp_avg_sq_c")):
+                assert bool(torch.isfinite(so[was]).all())
+                assert max_err(st[key], so[was], REL, 1e-30) <= 1.0, (t, EDGES[i], key)
 
 
 def _own(m):
