@@ -473,11 +473,11 @@ class ELO_CELO2_CUDA(Optimizer):
                 items = [(k, t) for k, t in state.items() if torch.is_tensor(t) and t.dim() > 0]
                 return items if len(tensors) <= _WATCH_ALL else items[:1]
             alive = [(self.state[p], k, t) for _, p, _a in tensors for k, t in watched(self.state[p])]
-            dtypes = [p.dtype for _, p, _a in tensors]
+            halves = any(t.itemsize == 2 for t in {row[2] for row in self._plan_key})
             self._fast = dict(tensors=tensors, params=[p for _, p, _a in tensors], groups=list(self.param_groups),
                               sizes=[len(g["params"]) for g in self.param_groups], owners=list(self.state),
                               states=list(self.state.values()), nbytes=[p.nbytes for _, p, _a in tensors],
-                              dtypes=dtypes if any(t.itemsize == 2 for t in dtypes) else None, alive=alive,
+                              dtypes=[p.dtype for _, p, _a in tensors] if halves else None, alive=alive,
                               routing=[(g["use_adamw_for_1d"], g["is_embedding"]) for g in self.param_groups],
                               gidx=np.asarray([index[id(g)] for g, _p, _a in tensors], dtype=np.int64),
                               adam=np.asarray([a for _g, _p, a in tensors], dtype=bool))
