@@ -409,7 +409,7 @@ __global__ __launch_bounds__(kThreads) void k_gnorm(NormArgs na, Globals* __rest
 
 // Where k_p0 had few blocks, every block of the launch behind it adds their partials up for itself -- the same sum in the same
 // order -- and one leaves the result for the launches that follow: a launch of one block and the gap behind it, 4 to 8 us of a
-// step of 60 to 150, for 1 us of loads that hit L2.  (kNormBlocks: two partials a thread; at 512 blocks of k_p0 3 MB for all.)
+// step of 60 to 150, for 1 us of loads that hit L2.  (kNormBlocks: two partials a thread, 6 KB a block: 25 MB from L2 where that launch has 4096.)
 constexpr int kNormBlocks = 512;
 __device__ __forceinline__ void own_norm(const NormArgs& na, Globals* __restrict__ gl, Globals* own) {
   gnorm_block(na.gsq_part, na.flag_part, na.nblk, na.use_flags, own);

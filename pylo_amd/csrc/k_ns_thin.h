@@ -15,7 +15,7 @@
 //   sum of squares of the result = tr(Q A Q);  X <- Q X / (sqrt(tr G) + eps), normalised, applied to the parameter.
 // The chain that k_ns_small has for larger ones, with a class for these, passed over X eight times and met five times.  What
 // bounds this: the latency of two passes of loads, and five iterations of three dependent products (0.3 to 0.5 us each with its
-// barriers).  Whole ELO-CELO2 steps, then / now: three thousand odd tensors 2.72 / 2.19 ms (its launch 651 -> 72 us), one and
+// barriers).  Whole ELO-CELO2 steps, then / now: three thousand odd tensors 2.72 / 2.19 ms (one launch of 651 us, now two of 64 and 75), one and
 // sixty-four of 32 x 32768 294 / 135 and 2072 / 1441 us, sixteen of 16 x 8192 455 / 131, one of 32 x 1024 93 / 98.  Against the
 // formula in fp64 the result is off by the roundings of its last three operations (2e-8 to 7e-7 of its RMS; 2e-7 to 2e-5 in fp32 products).
 //

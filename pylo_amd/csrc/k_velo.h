@@ -838,9 +838,11 @@ __global__ __launch_bounds__(kThreads) void k_velo_gates(const float* __restrict
 // three launches of both on the caller's stream.  Such a step is bound by its launches: on a second stream the LSTM's chain took
 // four of its own, two events and two waits for them, 78 us of host time a step where these take 24, and the GPU stood still between
 // dependent launches of 4 to 12 us.  Where k_p0 streams for longer than the LSTM's chain takes, that chain is better hidden under
-// it on a stream of its own (kVeloPaired).  Whole steps, apart / paired: MLP of width 32 91 / 58 us, 128 89 / 65, 1024 122 / 105,
-// ViT of 12 layers and width 64 165 / 131, 192 (400 blocks) 167 / 145, 256 (455) 197 / 192, 320 291 / 295, of 7 of 384 (610) 226 / 226,
-// 12 of 384 (970) 325 / 337; ResNet-50 of width 32 218 / 189, 40 237 / 242, 64 464 / 514; 250 tensors 315 / 258.
+// it on a stream of its own (kVeloPaired).  Only steps that carry sums have the two chains: the first one, and one after a
+// parameter was written from outside, takes the separate passes as before (MLP of width 128: 180 us on a new state).  Whole steps,
+// apart / paired: MLP of width 32 91 / 58 us, 128 89 / 65, 1024 122 / 105, ViT of 12 layers and width 64 165 / 131, 192 (400
+// blocks) 167 / 145, 256 (455) 197 / 192, 320 291 / 295, of 7 of 384 (610) 226 / 226, 12 of 384 (970) 325 / 337; ResNet-50 of width 32
+// 218 / 189, 40 237 / 242, 64 464 / 514; 250 tensors 315 / 258.
 template <bool SPLIT>
 __global__ __launch_bounds__(kFoldThreads) void k_velo_p0_feat(
     const TDesc* __restrict__ descs, const PyloTensorArgs* __restrict__ dyn, const Item* __restrict__ items, float* __restrict__ part,

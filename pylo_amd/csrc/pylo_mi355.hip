@@ -500,10 +500,10 @@ int ns_small_part(int cls) { return cls == 0 ? ThinDims<1>::NT * 512 : cls == 1 
 //   m = 64, 1, 4, 16, 64 of them: 16384 213 / 232, 258 / 314, 737 / 786, 1974 / 2457      32768 317 / 284, 446 / 497, 1219 / 1453,
 //     4028 / 4528
 //   m = 48: 24000 229 / 248, 286 / 342, 823 / 874, 2573 / 2806      32768 267 / 271, 358 / 418, 1043 / 1299, 3110 / 3748
-//   m = 32 (k_ns_thin, no line below its limits): 1024 98 / 172, 99 / 173, 102 / 174, 125 / 236      16384 106 / 209, 138 / 257,
-//     327 / 491, 764 / 1404      32768 135 / 235, 192 / 310, 538 / 929, 1441 / 2471
-//   m = 16, 1, 16 of them: 8192 89 / 185, 131 / 264      32768 99 / 220, 347 / 719      65536 127 / 242, 550 / 1160
-//   m = 4: 65536 97 / 228, 264 / 934
+//   m = 32 (k_ns_thin, no line below its limits: from one matrix to 256 of any length it is the faster): 1024 101 / 172, 104 / 182,
+//     110 / 192, 145 / 262      16384 110 / 222, 154 / 279, 335 / 515, 850 / 1499      32768 141 / 255, 206 / 327, 549 / 965, 1622 / 2659
+//   m = 16, 1, 16 of them: 8192 100 / 205, 146 / 289      32768 104 / 235, 354 / 745      65536 131 / 257, 571 / 1200
+//   m = 4: 65536 101 / 237, 271 / 963
 //   decoders of width 128 with two embeddings: 12 layers (74 matrices) 2000 239 / 266, 4000 324 / 291; 24 (146) 2000 287 / 345,
 //     4000 374 / 402, 8000 549 / 472; 40 (242) 4000 424 / 559, 8000 571 / 688
 struct NsSmallRule {
